@@ -58,7 +58,11 @@ struct egg_ctx {
     unsigned long long *d_loss_acc = nullptr, *d_counter = nullptr;
     int32_t *d_loss = nullptr, *d_fit = nullptr;
     Scalars *d_scal = nullptr;
-    int8_t *d_panel_a = nullptr, *d_panel_b = nullptr; int pairs_pad = 0;
+    // votes and optimizer step (egg_votes.hip): the noise table, and the matrices' descriptors in lists that one launch walks
+    NoiseTable noise = {nullptr, 0, 0, nullptr, nullptr, 0, nullptr};
+    struct MatList { int first, count, tiles; };
+    MatDesc *d_mat = nullptr;
+    MatList mat_all, mat_adam; std::vector<MatList> mat_muon, mat_one;     // every matrix; the AdamW ones; each Muon batch; each on its own (by tensor id)
     // taps
     bool taps = false; int8_t *d_tap = nullptr; int32_t *d_tap_logits = nullptr; int tap_members = 0;
     // per-kernel-class event timing (egg_ctx_enable_timing)
@@ -71,7 +75,8 @@ struct egg_ctx {
     int8_t *d_gen_kv = nullptr; bool gen_kv_cache = true;      // per-layer K / V rows of the generated sequence (egg_ctx_generate_kv_cache)
     int mask_override = -1; int32_t *logits_override = nullptr;
     bool first_dedup = true;        // first block once per distinct byte value of a member's window (egg_ctx_first_block_dedup)
-    VecDesc *d_vec_desc = nullptr; int n_vec = 0, vec_total = 0;       // all vector tensors, for the one-launch update
+    VecDesc *d_vec_desc = nullptr; int n_vec = 0, vec_total = 0;       // all vector tensors, then each on its own
+    std::vector<int> vec_one;                                          // by tensor id: its place behind the first n_vec
     // adaptive noise overlay (egg_adaptive_enable): raw overlay values, q = clamp(overlay, 0, 64) and change flags, all
     // laid out like the model blob; one segment (rows + cols, or len) per tensor
     bool adaptive = false; int ov_inc = 5, ov_dec = 1;
@@ -258,14 +263,72 @@ extern "C" int egg_describe_layout(const egg_config *cfg, int tensor_id, egg_ten
 static void free_all(egg_ctx *ctx) {
     void *ptrs[] = {ctx->muon.x, ctx->muon.swap, ctx->muon.bterm, ctx->muon.partials, ctx->muon.norm,
                     ctx->d_wfrag, ctx->d_plin_frag, ctx->d_model, ctx->d_state, ctx->d_exp, ctx->d_act, ctx->d_rope, ctx->d_x, ctx->d_q, ctx->d_k, ctx->d_v,
-                    ctx->d_ao, ctx->d_loss_acc, ctx->d_counter, ctx->d_loss, ctx->d_fit, ctx->d_scal, ctx->d_panel_a,
-                    ctx->d_panel_b, ctx->d_tap, ctx->d_tap_logits, ctx->d_gen_tok, ctx->d_gen_logits, ctx->d_gen_ws, ctx->d_gen_scal, ctx->d_gen_kv, ctx->d_vec_desc,
+                    ctx->d_ao, ctx->d_loss_acc, ctx->d_counter, ctx->d_loss, ctx->d_fit, ctx->d_scal, ctx->noise.table,
+                    ctx->noise.neg, ctx->noise.nonzero, ctx->noise.general, ctx->d_mat, ctx->d_tap, ctx->d_tap_logits, ctx->d_gen_tok, ctx->d_gen_logits, ctx->d_gen_ws, ctx->d_gen_scal, ctx->d_gen_kv, ctx->d_vec_desc,
                     ctx->d_overlay, ctx->d_overlay_q, ctx->d_flags, ctx->d_ov_segs};
     for (void *p : ptrs) if (p) (void)hipFree(p);
     for (auto &sp : ctx->spans) { (void)hipEventDestroy(sp.a); (void)hipEventDestroy(sp.b); }
     if (ctx->gexec) (void)hipGraphExecDestroy(ctx->gexec);
     if (ctx->graph) (void)hipGraphDestroy(ctx->graph);
     if (ctx->own_stream && ctx->stream) (void)hipStreamDestroy(ctx->stream);
+}
+
+// entries of a noise table row: the highest seed offset of any tensor and its window of pairs, to a multiple of 16
+static int noise_entries(const egg_config &c, int pairs_pad) {
+    const int layers = 1000 * (c.n_layers - 1) + EGG_LAYER_SEEDS;
+    return std::max(EGG_MODEL_SEEDS, layers) + pairs_pad + 16;
+}
+// one descriptor per vector tensor, in table order
+static std::vector<VecDesc> vector_descs(const egg_ctx *ctx) {
+    std::vector<VecDesc> vd;
+    int first = 0;
+    for (size_t id = 0; id < ctx->tensors.size(); id++) {
+        const egg_tensor_info &t = ctx->tensors[id];
+        if (t.is_matrix) continue;
+        VecDesc d; d.W = ctx->d_model + t.offset; d.state = reinterpret_cast<float *>(ctx->d_state + ctx->t_state_off[id]);
+        d.n = t.cols; d.first = first; d.off_a = t.off_a; d.off_b = t.off_b; d.seed_base = t.seed_base; d.lr_scale = t.lr_scale;
+        d.flags = ctx->d_flags ? ctx->d_flags + t.offset : nullptr;
+        vd.push_back(d); first += t.cols;
+    }
+    return vd;
+}
+// The lists of matrix descriptors: all matrices, the AdamW ones, the batches of the Muon plan (each matrix with its slot of the
+// workspace), and every matrix on its own for the calls that name one.
+static std::vector<MatDesc> matrix_descs(egg_ctx *ctx) {
+    const egg_config &c = ctx->cfg;
+    std::vector<MatDesc> md;
+    auto list = [&](const std::vector<int> &ids, bool muon) {
+        egg_ctx::MatList l = {(int)md.size(), (int)ids.size(), 0};
+        for (size_t b = 0; b < ids.size(); b++) {
+            const egg_tensor_info &t = ctx->tensors[ids[b]];
+            MatDesc d;
+            d.W = ctx->d_model + t.offset; d.frag = ctx->d_wfrag + t.offset; d.offset = t.offset;
+            d.state = reinterpret_cast<float *>(ctx->d_state + ctx->t_state_off[ids[b]]);
+            d.muon_x = muon ? ctx->muon.x + b * (size_t)t.rows * t.cols : nullptr;
+            d.rows = t.rows; d.cols = t.cols; d.tile_first = l.tiles;
+            // hidden x hidden blocks for the layer matrices; the embedding (hidden x vocab) is cut into <= 256-wide blocks
+            d.block = (t.cols == c.vocab && t.rows == c.hidden && c.hidden > 256) ? 256 : c.hidden;
+            d.t_a = t.seed_base + t.off_a; d.t_b = t.seed_base + t.off_b;
+            d.limit = c.weight_limit;
+            d.lr_scale = muon ? t.lr_scale * c.muon_lr_scale : t.lr_scale;
+            l.tiles += (t.rows / 64) * (t.cols / 64);
+            md.push_back(d);
+        }
+        return l;
+    };
+    std::vector<int> all, adam;
+    for (int id = 0; id < (int)ctx->tensors.size(); id++)
+        if (ctx->tensors[id].is_matrix) { all.push_back(id); if (!(c.use_muon && ctx->tensors[id].muon)) adam.push_back(id); }
+    ctx->mat_all = list(all, false);
+    ctx->mat_adam = list(adam, false);
+    for (size_t gi = 0; gi < ctx->muon_groups.size(); gi++) {
+        const std::vector<int> &g = ctx->muon_groups[gi];
+        for (size_t first = 0; first < g.size(); first += (size_t)ctx->muon_group_batch[gi])
+            ctx->mat_muon.push_back(list(std::vector<int>(g.begin() + first, g.begin() + std::min(g.size(), first + (size_t)ctx->muon_group_batch[gi])), true));
+    }
+    ctx->mat_one.assign(ctx->tensors.size(), egg_ctx::MatList{0, 0, 0});
+    for (int id : all) ctx->mat_one[id] = list(std::vector<int>(1, id), c.use_muon && ctx->tensors[id].muon);
+    return md;
 }
 
 // why the last egg_ctx_create of this thread failed (there is no context to hold the message yet)
@@ -344,17 +407,11 @@ extern "C" int egg_ctx_create(const egg_config *cfg, egg_ctx **out) {
     ctx->state_bytes = state_offsets(c, ctx->tensors, ctx->t_state_off);
     CR(hipMalloc(&ctx->d_state, ctx->state_bytes)); CR(hipMemset(ctx->d_state, 0, ctx->state_bytes));
     {
-        std::vector<VecDesc> vd;
-        int first = 0;
-        for (size_t id = 0; id < ctx->tensors.size(); id++) {
-            const egg_tensor_info &t = ctx->tensors[id];
-            if (t.is_matrix) continue;
-            VecDesc d; d.W = ctx->d_model + t.offset; d.state = reinterpret_cast<float *>(ctx->d_state + ctx->t_state_off[id]);
-            d.n = t.cols; d.first = first; d.off_a = t.off_a; d.off_b = t.off_b; d.seed_base = t.seed_base; d.lr_scale = t.lr_scale;
-            d.flags = nullptr;
-            vd.push_back(d); first += t.cols;
-        }
-        ctx->n_vec = (int)vd.size(); ctx->vec_total = first;
+        std::vector<VecDesc> vd = vector_descs(ctx), one = vd;
+        ctx->n_vec = (int)vd.size(); ctx->vec_total = vd.empty() ? 0 : vd.back().first + vd.back().n;
+        ctx->vec_one.assign(ctx->tensors.size(), -1);
+        for (size_t id = 0; id < ctx->tensors.size(); id++)
+            if (!ctx->tensors[id].is_matrix) { ctx->vec_one[id] = (int)vd.size(); vd.push_back(one[vd.size() - one.size()]); vd.back().first = 0; }
         CR(hipMalloc(&ctx->d_vec_desc, vd.size() * sizeof(VecDesc)));
         CR(hipMemcpy(ctx->d_vec_desc, vd.data(), vd.size() * sizeof(VecDesc), hipMemcpyHostToDevice));
     }
@@ -385,24 +442,26 @@ extern "C" int egg_ctx_create(const egg_config *cfg, egg_ctx **out) {
     CR(hipMemset(ctx->d_counter, 0, 8));
     CR(hipMalloc(&ctx->d_loss, (size_t)c.population * 4)); CR(hipMalloc(&ctx->d_fit, (size_t)(c.population / 2) * 4));
     CR(hipMalloc(&ctx->d_scal, sizeof(Scalars)));
-    ctx->pairs_pad = ((c.population / 2) + 63) / 64 * 64;
-    const size_t panel_rows = std::max(4 * c.hidden, c.vocab);       // the widest side of any matrix: 4 * hidden, or the embedding's vocabulary
-    CR(hipMalloc(&ctx->d_panel_a, panel_rows * ctx->pairs_pad));
-    CR(hipMalloc(&ctx->d_panel_b, panel_rows * ctx->pairs_pad));
+    // noise table: the rows of the widest side of any matrix (4 * hidden, or the embedding's vocabulary), every layer's seeds
+    ctx->noise.pairs_pad = ((c.population / 2) + 127) / 128 * 128;
+    ctx->noise.rows = std::max(4 * c.hidden, c.vocab);
+    ctx->noise.ld = (size_t)(noise_entries(c, ctx->noise.pairs_pad) + 127) / 128 * 128;
+    CR(hipMalloc(&ctx->noise.table, ctx->noise.rows * ctx->noise.ld));
+    CR(hipMalloc(&ctx->noise.neg, ctx->noise.pairs_pad)); CR(hipMalloc(&ctx->noise.nonzero, ctx->noise.pairs_pad));
+    CR(hipMalloc(&ctx->noise.general, sizeof(int)));
+    {
+        const std::vector<MatDesc> md = matrix_descs(ctx);
+        CR(hipMalloc(&ctx->d_mat, md.size() * sizeof(MatDesc)));
+        CR(hipMemcpy(ctx->d_mat, md.data(), md.size() * sizeof(MatDesc), hipMemcpyHostToDevice));
+    }
 #undef CR
     *out = ctx;
     return EGG_OK;
 }
 
-// refresh the fragment-major copy of one matrix (tensor id) or of all matrices (id < 0); enqueued on the stream
-static int refresh_frag(egg_ctx *ctx, int id) {
-    for (int i = 0; i < (int)ctx->tensors.size(); i++) {
-        const egg_tensor_info &t = ctx->tensors[i];
-        if (!t.is_matrix || (id >= 0 && i != id)) continue;
-        // hidden x hidden blocks for the layer matrices; the embedding (hidden x 256) is cut into <= 256-wide blocks
-        const int B = (t.cols == ctx->cfg.vocab && t.rows == ctx->cfg.hidden && ctx->cfg.hidden > 256) ? 256 : ctx->cfg.hidden;
-        HIP_TRY(egg_launch_swizzle(ctx->d_model + t.offset, ctx->d_wfrag + t.offset, t.rows, t.cols, B, 0, ctx->stream));
-    }
+// refresh the fragment-major copy of every matrix; enqueued on the stream
+static int refresh_frag(egg_ctx *ctx) {
+    HIP_TRY(egg_launch_frag(ctx->d_mat + ctx->mat_all.first, ctx->mat_all.count, ctx->mat_all.tiles, ctx->stream));
     return EGG_OK;
 }
 
@@ -464,13 +523,13 @@ extern "C" int egg_model_init(egg_ctx *ctx, uint32_t seed) {
     for (int i = 0; i < H; i++) m[L.ln_f + i] = 16;
     HIP_TRY(hipStreamSynchronize(ctx->stream));
     HIP_TRY(hipMemcpy(ctx->d_model, m.data(), m.size(), hipMemcpyHostToDevice));
-    return refresh_frag(ctx, -1);
+    return refresh_frag(ctx);
 }
 extern "C" int egg_model_upload(egg_ctx *ctx, const void *h, size_t bytes) {
     if (!ctx || !h || (int64_t)bytes != ctx->L.total) return fail(ctx, EGG_E_INVALID, "model size mismatch");
     HIP_TRY(hipStreamSynchronize(ctx->stream));
     HIP_TRY(hipMemcpy(ctx->d_model, h, bytes, hipMemcpyHostToDevice));
-    return refresh_frag(ctx, -1);
+    return refresh_frag(ctx);
 }
 extern "C" int egg_model_download(egg_ctx *ctx, void *h, size_t bytes) {
     if (!ctx || !h || (int64_t)bytes != ctx->L.total) return fail(ctx, EGG_E_INVALID, "model size mismatch");
@@ -514,7 +573,7 @@ extern "C" int egg_model_upload_ternary(egg_ctx *ctx, const void *h, size_t byte
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
     (void)hipFree(d_packed);
     if (e != hipSuccess) return fail(ctx, EGG_E_HIP, "egg_model_upload_ternary", e);
-    return refresh_frag(ctx, -1);
+    return refresh_frag(ctx);
 }
 extern "C" int egg_model_download_ternary(egg_ctx *ctx, void *h, size_t bytes) {
     if (!ctx || !h || (int64_t)bytes != egg_ternary_model_bytes(ctx)) return fail(ctx, EGG_E_INVALID, "ternary model size mismatch");
@@ -768,107 +827,81 @@ extern "C" int egg_fitness(egg_ctx *ctx, const int32_t *d_loss, int32_t *d_fit, 
 }
 
 // ------------------------------------------------------------------ update
-static UpdParams make_upd(egg_ctx *ctx, int id, const int32_t *d_fit, const uint32_t *d_seed, const float *d_lr) {
-    const egg_tensor_info &t = ctx->tensors[id];
+static UpdLaunch make_upd(egg_ctx *ctx, const egg_ctx::MatList &l, const int32_t *d_fit, const float *d_lr) {
     const egg_config &c = ctx->cfg;
-    UpdParams p; memset(&p, 0, sizeof(p));
-    p.W = ctx->d_model + t.offset; p.state = reinterpret_cast<float *>(ctx->d_state + ctx->t_state_off[id]);
-    p.rows = t.rows; p.cols = t.cols; p.off_a = t.off_a; p.off_b = t.off_b; p.seed_base = t.seed_base;
-    p.fit = d_fit; p.pairs = c.population / 2; p.d_seed = d_seed; p.d_lr = d_lr; p.lr_scale = t.lr_scale;
-    p.limit = t.is_matrix ? c.weight_limit : 127;
-    p.mask = noise_word(c); p.beta1 = c.adam_beta1; p.beta2 = c.adam_beta2; p.eps = c.adam_eps; p.wd = c.adam_weight_decay;
-    p.panel_a = ctx->d_panel_a; p.panel_b = ctx->d_panel_b; p.pairs_pad = ctx->pairs_pad; p.counter = ctx->d_counter;
+    UpdLaunch p; memset(&p, 0, sizeof(p));
+    p.mat = ctx->d_mat + l.first; p.n_mat = l.count; p.tiles = l.tiles;
+    p.noise = ctx->noise; p.fit = d_fit; p.pairs = c.population / 2; p.d_lr = d_lr;
+    p.beta1 = c.adam_beta1; p.beta2 = c.adam_beta2; p.eps = c.adam_eps; p.wd = c.adam_weight_decay; p.muon_momentum = c.muon_momentum;
+    p.counter = ctx->d_counter;
     return p;
 }
-static int update_one(egg_ctx *ctx, int id, const int32_t *d_fit, const uint32_t *d_seed, const float *d_lr, bool record_flags = false) {
-    const egg_tensor_info &t = ctx->tensors[id];
-    UpdParams p = make_upd(ctx, id, d_fit, d_seed, d_lr);
-    if (record_flags) p.flags = ctx->d_flags + t.offset;
-    if (t.is_matrix && t.muon && ctx->cfg.use_muon) {
-        // LAUNCH_ADAM_MATRIX under USE_MUON (mgpu.cu:1587-1595)
-        {
-            SpanScope span(ctx, EGG_K_UPDATE_MATRIX);
-            p.muon_momentum = ctx->cfg.muon_momentum; p.muon_x = ctx->muon.x;
-            HIP_TRY(egg_launch_muon_momentum(p, ctx->stream));
-            HIP_TRY(egg_launch_newton_schulz(ctx->muon, t.rows, t.cols, 5, ctx->stream));
-            p.lr_scale = t.lr_scale * ctx->cfg.muon_lr_scale;
-            HIP_TRY(egg_launch_muon_apply(p, ctx->cfg.adam_weight_decay, ctx->stream));
-        }
-        int rc = refresh_frag(ctx, id);
-        if (rc) return rc;
-    } else if (t.is_matrix) {
-        { SpanScope span(ctx, EGG_K_UPDATE_MATRIX); HIP_TRY(egg_launch_update_matrix(p, ctx->stream)); }
-        int rc = refresh_frag(ctx, id);
-        if (rc) return rc;
-    }
-    else { SpanScope span(ctx, EGG_K_UPDATE_VECTOR); HIP_TRY(egg_launch_update_vector(p, ctx->stream)); }
+// the part of the noise table that one tensor reads, and the fitness masks
+static int table_of_tensor(egg_ctx *ctx, int id, const int32_t *d_fit, const uint32_t *d_seed) {
+    const egg_config &c = ctx->cfg; const egg_tensor_info &t = ctx->tensors[id];
+    const int lo = t.seed_base + std::min(t.off_a, t.off_b), hi = t.seed_base + std::max(t.off_a, t.off_b) + ctx->noise.pairs_pad;
+    HIP_TRY(egg_launch_noise_table(ctx->noise, d_seed, d_fit, c.population / 2, noise_word(c), t.is_matrix ? std::max(t.rows, t.cols) : t.cols,
+                                   4 * c.hidden, lo, hi, t.off_a + ctx->noise.pairs_pad + 16, c.n_layers, nullptr, ctx->stream));
     return EGG_OK;
 }
 extern "C" int egg_update_tensor(egg_ctx *ctx, int id, const int32_t *d_fit, const uint32_t *d_seed, const float *d_lr) {
     if (!ctx || id < 0 || id >= (int)ctx->tensors.size() || !d_fit || !d_seed || !d_lr) return fail(ctx, EGG_E_INVALID, "egg_update_tensor arguments");
-    return update_one(ctx, id, d_fit, d_seed, d_lr);
+    const egg_tensor_info &t = ctx->tensors[id];
+    UpdLaunch p = make_upd(ctx, ctx->mat_one[id], d_fit, d_lr);
+    if (!t.is_matrix) { p.vec = ctx->d_vec_desc + ctx->vec_one[id]; p.n_vec = 1; p.vec_total = t.cols; }
+    SpanScope span(ctx, t.is_matrix ? EGG_K_UPDATE_MATRIX : EGG_K_UPDATE_VECTOR);
+    int rc = table_of_tensor(ctx, id, d_fit, d_seed);
+    if (rc) return rc;
+    HIP_TRY(egg_launch_update(p, ctx->stream));
+    if (t.is_matrix && t.muon && ctx->cfg.use_muon) {
+        // LAUNCH_ADAM_MATRIX under USE_MUON (mgpu.cu:1587-1595)
+        HIP_TRY(egg_launch_newton_schulz(ctx->muon, t.rows, t.cols, 5, ctx->stream));
+        HIP_TRY(egg_launch_muon_apply(p, ctx->cfg.adam_weight_decay, ctx->stream));
+    }
+    return EGG_OK;
 }
 extern "C" int egg_matrix_votes(egg_ctx *ctx, int id, const int32_t *d_fit, const uint32_t *d_seed, int32_t *d_votes) {
     if (!ctx || id < 0 || id >= (int)ctx->tensors.size() || !d_fit || !d_seed || !d_votes || !ctx->tensors[id].is_matrix)
         return fail(ctx, EGG_E_INVALID, "egg_matrix_votes arguments");
-    UpdParams p = make_upd(ctx, id, d_fit, d_seed, nullptr);
+    UpdLaunch p = make_upd(ctx, ctx->mat_one[id], d_fit, nullptr);
     p.votes_out = d_votes;
-    HIP_TRY(egg_launch_update_matrix(p, ctx->stream));
+    int rc = table_of_tensor(ctx, id, d_fit, d_seed);
+    if (rc) return rc;
+    HIP_TRY(egg_launch_update(p, ctx->stream));
     return EGG_OK;
 }
 extern "C" int egg_es_update(egg_ctx *ctx, const int32_t *d_fit, const uint32_t *d_seed, const float *d_lr) {
     if (!ctx || !d_fit || !d_seed || !d_lr) return fail(ctx, EGG_E_INVALID, "egg_es_update arguments");
-    HIP_TRY(egg_launch_zero_u64(ctx->d_counter, 1, ctx->stream));
-    // matrices one by one (each needs the panel workspace), then every vector tensor in one launch; tensors are
-    // independent, so the reference's launch order (mgpu.cu:1603-1643) does not matter
-    for (int id = 0; id < (int)ctx->tensors.size(); id++) {
-        if (!ctx->tensors[id].is_matrix || (ctx->cfg.use_muon && ctx->tensors[id].muon)) continue;
-        int rc = update_one(ctx, id, d_fit, d_seed, d_lr, ctx->adaptive);
-        if (rc) return rc;
+    const egg_config &c = ctx->cfg;
+    // tensors are independent, so the reference's launch order (mgpu.cu:1603-1643) does not matter: the noise of all of
+    // them, then every AdamW matrix and every vector tensor in one launch
+    {
+        SpanScope span(ctx, EGG_K_UPDATE_MATRIX);
+        HIP_TRY(egg_launch_noise_table(ctx->noise, d_seed, d_fit, c.population / 2, noise_word(c), ctx->noise.rows, 4 * c.hidden, 0,
+                                       noise_entries(c, ctx->noise.pairs_pad), ctx->noise.pairs_pad + 16, c.n_layers, ctx->d_counter, ctx->stream));
+        UpdLaunch p = make_upd(ctx, ctx->mat_adam, d_fit, d_lr);
+        p.vec = ctx->d_vec_desc; p.n_vec = ctx->n_vec; p.vec_total = ctx->vec_total;
+        p.flags = ctx->adaptive ? ctx->d_flags : nullptr;
+        HIP_TRY(egg_launch_update(p, ctx->stream));
     }
     // Muon matrices (LAUNCH_ADAM_MATRIX under USE_MUON, mgpu.cu:1587-1595), a batch of one shape at a time: momentum of
-    // each into its slot of the workspace, Newton-Schulz of the whole batch, then each matrix's apply rule
-    if (ctx->cfg.use_muon)
-        for (size_t gi = 0; gi < ctx->muon_groups.size(); gi++) {
-            const std::vector<int> &g = ctx->muon_groups[gi];
-            const egg_tensor_info &t0 = ctx->tensors[g[0]];
-            const size_t one = (size_t)t0.rows * t0.cols, k = (size_t)(t0.rows < t0.cols ? t0.rows : t0.cols);
-            const size_t limit = (size_t)ctx->muon_group_batch[gi];
-            // the group's own limit, never the largest group's: the buffers hold `limit` matrices of this shape
-            if (limit < 1 || limit * one > ctx->muon_elems || limit * k * k > ctx->muon_bterm || (int)limit > ctx->muon_batch_max)
-                return fail(ctx, EGG_E_STATE, "Muon batch does not fit the workspace");
-            for (size_t first = 0; first < g.size(); first += limit) {
-                const int nb = (int)std::min(g.size() - first, limit);
-                int rc = EGG_OK;
-                {
-                    SpanScope span(ctx, EGG_K_UPDATE_MATRIX);
-                    for (int b = 0; b < nb; b++) {
-                        UpdParams p = make_upd(ctx, g[first + b], d_fit, d_seed, d_lr);
-                        p.muon_momentum = ctx->cfg.muon_momentum; p.muon_x = ctx->muon.x + (size_t)b * one;
-                        HIP_TRY(egg_launch_muon_momentum(p, ctx->stream));
-                    }
-                }
-                { SpanScope span(ctx, EGG_K_MUON_NS); HIP_TRY(egg_launch_newton_schulz_batched(ctx->muon, t0.rows, t0.cols, 5, nb, ctx->stream)); }
-                {
-                    SpanScope span(ctx, EGG_K_UPDATE_MATRIX);
-                    // a failed launch must not leave earlier matrices of the batch with a stale fragment-major copy:
-                    // go on to the refresh below with what was applied, then report
-                    int applied = 0;
-                    for (; applied < nb; applied++) {
-                        const int id = g[first + applied];
-                        UpdParams p = make_upd(ctx, id, d_fit, d_seed, d_lr);
-                        p.muon_x = ctx->muon.x + (size_t)applied * one;
-                        p.lr_scale = ctx->tensors[id].lr_scale * ctx->cfg.muon_lr_scale;
-                        const hipError_t e = egg_launch_muon_apply(p, ctx->cfg.adam_weight_decay, ctx->stream);
-                        if (e != hipSuccess) { rc = fail(ctx, EGG_E_HIP, "egg_launch_muon_apply", e); break; }
-                    }
-                    for (int b = 0; b < applied; b++) { const int r2 = refresh_frag(ctx, g[first + b]); if (r2 && !rc) rc = r2; }
-                }
-                if (rc) return rc;
-            }
+    // each into its slot of the workspace, Newton-Schulz of the whole batch, then the apply rule
+    size_t batch = 0;
+    for (size_t gi = 0; gi < ctx->muon_groups.size(); gi++) {
+        const std::vector<int> &g = ctx->muon_groups[gi];
+        const egg_tensor_info &t0 = ctx->tensors[g[0]];
+        const size_t one = (size_t)t0.rows * t0.cols, k = (size_t)(t0.rows < t0.cols ? t0.rows : t0.cols);
+        const size_t limit = (size_t)ctx->muon_group_batch[gi];
+        // the group's own limit, never the largest group's: the buffers hold `limit` matrices of this shape
+        if (limit < 1 || limit * one > ctx->muon_elems || limit * k * k > ctx->muon_bterm || (int)limit > ctx->muon_batch_max)
+            return fail(ctx, EGG_E_STATE, "Muon batch does not fit the workspace");
+        for (size_t first = 0; first < g.size(); first += limit, batch++) {
+            const UpdLaunch p = make_upd(ctx, ctx->mat_muon[batch], d_fit, d_lr);
+            { SpanScope span(ctx, EGG_K_UPDATE_MATRIX); HIP_TRY(egg_launch_update(p, ctx->stream)); }
+            { SpanScope span(ctx, EGG_K_MUON_NS); HIP_TRY(egg_launch_newton_schulz_batched(ctx->muon, t0.rows, t0.cols, 5, p.n_mat, ctx->stream)); }
+            { SpanScope span(ctx, EGG_K_UPDATE_MATRIX); HIP_TRY(egg_launch_muon_apply(p, c.adam_weight_decay, ctx->stream)); }
         }
-    UpdParams common = make_upd(ctx, 0, d_fit, d_seed, d_lr);
-    { SpanScope span(ctx, EGG_K_UPDATE_VECTOR); HIP_TRY(egg_launch_update_vectors(common, ctx->d_vec_desc, ctx->n_vec, ctx->vec_total, ctx->stream)); }
+    }
     // d-eggs runs the overlay rule after each tensor's update (de/src/worker.cu:446-523); tensors and their overlay
     // entries are independent, so one launch over every tensor's segment at the end gives the same values
     if (ctx->adaptive)
@@ -889,21 +922,17 @@ extern "C" int egg_adaptive_enable(egg_ctx *ctx, int init_value, int inc, int de
     const size_t n = (size_t)ctx->L.total;
     if (!ctx->d_overlay) {
         HIP_TRY(hipMalloc(&ctx->d_overlay, n)); HIP_TRY(hipMalloc(&ctx->d_overlay_q, n)); HIP_TRY(hipMalloc(&ctx->d_flags, n));
-        std::vector<OvSeg> segs; std::vector<VecDesc> vd; int first = 0;
+        std::vector<OvSeg> segs;
         for (size_t id = 0; id < ctx->tensors.size(); id++) {
             const egg_tensor_info &t = ctx->tensors[id];
             OvSeg sg; sg.offset = (int)t.offset; sg.count = t.is_matrix ? t.rows + t.cols : t.cols;
             segs.push_back(sg);
             if (sg.count > ctx->ov_max_count) ctx->ov_max_count = sg.count;
-            if (t.is_matrix) continue;
-            VecDesc d; d.W = ctx->d_model + t.offset; d.state = reinterpret_cast<float *>(ctx->d_state + ctx->t_state_off[id]);
-            d.n = t.cols; d.first = first; d.off_a = t.off_a; d.off_b = t.off_b; d.seed_base = t.seed_base; d.lr_scale = t.lr_scale;
-            d.flags = ctx->d_flags + t.offset;
-            vd.push_back(d); first += t.cols;
         }
         ctx->n_ov_segs = (int)segs.size();
         HIP_TRY(hipMalloc(&ctx->d_ov_segs, segs.size() * sizeof(OvSeg)));
         HIP_TRY(hipMemcpy(ctx->d_ov_segs, segs.data(), segs.size() * sizeof(OvSeg), hipMemcpyHostToDevice));
+        const std::vector<VecDesc> vd = vector_descs(ctx);       // now with their flags
         HIP_TRY(hipMemcpy(ctx->d_vec_desc, vd.data(), vd.size() * sizeof(VecDesc), hipMemcpyHostToDevice));
     }
     HIP_TRY(hipMemset(ctx->d_overlay, init_value & 0xff, n));

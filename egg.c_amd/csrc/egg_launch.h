@@ -42,27 +42,44 @@ hipError_t egg_launch_sample(const int32_t *logits, const int32_t *exp_lut, int 
 hipError_t egg_launch_sample_deggs(const int32_t *logits, const int32_t *exp_lut, int vocab, int bt, uint32_t seed, int t,
                                    const void *tokens, float temp, int min_p_limit, int penalty_int, int *ws, void *out, int token_bytes, hipStream_t s);
 
-struct UpdParams {
-    int8_t *W; float *state;           // tensor weights and optimizer state ({m,v,acc} per element)
-    int rows, cols;                    // matrix: rows = input dim (k), cols = output dim (n); vector: cols = len
-    int off_a, off_b, seed_base;
-    const int32_t *fit; int pairs;
-    const uint32_t *d_seed; const float *d_lr; float lr_scale;
-    int mask; float beta1, beta2, eps, wd;
-    int limit;                         // weights saturate at +-limit: 127 (mgpu.cu:1056-1062), or the configured limit for matrices
-    int8_t *panel_a, *panel_b; int pairs_pad;   // workspace: [cols][pairs_pad], [rows][pairs_pad]
-    unsigned long long *counter;
-    int32_t *votes_out;                // optional: only compute votes (blocked order), no update
-    int8_t *flags;                     // optional (adaptive noise overlay): [rows] then [cols], set to 1 where a weight of
-                                       // that input row / output column changed (de/include/optimizer/adam.cuh:77-83)
-    // Muon (state is {m, acc} per element): momentum pass writes m and the row-major gather buffer
-    float muon_momentum; float *muon_x; // [rows][cols] row-major
+// ---- votes and optimizer step (egg_votes.hip)
+// the noise of every tensor as shifted windows of one table, see egg_votes.hip
+#define EGG_MODEL_SEEDS 920        // seed offsets of the tensors outside the layers and of layer 0 lie below this
+#define EGG_LAYER_SEEDS 416        // those of a layer's tensors, above its 1000 * layer
+struct NoiseTable {
+    int8_t *table; size_t ld; int rows;        // [rows][ld]
+    int8_t *neg, *nonzero; int pairs_pad;      // [pairs_pad] each (a multiple of 128): 0xff where the fitness is -1 / is not 0
+    int *general;                              // 1: some fitness lies outside {-1, 0, 1}
 };
-hipError_t egg_launch_update_matrix(const UpdParams &p, hipStream_t s);
-hipError_t egg_launch_update_vector(const UpdParams &p, hipStream_t s);
-// every vector tensor of the model in one launch: descriptors live on the device, `first` is the running element count
-struct VecDesc { int8_t *W; float *state; int n, first, off_a, off_b, seed_base; float lr_scale; int8_t *flags; };   // flags: as above, per element, or null
-hipError_t egg_launch_update_vectors(const UpdParams &common, const VecDesc *d_desc, int n_desc, int total, hipStream_t s);
+// rows [0, rows) of the entries [t_lo, t_hi) (rows from layer_rows on only below emb_t), the fitness masks, and *counter = 0
+// unless it is null
+hipError_t egg_launch_noise_table(const NoiseTable &nt, const uint32_t *d_seed, const int32_t *d_fit, int pairs, int mask, int rows,
+                                  int layer_rows, int t_lo, int t_hi, int emb_t, int n_layers, unsigned long long *counter, hipStream_t s);
+struct MatDesc {
+    int8_t *W, *frag; float *state;    // canonical weights, their fragment-major copy, optimizer state ({m,v,acc} or Muon's {m,acc})
+    float *muon_x;                     // Muon: the matrix's [rows][cols] slot of the workspace, else null
+    int64_t offset;                    // in the model blob (and in the overlay's flags)
+    int rows, cols, block;             // rows = input dim (k), cols = output dim (n); block: edge of the fragment-major blocks
+    int tile_first;                    // number of 64 x 64 tiles of the matrices in front of it in its list
+    int t_a, t_b;                      // first table entry of its output-side and input-side noise
+    int limit; float lr_scale;         // weights saturate at +-limit: 127 (mgpu.cu:1056-1062), or the configured limit
+};
+// a vector tensor; `first` is the running element count.  flags (adaptive noise overlay), per element, or null
+struct VecDesc { int8_t *W; float *state; int n, first, off_a, off_b, seed_base; float lr_scale; int8_t *flags; };
+struct UpdLaunch {
+    const MatDesc *mat; int n_mat, tiles;          // device array and its number of 64 x 64 tiles
+    const VecDesc *vec; int n_vec, vec_total;      // device array; may be empty
+    NoiseTable noise;
+    const int32_t *fit; int pairs;
+    const float *d_lr; float beta1, beta2, eps, wd, muon_momentum;
+    unsigned long long *counter;
+    int32_t *votes_out;                // optional, one matrix: only its votes (blocked order), no update
+    int8_t *flags;                     // optional (adaptive noise overlay), laid out like the model blob: a matrix's rows, then its
+                                       // cols, set to 1 where a weight changed (de/include/optimizer/adam.cuh:77-83)
+};
+hipError_t egg_launch_update(const UpdLaunch &p, hipStream_t s);
+hipError_t egg_launch_muon_apply(const UpdLaunch &p, float wd, hipStream_t s);
+hipError_t egg_launch_frag(const MatDesc *d_mat, int n_mat, int tiles, hipStream_t s);
 
 // adaptive noise overlay (de/src/kernels.cu:61-77): for every entry of every segment, +inc where the flag is set, -dec
 // elsewhere, clamped to [-127, 127]; also writes q = clamp(overlay, 0, 64) and clears the flag
@@ -75,13 +92,11 @@ hipError_t egg_launch_overlay_q(const int8_t *overlay, int8_t *q, int64_t n, hip
 hipError_t egg_launch_ternary_unpack(const uint8_t *packed, int8_t *dst, int n_elems, hipStream_t s);
 hipError_t egg_launch_ternary_pack(const int8_t *src, uint8_t *packed, int n_elems, int *d_bad, hipStream_t s);
 
-// Muon chain (muon_internal.cuh:15-342): momentum + gather (vote GEMM epilogue), Frobenius normalisation,
-// 5 Newton-Schulz iterations on fp32 MFMA, quantised apply.
-hipError_t egg_launch_muon_momentum(const UpdParams &p, hipStream_t s);
+// Muon chain (muon_internal.cuh:15-342): momentum + gather (epilogue of the votes), Frobenius normalisation,
+// 5 Newton-Schulz iterations on fp32 MFMA, quantised apply (egg_launch_muon_apply).
 struct MuonWork { float *x, *swap, *gram, *bterm, *partials, *norm; };   // x/swap: rows*cols, gram/bterm: K*K, partials: 1024
 hipError_t egg_launch_newton_schulz(const MuonWork &w, int rows, int cols, int iters, hipStream_t s);
 hipError_t egg_launch_newton_schulz_batched(const MuonWork &w, int rows, int cols, int iters, int batch, hipStream_t s);
-hipError_t egg_launch_muon_apply(const UpdParams &p, float wd, hipStream_t s);
 // message returned by egg_last_error(NULL) on this thread, for entry points that take no context
 void egg_set_thread_error(const char *what);
 #define EGG_MAX_DEVICES 64

@@ -1,10 +1,8 @@
-// egg_update.hip -- fitness, vote reconstruction and the ES-AdamW step on gfx950.
+// egg_update.hip -- fitness, the adaptive overlay's rule, ternary packing, sampling and the Newton-Schulz chain on gfx950
+// (votes and the optimizer step: egg_votes.hip).
 //
-// Reference: compute_fitness_kernel, apply_adam_update, update_matrix_adam_kernel and
-// update_vector_adam_kernel, full_cuda_train_transformer_adam_mgpu.cu:1031-1152 ("mgpu.cu").
-// The reference recomputes two noise hashes per (weight, pair); here the (rows+cols) x pairs noise
-// panels are generated once per matrix and the vote  sum_p fit_p A_p[n] B_p[k]  is an int8 MFMA GEMM
-// over the population axis whose epilogue applies AdamW in place (blocked element order).
+// Reference: compute_fitness_kernel, mgpu.cu:1031-1036 ("mgpu.cu" = full_cuda_train_transformer_adam_mgpu.cu);
+// update_overlay_kernel, de/src/kernels.cu:61-77; generate_sequence_kernel's sampling; perform_newton_schulz.
 #include "../../include/egg_hip.h"
 #include "egg_device.h"
 #include "egg_launch.h"
@@ -57,192 +55,6 @@ hipError_t egg_launch_fitness(const int32_t *loss, int32_t *fit, int pairs, hipS
     return hipGetLastError();
 }
 
-// apply_adam_update (mgpu.cu:1040-1064); every float operation is a single IEEE-754 operation
-struct AdamHyper { float b1, b2, eps, wd; int limit; };     // limit: the weight saturates at +-limit (127 in the reference)
-__device__ __forceinline__ int adam_apply(float &m, float &v, float &acc, int &w, float gr, float lr, const AdamHyper &h) {
-    float t1 = h.b1 * m; float t2 = (1.0f - h.b1) * gr; m = t1 + t2;
-    float t3 = h.b2 * v; float gg = gr * gr; float t4 = (1.0f - h.b2) * gg; v = t3 + t4;
-    float den = sqrtf(v) + h.eps;
-    float q = m / den;
-    float wdw = h.wd * (float)w;
-    float step = (-lr) * (q + wdw);
-    acc += step;
-    int change = 0;
-    if (acc >= 1.0f) {
-        if (w < h.limit) { w++; change = 1; acc -= 1.0f; } else acc = 1.0f;
-    } else if (acc <= -1.0f) {
-        if (w > -h.limit) { w--; change = 1; acc += 1.0f; } else acc = -1.0f;
-    }
-    return change;
-}
-
-// noise panels, pair index contiguous: pa[n][p] = fit_p * A_p[n], pb[k][p] = B_p[k]; zero beyond `pairs`
-__global__ void k_panels(UpdParams p) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    int64_t total = (int64_t)(p.rows + p.cols) * p.pairs_pad;
-    if (i >= total) return;
-    int pr = (int)(i % p.pairs_pad); int r = (int)(i / p.pairs_pad);
-    int val = 0;
-    if (pr < p.pairs) {
-        uint32_t s = *p.d_seed + (uint32_t)pr + (uint32_t)p.seed_base;
-        if (r < p.cols) val = p.fit[pr] * noise_from_hash(s + p.off_a, r, p.mask);
-        else val = noise_from_hash(s + p.off_b, r - p.cols, p.mask);
-    }
-    if (r < p.cols) p.panel_a[(size_t)r * p.pairs_pad + pr] = (int8_t)val;
-    else p.panel_b[(size_t)(r - p.cols) * p.pairs_pad + pr] = (int8_t)val;
-}
-
-// One workgroup per 32(k) x 32(n) tile of the vote matrix.  The reduction over pairs runs on the MFMA, split four
-// ways over the waves (wave w takes the 32-pair steps w, w+4, ...; integer sums do not depend on the order); the
-// partial tiles meet in LDS and wave q finishes the four k-rows 8q+4g+e of the tile (the Adam / Muon / raw-vote
-// epilogue).  The operand loads are issued several steps ahead of the MFMAs that consume them.
-__global__ void __launch_bounds__(EGG_THREADS) k_vote_adam(UpdParams p) {
-    __shared__ int red[EGG_WAVES][16][64];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 5, j = lane & 31;
-    const int tiles_n = p.cols / 32;
-    const int tile = blockIdx.x;
-    const int k0 = (tile / tiles_n) * 32, n0 = (tile % tiles_n) * 32;
-    const int8_t *pb = p.panel_b + (size_t)(k0 + j) * p.pairs_pad + 16 * g;
-    const int8_t *pa = p.panel_a + (size_t)(n0 + j) * p.pairs_pad + 16 * g;
-    v16i acc;
-#pragma unroll
-    for (int r = 0; r < 16; r++) acc[r] = 0;
-#pragma unroll 8
-    for (int s = wave * 32; s < p.pairs_pad; s += 32 * EGG_WAVES) {
-        v4i a = *reinterpret_cast<const v4i *>(pb + s);
-        v4i b = *reinterpret_cast<const v4i *>(pa + s);
-        acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, acc, 0, 0, 0);
-    }
-#pragma unroll
-    for (int r = 0; r < 16; r++) red[wave][r][lane] = acc[r];
-    __syncthreads();
-    const int q = wave;
-    int vote[4];
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-        int v = 0;
-#pragma unroll
-        for (int w = 0; w < EGG_WAVES; w++) v += red[w][4 * q + e][lane];
-        vote[e] = v;
-    }
-    // lane (n = n0 + j, half g), element e -> k = k0 + 8q + 4g + e ; blocked index of (k, n) (mgpu.cu:1085-1089)
-    const int n = n0 + j;
-    const size_t idx0 = ((size_t)((k0 >> 2) + 2 * q + g) * p.cols + n) * 4;
-    if (p.muon_x) {
-        // muon_momentum_update_kernel + muon_gather_m_kernel (muon_internal.cuh:15-74): m = mu*m + vote
-        float4 *sp = reinterpret_cast<float4 *>(p.state + idx0 * 2);
-        float4 s0 = sp[0], s1 = sp[1];
-        float mv[4] = {s0.x, s0.z, s1.x, s1.z};
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            float t = p.muon_momentum * mv[e];
-            mv[e] = t + (float)vote[e];
-            p.muon_x[(size_t)(k0 + 8 * q + 4 * g + e) * p.cols + n] = mv[e];
-        }
-        sp[0] = make_float4(mv[0], s0.y, mv[1], s0.w);
-        sp[1] = make_float4(mv[2], s1.y, mv[3], s1.w);
-        return;
-    }
-    if (p.votes_out) {
-        v4i o4;
-#pragma unroll
-        for (int e = 0; e < 4; e++) o4[e] = vote[e];
-        *reinterpret_cast<v4i *>(p.votes_out + idx0) = o4;
-        return;
-    }
-    const float lr = (*p.d_lr) * p.lr_scale;
-    const AdamHyper hy = {p.beta1, p.beta2, p.eps, p.wd, p.limit};
-    int changes = 0;
-    int w4 = *reinterpret_cast<const int *>(p.W + idx0);
-    float st[12];
-    float4 *sp = reinterpret_cast<float4 *>(p.state + idx0 * 3);
-    float4 s0 = sp[0], s1 = sp[1], s2 = sp[2];
-    st[0] = s0.x; st[1] = s0.y; st[2] = s0.z; st[3] = s0.w; st[4] = s1.x; st[5] = s1.y; st[6] = s1.z; st[7] = s1.w;
-    st[8] = s2.x; st[9] = s2.y; st[10] = s2.z; st[11] = s2.w;
-    int wv[4];
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-        wv[e] = sx8(w4, e);
-        const int ch = adam_apply(st[3 * e], st[3 * e + 1], st[3 * e + 2], wv[e], -(float)vote[e], lr, hy);
-        changes += ch;
-        // every writer stores the same value, so plain stores do (the overlay rule only asks "any change?")
-        if (ch && p.flags) { p.flags[k0 + 8 * q + 4 * g + e] = 1; p.flags[p.rows + n] = 1; }
-    }
-    *reinterpret_cast<int *>(p.W + idx0) = pack4(wv[0], wv[1], wv[2], wv[3]);
-    sp[0] = make_float4(st[0], st[1], st[2], st[3]);
-    sp[1] = make_float4(st[4], st[5], st[6], st[7]);
-    sp[2] = make_float4(st[8], st[9], st[10], st[11]);
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) changes += __shfl_xor(changes, off, 64);
-    if (lane == 0 && changes) atomicAdd(p.counter, (unsigned long long)changes);
-}
-hipError_t egg_launch_update_matrix(const UpdParams &p, hipStream_t s) {
-    if (p.rows % 32 || p.cols % 32 || p.pairs_pad % 32) return hipErrorInvalidValue;
-    int64_t total = (int64_t)(p.rows + p.cols) * p.pairs_pad;
-    hipLaunchKernelGGL(k_panels, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, p);
-    int tiles = (p.rows / 32) * (p.cols / 32);
-    hipLaunchKernelGGL(k_vote_adam, dim3(tiles), dim3(EGG_THREADS), 0, s, p);
-    return hipGetLastError();
-}
-
-// update_vector_adam_kernel (mgpu.cu:1114-1152): one wave per element, lanes stride over pairs
-__global__ void __launch_bounds__(EGG_THREADS) k_vector_adam(UpdParams p) {
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int idx = blockIdx.x * EGG_WAVES + wave;
-    if (idx >= p.cols) return;
-    const uint32_t base = *p.d_seed + (uint32_t)p.seed_base;
-    int vote = 0;
-    for (int pr = lane; pr < p.pairs; pr += 64) {
-        int f = p.fit[pr];
-        if (f == 0) continue;
-        uint32_t s = base + (uint32_t)pr;
-        vote += f * noise_from_hash(s + p.off_a, idx, p.mask) * noise_from_hash(s + p.off_b, idx, p.mask);
-    }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) vote += __shfl_xor(vote, off, 64);
-    if (lane == 0) {
-        const AdamHyper hy = {p.beta1, p.beta2, p.eps, p.wd, 127};     // vector tensors keep the reference's +-127
-        const float lr = (*p.d_lr) * p.lr_scale;
-        float *st = p.state + (size_t)idx * 3;
-        float m = st[0], v = st[1], acc = st[2];
-        int w = p.W[idx];
-        int ch = adam_apply(m, v, acc, w, -(float)vote, lr, hy);
-        p.W[idx] = (int8_t)w; st[0] = m; st[1] = v; st[2] = acc;
-        if (ch) atomicAdd(p.counter, 1ull);
-    }
-}
-// the same for all vector tensors at once (one wave per element of any of them), so that the small per-tensor
-// launches do not leave most of the GPU idle
-__global__ void __launch_bounds__(EGG_THREADS) k_vectors_adam(UpdParams p, const VecDesc *desc, int n_desc, int total) {
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int gi = blockIdx.x * EGG_WAVES + wave;
-    if (gi >= total) return;
-    int d = 0;
-    while (d + 1 < n_desc && desc[d + 1].first <= gi) d++;
-    const VecDesc t = desc[d];
-    const int idx = gi - t.first;
-    const uint32_t base = *p.d_seed + (uint32_t)t.seed_base;
-    int vote = 0;
-    for (int pr = lane; pr < p.pairs; pr += 64) {
-        int f = p.fit[pr];
-        if (f == 0) continue;
-        uint32_t s = base + (uint32_t)pr;
-        vote += f * noise_from_hash(s + t.off_a, idx, p.mask) * noise_from_hash(s + t.off_b, idx, p.mask);
-    }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) vote += __shfl_xor(vote, off, 64);
-    if (lane == 0) {
-        const AdamHyper hy = {p.beta1, p.beta2, p.eps, p.wd, 127};     // vector tensors keep the reference's +-127
-        const float lr = (*p.d_lr) * t.lr_scale;
-        float *st = t.state + (size_t)idx * 3;
-        float m = st[0], v = st[1], acc = st[2];
-        int w = t.W[idx];
-        int ch = adam_apply(m, v, acc, w, -(float)vote, lr, hy);
-        t.W[idx] = (int8_t)w; st[0] = m; st[1] = v; st[2] = acc;
-        if (ch) atomicAdd(p.counter, 1ull);
-        if (ch && t.flags) t.flags[idx] = 1;
-    }
-}
 // Ternary-packed matrix weights (no counterpart in the reference, whose weights are plain int8): four consecutive
 // elements of the blocked matrix -- the four input rows that share one dword -- per byte, element e in bits 2e+1..2e
 // as a 2-bit two's complement number (00 = 0, 01 = +1, 11 = -1).  Unpacking writes the canonical int8 blob, from which
@@ -309,16 +121,6 @@ __global__ void k_overlay_q(const int8_t *overlay, int8_t *q, int64_t n) {
 }
 hipError_t egg_launch_overlay_q(const int8_t *overlay, int8_t *q, int64_t n, hipStream_t s) {
     hipLaunchKernelGGL(k_overlay_q, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, overlay, q, n);
-    return hipGetLastError();
-}
-
-hipError_t egg_launch_update_vectors(const UpdParams &common, const VecDesc *d_desc, int n_desc, int total, hipStream_t s) {
-    if (total <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_vectors_adam, dim3((total + EGG_WAVES - 1) / EGG_WAVES), dim3(EGG_THREADS), 0, s, common, d_desc, n_desc, total);
-    return hipGetLastError();
-}
-hipError_t egg_launch_update_vector(const UpdParams &p, hipStream_t s) {
-    hipLaunchKernelGGL(k_vector_adam, dim3((p.cols + EGG_WAVES - 1) / EGG_WAVES), dim3(EGG_THREADS), 0, s, p);
     return hipGetLastError();
 }
 
@@ -457,11 +259,6 @@ hipError_t egg_launch_swizzle(const int8_t *W, int8_t *Wf, int K, int N, int B, 
     hipLaunchKernelGGL(k_swizzle, dim3((chunks + 255) / 256), dim3(256), 0, s, reinterpret_cast<const uint32_t *>(W),
                        reinterpret_cast<v4i *>(Wf), K, N, B, nat);
     return hipGetLastError();
-}
-
-hipError_t egg_launch_muon_momentum(const UpdParams &p, hipStream_t s) {
-    if (!p.muon_x) return hipErrorInvalidValue;
-    return egg_launch_update_matrix(p, s);
 }
 
 // ---------------------------------------------------------------- Newton-Schulz (muon_internal.cuh:182-342)
@@ -776,31 +573,4 @@ extern "C" int egg_newton_schulz_static(float *d_X, int rows, int cols, int iter
         return EGG_E_HIP;
     }
     return EGG_OK;
-}
-
-// muon_apply_update_kernel (muon_internal.cuh:112-170)
-__global__ void __launch_bounds__(256) k_muon_apply(UpdParams p, float wd) {
-    int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    int change = 0;
-    if (idx < p.rows * p.cols) {
-        int byte_off = idx & 3, word = idx >> 2, n = word % p.cols, k = (word / p.cols) * 4 + byte_off;
-        int w = p.W[idx];
-        float *st = p.state + (size_t)idx * 2;
-        float acc = st[1];
-        float u = p.muon_x[(size_t)k * p.cols + n];
-        float lr = (*p.d_lr) * p.lr_scale;
-        float wdw = wd * (float)w;
-        float step = (-lr) * (u + wdw);
-        acc += step;
-        if (acc >= 1.0f) { if (w < p.limit) { w++; change = 1; acc -= 1.0f; } else acc = 1.0f; }
-        else if (acc <= -1.0f) { if (w > -p.limit) { w--; change = 1; acc += 1.0f; } else acc = -1.0f; }
-        p.W[idx] = (int8_t)w; st[1] = acc;
-    }
-    unsigned long long m = __ballot(change);
-    if ((threadIdx.x & 63) == 0 && m) atomicAdd(p.counter, (unsigned long long)__popcll(m));
-}
-hipError_t egg_launch_muon_apply(const UpdParams &p, float wd, hipStream_t s) {
-    int n = p.rows * p.cols;
-    hipLaunchKernelGGL(k_muon_apply, dim3((n + 255) / 256), dim3(256), 0, s, p, wd);
-    return hipGetLastError();
 }

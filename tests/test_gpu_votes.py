@@ -1,0 +1,39 @@
+"""The vote kernel at the edges of its pair chunks (128 pairs, masks padded with zeros) and of its fitness forms."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("values", [(-1, 0, 1), (-3, 2, 5)], ids=["ternary", "any"])
+@pytest.mark.parametrize("pairs", [1, 127, 128, 129, 640])
+def test_votes_and_update_at_chunk_edges(pkg, orc, dev, pairs, values):
+    import torch
+    kw = dict(hidden=64, head_dim=32, n_layers=3, seq_len=32, population=2 * pairs)
+    ocfg = orc.config(**kw)
+    ctx = pkg.Context(pkg.default_config(**kw))
+    model = orc.init_model(ocfg, 42)
+    state = np.zeros(model.size, orc.ADAM_DTYPE)
+    ctx.model_upload(model)
+    fit = np.random.default_rng(pairs).choice(np.array(values, np.int32), pairs)
+    seed, lr = 0xFFFFFF00, 5.0                       # pair seeds that wrap around 2^32
+    d_fit = torch.from_numpy(fit).to(dev)
+    d_seed = torch.from_numpy(np.array([seed], np.uint32).view(np.int32)).to(dev)
+    d_lr = torch.tensor([lr], dtype=torch.float32, device=dev)
+    for t in (t for t in ctx.tensors() if t["is_matrix"]):
+        d_votes = torch.zeros(t["rows"] * t["cols"], dtype=torch.int32, device=dev)
+        ctx.matrix_votes(t["id"], d_fit.data_ptr(), d_seed.data_ptr(), d_votes.data_ptr())
+        ctx.sync()
+        ref = np.zeros(t["rows"] * t["cols"], np.int32)
+        orc.lib().orc_matrix_votes(C.byref(ocfg), t["rows"], t["cols"], t["off_a"], t["off_b"], t["seed_base"],
+                                   fit.ctypes.data_as(C.c_void_p), pairs, C.c_uint32(seed), ref.ctypes.data_as(C.c_void_p))
+        assert np.array_equal(d_votes.cpu().numpy(), ref), t["name"]
+    for _ in range(2):
+        ctx.es_update(d_fit.data_ptr(), d_seed.data_ptr(), d_lr.data_ptr())
+        n_ref = orc.es_update_adam(ocfg, model, state, fit, seed, lr)
+        assert np.array_equal(ctx.model_download(), model)
+        assert np.array_equal(ctx.opt_state_download().view(np.int32), state.view(np.int32))
+        assert ctx.last_update_count() == n_ref
+    ctx.close()
