@@ -72,7 +72,8 @@ struct egg_ctx {
     double t_ms[EGG_KCLASS_COUNT] = {0}; long t_n[EGG_KCLASS_COUNT] = {0};
     // generation (egg_generate): token buffer [T + 1], logits of one member [T][vocab], a zero start index / seed
     uint8_t *d_gen_tok = nullptr; int32_t *d_gen_logits = nullptr, *d_gen_ws = nullptr; Scalars *d_gen_scal = nullptr;
-    int8_t *d_gen_kv = nullptr; bool gen_kv_cache = true;      // per-layer K / V rows of the generated sequence (egg_ctx_generate_kv_cache)
+    int8_t *d_gen_kv = nullptr; bool gen_kv_cache = true;      // per-layer K / V rows of the prompt (egg_ctx_generate_kv_cache)
+    int8_t *d_dec_kv = nullptr; unsigned long long *d_dec_slots = nullptr; uint32_t *d_dec_epoch = nullptr; int *h_dec_fail = nullptr;    // egg_decode.hip
     int mask_override = -1; int32_t *logits_override = nullptr;
     bool first_dedup = true;        // first block once per distinct byte value of a member's window (egg_ctx_first_block_dedup)
     VecDesc *d_vec_desc = nullptr; int n_vec = 0, vec_total = 0;       // all vector tensors, then each on its own
@@ -264,9 +265,10 @@ static void free_all(egg_ctx *ctx) {
     void *ptrs[] = {ctx->muon.x, ctx->muon.swap, ctx->muon.bterm, ctx->muon.partials, ctx->muon.norm,
                     ctx->d_wfrag, ctx->d_plin_frag, ctx->d_model, ctx->d_state, ctx->d_exp, ctx->d_act, ctx->d_rope, ctx->d_x, ctx->d_q, ctx->d_k, ctx->d_v,
                     ctx->d_ao, ctx->d_loss_acc, ctx->d_counter, ctx->d_loss, ctx->d_fit, ctx->d_scal, ctx->noise.table,
-                    ctx->noise.neg, ctx->noise.nonzero, ctx->noise.general, ctx->d_mat, ctx->d_tap, ctx->d_tap_logits, ctx->d_gen_tok, ctx->d_gen_logits, ctx->d_gen_ws, ctx->d_gen_scal, ctx->d_gen_kv, ctx->d_vec_desc,
+                    ctx->noise.neg, ctx->noise.nonzero, ctx->noise.general, ctx->d_mat, ctx->d_tap, ctx->d_tap_logits, ctx->d_gen_tok, ctx->d_gen_logits, ctx->d_gen_ws, ctx->d_gen_scal, ctx->d_gen_kv, ctx->d_dec_kv, ctx->d_dec_slots, ctx->d_dec_epoch, ctx->d_vec_desc,
                     ctx->d_overlay, ctx->d_overlay_q, ctx->d_flags, ctx->d_ov_segs};
     for (void *p : ptrs) if (p) (void)hipFree(p);
+    if (ctx->h_dec_fail) (void)hipHostFree(ctx->h_dec_fail);
     for (auto &sp : ctx->spans) { (void)hipEventDestroy(sp.a); (void)hipEventDestroy(sp.b); }
     if (ctx->gexec) (void)hipGraphExecDestroy(ctx->gexec);
     if (ctx->graph) (void)hipGraphDestroy(ctx->graph);
@@ -482,6 +484,7 @@ extern "C" int egg_ctx_set_stream(egg_ctx *ctx, void *s) {
 extern "C" int egg_sync(egg_ctx *ctx) {
     if (!ctx) return EGG_E_INVALID;
     HIP_TRY(hipStreamSynchronize(ctx->stream));
+    if (ctx->h_dec_fail && *(volatile int *)ctx->h_dec_fail) return fail(ctx, EGG_E_HIP, "a generation did not finish: its workgroups were not on the GPU together");
     return EGG_OK;
 }
 
@@ -708,7 +711,8 @@ static int8_t *tap_ptr(egg_ctx *ctx, int slot) {
 // `range` (generation only): evaluate the token positions [t0, t0 + tn) of the chunk's members and keep every layer's
 // K / V rows in `kv` ([layer][K, V][nm][T][H]) instead of the shared k / v buffers, so that a later call on a later
 // range finds the rows of the positions in front of it (the reference's d_gen_kv, mgpu.cu:1160-1170)
-struct FwdRange { int t0, tn; int8_t *kv; };
+// kv_only: nothing behind the last layer's K / V rows is wanted.
+struct FwdRange { int t0, tn; int8_t *kv; bool kv_only; };
 static int forward_chunk(egg_ctx *ctx, const uint8_t *d_data, int64_t len, const int64_t *d_start, const uint32_t *d_seed,
                          int first_member, int nm, const FwdRange *range = nullptr) {
     const egg_config &c = ctx->cfg; const Layout &L = ctx->L; const int8_t *M = ctx->d_model; const int H = c.hidden;
@@ -755,6 +759,7 @@ static int forward_chunk(egg_ctx *ctx, const uint8_t *d_data, int64_t len, const
                 HIP_TRY(hipMemcpyAsync(tap_ptr(ctx, 1 + 6 * l + 1), ctx->d_k, act_bytes, hipMemcpyDeviceToDevice, s));
                 HIP_TRY(hipMemcpyAsync(tap_ptr(ctx, 1 + 6 * l + 2), ctx->d_v, act_bytes, hipMemcpyDeviceToDevice, s));
             }
+            if (range && range->kv_only && l + 1 == c.n_layers) return EGG_OK;
         }
         {
             AttnParams p; memset(&p, 0, sizeof(p)); p.c = f; p.q = ctx->d_q; p.k = ctx->d_k; p.v = ctx->d_v; p.ao = ctx->d_ao;
@@ -1085,18 +1090,36 @@ extern "C" uint32_t egg_next_seed(uint32_t seed, uint64_t step) {
 // ------------------------------------------------------------------ taps
 // generate_sequence_kernel (mgpu.cu:1154-1283) and its call site (:1701-1708).  The reference walks the sequence
 // token by token with a per-layer KV cache (d_gen_kv).  Here the unperturbed forward of one member (noise mask 0 makes
-// every perturbation term vanish, i.e. noise_sign = 0) runs once over the whole window for the prompt and fills every
-// layer's K / V rows; each new token then re-evaluates only the 32-token tile that holds position t -- embedding,
-// projections, the tile's queries against the cached K / V rows of everything in front of them, MLP, head -- and
-// samples from the logits of position t.  Causality makes what position t sees independent of the not yet generated
-// tail, and a tile's K / V rows are final once its last position has been generated.  With the cache switched off
-// (egg_ctx_generate_kv_cache) every new token re-runs the whole window instead; the tokens are the same.
+// every perturbation term vanish, i.e. noise_sign = 0) runs once over the prompt's tiles and leaves every layer's K / V
+// rows of the positions in front of the prompt's last token; from that token on one launch evaluates and samples token
+// by token (egg_decode.hip).  With the cache switched off (egg_ctx_generate_kv_cache) every new token runs the forward
+// over the whole window instead and is sampled by a launch of its own; the tokens are the same.
 struct DeggsSampling { float temp; int min_p_limit, penalty_int; };
+// the persistent launch's buffers; a launch that gave up leaves them in no defined state
+static int decode_buffers(egg_ctx *ctx) {
+    const egg_config &c = ctx->cfg; const size_t strips = c.hidden / 16, slots = (size_t)egg_decode_slots(c.hidden) * 8;
+    if (!ctx->h_dec_fail) {
+        HIP_TRY(egg_prepare_decode(c.hidden, c.vocab));
+        HIP_TRY(hipMalloc(&ctx->d_dec_kv, strips * c.n_layers * c.seq_len * (c.head_dim + 16)));
+        HIP_TRY(hipMalloc(&ctx->d_dec_slots, slots)); HIP_TRY(hipMalloc(&ctx->d_dec_epoch, 4));
+        HIP_TRY(hipMemset(ctx->d_dec_slots, 0, slots)); HIP_TRY(hipMemset(ctx->d_dec_epoch, 0, 4));
+        HIP_TRY(hipHostMalloc(&ctx->h_dec_fail, sizeof(int)));
+        *ctx->h_dec_fail = 0;
+    }
+    if (*(volatile int *)ctx->h_dec_fail) {
+        HIP_TRY(hipStreamSynchronize(ctx->stream));
+        HIP_TRY(hipMemset(ctx->d_dec_slots, 0, slots)); HIP_TRY(hipMemset(ctx->d_dec_epoch, 0, 4));
+        *ctx->h_dec_fail = 0;
+        return fail(ctx, EGG_E_HIP, "the generation before this one did not finish: its workgroups were not on the GPU together");
+    }
+    return EGG_OK;
+}
 static int generate_impl(egg_ctx *ctx, uint8_t *d_buffer, int seed_len, int gen_len, uint32_t seed, const DeggsSampling *de) {
     if (!ctx || !d_buffer) return EGG_E_INVALID;
     const egg_config &c = ctx->cfg; const int T = c.seq_len, total = seed_len + gen_len;
     if (seed_len < 1 || gen_len < 0 || total > T) return fail(ctx, EGG_E_INVALID, "egg_generate: need 1 <= seed_len and seed_len + gen_len <= seq_len");
     if (ctx->captured) return fail(ctx, EGG_E_STATE, "egg_generate cannot run on a context whose step is captured");
+    if (gen_len == 0) return EGG_OK;
     const int tb = c.vocab > 256 ? 4 : 1;          // bytes per token of the buffer
     hipStream_t s = ctx->stream;
     if (!ctx->d_gen_tok) {
@@ -1107,19 +1130,51 @@ static int generate_impl(egg_ctx *ctx, uint8_t *d_buffer, int seed_len, int gen_
         HIP_TRY(hipMemset(ctx->d_gen_scal, 0, sizeof(Scalars)));
         HIP_TRY(hipMalloc(&ctx->d_gen_kv, (size_t)c.n_layers * 2 * T * c.hidden));
     }
-    HIP_TRY(egg_launch_zero_u64(reinterpret_cast<unsigned long long *>(ctx->d_gen_tok), (T + 16) * tb / 8, s));   // a fill kernel, not a memset node: a caller may be capturing this stream
-    HIP_TRY(hipMemcpyAsync(ctx->d_gen_tok, d_buffer, (size_t)seed_len * tb, hipMemcpyDeviceToDevice, s));
-    int bt = (c.hidden + 31) & ~31; if (bt > 1024) bt = 1024;          // BLOCK_THREADS (mgpu.cu:74-75)
+    int rc = decode_buffers(ctx);
+    if (rc) return rc;
+    const bool cached = ctx->gen_kv_cache && ctx->L.total < ((int64_t)1 << 32);        // the persistent launch addresses the blob with 32 bits
+    if (!cached || seed_len > 1) {
+        HIP_TRY(egg_launch_zero_u64(reinterpret_cast<unsigned long long *>(ctx->d_gen_tok), (T + 16) * tb / 8, s));   // a fill kernel, not a memset node: a caller may be capturing this stream
+        HIP_TRY(hipMemcpyAsync(ctx->d_gen_tok, d_buffer, (size_t)seed_len * tb, hipMemcpyDeviceToDevice, s));
+    }
     const bool taps = ctx->taps; ctx->taps = false;
     ctx->mask_override = 0; ctx->logits_override = ctx->d_gen_logits;
-    int rc = EGG_OK;
-    for (int t = seed_len - 1; t < total - 1 && rc == EGG_OK; t++) {
-        // data_len = T + 1 puts the member's stream position at 0 (mgpu.cu:864-870 with len - T == 1)
-        FwdRange range = {0, T, ctx->d_gen_kv};
-        if (t > seed_len - 1) { range.t0 = t & ~31; range.tn = 32; }       // the prompt: whole window; then the tile of position t
-        rc = forward_chunk(ctx, ctx->d_gen_tok, (int64_t)T + 1, &ctx->d_gen_scal->start, &ctx->d_gen_scal->seed, 0, 1,
-                           ctx->gen_kv_cache ? &range : nullptr);
+    // data_len = T + 1 puts the member's stream position at 0 (mgpu.cu:864-870 with len - T == 1)
+    auto forward = [&](const FwdRange *range) {
+        return forward_chunk(ctx, ctx->d_gen_tok, (int64_t)T + 1, &ctx->d_gen_scal->start, &ctx->d_gen_scal->seed, 0, 1, range);
+    };
+    if (cached) {
+        if (seed_len > 1) {
+            int tn = 32;                             // the kernels walk 1, 2, 4, ... tiles of a member
+            while (tn < seed_len - 1) tn *= 2;
+            const FwdRange prompt = {0, tn, ctx->d_gen_kv, true};
+            rc = forward(&prompt);
+        }
         if (rc == EGG_OK) {
+            DecodeParams p;
+            const Layout &L = ctx->L;
+            p.model = ctx->d_model; p.frag = ctx->d_wfrag;
+            p.embedding = (uint32_t)L.embedding; p.emb_bias = (uint32_t)L.emb_bias; p.ln_init = (uint32_t)L.ln_init; p.ln_init_bias = (uint32_t)L.ln_init_bias;
+            p.w_up_init = (uint32_t)L.w_emb_mlp_up; p.b_up_init = (uint32_t)L.mlp_emb_bias_up; p.w_dn_init = (uint32_t)L.w_emb_mlp_down; p.b_dn_init = (uint32_t)L.mlp_emb_bias_down;
+            p.ln_1 = (uint32_t)L.ln_1; p.ln_1_bias = (uint32_t)L.ln_1_bias; p.w_q = (uint32_t)L.w_q; p.w_k = (uint32_t)L.w_k; p.w_v = (uint32_t)L.w_v; p.w_o = (uint32_t)L.w_o;
+            p.ln_2 = (uint32_t)L.ln_2; p.ln_2_bias = (uint32_t)L.ln_2_bias; p.w_up = (uint32_t)L.w_up; p.b_up = (uint32_t)L.mlp_bias_up; p.w_dn = (uint32_t)L.w_down;
+            p.b_dn = (uint32_t)L.mlp_bias_down; p.ln_f = (uint32_t)L.ln_f; p.ln_f_bias = (uint32_t)L.ln_f_bias;
+            p.exp_lut = ctx->d_exp; p.act_lut = ctx->d_act; p.rope_lut = ctx->d_rope;
+            p.n_layers = c.n_layers; p.head_dim = c.head_dim; p.T = T; p.vocab = c.vocab;
+            p.shift_attn = c.shift_attn; p.shift_out = c.shift_out; p.shift_logit = c.shift_logit; p.shift_up = c.shift_mlp_up; p.shift_dn = c.shift_mlp_down;
+            p.rope_bit = c.rope_scale_bit;
+            p.tokens = d_buffer; p.out = d_buffer; p.token_bytes = tb; p.t_first = seed_len - 1; p.count = gen_len;
+            p.prompt_kv = ctx->d_gen_kv; p.kcache = ctx->d_dec_kv; p.vcache = ctx->d_dec_kv + (size_t)(c.hidden / 16) * c.n_layers * T * c.head_dim;
+            p.slots = ctx->d_dec_slots; p.epoch = ctx->d_dec_epoch; p.fail = ctx->h_dec_fail;
+            p.seed = seed; p.deggs = de != nullptr; p.temp = de ? de->temp : 1.f; p.min_p_limit = de ? de->min_p_limit : 0; p.penalty_int = de ? de->penalty_int : 0;
+            const hipError_t e = egg_launch_decode(p, c.hidden, s);
+            if (e != hipSuccess) rc = fail(ctx, EGG_E_HIP, "egg_launch_decode", e);
+        }
+    } else {
+        int bt = (c.hidden + 31) & ~31; if (bt > 1024) bt = 1024;          // BLOCK_THREADS (mgpu.cu:74-75)
+        for (int t = seed_len - 1; t < total - 1 && rc == EGG_OK; t++) {
+            rc = forward(nullptr);
+            if (rc != EGG_OK) break;
             const int32_t *row = ctx->d_gen_logits + (size_t)t * c.vocab;
             uint8_t *next = ctx->d_gen_tok + (size_t)(t + 1) * tb;
             hipError_t e = de ? egg_launch_sample_deggs(row, ctx->d_exp, c.vocab, bt, seed, t, ctx->d_gen_tok, de->temp, de->min_p_limit, de->penalty_int,
@@ -1130,7 +1185,7 @@ static int generate_impl(egg_ctx *ctx, uint8_t *d_buffer, int seed_len, int gen_
     }
     ctx->mask_override = -1; ctx->logits_override = nullptr; ctx->taps = taps;
     if (rc) return rc;
-    HIP_TRY(hipMemcpyAsync(d_buffer, ctx->d_gen_tok, (size_t)total * tb, hipMemcpyDeviceToDevice, s));
+    if (!cached) HIP_TRY(hipMemcpyAsync(d_buffer, ctx->d_gen_tok, (size_t)total * tb, hipMemcpyDeviceToDevice, s));
     return EGG_OK;
 }
 extern "C" int egg_ctx_generate_kv_cache(egg_ctx *ctx, int enable) {

@@ -88,6 +88,27 @@ hipError_t egg_launch_overlay_update(int8_t *overlay, int8_t *q, int8_t *flags, 
                                      int inc, int dec, hipStream_t s);
 hipError_t egg_launch_overlay_q(const int8_t *overlay, int8_t *q, int64_t n, hipStream_t s);
 
+// ---- continuation of one sequence (egg_decode.hip)
+struct DecodeParams {
+    const int8_t *model, *frag;        // the model blob and the fragment-major copies of its matrices; offsets in both:
+    uint32_t embedding, emb_bias, ln_init, ln_init_bias, w_up_init, b_up_init, w_dn_init, b_dn_init, ln_1, ln_1_bias, w_q, w_k, w_v, w_o,
+        ln_2, ln_2_bias, w_up, b_up, w_dn, b_dn, ln_f, ln_f_bias;
+    const int32_t *exp_lut; const int8_t *act_lut; const int32_t *rope_lut;
+    int n_layers, head_dim, T, vocab, shift_attn, shift_out, shift_logit, shift_up, shift_dn, rope_bit;
+    const uint8_t *tokens;             // the prompt: tokens 0..t_first of token_bytes each
+    void *out; int token_bytes;        // token t + 1 goes to out[t + 1]
+    int t_first, count;                // positions t_first .. t_first + count - 1 are evaluated and sampled from
+    const int8_t *prompt_kv;           // [layer][K, V][T][H] slot order: the rows of the positions in front of t_first
+    int8_t *kcache, *vcache;           // [H / 16][layer][T][head_dim], [H / 16][layer][T][16]
+    unsigned long long *slots;         // egg_decode_slots, zero before the first launch
+    uint32_t *epoch;                   // number of the last exchange, zero before the first launch
+    int *fail;                         // host memory: set when a wait ran into its bound
+    uint32_t seed; int deggs; float temp; int min_p_limit, penalty_int;
+};
+int64_t egg_decode_slots(int H);
+hipError_t egg_prepare_decode(int H, int vocab);      // before the first launch
+hipError_t egg_launch_decode(const DecodeParams &p, int H, hipStream_t s);
+
 // ternary-packed matrix weights <-> canonical int8 (n_elems a multiple of 4); *d_bad is set when a weight is not in {-1,0,1}
 hipError_t egg_launch_ternary_unpack(const uint8_t *packed, int8_t *dst, int n_elems, hipStream_t s);
 hipError_t egg_launch_ternary_pack(const int8_t *src, uint8_t *packed, int n_elems, int *d_bad, hipStream_t s);
