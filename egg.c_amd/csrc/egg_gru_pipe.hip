@@ -12,11 +12,12 @@
 // L).  Before, a tick was one stage of single tokens: 2 T + 6 L + 1 launches of 9.6 us, each streaming the weights again.
 // Here there are T / 32 + 4 L, and R's chain of T steps that never leaves a CU is what a sequence takes.
 //
-// R: a workgroup of eight waves keeps W1 and W3 (512 KB at hidden 512) in its CU: all of W1 and half of W3 in registers, the
-// other half of W3 in LDS.  Wave w owns 64 rows of both; a token is two products of 4 strips of 16 rows by 8 members on
+// R: a workgroup of eight waves keeps W1 and W3 (512 KB at hidden 512) in its CU: all of W1 and a part of W3 in registers, the
+// larger part of W3 in LDS.  Wave w owns 64 rows of both; a token is two products of 4 strips of 16 rows by 8 members on
 // v_mfma_i32_16x16x64_i8 with a barrier behind each.  The 16 columns hold the 8 members twice: lanes of the first copy finish
 // strips 0 and 2, lanes of the second strips 1 and 3, so the elementwise arithmetic -- more than the products -- uses every
-// lane.  "Pipe order" (egg_gru.h) of a row is the order in which those lanes hold 64 rows' results, so what a wave stores is
+// lane.  What bounds a token (2.35 us at hidden 512) is one wave per SIMD issuing, one behind the other, the reads of operand and
+// LDS fragments, 64 MFMAs and about 300 vector instructions; the order between them changed nothing.  "Pipe order" (egg_gru.h) of a row is the order in which those lanes hold 64 rows' results, so what a wave stores is
 // operand for the next product as it stands.
 //
 // A, E, D, head: a workgroup of eight waves takes 8 members; a wave has 32 tokens of one member as the columns of
@@ -40,6 +41,10 @@ __device__ __forceinline__ int8_t *buf_g(const PipeParams &p, int H, int l, int 
 }
 __device__ __forceinline__ int8_t *buf_m(const PipeParams &p, int H, int l, int c) { return p.act + unit(p.members, H) * (4 * (p.L + 1) + 8 * p.L + 8 * l + 4 * (c & 1)); }
 
+__device__ __forceinline__ int *buf_xb(const PipeParams &p, int H, int l, int c) {      // [member][token] of a layer's E, for its D
+    return reinterpret_cast<int *>(p.act + unit(p.members, H) * (20 * p.L + 4)) + (size_t)(2 * l + (c & 1)) * p.members * C;
+}
+
 __device__ __forceinline__ const int8_t *row_bias(const PipeParams &p, int H, int l, int which) { return p.rows + (size_t)(p.V + 2 * l + which) * H; }
 __device__ __forceinline__ const int8_t *row_gain(const PipeParams &p, int H, int l, int which) { return p.rows + (size_t)(p.V + 2 * p.L + 2 * l + which) * H; }
 __device__ __forceinline__ const int8_t *row_gain_out(const PipeParams &p, int H) { return p.rows + (size_t)(p.V + 4 * p.L) * H; }
@@ -48,8 +53,10 @@ __device__ __forceinline__ const int8_t *row_gain_out(const PipeParams &p, int H
 template <int H>
 struct Rec {
     static constexpr int KS = H / 64;              // k-steps of 64, and waves with rows
-    static constexpr int REG = KS == 8 ? 4 : KS;   // k-steps of W3 in registers, the others in LDS
-    static constexpr int LDS_W = WAVES * 4 * (KS - REG) * 1024, OPERAND = KS * 512;
+    // fragments (strip s, k-step ks) of W3 that do not fit the registers beside W1: the k-steps from 4 on, and two more
+    static constexpr bool in_lds(int s, int ks) { return KS == 8 && (ks >= 4 || (ks == 3 && s < 2)); }
+    static constexpr int lds_slot(int s, int ks) { return ks >= 4 ? 4 * (ks - 4) + s : 16 + s; }
+    static constexpr int LDS_W = KS == 8 ? WAVES * 18 * 1024 : 0, OPERAND = KS * 512;
     static constexpr int LDS = LDS_W + 2 * OPERAND + 2 * 256;
 };
 // Fragments of W1 / W3: [strip of 16 rows][k-step][lane (row, k quarter)][16 bytes], 1 KB per (strip, k-step)
@@ -74,21 +81,21 @@ __device__ __forceinline__ void stage_rec(const PipeParams &p, int l, int tile, 
     const int m = lane & 7, g = lane >> 4, local = tile * 8 + m;
     const bool second = lane & 8;                  // this lane finishes strips 1 and 3
     const int tokens = min(C, p.T - chunk * C);
-    int8_t *const w3l = lds + wave * (4 * (KS - R::REG) * 1024), *const op_h = lds + R::LDS_W, *const op_g = op_h + R::OPERAND;
+    int8_t *const w3l = lds + wave * 18 * 1024 + lane * 16, *const op_h = lds + R::LDS_W, *const op_g = op_h + R::OPERAND;
     int *const xb_h = reinterpret_cast<int *>(op_g + R::OPERAND), *const xb_g = xb_h + 64;      // [member][wave]
     if (wave >= KS) {                              // hidden below 512: the waves without rows only keep the barriers
         for (int t = 0; t < 2 * tokens + 1; t++) __syncthreads();
         return;
     }
     const PipeMat m1 = p.m[6 * l + 1], m3 = p.m[6 * l + 3];
-    v4i w1[4][KS], w3[4][R::REG];
+    v4i w1[4][KS], w3[4][KS];
 #pragma unroll
     for (int s = 0; s < 4; s++)
 #pragma unroll
         for (int ks = 0; ks < KS; ks++) {
             w1[s][ks] = rec_frag(p.frag + m1.w_off, 4 * wave + s, ks, KS, lane);
-            if (ks < R::REG) w3[s][ks] = rec_frag(p.frag + m3.w_off, 4 * wave + s, ks, KS, lane);
-            else *reinterpret_cast<v4i *>(w3l + (s * (KS - R::REG) + ks - R::REG) * 1024 + lane * 16) = rec_frag(p.frag + m3.w_off, 4 * wave + s, ks, KS, lane);
+            if (!R::in_lds(s, ks)) w3[s][ks] = rec_frag(p.frag + m3.w_off, 4 * wave + s, ks, KS, lane);
+            else *reinterpret_cast<v4i *>(w3l + R::lds_slot(s, ks) * 1024) = rec_frag(p.frag + m3.w_off, 4 * wave + s, ks, KS, lane);
         }
     const uint32_t at = 64 * wave + 16 * g + (second ? 8 : 0);          // this lane's 8 bytes of a row: strips 0 and 2, or 1 and 3
     const long long pair = (p.first + local) >> 1;
@@ -97,12 +104,13 @@ __device__ __forceinline__ void stage_rec(const PipeParams &p, int l, int tile, 
                a3 = ld8(p.noise_pipe + m3.a_off + pair * H + at), b3 = ld8(p.noise_pipe + m3.b_off + pair * H + at),
                bf = ld8(row_bias(p, H, l, 0) + at), bh = ld8(row_bias(p, H, l, 1) + at);
     int8_t *const hs = p.h + ((size_t)l * p.members + local) * H + at;
-    const size_t row0 = (size_t)local * C * H + at;
-    const int8_t *const g0p = buf_g(p, H, l, 0, chunk) + row0, *const g2p = buf_g(p, H, l, 1, chunk) + row0, *const xp = buf_x(p, H, l, chunk) + row0;
-    int8_t *const op = buf_x1(p, H, l, chunk) + row0;
-    const uint32_t put = ((wave * 4 + g) * 8 + m) * 16 + (second ? 8 : 0), get = g * 128 + m * 16;
+    // uniform bases, one offset
+    const int8_t *const g0p = buf_g(p, H, l, 0, chunk), *const g2p = buf_g(p, H, l, 1, chunk), *const xp = buf_x(p, H, l, chunk);
+    int8_t *const op = buf_x1(p, H, l, chunk);
+    uint32_t off = (uint32_t)local * C * H + at;
+    const uint32_t put = ((wave * 4 + g) * 8 + m) * 16 + (second ? 8 : 0);
+    uint32_t get = g * 128 + m * 16;
     int2 h = ld8(hs);
-    int2 g0 = ld8(g0p), g2 = ld8(g2p), x = ld8(xp);
     auto publish = [&](int2 v, int8_t *operand, int2 b, int *xb) {
         *reinterpret_cast<int2 *>(operand + put) = v;
         const int part = member_sum(dot4(v.x, b.x, dot4(v.y, b.y, 0)));
@@ -117,63 +125,64 @@ __device__ __forceinline__ void stage_rec(const PipeParams &p, int l, int tile, 
     auto value = [&](int acc, int xb, int a) { return clip127((acc + (mul24(xb, a) >> p.sigma)) >> 8); };     // egg.c:167-175, shift 8
     publish(h, op_h, b1, xb_h);
     __syncthreads();
-    for (int t = 0; t < tokens; t++) {
-        // W1 h, ft = cadd(cadd(W0 x, W1 h), b_f), gated = ((ft + 127) h) >> 8 (egg.c:246-258)
-        v4i acc[4];
+    // Two passes of two strips that each read the operand again: with the four accumulators of one pass, or the operand kept,
+    // fragments go to scratch (2.8 us a token at hidden 512; 2.35 as it is, of which the matrix unit has 0.9).
+    auto product = [&](const v4i (&w)[4][KS], bool third, const int8_t *operand, auto one) {
+        v4i mine = {0, 0, 0, 0};
 #pragma unroll
-        for (int s = 0; s < 4; s++) acc[s] = v4i{0, 0, 0, 0};
+        for (int v = 0; v < 2; v++) {
+            v4i c0 = {0, 0, 0, 0}, c1 = {0, 0, 0, 0};
 #pragma unroll
-        for (int ks = 0; ks < KS; ks++) {
-            const v4i b = *reinterpret_cast<const v4i *>(op_h + ks * 512 + get);
-#pragma unroll
-            for (int s = 0; s < 4; s++) acc[s] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w1[s][ks], b, acc[s], 0, 0, 0);
-        }
-        const int xb1 = total(xb_h);
-        int ft[8];
-        {
-            int gt[8];
-#pragma unroll
-            for (int v = 0; v < 2; v++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const int a = second ? acc[2 * v + 1][e] : acc[2 * v][e];
-                    const int r = value(a, xb1, sx8(v ? a1.y : a1.x, e));
-                    ft[4 * v + e] = cadd(cadd(sx8(v ? g0.y : g0.x, e), r), sx8(v ? bf.y : bf.x, e)) + 127;
-                    gt[4 * v + e] = mul24(ft[4 * v + e], sx8(v ? h.y : h.x, e)) >> 8;
-                }
-            publish(make_int2(pack4(gt[0], gt[1], gt[2], gt[3]), pack4(gt[4], gt[5], gt[6], gt[7])), op_g, b3, xb_g);
-        }
-        const int next = t + 1 < tokens ? t + 1 : t;
-        const int2 g0n = ld8(g0p + next * H), g2n = ld8(g2p + next * H), xn = ld8(xp + next * H);
-        __syncthreads();
-        // W3 gated, ht = cadd(cadd(W2 x, W3 gated), b_h), h += ((ft + 127) (ht - h)) >> 8, x = cadd(h, x) (egg.c:260-271)
-#pragma unroll
-        for (int s = 0; s < 4; s++) acc[s] = v4i{0, 0, 0, 0};
-#pragma unroll
-        for (int ks = 0; ks < KS; ks++) {
-            const v4i b = *reinterpret_cast<const v4i *>(op_g + ks * 512 + get);
-#pragma unroll
-            for (int s = 0; s < 4; s++) {
-                const v4i w = ks < R::REG ? w3[s][ks < R::REG ? ks : 0] : *reinterpret_cast<const v4i *>(w3l + (s * (KS - R::REG) + ks - R::REG) * 1024 + lane * 16);
-                acc[s] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w, b, acc[s], 0, 0, 0);
+            for (int ks = 0; ks < KS; ks++) {
+                const v4i b = *reinterpret_cast<const v4i *>(operand + ks * 512 + get);
+                const v4i f0 = third && R::in_lds(2 * v, ks) ? *reinterpret_cast<const v4i *>(w3l + R::lds_slot(2 * v, ks) * 1024) : w[2 * v][ks],
+                          f1 = third && R::in_lds(2 * v + 1, ks) ? *reinterpret_cast<const v4i *>(w3l + R::lds_slot(2 * v + 1, ks) * 1024) : w[2 * v + 1][ks];
+                c0 = __builtin_amdgcn_mfma_i32_16x16x64_i8(f0, b, c0, 0, 0, 0);
+                c1 = __builtin_amdgcn_mfma_i32_16x16x64_i8(f1, b, c1, 0, 0, 0);
             }
-        }
-        const int xb3 = total(xb_g);
-        int hn[8], xo[8];
-#pragma unroll
-        for (int v = 0; v < 2; v++)
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                const int a = second ? acc[2 * v + 1][e] : acc[2 * v][e];
-                const int r = value(a, xb3, sx8(v ? a3.y : a3.x, e));
-                const int ht = cadd(cadd(sx8(v ? g2.y : g2.x, e), r), sx8(v ? bh.y : bh.x, e)), hv = sx8(v ? h.y : h.x, e);
-                hn[4 * v + e] = cadd(hv, mul24(ft[4 * v + e], ht - hv) >> 8);
-                xo[4 * v + e] = cadd(hn[4 * v + e], sx8(v ? x.y : x.x, e));
+                if (v == 1) one(0, e, mine[e]);
+                mine[e] = second ? c1[e] : c0[e];
             }
-        h = make_int2(pack4(hn[0], hn[1], hn[2], hn[3]), pack4(hn[4], hn[5], hn[6], hn[7]));
-        publish(h, op_h, b1, xb_h);
-        *reinterpret_cast<int2 *>(op + t * H) = make_int2(pack4(xo[0], xo[1], xo[2], xo[3]), pack4(xo[4], xo[5], xo[6], xo[7]));
-        g0 = g0n; g2 = g2n; x = xn;
+            asm volatile("" : "+v"(get));          // the operand is read again for the other two strips, not kept
+        }
+#pragma unroll
+        for (int e = 0; e < 4; e++) one(1, e, mine[e]);
+    };
+    int2 g0 = ld8(g0p + off);
+    __builtin_amdgcn_s_waitcnt(0x0F70);            // vmcnt(0) here, so that no wait inside the loop has to allow for it
+    for (int t = 0; t < tokens; t++, off += H) {
+        int2 ft, xo;
+        {   // W1 h, ft = cadd(cadd(W0 x, W1 h), b_f), gated = ((ft + 127) h) >> 8 (egg.c:246-258)
+            const int xb1 = total(xb_h);
+            int f[4], gt[4];
+            int2 gated;
+            product(w1, false, op_h, [&](int v, int e, int a) {
+                const int r = value(a, xb1, sx8(v ? a1.y : a1.x, e));
+                f[e] = cadd(cadd(sx8(v ? g0.y : g0.x, e), r), sx8(v ? bf.y : bf.x, e));
+                gt[e] = mul24(f[e] + 127, sx8(v ? h.y : h.x, e)) >> 8;
+                if (e == 3) { (v ? ft.y : ft.x) = pack4(f[0], f[1], f[2], f[3]); (v ? gated.y : gated.x) = pack4(gt[0], gt[1], gt[2], gt[3]); }
+            });
+            publish(gated, op_g, b3, xb_g);
+        }
+        __syncthreads();
+        {   // W3 gated, ht = cadd(cadd(W2 x, W3 gated), b_h), h += ((ft + 127) (ht - h)) >> 8, x = cadd(h, x) (egg.c:260-271)
+            // the next token's loads go in front of this token's store: a wait for a load waits for the stores before it
+            const int2 g2 = ld8(g2p + off), x = ld8(xp + off);
+            g0 = ld8(g0p + off + (t + 1 < tokens ? H : 0));
+            const int xb3 = total(xb_g);
+            int hv[4], xv[4];
+            product(w3, true, op_g, [&](int v, int e, int a) {
+                const int r = value(a, xb3, sx8(v ? a3.y : a3.x, e));
+                const int ht = cadd(cadd(sx8(v ? g2.y : g2.x, e), r), sx8(v ? bh.y : bh.x, e)), h0 = sx8(v ? h.y : h.x, e);
+                hv[e] = cadd(h0, mul24(sx8(v ? ft.y : ft.x, e) + 127, ht - h0) >> 8);
+                xv[e] = cadd(hv[e], sx8(v ? x.y : x.x, e));
+                if (e == 3) { (v ? h.y : h.x) = pack4(hv[0], hv[1], hv[2], hv[3]); (v ? xo.y : xo.x) = pack4(xv[0], xv[1], xv[2], xv[3]); }
+            });
+            publish(h, op_h, b1, xb_h);
+        }
+        *reinterpret_cast<int2 *>(op + off) = xo;
         __syncthreads();
     }
     *reinterpret_cast<int2 *>(hs) = h;
@@ -236,6 +245,12 @@ __device__ __forceinline__ void load_row(v4i (&x)[NK], const int8_t *row, int g)
 #pragma unroll
     for (int ks = 0; ks < NK; ks++) x[ks] = *reinterpret_cast<const v4i *>(row + 32 * ks + 16 * g);
 }
+// the same from the MLP's intermediate, which is kept in the order of these loads: [member][k-step][half][token][16 bytes]
+template <int NK>
+__device__ __forceinline__ void load_ops(v4i (&x)[NK], const int8_t *ops, uint32_t lane16) {      // ops: uniform
+#pragma unroll
+    for (int ks = 0; ks < NK; ks++) x[ks] = *reinterpret_cast<const v4i *>(ops + 1024 * ks + lane16);
+}
 template <int NK>
 __device__ __forceinline__ int noise_dot(const v4i (&x)[NK], const int8_t *b, int g) {
     int s = 0;
@@ -267,11 +282,22 @@ __device__ __forceinline__ void norm(v4i (&x)[NK], const int8_t *gains, int g) {
         }
     }
 }
+// the accumulators of a block start from the rank-1 term, (x.B A ns) >> sigma (egg.c:167-175); xbn: x.B times the member's sign
+__device__ __forceinline__ void begin_block(v16i (&acc)[2], int xbn, const v4i &a0, const v4i &a1, int sigma) {
+#pragma unroll
+    for (int r = 0; r < 16; r++) { acc[0][r] = mul24(xbn, sx8(a0[r >> 2], r & 3)) >> sigma; acc[1][r] = mul24(xbn, sx8(a1[r >> 2], r & 3)) >> sigma; }
+}
+__device__ __forceinline__ v4i clamped(const v16i &acc, int shift) {
+    v4i o;
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+        o[q] = pack4(clip127(acc[4 * q] >> shift), clip127(acc[4 * q + 1] >> shift), clip127(acc[4 * q + 2] >> shift), clip127(acc[4 * q + 3] >> shift));
+    return o;
+}
 // a block's 64 results of the lane's token, its half: the 16-byte pieces g and g + 2 of the row's 64-group in pipe order
 struct Pieces { v4i lo, hi; };
-__device__ __forceinline__ Pieces finish_block(const v16i (&acc)[2], int xb, const int8_t *a, int ns, int sigma, int shift, int g) {
-    const v4i r0 = gru_finish(acc[0], xb, *reinterpret_cast<const v4i *>(a + 16 * g), ns, sigma, shift),
-              r1 = gru_finish(acc[1], xb, *reinterpret_cast<const v4i *>(a + 32 + 16 * g), ns, sigma, shift);
+__device__ __forceinline__ Pieces finish_block(const v16i (&acc)[2], int shift) {
+    const v4i r0 = clamped(acc[0], shift), r1 = clamped(acc[1], shift);
     Pieces o;
     o.lo = v4i{r0[0], r1[0], r0[2], r1[2]};
     o.hi = v4i{r0[1], r1[1], r0[3], r1[3]};
@@ -296,7 +322,7 @@ __device__ __forceinline__ long long stream_pos(const PipeParams &p, int member)
     const long long stride = p.data_len / (p.population / 2);                    // egg.c:553-554
     return (p.start_idx + (long long)(member >> 1) * stride) % (p.data_len - p.T);
 }
-__device__ __forceinline__ void clear(v16i (&acc)[2]) { zero_acc<2>(acc); }
+__device__ __forceinline__ v4i ld16(const int8_t *p) { return *reinterpret_cast<const v4i *>(p); }
 
 struct Tile { int local, member, ns, g, lane, token; long long pair; };
 __device__ __forceinline__ Tile tile_of(const PipeParams &p, int unit8, int chunk) {
@@ -325,15 +351,17 @@ __device__ __forceinline__ void stage_a(const PipeParams &p, int l, int unit8, i
     } else
         load_row<NK>(x, buf_x(p, H, l, chunk) + row, t.g);
     norm<NK>(x, row_gain(p, H, l, 0), t.g);
-    const int xb0 = sum_halves(noise_dot<NK>(x, p.noise_pipe + m0.b_off + t.pair * H, t.g)), xb2 = sum_halves(noise_dot<NK>(x, p.noise_pipe + m2.b_off + t.pair * H, t.g));
+    const int xb0 = t.ns * sum_halves(noise_dot<NK>(x, p.noise_pipe + m0.b_off + t.pair * H, t.g)),
+              xb2 = t.ns * sum_halves(noise_dot<NK>(x, p.noise_pipe + m2.b_off + t.pair * H, t.g));
     for (int b = 0; b < 2 * NB; b++) {
         const int which = b >= NB, nb = which ? b - NB : b;
+        const int8_t *a = p.noise_slot + (which ? m2.a_off : m0.a_off) + t.pair * H + 64 * nb + 16 * t.g;
+        const v4i a0 = ld16(a), a1 = ld16(a + 32);
         const int8_t *w = blocks.take();
         v16i acc[2];
-        clear(acc);
+        begin_block(acc, which ? xb2 : xb0, a0, a1, p.sigma);
         multiply<NK>(acc, x, w, t.lane);
-        const Pieces o = finish_block(acc, which ? xb2 : xb0, p.noise_slot + (which ? m2.a_off : m0.a_off) + t.pair * H + 64 * nb, t.ns, p.sigma, 8, t.g);
-        store_pieces(buf_g(p, H, l, which, chunk) + row + 64 * nb, o, t.g);
+        store_pieces(buf_g(p, H, l, which, chunk) + row + 64 * nb, finish_block(acc, 8), t.g);
     }
 }
 template <int H>
@@ -347,15 +375,24 @@ __device__ __forceinline__ void stage_e(const PipeParams &p, int l, int unit8, i
     v4i x[NK];
     load_row<NK>(x, buf_x1(p, H, l, chunk) + row * H, t.g);
     norm<NK>(x, row_gain(p, H, l, 1), t.g);
-    const int xb = sum_halves(noise_dot<NK>(x, p.noise_pipe + m.b_off + t.pair * H, t.g));
+    const int xb = t.ns * sum_halves(noise_dot<NK>(x, p.noise_pipe + m.b_off + t.pair * H, t.g));
+    const int8_t *a = p.noise_slot + m.a_off + t.pair * 4 * H + 16 * t.g, *bd = p.noise_pipe + p.m[6 * l + 5].b_off + t.pair * 4 * H + 16 * t.g;
+    int8_t *out = buf_m(p, H, l, chunk) + (size_t)t.local * C * 4 * H + t.lane * 16;
+    int xbd = 0;                                   // the projection's x . B, of the results as they leave
     for (int b = 0; b < NB; b++) {
+        const v4i a0 = ld16(a + 64 * b), a1 = ld16(a + 64 * b + 32), n0 = ld16(bd + 64 * b), n1 = ld16(bd + 64 * b + 32);
         const int8_t *w = blocks.take();
         v16i acc[2];
-        clear(acc);
+        begin_block(acc, xb, a0, a1, p.sigma);
         multiply<NK>(acc, x, w, t.lane);
-        const Pieces o = finish_block(acc, xb, p.noise_slot + m.a_off + t.pair * 4 * H + 64 * b, t.ns, p.sigma, 8, t.g);
-        store_pieces(buf_m(p, H, l, chunk) + row * 4 * H + 64 * b, o, t.g);
+        const Pieces o = finish_block(acc, 8);
+#pragma unroll
+        for (int q = 0; q < 4; q++) xbd = dot4(o.lo[q], n0[q], dot4(o.hi[q], n1[q], xbd));
+        *reinterpret_cast<v4i *>(out + 2048 * b) = o.lo;
+        *reinterpret_cast<v4i *>(out + 2048 * b + 1024) = o.hi;
     }
+    xbd = t.ns * sum_halves(xbd);
+    if (t.g == 0) buf_xb(p, H, l, chunk)[row] = xbd;
 }
 template <int H>
 __device__ __forceinline__ void stage_d(const PipeParams &p, int l, int unit8, int chunk, int8_t *lds) {
@@ -365,23 +402,31 @@ __device__ __forceinline__ void stage_d(const PipeParams &p, int l, int unit8, i
     Blocks<H> blocks;
     blocks.begin(lds, p.frag + m.w_off, 4 * NB, nullptr, 0);
     const size_t row = (size_t)t.local * C + (t.lane & 31);
-    const int8_t *in = buf_m(p, H, l, chunk) + row * 4 * H;
-    int xb = 0;
+    const uint32_t lane16 = t.lane * 16;
+    const int8_t *in = buf_m(p, H, l, chunk) + (size_t)t.local * C * 4 * H, *res = buf_x1(p, H, l, chunk) + row * H + 16 * t.g,
+                 *a = p.noise_slot + m.a_off + t.pair * H + 16 * t.g;
+    int8_t *out = buf_x(p, H, l + 1, chunk) + row * H;
+    const int xb = buf_xb(p, H, l, chunk)[row];
+    // a quarter of the input row at a time, the next one on its way while a block of weights is multiplied with this one
+    v4i x0[NK], x1[NK];
+    load_ops<NK>(x0, in, lane16);
     for (int b = 0; b < NB; b++) {
+        const v4i a0 = ld16(a + 64 * b), a1 = ld16(a + 64 * b + 32), r0 = ld16(res + 64 * b), r1 = ld16(res + 64 * b + 32);
         v16i acc[2];
-        clear(acc);
-        for (int kc = 0; kc < 4; kc++) {
-            v4i x[NK];
-            load_row<NK>(x, in + kc * H, t.g);
-            if (b == 0) xb += noise_dot<NK>(x, p.noise_pipe + m.b_off + t.pair * 4 * H + kc * H, t.g);
-            multiply<NK>(acc, x, blocks.take(), t.lane);
+        begin_block(acc, xb, a0, a1, p.sigma);
+#pragma unroll
+        for (int kc = 0; kc < 4; kc += 2) {
+            const int8_t *w = blocks.take();
+            load_ops<NK>(x1, in + (kc + 1) * NK * 1024, lane16);
+            multiply<NK>(acc, x0, w, t.lane);
+            w = blocks.take();
+            load_ops<NK>(x0, in + ((kc + 2) & 3) * NK * 1024, lane16);
+            multiply<NK>(acc, x1, w, t.lane);
         }
-        if (b == 0) xb = sum_halves(xb);
-        Pieces o = finish_block(acc, xb, p.noise_slot + m.a_off + t.pair * H + 64 * b, t.ns, p.sigma, 9, t.g);
-        const int8_t *res = buf_x1(p, H, l, chunk) + row * H + 64 * b;
-        o.lo = cadd16(o.lo, *reinterpret_cast<const v4i *>(res + 16 * t.g));
-        o.hi = cadd16(o.hi, *reinterpret_cast<const v4i *>(res + 32 + 16 * t.g));
-        store_pieces(buf_x(p, H, l + 1, chunk) + row * H + 64 * b, o, t.g);
+        Pieces o = finish_block(acc, 9);
+        o.lo = cadd16(o.lo, r0);
+        o.hi = cadd16(o.hi, r1);
+        store_pieces(out + 64 * b, o, t.g);
     }
 }
 // output norm, logits (egg.c:288-294), loss (egg.c:321-330)
@@ -397,17 +442,19 @@ __device__ __forceinline__ void stage_head(const PipeParams &p, int unit8, int c
     v4i x[NK];
     load_row<NK>(x, buf_x(p, H, p.L, chunk) + ((size_t)t.local * C + (t.lane & 31)) * H, t.g);
     norm<NK>(x, row_gain_out(p, H), t.g);
-    const int xb = sum_halves(noise_dot<NK>(x, p.noise_pipe + m.b_off + t.pair * H, t.g));
+    const int xb = t.ns * sum_halves(noise_dot<NK>(x, p.noise_pipe + m.b_off + t.pair * H, t.g));
+    const int8_t *a = p.noise_slot + m.a_off + t.pair * p.V + 16 * t.g;
     const int target = p.data[stream_pos(p, t.member) + t.token + 1];
     int sum_exp = 0, tl = 0;
     for (int b = 0; b < p.V / 64; b++) {
+        const v4i a0 = ld16(a + 64 * b), a1 = ld16(a + 64 * b + 32);
         const int8_t *w = blocks.take();
         v16i acc[2];
-        clear(acc);
+        begin_block(acc, xb, a0, a1, p.sigma);
         multiply<NK>(acc, x, w, t.lane);
 #pragma unroll
         for (int half = 0; half < 2; half++) {
-            const v4i r = gru_finish(acc[half], xb, *reinterpret_cast<const v4i *>(p.noise_slot + m.a_off + t.pair * p.V + 64 * b + 32 * half + 16 * t.g), t.ns, p.sigma, 8);
+            const v4i r = clamped(acc[half], 8);
 #pragma unroll
             for (int q = 0; q < 4; q++)
 #pragma unroll
@@ -495,7 +542,7 @@ hipError_t forward(const PipeParams &p, hipStream_t s) {
 
 }  // namespace
 
-size_t gru_pipe_act_bytes(int members, int H, int L) { return unit(members, H) * (20 * L + 4); }
+size_t gru_pipe_act_bytes(int members, int H, int L) { return unit(members, H) * (20 * L + 4) + (size_t)2 * L * members * C * sizeof(int); }
 size_t gru_pipe_rows_bytes(int H, int L, int V) { return (size_t)(V + 4 * L + 1) * H; }
 hipError_t gru_pipe_prepare(int H) {
 #define EGG_PREP(HH) hipFuncSetAttribute(reinterpret_cast<const void *>(&k_gru_tick<HH>), hipFuncAttributeMaxDynamicSharedMemorySize, tick_lds<HH>())
