@@ -34,32 +34,69 @@ struct GruParams {
 };
 
 __device__ __forceinline__ uint32_t xorshift32(uint32_t &x) { x ^= x << 13; x ^= x >> 17; x ^= x << 5; return x; }
-__device__ __forceinline__ int slot_pos(int n) { int w = n & 31; return (n & ~31) + 16 * ((w >> 2) & 1) + 4 * (w >> 3) + (w & 3); }
+constexpr int NOISE_SEG = 64;
+
+// xorshift32 is linear over GF(2), so 80 << k steps at once are a 32 x 32 matrix: jump.col[k][j] is what they make of 1 << j
+struct Jump {
+    uint32_t col[6][32];
+    constexpr Jump() : col() {
+        for (int j = 0; j < 32; j++) {
+            uint32_t x = 1u << j;
+            for (int s = 0; s < NOISE_SEG / 16 * 20; s++) { x ^= x << 13; x ^= x >> 17; x ^= x << 5; }
+            col[0][j] = x;
+        }
+        for (int k = 1; k < 6; k++)
+            for (int j = 0; j < 32; j++) {
+                uint32_t x = 0;
+                for (int b = 0; b < 32; b++) if (col[k - 1][j] >> b & 1) x ^= col[k - 1][b];
+                col[k][j] = x;
+            }
+    }
+};
+__constant__ const Jump jump;
 
 // gen_noise_vector_neon (egg.c:87-105) for every (matrix, pair): A[rows] then B[cols] from one stream seeded
 // step_seed + pair + seed_off.  Writes the vectors in slot order and in pipe order, [pair][count] each, and the raw panels
-// for the vote.
-__global__ void k_gru_noise(const GruMat *mats, int n_mats, int pairs, int pairs_pad, uint32_t step_seed,
-                            int8_t *noise, int8_t *npipe, int8_t *panels) {
-    int id = blockIdx.x * blockDim.x + threadIdx.x;
-    if (id >= n_mats * pairs) return;
-    const GruMat m = mats[id / pairs]; const int p = id % pairs;
+// for the vote.  A thread replays 64 values (80 steps) of a pair's stream: its start is reached by jumping, one matrix for each bit of
+// the segment's number, which is the same for all threads of the block.  At the reference's sizes (64 pairs, 25 matrices)
+// that is 28,800 threads where one thread to a stream was 1,600 with chains of up to 3,200 steps: 250 -> 8 us.
+__global__ void __launch_bounds__(64) k_gru_noise(const GruMat *mats, int pairs, int pairs_pad, uint32_t step_seed,
+                                                  int8_t *noise, int8_t *npipe, int8_t *panels) {
+    const GruMat m = mats[blockIdx.z];
+    const int p = blockIdx.x * 64 + threadIdx.x, seg = blockIdx.y;
+    if (p >= pairs || seg * NOISE_SEG >= m.rows + m.cols) return;
     uint32_t rng = step_seed + (uint32_t)p + (uint32_t)m.seed_off;
-    for (int part = 0; part < 2; part++) {
-        const int count = part ? m.cols : m.rows;
-        int8_t *vec = noise + (part ? m.b_off + (long long)p * m.cols : m.a_off + (long long)p * m.rows);
-        int8_t *pvec = npipe + (part ? m.b_off + (long long)p * m.cols : m.a_off + (long long)p * m.rows);
-        int8_t *pan = panels + (part ? m.pb_off : m.pa_off);
-        for (int i = 0; i < count; i += 16) {
-            xorshift32(rng); xorshift32(rng); xorshift32(rng); xorshift32(rng);
-            for (int jj = 0; jj < 16 && i + jj < count; jj++) {
-                uint32_t r = xorshift32(rng);
-                int v = (int)((r >> 1) & 31u); if (!(r & 1)) v = -v;
-                vec[slot_pos(i + jj)] = (int8_t)v;
-                pvec[pipe_pos(i + jj)] = (int8_t)v;
-                pan[(long long)(i + jj) * pairs_pad + p] = (int8_t)v;
-            }
+#pragma unroll 1
+    for (int k = 0; k < 6; k++)
+        if (seg >> k & 1) {
+            uint32_t x = 0;
+#pragma unroll
+            for (int j = 0; j < 32; j++) x ^= jump.col[k][j] & (uint32_t)((int32_t)(rng << (31 - j)) >> 31);
+            rng = x;
         }
+    const bool second = seg * NOISE_SEG >= m.rows;
+    const int at = seg * NOISE_SEG - (second ? m.rows : 0);
+    const long long out = (second ? m.b_off + (long long)p * m.cols : m.a_off + (long long)p * m.rows) + at;
+    int8_t *pan = panels + (second ? m.pb_off : m.pa_off) + (long long)at * pairs_pad + p;
+    int d[NOISE_SEG / 4];                                       // natural order
+#pragma unroll
+    for (int i = 0; i < NOISE_SEG; i++) {
+        if (i % 16 == 0) { xorshift32(rng); xorshift32(rng); xorshift32(rng); xorshift32(rng); }
+        const uint32_t r = xorshift32(rng);
+        const int n = (int)((r >> 1) & 31u), v = r & 1 ? n : -n;
+        d[i / 4] = i % 4 ? d[i / 4] | (v & 255) << 8 * (i % 4) : v & 255;
+        pan[(long long)i * pairs_pad] = (int8_t)v;
+    }
+#pragma unroll
+    for (int q = 0; q < NOISE_SEG / 16; q++) {
+        v4i slot, pipe;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            slot[e] = d[8 * (q >> 1) + 2 * e + (q & 1)];
+            pipe[e] = d[pipe_dword(4 * q + e)];
+        }
+        reinterpret_cast<v4i *>(noise + out)[q] = slot;
+        reinterpret_cast<v4i *>(npipe + out)[q] = pipe;
     }
 }
 
@@ -340,17 +377,23 @@ __global__ void __launch_bounds__(GRU_THREADS) k_gru_forward(GruParams p) {
     if (wave == 0 && g == 0) p.loss[member] = loss;
 }
 
-// A panel *= fitness of the pair (A_T[r][p] = A[r] * f, egg.c:362-366)
-__global__ void k_gru_scale_panel(int8_t *panel, long long n, int pairs_pad, int pairs, const int32_t *fit) {
-    long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    int pp = (int)(i % pairs_pad);
-    panel[i] = (pp < pairs) ? (int8_t)(panel[i] * fit[pp]) : (int8_t)0;
+// the A panels of all matrices *= fitness of the pair (A_T[r][p] = A[r] * f, egg.c:362-366)
+__global__ void k_gru_scale_panels(const GruMat *mats, int8_t *panels, int pairs_pad, int pairs, const int32_t *fit) {
+    const GruMat m = mats[blockIdx.y];
+    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= (long long)m.rows * pairs_pad) return;
+    const int pp = (int)(i % pairs_pad);
+    panels[m.pa_off + i] = (pp < pairs) ? (int8_t)(panels[m.pa_off + i] * fit[pp]) : (int8_t)0;
 }
 
-// update_matrix (egg.c:332-409): vote[r][c] = sum_p A_T[r][p] B_T[c][p] on the MFMA, then the +-1 threshold rule
-__global__ void __launch_bounds__(256) k_gru_vote_update(int8_t *W, const int8_t *pa, const int8_t *pb, int rows, int cols,
-                                                        int pairs_pad, int threshold) {
+// update_matrix (egg.c:332-409) of all matrices: vote[r][c] = sum_p A_T[r][p] B_T[c][p] on the MFMA, then the +-1 threshold
+// rule.  One launch for the 25 matrices of the reference's sizes and one for their panels, where each matrix had two of its
+// own: 400 -> 24 us a step.
+__global__ void __launch_bounds__(256) k_gru_vote_update(const GruMat *mats, int8_t *model, const int8_t *panels, int pairs_pad, int threshold) {
+    const GruMat m = mats[blockIdx.y];
+    const int rows = m.rows, cols = m.cols;
+    int8_t *W = model + m.w_off;
+    const int8_t *pa = panels + m.pa_off, *pb = panels + m.pb_off;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 5, j = lane & 31;
     const int tiles_c = cols / 32, tile = blockIdx.x * 4 + wave;
     if (tile >= (rows / 32) * tiles_c) return;
@@ -581,8 +624,9 @@ extern "C" int egg_gru_step(egg_gru_ctx *ctx, const uint8_t *d_data, int64_t dat
     if (!ctx || !d_data || data_len <= ctx->cfg.seq_len + 1) return gfail(ctx, EGG_E_INVALID, "egg_gru_step arguments");
     const egg_gru_config &c = ctx->cfg;
     const int pairs = c.population / 2, nm = (int)ctx->mats.size();
-    hipLaunchKernelGGL(k_gru_noise, dim3((nm * pairs + 63) / 64), dim3(64), 0, ctx->stream, ctx->d_mats, nm, pairs, ctx->pairs_pad,
-                       step_seed, ctx->d_noise, ctx->d_npipe, ctx->d_panels);
+    static_assert(5 * 512 / NOISE_SEG <= 64, "six bits of segments");
+    hipLaunchKernelGGL(k_gru_noise, dim3((pairs + 63) / 64, 5 * c.hidden / NOISE_SEG, nm), dim3(64), 0, ctx->stream, ctx->d_mats, pairs,
+                       ctx->pairs_pad, step_seed, ctx->d_noise, ctx->d_npipe, ctx->d_panels);
     { const int rc = gru_refresh_frag(ctx); if (rc) return rc; }
     GruParams p;
     p.mats = ctx->d_mats; p.model = ctx->d_model; p.frag = ctx->d_frag; p.noise = ctx->d_noise;
@@ -606,14 +650,12 @@ extern "C" int egg_gru_step(egg_gru_ctx *ctx, const uint8_t *d_data, int64_t dat
     // pair fitness (egg.c:559-561) has the same rule as the transformer's
     GTRY(egg_launch_fitness(ctx->d_loss, ctx->d_fit, pairs, ctx->stream));
     if (do_update) {
-        for (const GruMat &m : ctx->mats) {
-            long long n = (long long)m.rows * ctx->pairs_pad;
-            hipLaunchKernelGGL(k_gru_scale_panel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, ctx->stream, ctx->d_panels + m.pa_off, n,
-                               ctx->pairs_pad, pairs, ctx->d_fit);
-            int tiles = (m.rows / 32) * (m.cols / 32);
-            hipLaunchKernelGGL(k_gru_vote_update, dim3((tiles + 3) / 4), dim3(256), 0, ctx->stream, ctx->d_model + m.w_off,
-                               ctx->d_panels + m.pa_off, ctx->d_panels + m.pb_off, m.rows, m.cols, ctx->pairs_pad, c.update_threshold);
-        }
+        int most_rows = 0, most_tiles = 0;
+        for (const GruMat &m : ctx->mats) { most_rows = std::max(most_rows, m.rows); most_tiles = std::max(most_tiles, (m.rows / 32) * (m.cols / 32)); }
+        hipLaunchKernelGGL(k_gru_scale_panels, dim3((unsigned)(((long long)most_rows * ctx->pairs_pad + 255) / 256), nm), dim3(256), 0, ctx->stream,
+                           ctx->d_mats, ctx->d_panels, ctx->pairs_pad, pairs, ctx->d_fit);
+        hipLaunchKernelGGL(k_gru_vote_update, dim3((most_tiles + 3) / 4, nm), dim3(256), 0, ctx->stream, ctx->d_mats, ctx->d_model, ctx->d_panels,
+                           ctx->pairs_pad, c.update_threshold);
         GTRY(hipGetLastError());
         gru_weights_changed(ctx);
         return gru_refresh_frag(ctx);
