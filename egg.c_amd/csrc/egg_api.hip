@@ -57,6 +57,12 @@ struct egg_ctx {
     int8_t *d_x = nullptr, *d_q = nullptr, *d_k = nullptr, *d_v = nullptr, *d_ao = nullptr;
     unsigned long long *d_loss_acc = nullptr, *d_counter = nullptr;
     int32_t *d_loss = nullptr, *d_fit = nullptr;
+    bool acc_dirty = false;         // the loss sums may hold something (a forward ended early): the next one clears them
+    // what the host reads after a step, written by the step itself: changed weights | losses | fitness
+    unsigned long long *h_result = nullptr;
+    HostOut out;
+    int32_t *h_loss() { return reinterpret_cast<int32_t *>(h_result + 2); }
+    int32_t *h_fit() { return h_loss() + cfg.population; }
     Scalars *d_scal = nullptr;
     // votes and optimizer step (egg_votes.hip): the noise table, and the matrices' descriptors in lists that one launch walks
     NoiseTable noise = {nullptr, 0, 0, nullptr, nullptr, 0, nullptr};
@@ -269,6 +275,8 @@ static void free_all(egg_ctx *ctx) {
                     ctx->d_overlay, ctx->d_overlay_q, ctx->d_flags, ctx->d_ov_segs};
     for (void *p : ptrs) if (p) (void)hipFree(p);
     if (ctx->h_dec_fail) (void)hipHostFree(ctx->h_dec_fail);
+    if (ctx->h_result) (void)hipHostFree(ctx->h_result);
+    egg_host_out_destroy(&ctx->out);
     for (auto &sp : ctx->spans) { (void)hipEventDestroy(sp.a); (void)hipEventDestroy(sp.b); }
     if (ctx->gexec) (void)hipGraphExecDestroy(ctx->gexec);
     if (ctx->graph) (void)hipGraphDestroy(ctx->graph);
@@ -440,10 +448,13 @@ extern "C" int egg_ctx_create(const egg_config *cfg, egg_ctx **out) {
     size_t act_bytes = (size_t)chunk * c.seq_len * c.hidden;
     CR(hipMalloc(&ctx->d_x, act_bytes)); CR(hipMalloc(&ctx->d_q, act_bytes)); CR(hipMalloc(&ctx->d_k, act_bytes));
     CR(hipMalloc(&ctx->d_v, act_bytes)); CR(hipMalloc(&ctx->d_ao, act_bytes));
-    CR(hipMalloc(&ctx->d_loss_acc, (size_t)c.population * 8)); CR(hipMalloc(&ctx->d_counter, 8));
-    CR(hipMemset(ctx->d_counter, 0, 8));
+    CR(hipMalloc(&ctx->d_loss_acc, (size_t)c.population * 8)); CR(hipMalloc(&ctx->d_counter, 16));     // and the loss sum of a generation
+    CR(hipMemset(ctx->d_loss_acc, 0, (size_t)c.population * 8)); CR(hipMemset(ctx->d_counter, 0, 16));
     CR(hipMalloc(&ctx->d_loss, (size_t)c.population * 4)); CR(hipMalloc(&ctx->d_fit, (size_t)(c.population / 2) * 4));
     CR(hipMalloc(&ctx->d_scal, sizeof(Scalars)));
+    CR(hipHostMalloc(reinterpret_cast<void **>(&ctx->h_result), 16 + (size_t)c.population * 4 + (size_t)(c.population / 2) * 4, hipHostMallocCoherent));
+    memset(ctx->h_result, 0, 16 + (size_t)c.population * 4 + (size_t)(c.population / 2) * 4);
+    CR(egg_host_out_create(&ctx->out, (size_t)std::max<int64_t>(ctx->L.total, ctx->state_bytes)));
     // noise table: the rows of the widest side of any matrix (4 * hidden, or the embedding's vocabulary), every layer's seeds
     ctx->noise.pairs_pad = ((c.population / 2) + 127) / 128 * 128;
     ctx->noise.rows = std::max(4 * c.hidden, c.vocab);
@@ -536,8 +547,7 @@ extern "C" int egg_model_upload(egg_ctx *ctx, const void *h, size_t bytes) {
 }
 extern "C" int egg_model_download(egg_ctx *ctx, void *h, size_t bytes) {
     if (!ctx || !h || (int64_t)bytes != ctx->L.total) return fail(ctx, EGG_E_INVALID, "model size mismatch");
-    HIP_TRY(hipStreamSynchronize(ctx->stream));
-    HIP_TRY(hipMemcpy(h, ctx->d_model, bytes, hipMemcpyDeviceToHost));
+    HIP_TRY(egg_host_out(ctx->out, h, ctx->d_model, bytes, ctx->stream));
     return EGG_OK;
 }
 // ------------------------------------------------------------------ ternary-packed model (no reference counterpart)
@@ -616,8 +626,7 @@ extern "C" int egg_opt_state_upload(egg_ctx *ctx, const void *h, size_t bytes) {
 }
 extern "C" int egg_opt_state_download(egg_ctx *ctx, void *h, size_t bytes) {
     if (!ctx || !h || (int64_t)bytes != ctx->state_bytes) return fail(ctx, EGG_E_INVALID, "state size mismatch");
-    HIP_TRY(hipStreamSynchronize(ctx->stream));
-    HIP_TRY(hipMemcpy(h, ctx->d_state, bytes, hipMemcpyDeviceToHost));
+    HIP_TRY(egg_host_out(ctx->out, h, ctx->d_state, bytes, ctx->stream));
     return EGG_OK;
 }
 extern "C" int egg_opt_state_reset(egg_ctx *ctx) {
@@ -789,26 +798,40 @@ static int forward_chunk(egg_ctx *ctx, const uint8_t *d_data, int64_t len, const
     {
         HeadParams p; memset(&p, 0, sizeof(p)); p.c = f;
         p.ln_w = M + L.ln_f; p.ln_b = M + L.ln_f_bias; p.embedding_frag = F + L.embedding; p.x = ctx->d_x;
-        p.loss_acc = ctx->d_loss_acc; p.logits_tap = ctx->logits_override ? ctx->logits_override : (taps ? ctx->d_tap_logits : nullptr);
+        p.loss_acc = ctx->logits_override ? ctx->d_counter + 1 : ctx->d_loss_acc; p.logits_tap = ctx->logits_override ? ctx->logits_override : (taps ? ctx->d_tap_logits : nullptr);
         if (Q) { p.q_ln_w = Q + L.ln_f; p.q_ln_b = Q + L.ln_f_bias; p.q_emb = Q + L.embedding; }
         { SpanScope span(ctx, EGG_K_HEAD); HIP_TRY(egg_launch_head(p, s)); }
     }
     return EGG_OK;
 }
 
+// Every forward leaves the loss sums of its members at zero; only one that ended early does not.  (Cleared inside a
+// caller's capture, they are cleared when that graph runs, not now.)
+static int clear_loss_sums(egg_ctx *ctx) {
+    if (!ctx->acc_dirty) return EGG_OK;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    HIP_TRY(hipStreamIsCapturing(ctx->stream, &st));
+    HIP_TRY(egg_launch_zero_u64(ctx->d_loss_acc, ctx->cfg.population, ctx->stream));
+    ctx->acc_dirty = st != hipStreamCaptureStatusNone;
+    return EGG_OK;
+}
+// in_step: the losses are taken from the sums by what follows
 static int forward_range(egg_ctx *ctx, const uint8_t *d_data, int64_t len, const int64_t *d_start, const uint32_t *d_seed,
-                         int pop_offset, int pop_count, int32_t *d_loss) {
+                         int pop_offset, int pop_count, int32_t *d_loss, bool in_step = false) {
     const egg_config &c = ctx->cfg;
     if (!d_data || !d_loss || pop_offset < 0 || pop_count < 1 || pop_offset + pop_count > c.population)
         return fail(ctx, EGG_E_INVALID, "population range");
     if (len <= c.seq_len + 1) return fail(ctx, EGG_E_INVALID, "data_len must exceed seq_len + 1");
-    HIP_TRY(egg_launch_zero_u64(ctx->d_loss_acc + pop_offset, pop_count, ctx->stream));
+    if (int rc = clear_loss_sums(ctx)) return rc;
+    const bool dirty = ctx->acc_dirty;
+    ctx->acc_dirty = true;
     for (int done = 0; done < pop_count; done += ctx->chunk) {
         int nm = pop_count - done < ctx->chunk ? pop_count - done : ctx->chunk;
         int rc = forward_chunk(ctx, d_data, len, d_start, d_seed, pop_offset + done, nm);
         if (rc) return rc;
     }
-    HIP_TRY(egg_launch_loss_finalize(ctx->d_loss_acc, d_loss, pop_offset, pop_count, ctx->stream));
+    if (!in_step) HIP_TRY(egg_launch_loss_finalize(ctx->d_loss_acc, d_loss, pop_offset, pop_count, ctx->stream));
+    ctx->acc_dirty = dirty;
     return EGG_OK;
 }
 
@@ -838,14 +861,14 @@ static UpdLaunch make_upd(egg_ctx *ctx, const egg_ctx::MatList &l, const int32_t
     p.mat = ctx->d_mat + l.first; p.n_mat = l.count; p.tiles = l.tiles;
     p.noise = ctx->noise; p.fit = d_fit; p.pairs = c.population / 2; p.d_lr = d_lr;
     p.beta1 = c.adam_beta1; p.beta2 = c.adam_beta2; p.eps = c.adam_eps; p.wd = c.adam_weight_decay; p.muon_momentum = c.muon_momentum;
-    p.counter = ctx->d_counter;
+    p.counter = ctx->d_counter; p.h_counter = ctx->h_result;
     return p;
 }
 // the part of the noise table that one tensor reads, and the fitness masks
 static int table_of_tensor(egg_ctx *ctx, int id, const int32_t *d_fit, const uint32_t *d_seed) {
     const egg_config &c = ctx->cfg; const egg_tensor_info &t = ctx->tensors[id];
     const int lo = t.seed_base + std::min(t.off_a, t.off_b), hi = t.seed_base + std::max(t.off_a, t.off_b) + ctx->noise.pairs_pad;
-    HIP_TRY(egg_launch_noise_table(ctx->noise, d_seed, d_fit, c.population / 2, noise_word(c), t.is_matrix ? std::max(t.rows, t.cols) : t.cols,
+    HIP_TRY(egg_launch_noise_table(ctx->noise, d_seed, d_fit, StepEnd{}, c.population / 2, noise_word(c), t.is_matrix ? std::max(t.rows, t.cols) : t.cols,
                                    4 * c.hidden, lo, hi, t.off_a + ctx->noise.pairs_pad + 16, c.n_layers, nullptr, ctx->stream));
     return EGG_OK;
 }
@@ -854,6 +877,7 @@ extern "C" int egg_update_tensor(egg_ctx *ctx, int id, const int32_t *d_fit, con
     const egg_tensor_info &t = ctx->tensors[id];
     UpdLaunch p = make_upd(ctx, ctx->mat_one[id], d_fit, d_lr);
     if (!t.is_matrix) { p.vec = ctx->d_vec_desc + ctx->vec_one[id]; p.n_vec = 1; p.vec_total = t.cols; }
+    p.count_of = egg_update_blocks(p);
     SpanScope span(ctx, t.is_matrix ? EGG_K_UPDATE_MATRIX : EGG_K_UPDATE_VECTOR);
     int rc = table_of_tensor(ctx, id, d_fit, d_seed);
     if (rc) return rc;
@@ -875,19 +899,22 @@ extern "C" int egg_matrix_votes(egg_ctx *ctx, int id, const int32_t *d_fit, cons
     HIP_TRY(egg_launch_update(p, ctx->stream));
     return EGG_OK;
 }
-extern "C" int egg_es_update(egg_ctx *ctx, const int32_t *d_fit, const uint32_t *d_seed, const float *d_lr) {
-    if (!ctx || !d_fit || !d_seed || !d_lr) return fail(ctx, EGG_E_INVALID, "egg_es_update arguments");
+static int es_update(egg_ctx *ctx, const int32_t *d_fit, const StepEnd &end, const uint32_t *d_seed, const float *d_lr) {
     const egg_config &c = ctx->cfg;
     // tensors are independent, so the reference's launch order (mgpu.cu:1603-1643) does not matter: the noise of all of
     // them, then every AdamW matrix and every vector tensor in one launch
+    UpdLaunch adam = make_upd(ctx, ctx->mat_adam, d_fit, d_lr);
+    adam.vec = ctx->d_vec_desc; adam.n_vec = ctx->n_vec; adam.vec_total = ctx->vec_total;
+    adam.flags = ctx->adaptive ? ctx->d_flags : nullptr;
+    int count_of = egg_update_blocks(adam);
+    for (const egg_ctx::MatList &l : ctx->mat_muon) count_of += l.tiles;
+    if (count_of >= 1 << 24) return fail(ctx, EGG_E_STATE, "too many tiles to count");
+    adam.count_of = count_of;
     {
         SpanScope span(ctx, EGG_K_UPDATE_MATRIX);
-        HIP_TRY(egg_launch_noise_table(ctx->noise, d_seed, d_fit, c.population / 2, noise_word(c), ctx->noise.rows, 4 * c.hidden, 0,
+        HIP_TRY(egg_launch_noise_table(ctx->noise, d_seed, d_fit, end, c.population / 2, noise_word(c), ctx->noise.rows, 4 * c.hidden, 0,
                                        noise_entries(c, ctx->noise.pairs_pad), ctx->noise.pairs_pad + 16, c.n_layers, ctx->d_counter, ctx->stream));
-        UpdLaunch p = make_upd(ctx, ctx->mat_adam, d_fit, d_lr);
-        p.vec = ctx->d_vec_desc; p.n_vec = ctx->n_vec; p.vec_total = ctx->vec_total;
-        p.flags = ctx->adaptive ? ctx->d_flags : nullptr;
-        HIP_TRY(egg_launch_update(p, ctx->stream));
+        HIP_TRY(egg_launch_update(adam, ctx->stream));
     }
     // Muon matrices (LAUNCH_ADAM_MATRIX under USE_MUON, mgpu.cu:1587-1595), a batch of one shape at a time: momentum of
     // each into its slot of the workspace, Newton-Schulz of the whole batch, then the apply rule
@@ -901,7 +928,8 @@ extern "C" int egg_es_update(egg_ctx *ctx, const int32_t *d_fit, const uint32_t 
         if (limit < 1 || limit * one > ctx->muon_elems || limit * k * k > ctx->muon_bterm || (int)limit > ctx->muon_batch_max)
             return fail(ctx, EGG_E_STATE, "Muon batch does not fit the workspace");
         for (size_t first = 0; first < g.size(); first += limit, batch++) {
-            const UpdLaunch p = make_upd(ctx, ctx->mat_muon[batch], d_fit, d_lr);
+            UpdLaunch p = make_upd(ctx, ctx->mat_muon[batch], d_fit, d_lr);
+            p.count_of = count_of;
             { SpanScope span(ctx, EGG_K_UPDATE_MATRIX); HIP_TRY(egg_launch_update(p, ctx->stream)); }
             { SpanScope span(ctx, EGG_K_MUON_NS); HIP_TRY(egg_launch_newton_schulz_batched(ctx->muon, t0.rows, t0.cols, 5, p.n_mat, ctx->stream)); }
             { SpanScope span(ctx, EGG_K_UPDATE_MATRIX); HIP_TRY(egg_launch_muon_apply(p, c.adam_weight_decay, ctx->stream)); }
@@ -913,6 +941,10 @@ extern "C" int egg_es_update(egg_ctx *ctx, const int32_t *d_fit, const uint32_t 
         HIP_TRY(egg_launch_overlay_update(ctx->d_overlay, ctx->d_overlay_q, ctx->d_flags, ctx->d_ov_segs, ctx->n_ov_segs,
                                           ctx->ov_max_count, ctx->ov_inc, ctx->ov_dec, ctx->stream));
     return EGG_OK;
+}
+extern "C" int egg_es_update(egg_ctx *ctx, const int32_t *d_fit, const uint32_t *d_seed, const float *d_lr) {
+    if (!ctx || !d_fit || !d_seed || !d_lr) return fail(ctx, EGG_E_INVALID, "egg_es_update arguments");
+    return es_update(ctx, d_fit, StepEnd{}, d_seed, d_lr);
 }
 
 // ------------------------------------------------------------------ adaptive noise overlay (d-eggs)
@@ -961,8 +993,7 @@ extern "C" int egg_overlay_upload(egg_ctx *ctx, const void *h, size_t bytes) {
 extern "C" int egg_overlay_download(egg_ctx *ctx, void *h, size_t bytes) {
     if (!ctx || !h || (int64_t)bytes != ctx->L.total) return fail(ctx, EGG_E_INVALID, "overlay size mismatch");
     if (!ctx->adaptive) return fail(ctx, EGG_E_STATE, "egg_adaptive_enable has not been called");
-    HIP_TRY(hipStreamSynchronize(ctx->stream));
-    HIP_TRY(hipMemcpy(h, ctx->d_overlay, bytes, hipMemcpyDeviceToHost));
+    HIP_TRY(egg_host_out(ctx->out, h, ctx->d_overlay, bytes, ctx->stream));
     return EGG_OK;
 }
 extern "C" int64_t egg_opt_state_bytes(const egg_ctx *ctx) { return ctx ? ctx->state_bytes : 0; }
@@ -990,18 +1021,19 @@ extern "C" int egg_tensor_info_get(const egg_ctx *ctx, int id, egg_tensor_info *
 extern "C" int egg_last_update_count(egg_ctx *ctx, uint64_t *out) {
     if (!ctx || !out) return EGG_E_INVALID;
     HIP_TRY(hipStreamSynchronize(ctx->stream));
-    unsigned long long v = 0;
-    HIP_TRY(hipMemcpy(&v, ctx->d_counter, 8, hipMemcpyDeviceToHost));
-    *out = v;
+    *out = *ctx->h_result;
     return EGG_OK;
 }
 
 // ------------------------------------------------------------------ whole step
 static int enqueue_step(egg_ctx *ctx, const uint8_t *d_data, int64_t len) {
-    int rc = forward_range(ctx, d_data, len, &ctx->d_scal->start, &ctx->d_scal->seed, 0, ctx->cfg.population, ctx->d_loss);
+    int rc = forward_range(ctx, d_data, len, &ctx->d_scal->start, &ctx->d_scal->seed, 0, ctx->cfg.population, ctx->d_loss, true);
     if (rc) return rc;
-    HIP_TRY(egg_launch_fitness(ctx->d_loss, ctx->d_fit, ctx->cfg.population / 2, ctx->stream));
-    return egg_es_update(ctx, ctx->d_fit, &ctx->d_scal->seed, &ctx->d_scal->lr);
+    const bool dirty = ctx->acc_dirty;
+    ctx->acc_dirty = true;
+    rc = es_update(ctx, ctx->d_fit, StepEnd{ctx->d_loss_acc, ctx->d_loss, ctx->d_fit, ctx->h_loss(), ctx->h_fit()}, &ctx->d_scal->seed, &ctx->d_scal->lr);
+    if (!rc) ctx->acc_dirty = dirty;
+    return rc;
 }
 extern "C" int egg_step(egg_ctx *ctx, const uint8_t *d_data, int64_t len, int64_t start_idx, uint32_t step_seed, float lr) {
     if (!ctx) return EGG_E_INVALID;
@@ -1014,6 +1046,7 @@ extern "C" int egg_step_capture(egg_ctx *ctx, const uint8_t *d_data, int64_t len
     if (ctx->captured) return fail(ctx, EGG_E_STATE, "step already captured");
     if (ctx->taps) return fail(ctx, EGG_E_STATE, "disable taps before capturing");
     if (ctx->timing) return fail(ctx, EGG_E_STATE, "disable timing before capturing");
+    if (int rc = clear_loss_sums(ctx)) return rc;          // the captured step finds them at zero
     HIP_TRY(hipStreamSynchronize(ctx->stream));
     HIP_TRY(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
     int rc = enqueue_step(ctx, d_data, len);
@@ -1031,14 +1064,15 @@ extern "C" int egg_step_launch(egg_ctx *ctx, int64_t start_idx, uint32_t step_se
     if (!ctx->captured) return fail(ctx, EGG_E_STATE, "egg_step_capture has not been called");
     hipLaunchKernelGGL(k_set_scalars, dim3(1), dim3(1), 0, ctx->stream, ctx->d_scal, step_seed, lr, start_idx);
     HIP_TRY(hipGetLastError());
+    if (int rc = clear_loss_sums(ctx)) return rc;
     HIP_TRY(hipGraphLaunch(ctx->gexec, ctx->stream));
     return EGG_OK;
 }
 extern "C" int egg_step_losses(egg_ctx *ctx, int32_t *h_loss, int32_t *h_fit) {
     if (!ctx) return EGG_E_INVALID;
     HIP_TRY(hipStreamSynchronize(ctx->stream));
-    if (h_loss) HIP_TRY(hipMemcpy(h_loss, ctx->d_loss, (size_t)ctx->cfg.population * 4, hipMemcpyDeviceToHost));
-    if (h_fit) HIP_TRY(hipMemcpy(h_fit, ctx->d_fit, (size_t)(ctx->cfg.population / 2) * 4, hipMemcpyDeviceToHost));
+    if (h_loss) memcpy(h_loss, ctx->h_loss(), (size_t)ctx->cfg.population * 4);
+    if (h_fit) memcpy(h_fit, ctx->h_fit(), (size_t)(ctx->cfg.population / 2) * 4);
     return EGG_OK;
 }
 

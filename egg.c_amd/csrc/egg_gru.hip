@@ -436,6 +436,7 @@ struct egg_gru_ctx {
     // Each way of evaluating has its own copy of the weights, brought up to date when it is used.
     bool staged = true, frag_stale = true, pipe_stale = true;
     int8_t *d_act = nullptr, *d_h = nullptr, *d_pfrag = nullptr, *d_rows = nullptr, *d_npipe = nullptr;
+    HostOut out;
     std::string err;
 };
 static int gfail(egg_gru_ctx *c, int code, const char *what, hipError_t e = hipSuccess) {
@@ -529,6 +530,7 @@ extern "C" int egg_gru_create(const egg_gru_config *cfg, egg_gru_ctx **out) {
     for (int i = 0; i < 256; i++) ex[i] = (int32_t)(pow(2.0, (double)i / (1 << c.fixed_point)) * (1 << c.fixed_point));   // egg.c:57-60
     CR(hipMalloc(&ctx->d_exp2, 1024)); CR(hipMemcpy(ctx->d_exp2, ex, 1024, hipMemcpyHostToDevice));
     const int at_once = std::min(c.population, GRU_PIPE_MEMBERS);
+    CR(egg_host_out_create(&ctx->out, (size_t)ctx->model_bytes));
     CR(gru_pipe_prepare(c.hidden));
     CR(hipMalloc(&ctx->d_act, gru_pipe_act_bytes(at_once, c.hidden, c.n_layers)));
     CR(hipMalloc(&ctx->d_h, (size_t)at_once * L * H));
@@ -545,6 +547,7 @@ extern "C" void egg_gru_destroy(egg_gru_ctx *ctx) {
     void *ptrs[] = {ctx->d_model, ctx->d_frag, ctx->d_noise, ctx->d_panels, ctx->d_states, ctx->d_mats, ctx->d_loss, ctx->d_fit, ctx->d_exp2,
                     ctx->d_act, ctx->d_h, ctx->d_pfrag, ctx->d_rows, ctx->d_npipe};
     for (void *q : ptrs) if (q) (void)hipFree(q);
+    egg_host_out_destroy(&ctx->out);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
 }
@@ -580,8 +583,7 @@ extern "C" int egg_gru_model_upload(egg_gru_ctx *ctx, const void *h, size_t byte
 }
 extern "C" int egg_gru_model_download(egg_gru_ctx *ctx, void *h, size_t bytes) {
     if (!ctx || !h || (long long)bytes != ctx->model_bytes) return gfail(ctx, EGG_E_INVALID, "model size mismatch");
-    GTRY(hipStreamSynchronize(ctx->stream));
-    GTRY(hipMemcpy(h, ctx->d_model, bytes, hipMemcpyDeviceToHost));
+    GTRY(egg_host_out(ctx->out, h, ctx->d_model, bytes, ctx->stream));
     return EGG_OK;
 }
 extern "C" int egg_gru_state_reset(egg_gru_ctx *ctx) {
@@ -594,8 +596,7 @@ extern "C" int egg_gru_state_download(egg_gru_ctx *ctx, void *h, size_t bytes) {
     if (!ctx) return EGG_E_INVALID;
     const size_t want = (size_t)ctx->cfg.population * ctx->cfg.n_layers * ctx->cfg.hidden;
     if (!h || bytes != want) return gfail(ctx, EGG_E_INVALID, "state size mismatch");
-    GTRY(hipStreamSynchronize(ctx->stream));
-    GTRY(hipMemcpy(h, ctx->d_states, want, hipMemcpyDeviceToHost));
+    GTRY(egg_host_out(ctx->out, h, ctx->d_states, want, ctx->stream));
     return EGG_OK;
 }
 

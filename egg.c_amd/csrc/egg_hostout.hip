@@ -1,0 +1,107 @@
+// egg_hostout.hip -- device memory into the caller's (pageable) memory.
+//
+// hipMemcpy moves such a copy in pieces of 1 MB, each first by the GPU into pinned memory (20 us) and then by one host thread
+// into the caller's (65 us): 12 GB/s, and 25 us for a few bytes.  Here the two overlap: a context keeps eight pinned slots, a
+// kernel fills them in turn (one PCIe transfer after the other), and what has arrived is copied out meanwhile -- by this thread
+// for short pieces, by up to five helpers for long ones, because a caller's fresh memory is mapped and cleared page by
+// page as it is first written, which one thread cannot do at PCIe speed.
+// 27 MB of weights: 2.3 -> 0.8 ms; 11 MB of optimizer state: 0.95 -> 0.4 ms.
+#include "egg_launch.h"
+#include <string.h>
+#include <algorithm>
+#include <atomic>
+#include <thread>
+#include <vector>
+
+namespace {
+
+constexpr int SLOTS = 8;
+constexpr size_t SLOT_MAX = 1 << 20;         // at most 8 MB pinned per context
+constexpr size_t HELPER_BYTES = 1 << 21;     // bytes that are worth another thread (starting one takes about 20 us)
+constexpr int HELPERS = 5;
+
+typedef int v4i __attribute__((ext_vector_type(4)));
+// PCIe-bound: 64 workgroups keep its writes busy (1 MB in 20 us)
+__global__ void __launch_bounds__(256) k_out(v4i *dst, const v4i *src, size_t bytes) {
+    const size_t n = bytes / 16;
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) dst[i] = src[i];
+    if (blockIdx.x == 0 && threadIdx.x < bytes % 16)
+        reinterpret_cast<int8_t *>(dst + n)[threadIdx.x] = reinterpret_cast<const int8_t *>(src + n)[threadIdx.x];
+}
+
+}  // namespace
+
+hipError_t egg_host_out_create(HostOut *o, size_t largest) {
+    o->slot = std::max<size_t>(4096, std::min(SLOT_MAX, ((largest + SLOTS - 1) / SLOTS + 4095) & ~(size_t)4095));
+    hipError_t e = hipHostMalloc(reinterpret_cast<void **>(&o->mem), SLOTS * o->slot, hipHostMallocCoherent);
+    for (int i = 0; i < SLOTS && e == hipSuccess; i++) e = hipEventCreateWithFlags(&o->done[i], hipEventDisableTiming | hipEventReleaseToSystem);
+    return e;
+}
+void egg_host_out_destroy(HostOut *o) {
+    for (hipEvent_t &d : o->done) if (d) { (void)hipEventDestroy(d); d = nullptr; }
+    if (o->mem) (void)hipHostFree(o->mem);
+    o->mem = nullptr;
+}
+
+hipError_t egg_host_out(HostOut &o, void *dst, const void *src, size_t bytes, hipStream_t s) {
+    if (!o.mem || (reinterpret_cast<uintptr_t>(src) & 15)) return hipErrorInvalidValue;
+    // a short piece goes as a whole, through as many slots as it covers: splitting it would cost more events than it overlaps
+    const size_t piece = bytes <= SLOT_MAX / 4 && bytes <= SLOTS * o.slot ? bytes : o.slot;
+    const int n = piece ? (int)((bytes + piece - 1) / piece) : 0;
+    auto slot = [&](int c) { return o.mem + (size_t)(c % SLOTS) * o.slot; };
+    auto size = [&](int c) { return std::min(piece, bytes - (size_t)c * piece); };
+    auto start = [&](int c) {
+        const unsigned blocks = (unsigned)std::min<size_t>(64, (size(c) + 4095) / 4096);
+        hipLaunchKernelGGL(k_out, dim3(blocks), dim3(256), 0, s, reinterpret_cast<v4i *>(slot(c)),
+                           reinterpret_cast<const v4i *>(static_cast<const int8_t *>(src) + (size_t)c * piece), size(c));
+        const hipError_t e = hipGetLastError();
+        return e != hipSuccess ? e : n == 1 ? hipSuccess : hipEventRecord(o.done[c % SLOTS], s);
+    };
+    auto take = [&](int c) { memcpy(static_cast<int8_t *>(dst) + (size_t)c * piece, slot(c), size(c)); };
+    hipError_t e = hipSuccess;
+    if (n <= 1) {
+        if (n) e = start(0);
+        if (e == hipSuccess) e = hipStreamSynchronize(s);
+        if (n && e == hipSuccess) take(0);
+        return e;
+    }
+    int started = 0, have = 0;
+    while (started < n && started < SLOTS && e == hipSuccess) e = start(started++);
+    // helpers claim pieces as they arrive; this thread starts transfers and follows their events
+    std::atomic<int> arrived{0}, next{0};
+    std::atomic<bool> stop{false};
+    std::vector<std::atomic<char>> taken(n);
+    for (auto &t : taken) t.store(0, std::memory_order_relaxed);
+    std::vector<std::thread> crew;
+    try {
+        const int helpers = (int)std::min<size_t>(HELPERS, bytes / HELPER_BYTES);
+        crew.reserve(helpers);
+        for (int h = 0; h < helpers; h++)
+            crew.emplace_back([&] {
+                for (int c = next++; c < n; c = next++) {
+                    while (arrived.load(std::memory_order_acquire) <= c) {
+                        if (stop.load(std::memory_order_relaxed)) return;
+                        std::this_thread::yield();
+                    }
+                    take(c);
+                    taken[c].store(1, std::memory_order_release);
+                }
+            });
+    } catch (...) {}                              // fewer helpers, or none
+    while (have < n && e == hipSuccess) {
+        if (crew.empty()) {
+            e = hipEventSynchronize(o.done[have % SLOTS]);
+            if (e == hipSuccess) { take(have); taken[have++].store(1, std::memory_order_relaxed); }
+        } else if (have < started) {
+            e = hipEventQuery(o.done[have % SLOTS]);
+            if (e == hipSuccess) arrived.store(++have, std::memory_order_release);
+            else if (e == hipErrorNotReady) { (void)hipGetLastError(); e = hipSuccess; }
+        }
+        if (started < n && e == hipSuccess && taken[started - SLOTS].load(std::memory_order_acquire)) e = start(started++);
+    }
+    if (e != hipSuccess) stop.store(true);
+    for (std::thread &t : crew) t.join();
+    // on an error the slots may still be written to: nothing may use them until the stream is idle
+    if (e != hipSuccess) (void)hipStreamSynchronize(s);
+    return e;
+}

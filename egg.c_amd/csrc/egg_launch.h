@@ -34,7 +34,7 @@ hipError_t egg_launch_swizzle(const int8_t *W_blocked, int8_t *W_frag, int K, in
 // small utility kernels (egg_update.hip)
 hipError_t egg_launch_noise_fill(uint32_t seed, uint32_t first, int n, int mask, int8_t *out, hipStream_t s);
 hipError_t egg_launch_zero_u64(unsigned long long *p, int64_t n, hipStream_t s);
-hipError_t egg_launch_loss_finalize(const unsigned long long *acc, int32_t *loss, int first, int count, hipStream_t s);
+hipError_t egg_launch_loss_finalize(unsigned long long *acc, int32_t *loss, int first, int count, hipStream_t s);
 hipError_t egg_launch_fitness(const int32_t *loss, int32_t *fit, int pairs, hipStream_t s);
 // ws: vocab ints (plain sampler) or 2 * vocab ints (d-eggs sampler) of device scratch; token_bytes: 1 or 4
 hipError_t egg_launch_sample(const int32_t *logits, const int32_t *exp_lut, int vocab, int bt, uint32_t seed, int t,
@@ -51,9 +51,12 @@ struct NoiseTable {
     int8_t *neg, *nonzero; int pairs_pad;      // [pairs_pad] each (a multiple of 128): 0xff where the fitness is -1 / is not 0
     int *general;                              // 1: some fitness lies outside {-1, 0, 1}
 };
+// what a whole step does between its forward and its update: losses and fitness from the loss sums, which go back to
+// zero, into device memory and the host's copies.  acc null: the fitness is given.
+struct StepEnd { unsigned long long *acc; int32_t *loss, *fit, *h_loss, *h_fit; };
 // rows [0, rows) of the entries [t_lo, t_hi) (rows from layer_rows on only below emb_t), the fitness masks, and *counter = 0
 // unless it is null
-hipError_t egg_launch_noise_table(const NoiseTable &nt, const uint32_t *d_seed, const int32_t *d_fit, int pairs, int mask, int rows,
+hipError_t egg_launch_noise_table(const NoiseTable &nt, const uint32_t *d_seed, const int32_t *d_fit, const StepEnd &end, int pairs, int mask, int rows,
                                   int layer_rows, int t_lo, int t_hi, int emb_t, int n_layers, unsigned long long *counter, hipStream_t s);
 struct MatDesc {
     int8_t *W, *frag; float *state;    // canonical weights, their fragment-major copy, optimizer state ({m,v,acc} or Muon's {m,acc})
@@ -72,11 +75,13 @@ struct UpdLaunch {
     NoiseTable noise;
     const int32_t *fit; int pairs;
     const float *d_lr; float beta1, beta2, eps, wd, muon_momentum;
-    unsigned long long *counter;
+    unsigned long long *counter, *h_counter;       // changed weights; the host's copy
+    int count_of;                      // workgroups that report changes in the whole update
     int32_t *votes_out;                // optional, one matrix: only its votes (blocked order), no update
     int8_t *flags;                     // optional (adaptive noise overlay), laid out like the model blob: a matrix's rows, then its
                                        // cols, set to 1 where a weight changed (de/include/optimizer/adam.cuh:77-83)
 };
+int egg_update_blocks(const UpdLaunch &p);             // its workgroups
 hipError_t egg_launch_update(const UpdLaunch &p, hipStream_t s);
 hipError_t egg_launch_muon_apply(const UpdLaunch &p, float wd, hipStream_t s);
 hipError_t egg_launch_frag(const MatDesc *d_mat, int n_mat, int tiles, hipStream_t s);
@@ -118,6 +123,12 @@ hipError_t egg_launch_ternary_pack(const int8_t *src, uint8_t *packed, int n_ele
 struct MuonWork { float *x, *swap, *gram, *bterm, *partials, *norm; };   // x/swap: rows*cols, gram/bterm: K*K, partials: 1024
 hipError_t egg_launch_newton_schulz(const MuonWork &w, int rows, int cols, int iters, hipStream_t s);
 hipError_t egg_launch_newton_schulz_batched(const MuonWork &w, int rows, int cols, int iters, int batch, hipStream_t s);
+// ---- device memory to the caller's memory (egg_hostout.hip)
+struct HostOut { int8_t *mem = nullptr; size_t slot = 0; hipEvent_t done[8] = {}; };
+hipError_t egg_host_out_create(HostOut *o, size_t largest);       // largest: the longest piece that is usually asked for
+void egg_host_out_destroy(HostOut *o);
+// in stream order; returns when the bytes are in `dst`.  src 16-byte aligned.
+hipError_t egg_host_out(HostOut &o, void *dst, const void *src, size_t bytes, hipStream_t s);
 // message returned by egg_last_error(NULL) on this thread, for entry points that take no context
 void egg_set_thread_error(const char *what);
 #define EGG_MAX_DEVICES 64

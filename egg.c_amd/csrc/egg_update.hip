@@ -31,12 +31,12 @@ hipError_t egg_launch_zero_u64(unsigned long long *p, int64_t n, hipStream_t s) 
     return hipGetLastError();
 }
 
-// accum_loss[p] = (int32_t) my_loss   (mgpu.cu:1028)
-__global__ void k_loss_finalize(const unsigned long long *acc, int32_t *loss, int first, int count) {
+// accum_loss[p] = (int32_t) my_loss   (mgpu.cu:1028); the sums go back to zero for the next forward
+__global__ void k_loss_finalize(unsigned long long *acc, int32_t *loss, int first, int count) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < count) loss[first + i] = (int32_t)(long long)acc[first + i];
+    if (i < count) { loss[first + i] = (int32_t)(long long)acc[first + i]; acc[first + i] = 0ull; }
 }
-hipError_t egg_launch_loss_finalize(const unsigned long long *acc, int32_t *loss, int first, int count, hipStream_t s) {
+hipError_t egg_launch_loss_finalize(unsigned long long *acc, int32_t *loss, int first, int count, hipStream_t s) {
     if (count <= 0) return hipSuccess;
     hipLaunchKernelGGL(k_loss_finalize, dim3((count + 255) / 256), dim3(256), 0, s, acc, loss, first, count);
     return hipGetLastError();

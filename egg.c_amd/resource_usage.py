@@ -17,7 +17,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off", "-fhip-fp32-correctly-rounded-divide-sqrt",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "--cuda-device-only", "-w"]
 EXTRA = {"egg_linear_ws.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
-SOURCES = ["egg_forward.hip", "egg_linear.hip", "egg_linear_ws.hip", "egg_update.hip", "egg_votes.hip", "egg_decode.hip", "egg_gru.hip", "egg_gru_pipe.hip"]
+SOURCES = ["egg_forward.hip", "egg_linear.hip", "egg_linear_ws.hip", "egg_update.hip", "egg_votes.hip", "egg_decode.hip", "egg_gru.hip", "egg_gru_pipe.hip", "egg_hostout.hip"]
 KEYS = ["VGPRs", "AGPRs", "ScratchSize [bytes/lane]", "Occupancy [waves/SIMD]", "VGPRs Spill", "LDS Size [bytes/block]"]
 
 
