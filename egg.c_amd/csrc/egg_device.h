@@ -27,6 +27,7 @@
 #pragma clang fp contract(off)
 
 typedef int v4i __attribute__((ext_vector_type(4)));
+typedef float v4f __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 
 #define EGG_WAVES 4
@@ -344,15 +345,21 @@ static inline int tile_map_sets(int T, int cs) { int tpm = T / 32, tpw = EGG_WAV
 
 // Combine a per-token value over the CS waves sharing a tile.  `site` is an LDS area of EGG_WAVES*64 ints that no
 // other exchange uses until every wave has passed another barrier.  Every wave of the workgroup must call it.
+// (xput and xget: its two halves, for a caller that passes a barrier of its own between them)
+__device__ __forceinline__ void xput(int v, int *site, int CS, const TileMap &tm, int lane) { site[(tm.tslot * CS + tm.cs) * 64 + lane] = v; }
 template <int CS, bool IS_MAX>
-__device__ __forceinline__ int xreduce(int v, int *site, const TileMap &tm, int lane) {
-    if (CS == 1) return v;
-    site[(tm.tslot * CS + tm.cs) * 64 + lane] = v;
-    __syncthreads();
+__device__ __forceinline__ int xget(const int *site, const TileMap &tm, int lane) {
     int r = site[(tm.tslot * CS) * 64 + lane];
 #pragma unroll
     for (int c = 1; c < CS; c++) { int o = site[(tm.tslot * CS + c) * 64 + lane]; r = IS_MAX ? max(r, o) : r + o; }
     return r;
+}
+template <int CS, bool IS_MAX>
+__device__ __forceinline__ int xreduce(int v, int *site, const TileMap &tm, int lane) {
+    if (CS == 1) return v;
+    xput(v, site, CS, tm, lane);
+    __syncthreads();
+    return xget<CS, IS_MAX>(site, tm, lane);
 }
 
 template <int N>
@@ -429,24 +436,36 @@ __device__ __forceinline__ int dot_noise(const v4i *xop, const int8_t *btab, int
     return sum_halves(s);
 }
 
-// x . B under the overlay: every term x[k] * B[k] is scaled by the input row's factor and truncated before it is added
-// (the reference converts each thread's term to int, de/include/model/layers.cuh:240).  qtab holds the rows' q values
-// in the order of btab.
-template <int KS, bool NAT>
-__device__ __forceinline__ int dot_noise_ov(const v4i *xop, const int8_t *btab, const int8_t *qtab, int k_off, int g) {
-    const int *b32 = reinterpret_cast<const int *>(btab + k_off);
-    const int *q32 = reinterpret_cast<const int *>(qtab + k_off);
-    int s = 0;
+// Input-side noise times the input row's factor q / 64, as floats: under the overlay a term x[k] * B[k] * factor is truncated
+// before it is added (the reference converts each thread's term to int, de/include/model/layers.cuh:240).  The products have
+// six fraction bits below 127 * 127, so float32 holds them exactly, and multiply, truncate and add are three instructions a
+// term (four with the conversion of x) where 32-bit integers took eleven.
+__device__ __forceinline__ void fill_noise_f32_ov(float *dst, uint32_t seed, int n, int mask, int lane, int nthr, const int8_t *q) {
+    for (int i = lane; i < n; i += nthr) dst[i] = (float)(noise_from_hash(seed, i, mask) * q[i]) * 0.015625f;
+}
+// x . B under the overlay for the NB tables at tab, tab + stride, ... (natural order; x in slot order).  The sums stay below
+// 512 * 127 * 127 < 2^24.
+template <int KS, int NB>
+__device__ __forceinline__ void dot_noise_ov(const v4i *xop, const float *tab, int stride, int g, int *sb) {
+    float s[NB];
+#pragma unroll
+    for (int i = 0; i < NB; i++) s[i] = 0.f;
 #pragma unroll
     for (int ks = 0; ks < KS; ks++)
 #pragma unroll
         for (int q = 0; q < 4; q++) {
-            int kd = NAT ? (8 * ks + 4 * g + q) : (8 * ks + 2 * q + g);
-            const int xb = xop[ks][q], nb = b32[kd], qb = q32[kd];
+            float x[4];
 #pragma unroll
-            for (int e = 0; e < 4; e++) s += div_pow2_trunc<6>(mul24(mul24(sx8(xb, e), sx8(nb, e)), sx8(qb, e)));
+            for (int e = 0; e < 4; e++) x[e] = (float)sx8(xop[ks][q], e);
+#pragma unroll
+            for (int i = 0; i < NB; i++) {
+                const v4f b = *reinterpret_cast<const v4f *>(tab + i * stride + 32 * ks + 8 * q + 4 * g);
+#pragma unroll
+                for (int e = 0; e < 4; e++) s[i] += truncf(x[e] * b[e]);
+            }
         }
-    return sum_halves(s);
+#pragma unroll
+    for (int i = 0; i < NB; i++) sb[i] = sum_halves((int)s[i]);
 }
 
 // ---------------------------------------------------------------- norms on a token held as a packed operand

@@ -147,8 +147,11 @@ struct MlpCfg {
     static constexpr int ACT = 256;          // GELU table: entry v + 128 holds the activation of the int8 value v
     // (behind the first block ex1 does not exist: 4H bytes less.  At hidden 256 the total stays at 52 KB: the LDS is
     // handed out in granules, three workgroups of 53 KB no longer share a CU, and the kernel then runs 9 % slower.)
-    static constexpr int per_set(bool first) { return PER_SET + (first ? 0 : UPA32 - 4 * H); }
-    static int total(int sets, bool first) { return WBYTES + ACT + sets * per_set(first) + XCHG + RED + (first ? DEDUP : 0); }
+    // The overlay's variants hold the input-side noise as floats: exB, upB and dnB take four times their bytes.
+    static constexpr int per_set(bool first, bool adapt) { return PER_SET + (first ? 0 : UPA32 - 4 * H) + (adapt ? 3 * 6 * H : 0); }
+    static int total(int sets, bool first, bool adapt) { return WBYTES + ACT + sets * per_set(first, adapt) + XCHG + RED + (first ? DEDUP : 0); }
+    // the overlay's variants need the registers of two workgroups per CU
+    static constexpr int occ(bool adapt) { return adapt && OCC > 2 ? 2 : OCC; }
 };
 
 // FUSE: the host has checked sigma <= 7 and |noise| <= 15, which bounds |acc| * 2^sigma + |sb * a| below 2^31 for
@@ -157,9 +160,10 @@ struct MlpCfg {
 // ADAPT: the d-eggs adaptive noise overlay is on (de/include/model/layers.cuh:215-296, :432-438,
 // de/src/kernels.cu:139-158); see k_qkv.  The down projection's input-side sum follows the reference thread of a
 // hidden unit, which adds its four terms (k = unit, unit + H, ...) into an int one float addition at a time; the
-// sub-chunks are therefore visited so that those four are consecutive.
+// sub-chunks are therefore visited so that those four are consecutive.  At hidden 256, 2048 members x 256 tokens the overlay's
+// kernel took 0.91 ms with integer terms, spilling at three workgroups per CU; 0.63 ms as it is (0.47 without the overlay).
 template <int H, bool FIRST, bool FUSE, bool ADAPT>
-__global__ void __launch_bounds__(EGG_THREADS, MlpCfg<H>::OCC) k_mlp(MlpParams p) {
+__global__ void __launch_bounds__(EGG_THREADS, MlpCfg<H>::occ(ADAPT)) k_mlp(MlpParams p) {
     typedef MlpCfg<H> M;
     constexpr bool FUSE_DN = FUSE && 4 * H <= 1024;
     constexpr int CS = M::CS, KS = M::KS, NTS = M::NTS, HS = M::HS, NTU = M::NTU, SC = M::SC;
@@ -171,19 +175,20 @@ __global__ void __launch_bounds__(EGG_THREADS, MlpCfg<H>::OCC) k_mlp(MlpParams p
     // that the dynamic LDS block starts at LDS address 0 (the kernel declares no static LDS); built from the `act`
     // pointer instead, every read carries an extra add of that (zero) base.
     typedef const __attribute__((address_space(3))) uint8_t *lds_u8_ptr;
+    typedef const __attribute__((address_space(3))) int8_t *lds_i8_ptr;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, g = lane >> 5, j = lane & 31;
     const FwdCommon &c = p.c;
     const int T = c.T;
     const TileMap tm = tile_map<CS>(c.tn, wave, blockIdx.x);
     const int col0 = tm.cs * HS;                      // first output column of this wave's slice
-    constexpr int PSET = M::per_set(FIRST);
+    constexpr int PSET = M::per_set(FIRST, ADAPT), WB = ADAPT ? 4 : 1;        // WB: bytes of an input-side noise entry
     constexpr bool UPA32 = !FIRST;
     int8_t *tb = act + M::ACT + tm.set * PSET;
     int *ex0 = reinterpret_cast<int *>(tb);           // FIRST: emb_bias + noise   | else: O-proj A noise * ns as int8
     int *ex1 = ex0 + H;                               // FIRST: b_dim noise * ns    | else: absent
     int *lnw = ex1 + (FIRST ? H : 0), *lnb = lnw + H, *bup = lnb + H, *bdn = bup + 4 * H;
     int8_t *exB = reinterpret_cast<int8_t *>(bdn + H);   // O-proj B noise
-    int8_t *upB = exB + H, *dnB = upB + H, *upA = dnB + 4 * H, *dnA = upA + (UPA32 ? 16 : 4) * H;
+    int8_t *upB = exB + WB * H, *dnB = upB + WB * H, *upA = dnB + 4 * WB * H, *dnA = upA + (UPA32 ? 16 : 4) * H;
     const int8_t *oA = reinterpret_cast<const int8_t *>(ex0);
     int8_t *xch = act + M::ACT + tm.sets * PSET;
     int *red = reinterpret_cast<int *>(xch + M::XCHG);
@@ -220,7 +225,7 @@ __global__ void __launch_bounds__(EGG_THREADS, MlpCfg<H>::OCC) k_mlp(MlpParams p
         const uint32_t pseed = *c.d_step_seed + (uint32_t)(mem / 2), sbx = pseed + (uint32_t)p.seed_base;
         int8_t *t2 = act + M::ACT + ss * PSET;
         int *e0 = reinterpret_cast<int *>(t2), *e1 = e0 + H, *lw = e1 + (FIRST ? H : 0), *lb = lw + H, *bu = lb + H, *bd = bu + 4 * H;
-        int8_t *eB = reinterpret_cast<int8_t *>(bd + H), *uB = eB + H, *dB = uB + H, *uA = dB + 4 * H, *dA = uA + (UPA32 ? 16 : 4) * H;
+        int8_t *eB = reinterpret_cast<int8_t *>(bd + H), *uB = eB + WB * H, *dB = uB + WB * H, *uA = dB + 4 * WB * H, *dA = uA + (UPA32 ? 16 : 4) * H;
         const int tid = threadIdx.x;
         if (ADAPT) {
             if (FIRST) {
@@ -229,7 +234,7 @@ __global__ void __launch_bounds__(EGG_THREADS, MlpCfg<H>::OCC) k_mlp(MlpParams p
                 for (int i = tid; i < H; i += EGG_THREADS) e1[i] = noise_from_hash(pseed + OFF_EMB + H, i, c.mask) * p.q_emb[i] * nsx;
             } else {
                 fill_noise_i8_ov(reinterpret_cast<int8_t *>(e0), sbx + OFF_O_A, H, c.mask, tid, EGG_THREADS, nsx, p.q_o + H);
-                fill_noise_i8(eB, sbx + OFF_O_B, H, c.mask, tid, EGG_THREADS);
+                fill_noise_f32_ov(reinterpret_cast<float *>(eB), sbx + OFF_O_B, H, c.mask, tid, EGG_THREADS, p.q_o);
             }
             fill_vec_i32_ov(lw, p.ln_w, sbx + p.off_ln_a, sbx + p.off_ln_b, H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS, 2, p.q_ln_w);
             fill_vec_i32_ov(lb, p.ln_b, sbx + p.off_lnb_a, sbx + p.off_lnb_b, H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS, 0, p.q_ln_b);
@@ -238,8 +243,8 @@ __global__ void __launch_bounds__(EGG_THREADS, MlpCfg<H>::OCC) k_mlp(MlpParams p
             fill_vec_i32_ov(bu, p.b_up, sbx + p.off_bup_a, sbx + p.off_bup_b, 4 * H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS, c.shift_mlp_up, p.q_b_up, 128);
             fill_noise_i8_ov(dA, sbx + p.off_dn_a, H, c.mask, tid, EGG_THREADS, nsx, p.q_dn + 4 * H);
             fill_vec_i32_ov(bd, p.b_dn, sbx + p.off_bdn_a, sbx + p.off_bdn_b, H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS, 0, p.q_b_dn);
-            fill_noise_i8(uB, sbx + p.off_up_b, H, c.mask, tid, EGG_THREADS);
-            fill_noise_i8(dB, sbx + p.off_dn_b, 4 * H, c.mask, tid, EGG_THREADS);
+            fill_noise_f32_ov(reinterpret_cast<float *>(uB), sbx + p.off_up_b, H, c.mask, tid, EGG_THREADS, p.q_up);
+            fill_noise_f32_ov(reinterpret_cast<float *>(dB), sbx + p.off_dn_b, 4 * H, c.mask, tid, EGG_THREADS, p.q_dn);
             continue;
         }
         if (FIRST) {
@@ -343,13 +348,28 @@ __global__ void __launch_bounds__(EGG_THREADS, MlpCfg<H>::OCC) k_mlp(MlpParams p
                 v4i aop[KS];
 #pragma unroll
                 for (int ks = 0; ks < KS; ks++) aop[ks] = load_op(p.ao + row, ks, gA);
-                sbo = ADAPT ? dot_noise_ov<KS, false>(aop, exB, p.q_o, 0, gA) : dot_noise<KS, false>(aop, exB, 0, gA);
+                int *const site = ADAPT && CS > 1 ? next_site() : nullptr;
+                if (ADAPT) {
+                    // the waves of a tile take a column slice of the row each
+                    v4i own[NTS];
+#pragma unroll
+                    for (int nt = 0; nt < NTS; nt++) {
+                        own[nt] = aop[nt];
+#pragma unroll
+                        for (int k = 1; k < CS; k++)
+#pragma unroll
+                            for (int q = 0; q < 4; q++) own[nt][q] = tm.cs == k ? aop[k * NTS + nt][q] : own[nt][q];
+                    }
+                    dot_noise_ov<NTS, 1>(own, reinterpret_cast<const float *>(exB) + col0, 0, gA, &sbo);
+                    if (CS > 1) xput(sbo, site, CS, tm, laneA);
+                } else sbo = dot_noise<KS, false>(aop, exB, 0, gA);
 #pragma unroll
                 for (int u = 0; u < M::OU; u++) {
                     const int8_t *cur = w_acquire(ws);
                     if (u + 1 < M::OU) pf_o(u + 1); else pf_up(0, 0);
                     mfma_cols<M::PRO / 2, NTS, MAXF>(acc, aop + u * (M::PRO / 2), cur, H, col0, laneA);
                 }
+                if (ADAPT && CS > 1) sbo = xget<CS, false>(site, tm, laneA);
             }
             perturb_shift_groups<NTS, FUSE>(acc, sbo, oA, col0, c.sigma, c.shift_out, gA);
 #pragma unroll
@@ -373,6 +393,7 @@ __global__ void __launch_bounds__(EGG_THREADS, MlpCfg<H>::OCC) k_mlp(MlpParams p
 
         // MLP (mgpu.cu:708-759)
         v4i nrm[KS];
+        int sbu;
         {
             int tot = sumabs_groups<NTS>(xs);
             tot = sum_halves(tot);
@@ -384,14 +405,26 @@ __global__ void __launch_bounds__(EGG_THREADS, MlpCfg<H>::OCC) k_mlp(MlpParams p
                 // next prefetch into it is issued only after the barrier of the next w_acquire
                 v4i mine[NTS];
                 standard_scale<NTS>(xs, mine, mn, lnw, lnb, col0, gA);
+                int *const site = ADAPT ? next_site() : nullptr;
+                if (ADAPT) {
+                    dot_noise_ov<NTS, 1>(mine, reinterpret_cast<const float *>(upB) + col0, 0, gA, &sbu);
+                    xput(sbu, site, CS, tm, laneA);
+                }
                 exchange_operand<CS, NTS, KS, M::TPW, M::UNIT>(ws.other, tm, laneA, mine, nrm);
+                if (ADAPT) sbu = xget<CS, false>(site, tm, laneA);
             }
         }
-        const int sbu = ADAPT ? dot_noise_ov<KS, false>(nrm, upB, p.q_up, 0, gA) : dot_noise<KS, false>(nrm, upB, 0, gA);
+        if (ADAPT && CS == 1) dot_noise_ov<KS, 1>(nrm, reinterpret_cast<const float *>(upB), 0, gA, &sbu);
+        if (!ADAPT) sbu = dot_noise<KS, false>(nrm, upB, 0, gA);
         v16i accd[NTS];
         zero_acc<NTS>(accd);
         int sbd = 0;
-        int pb[ADAPT ? NTU * 16 : 1];           // ADAPT: running sums of the reference threads this laneA stands in for
+        // ADAPT: running sums of the reference threads this lane stands in for; whole numbers and, with a term added, six
+        // fraction bits below 4 * 127 * 127: exact in float32
+        float pb[ADAPT ? NTU * 16 : 1];
+        if (ADAPT)
+#pragma unroll
+            for (int i = 0; i < (ADAPT ? NTU * 16 : 1); i++) pb[i] = 0.f;
         // ADAPT: iteration it visits sub-chunk (it % 4) * NSUB/4 + it / 4, so four consecutive iterations cover the
         // intermediate columns unit, unit + H, unit + 2H, unit + 3H of the same hidden units
         auto sub_chunk = [](int it) { return ADAPT ? (it & 3) * (M::NSUB / 4) + (it >> 2) : it; };
@@ -429,31 +462,31 @@ __global__ void __launch_bounds__(EGG_THREADS, MlpCfg<H>::OCC) k_mlp(MlpParams p
                         int a4 = 0; v4i a32 = {0, 0, 0, 0};
                         if (UPA32) a32 = *reinterpret_cast<const v4i *>(reinterpret_cast<const int *>(upA) + n0);
                         else a4 = *reinterpret_cast<const int *>(upA + n0);
-                        uint32_t r4[4];          // the activation of element e as an unsigned byte
+                        uint32_t r4[4];          // byte 0: the activation of element e (ADAPT: sign-extended)
 #pragma unroll
                         for (int e = 0; e < 4; e++) {
                             // the accumulator carries + 128 (see the bias table): clamping to 1..255 is the clamp to +-127,
                             // and the result is the table index as it stands
                             const int idx = min(255, max(1, perturb_shift<FUSE>(au[nt][4 * q + e], sbu, UPA32 ? a32[e] : sx8(a4, e), c.sigma, c.shift_mlp_up)));
-                            r4[e] = reinterpret_cast<lds_u8_ptr>((uintptr_t)(uint32_t)idx)[M::WBYTES];
+                            r4[e] = ADAPT ? (uint32_t)(int)reinterpret_cast<lds_i8_ptr>((uintptr_t)(uint32_t)idx)[M::WBYTES]
+                                          : reinterpret_cast<lds_u8_ptr>((uintptr_t)(uint32_t)idx)[M::WBYTES];
                         }
                         // bytes 0 of the four results side by side: two byte permutes and an or
                         mine[nt][q] = (int)(__builtin_amdgcn_perm(r4[1], r4[0], 0x0c0c0400u) | __builtin_amdgcn_perm(r4[3], r4[2], 0x04000c0cu));
                         if (!ADAPT) sbd = dot4(mine[nt][q], dnb32[8 * nt + 2 * q + gL], sbd);
                         else {
-                            const int nz4 = dnb32[8 * nt + 2 * q + gL], q4 = *reinterpret_cast<const int *>(p.q_dn + n0);
+                            const v4f n4 = *reinterpret_cast<const v4f *>(reinterpret_cast<const float *>(dnB) + n0);
 #pragma unroll
                             for (int e = 0; e < 4; e++) {
+                                // (int)((float)pb + x * n * q / 64)
                                 const int idx = ADAPT ? (nt * 4 + q) * 4 + e : 0;
-                                const int prev = (it & 3) ? pb[idx] : 0;
-                                // (int)((float)pb + x * n * q / 64): every value is a multiple of 1/64 below 2^24
-                                pb[idx] = div_pow2_trunc<6>((prev << 6) + mul24(mul24(sx8((int)r4[e], 0), sx8(nz4, e)), sx8(q4, e)));
+                                pb[idx] = truncf(fmaf((float)(int)r4[e], n4[e], pb[idx]));
                             }
                         }
                     }
                 if (ADAPT && (it & 3) == 3) {
 #pragma unroll
-                    for (int i2 = 0; i2 < (ADAPT ? NTU * 16 : 1); i2++) sbd += pb[i2];
+                    for (int i2 = 0; i2 < (ADAPT ? NTU * 16 : 1); i2++) { sbd += (int)pb[i2]; pb[i2] = 0.f; }
                 }
                 if (CS == 1) {
 #pragma unroll
@@ -526,9 +559,10 @@ struct QkvCfg {
     static constexpr int PER_SET = 5 * H * 4 + 3 * H;
     static constexpr int XCHG = 0;             // the normalised input is exchanged through the idle W buffer
     static constexpr int SITE = EGG_WAVES * 64;
-    static constexpr int RED = CS > 1 ? 2 * SITE * 4 : 0;       // two reduction sites used alternately
+    static constexpr int RED = CS > 1 ? 2 * SITE * 4 : 0;       // two reduction sites used alternately (overlay: and one for each input-side sum)
     static constexpr int OCC = H == 256 ? 3 : 2;               // workgroups per CU the kernel is built for
-    static int total(int sets) { return WBYTES + sets * PER_SET + XCHG + RED; }
+    static constexpr int per_set(bool adapt) { return PER_SET + (adapt ? 3 * 3 * H : 0); }        // the overlay's qB kB vB are floats
+    static int total(int sets, bool adapt) { return WBYTES + sets * per_set(adapt) + XCHG + RED + (adapt && CS > 1 ? 3 * SITE * 4 : 0); }
 };
 
 // apply_rope_integer (mgpu.cu:624-644) on the raw accumulators of one token.  The (cos, sin) pairs repeat every
@@ -561,9 +595,11 @@ __device__ __forceinline__ void rope_inplace(v16i *acc, const int32_t *rope_row,
 }
 
 // ADAPT: the d-eggs adaptive noise overlay is on (de/include/model/layers.cuh:313-351): output-side noise and vector
-// noise are scaled when the per-member tables are filled, the input-side sums take the slow term-by-term form.
+// noise are scaled when the per-member tables are filled, the input-side sums are taken term by term (dot_noise_ov), each
+// wave of a tile over its own column slice, and added up with the exchange of the normalised input.  Hidden 256, 2048
+// members x 256 tokens: 0.49 -> 0.32 ms with that and the float terms; without the overlay 0.29.
 template <int H, bool ADAPT>
-__global__ void __launch_bounds__(EGG_THREADS, ADAPT ? 2 : QkvCfg<H>::OCC) k_qkv(QkvParams p) {
+__global__ void __launch_bounds__(EGG_THREADS, QkvCfg<H>::OCC) k_qkv(QkvParams p) {
     typedef QkvCfg<H> Q;
     constexpr int CS = Q::CS, KS = Q::KS, NTS = Q::NTS, HS = Q::HS;
     extern __shared__ __align__(16) int8_t smem[];
@@ -572,11 +608,12 @@ __global__ void __launch_bounds__(EGG_THREADS, ADAPT ? 2 : QkvCfg<H>::OCC) k_qkv
     const int T = c.T;
     const TileMap tm = tile_map<CS>(c.tn, wave, blockIdx.x);
     const int col0 = tm.cs * HS;
-    int8_t *tb = smem + Q::WBYTES + tm.set * Q::PER_SET;
+    constexpr int PSET = Q::per_set(ADAPT);
+    int8_t *tb = smem + Q::WBYTES + tm.set * PSET;
     int *lnw = reinterpret_cast<int *>(tb), *lnb = lnw + H;
     int *qA = lnb + H, *kA = qA + H, *vA = kA + H;
     int8_t *qB = reinterpret_cast<int8_t *>(vA + H), *kB = qB + H, *vB = kB + H;
-    int8_t *xch = smem + Q::WBYTES + tm.sets * Q::PER_SET;
+    int8_t *xch = smem + Q::WBYTES + tm.sets * PSET;
     int *red = reinterpret_cast<int *>(xch + Q::XCHG);
 
     WStream ws; wstream_init(ws, smem, Q::UNIT);
@@ -588,7 +625,7 @@ __global__ void __launch_bounds__(EGG_THREADS, ADAPT ? 2 : QkvCfg<H>::OCC) k_qkv
         int ml = blockIdx.x * tm.sets + ss; if (ml >= c.n_members) ml = c.n_members - 1;
         const int mem = c.pop_offset + ml, nsx = (mem & 1) ? -1 : 1;
         const uint32_t sbx = *c.d_step_seed + (uint32_t)(mem / 2) + (uint32_t)p.seed_base;
-        int8_t *t2 = smem + Q::WBYTES + ss * Q::PER_SET;
+        int8_t *t2 = smem + Q::WBYTES + ss * PSET;
         int *lw = reinterpret_cast<int *>(t2), *lb = lw + H;
         int *a0 = lb + H, *a1 = a0 + H, *a2 = a1 + H;
         int8_t *b0 = reinterpret_cast<int8_t *>(a2 + H), *b1 = b0 + H, *b2 = b1 + H;
@@ -599,16 +636,20 @@ __global__ void __launch_bounds__(EGG_THREADS, ADAPT ? 2 : QkvCfg<H>::OCC) k_qkv
             fill_noise_i32_ov(a0, sbx + OFF_Q_A, H, c.mask, nsx, tid, EGG_THREADS, p.q_wq + H);
             fill_noise_i32_ov(a1, sbx + OFF_K_A, H, c.mask, nsx, tid, EGG_THREADS, p.q_wk + H);
             fill_noise_i32_ov(a2, sbx + OFF_V_A, H, c.mask, nsx, tid, EGG_THREADS, p.q_wv + H);
+            float *f0 = reinterpret_cast<float *>(b0);
+            fill_noise_f32_ov(f0, sbx + OFF_Q_B, H, c.mask, tid, EGG_THREADS, p.q_wq);
+            fill_noise_f32_ov(f0 + H, sbx + OFF_K_B, H, c.mask, tid, EGG_THREADS, p.q_wk);
+            fill_noise_f32_ov(f0 + 2 * H, sbx + OFF_V_B, H, c.mask, tid, EGG_THREADS, p.q_wv);
         } else {
             fill_vec_i32(lw, p.ln_w, sbx + OFF_LN_1_A, sbx + OFF_LN_1_B, H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS, 2);     // 4 * gain, see standard_scale
             fill_vec_i32(lb, p.ln_b, sbx + OFF_LN_1_BIAS_A, sbx + OFF_LN_1_BIAS_B, H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS);
             fill_noise_i32(a0, sbx + OFF_Q_A, H, c.mask, nsx, tid, EGG_THREADS);
             fill_noise_i32(a1, sbx + OFF_K_A, H, c.mask, nsx, tid, EGG_THREADS);
             fill_noise_i32(a2, sbx + OFF_V_A, H, c.mask, nsx, tid, EGG_THREADS);
+            fill_noise_i8(b0, sbx + OFF_Q_B, H, c.mask, tid, EGG_THREADS);
+            fill_noise_i8(b1, sbx + OFF_K_B, H, c.mask, tid, EGG_THREADS);
+            fill_noise_i8(b2, sbx + OFF_V_B, H, c.mask, tid, EGG_THREADS);
         }
-        fill_noise_i8(b0, sbx + OFF_Q_B, H, c.mask, tid, EGG_THREADS);
-        fill_noise_i8(b1, sbx + OFF_K_B, H, c.mask, tid, EGG_THREADS);
-        fill_noise_i8(b2, sbx + OFF_V_B, H, c.mask, tid, EGG_THREADS);
     }
     __syncthreads();
 
@@ -620,6 +661,7 @@ __global__ void __launch_bounds__(EGG_THREADS, ADAPT ? 2 : QkvCfg<H>::OCC) k_qkv
         const int t = c.t0 + (tm.tile0 + Q::TPW * pass) * 32 + j;
         const size_t row = ((size_t)mloc * T + t) * H;
         v4i nrm[KS];
+        int sb3[3];
         {
             v4i x[NTS];
 #pragma unroll
@@ -632,9 +674,15 @@ __global__ void __launch_bounds__(EGG_THREADS, ADAPT ? 2 : QkvCfg<H>::OCC) k_qkv
             else {
                 v4i mine[NTS];
                 standard_scale<NTS>(x, mine, mn, lnw, lnb, col0, g);
+                if (ADAPT) {
+                    dot_noise_ov<NTS, 3>(mine, reinterpret_cast<const float *>(qB) + col0, H, g, sb3);
+#pragma unroll
+                    for (int i = 0; i < 3; i++) xput(sb3[i], red + (2 + i) * Q::SITE, CS, tm, lane);
+                }
                 exchange_operand<CS, NTS, KS, Q::TPW, Q::UNIT>(ws.other, tm, lane, mine, nrm);
             }
         }
+        if (ADAPT && CS == 1) dot_noise_ov<KS, 3>(nrm, reinterpret_cast<const float *>(qB), H, g, sb3);
 #pragma unroll 1
         for (int which = 0; which < 3; which++) {
             const int8_t *W = which == 0 ? p.w_q : (which == 1 ? p.w_k : p.w_v);
@@ -642,8 +690,8 @@ __global__ void __launch_bounds__(EGG_THREADS, ADAPT ? 2 : QkvCfg<H>::OCC) k_qkv
             const int8_t *Bn = which == 0 ? qB : (which == 1 ? kB : vB);
             const int *An = which == 0 ? qA : (which == 1 ? kA : vA);
             int8_t *dst = which == 0 ? p.q : (which == 1 ? p.k : p.v);
-            const int sb = ADAPT ? dot_noise_ov<KS, false>(nrm, Bn, which == 0 ? p.q_wq : (which == 1 ? p.q_wk : p.q_wv), 0, g)
-                                 : dot_noise<KS, false>(nrm, Bn, 0, g);
+            const int sb = !ADAPT ? dot_noise<KS, false>(nrm, Bn, 0, g) : CS > 1 ? xget<CS, false>(red + (2 + which) * Q::SITE, tm, lane)
+                                  : which == 0 ? sb3[0] : which == 1 ? sb3[1] : sb3[2];
             v16i acc[NTS];
             zero_acc<NTS>(acc);
 #pragma unroll
@@ -1086,9 +1134,9 @@ __global__ void __launch_bounds__(EGG_THREADS, (AttnWg<HD, CT>::OCC)) k_attn_wg(
 // ============================================================================ head + loss
 template <int H>
 struct HeadLds {
-    static constexpr int PER_WAVE = (2 * H + 256) * 4 + H;   // lnw lnb hA[256] + hB[H]
+    static constexpr int per_wave(bool adapt) { return (2 * H + 256) * 4 + (adapt ? 4 : 1) * H; }   // lnw lnb hA[256] + hB[H] (overlay: floats)
     static constexpr int WBLOCK = 2 * WUnit<(H < 256 ? H : 256)>::BYTES;   // double-buffered W units
-    static constexpr int TOTAL = WBLOCK + 1024 + EGG_WAVES * PER_WAVE;
+    static constexpr int total(bool adapt) { return WBLOCK + 1024 + EGG_WAVES * per_wave(adapt); }
 };
 
 // ADAPT: adaptive noise overlay; the tied head takes the embedding's per-hidden q values on its input side and the
@@ -1101,7 +1149,7 @@ __global__ void __launch_bounds__(EGG_THREADS, (H > 256 ? 1 : 2)) k_head(HeadPar
     int8_t *wlds = smem;
     int *lut = reinterpret_cast<int *>(smem + HeadLds<H>::WBLOCK);
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 5, j = lane & 31;
-    int8_t *tb = smem + HeadLds<H>::WBLOCK + 1024 + wave * HeadLds<H>::PER_WAVE;
+    int8_t *tb = smem + HeadLds<H>::WBLOCK + 1024 + wave * HeadLds<H>::per_wave(ADAPT);
     int *lnw = reinterpret_cast<int *>(tb), *lnb = lnw + H, *hA = lnb + H;
     int8_t *hB = reinterpret_cast<int8_t *>(hA + 256);
 
@@ -1134,7 +1182,8 @@ __global__ void __launch_bounds__(EGG_THREADS, (H > 256 ? 1 : 2)) k_head(HeadPar
         if (ADAPT) fill_noise_i32_ov(hA, pair_seed + OFF_EMB, 256, c.mask, ns, lane, 64, p.q_emb + H);
         else fill_noise_i32(hA, pair_seed + OFF_EMB, 256, c.mask, ns, lane);
     }
-    fill_noise_i8(hB, pair_seed + OFF_EMB + H, H, c.mask, lane);
+    if (ADAPT) fill_noise_f32_ov(reinterpret_cast<float *>(hB), pair_seed + OFF_EMB + H, H, c.mask, lane, 64, p.q_emb);
+    else fill_noise_i8(hB, pair_seed + OFF_EMB + H, H, c.mask, lane);
     __syncthreads();
 
     const int64_t spos = stream_pos_of(c, member);
@@ -1147,7 +1196,9 @@ __global__ void __launch_bounds__(EGG_THREADS, (H > 256 ? 1 : 2)) k_head(HeadPar
 #pragma unroll
         for (int ks = 0; ks < KS; ks++) x[ks] = load_op(p.x + row, ks, g);
         standard_norm<KS>(x, nf, lnw, lnb, g);
-        const int sbh = ADAPT ? dot_noise_ov<KS, false>(nf, hB, p.q_emb, 0, g) : dot_noise<KS, false>(nf, hB, 0, g);
+        int sbh;
+        if (ADAPT) dot_noise_ov<KS, 1>(nf, reinterpret_cast<const float *>(hB), 0, g, &sbh);
+        else sbh = dot_noise<KS, false>(nf, hB, 0, g);
         int gmax = INT_MIN, target;
         long long sum_ex; int tl;
         // two-pass softmax statistics (mgpu.cu:969-1009)
@@ -1256,7 +1307,7 @@ template <int H>
 static hipError_t launch_mlp_h(const MlpParams &p, bool first, hipStream_t s) {
     const int sets = tile_map_sets(p.c.tn, MlpCfg<H>::CS);
     dim3 grid((p.c.n_members + sets - 1) / sets), block(EGG_THREADS);
-    size_t lds = MlpCfg<H>::total(sets, first);
+    size_t lds = MlpCfg<H>::total(sets, first, p.q_ln_w != nullptr);
     // The up accumulator is seeded with (bias + 128 + noise) << shift_mlp_up (see the bias table), so its range is the
     // GEMM's plus that seed; the fused perturb-and-shift needs |acc| * 2^sigma + |sb * a| below 2^31 for it as well.
     const long long mag = egg_noise_magnitude(p.c.mask);
@@ -1264,9 +1315,9 @@ static hipError_t launch_mlp_h(const MlpParams &p, bool first, hipStream_t s) {
     const bool up_fits = p.c.sigma >= 0 && p.c.sigma < 31 && (up_acc << p.c.sigma) + (long long)H * 127 * mag * mag < (1LL << 31);
     const bool fuse = p.c.sigma <= 7 && mag <= 15 && up_fits;
     if (up_acc >= (1LL << 31)) return hipErrorInvalidValue;      // egg_ctx_create refuses such shifts
-    if (p.q_ln_w) {      // adaptive noise overlay: one (unfused) variant
-        if (first) hipLaunchKernelGGL((k_mlp<H, true, false, true>), grid, block, lds, s, p);
-        else hipLaunchKernelGGL((k_mlp<H, false, false, true>), grid, block, lds, s, p);
+    if (p.q_ln_w) {      // adaptive noise overlay: its factors are at most 1, so the same bounds hold
+        if (first) { if (fuse) hipLaunchKernelGGL((k_mlp<H, true, true, true>), grid, block, lds, s, p); else hipLaunchKernelGGL((k_mlp<H, true, false, true>), grid, block, lds, s, p); }
+        else { if (fuse) hipLaunchKernelGGL((k_mlp<H, false, true, true>), grid, block, lds, s, p); else hipLaunchKernelGGL((k_mlp<H, false, false, true>), grid, block, lds, s, p); }
         return hipGetLastError();
     }
     if (first) { if (fuse) hipLaunchKernelGGL((k_mlp<H, true, true, false>), grid, block, lds, s, p); else hipLaunchKernelGGL((k_mlp<H, true, false, false>), grid, block, lds, s, p); }
@@ -1287,7 +1338,7 @@ template <int H>
 static hipError_t launch_qkv_h(const QkvParams &p, hipStream_t s) {
     const int sets = tile_map_sets(p.c.tn, QkvCfg<H>::CS);
     dim3 grid((p.c.n_members + sets - 1) / sets), block(EGG_THREADS);
-    size_t lds = QkvCfg<H>::total(sets);
+    size_t lds = QkvCfg<H>::total(sets, p.q_ln_w != nullptr);
     if (p.q_ln_w) hipLaunchKernelGGL((k_qkv<H, true>), grid, block, lds, s, p);
     else hipLaunchKernelGGL((k_qkv<H, false>), grid, block, lds, s, p);
     return hipGetLastError();
@@ -1337,7 +1388,7 @@ hipError_t egg_launch_attn(const AttnParams &p, hipStream_t s) {
 template <int H>
 static hipError_t launch_head_h(const HeadParams &p, hipStream_t s) {
     dim3 grid((p.c.n_members + EGG_WAVES - 1) / EGG_WAVES), block(EGG_THREADS);
-    size_t lds = HeadLds<H>::TOTAL;
+    size_t lds = HeadLds<H>::total(p.q_ln_w != nullptr);
     if (p.c.vocab < 256 || p.c.vocab % 256) return hipErrorInvalidValue;
     if (p.c.vocab > 256) {
         if (p.q_ln_w) hipLaunchKernelGGL((k_head<H, true, true>), grid, block, lds, s, p);
@@ -1375,20 +1426,23 @@ static hipError_t prepare_h(int T) {
     const int msets = std::max(tile_map_sets(T, MlpCfg<H>::CS), tile_map_sets(32, MlpCfg<H>::CS));
     for (hipError_t e : {no_static_lds(&k_mlp<H, true, true, false>), no_static_lds(&k_mlp<H, false, true, false>),
                          no_static_lds(&k_mlp<H, true, false, false>), no_static_lds(&k_mlp<H, false, false, false>),
+                         no_static_lds(&k_mlp<H, true, true, true>), no_static_lds(&k_mlp<H, false, true, true>),
                          no_static_lds(&k_mlp<H, true, false, true>), no_static_lds(&k_mlp<H, false, false, true>)})
         if (e != hipSuccess) return e;
-    SET_LDS((k_mlp<H, true, true, false>), MlpCfg<H>::total(msets, true));
-    SET_LDS((k_mlp<H, false, true, false>), MlpCfg<H>::total(msets, false));
-    SET_LDS((k_mlp<H, true, false, false>), MlpCfg<H>::total(msets, true));
-    SET_LDS((k_mlp<H, false, false, false>), MlpCfg<H>::total(msets, false));
-    SET_LDS((k_mlp<H, true, false, true>), MlpCfg<H>::total(msets, true));
-    SET_LDS((k_mlp<H, false, false, true>), MlpCfg<H>::total(msets, false));
-    SET_LDS((k_qkv<H, false>), QkvCfg<H>::total(sets));
-    SET_LDS((k_qkv<H, true>), QkvCfg<H>::total(sets));
-    SET_LDS((k_head<H, false, false>), HeadLds<H>::TOTAL);
-    SET_LDS((k_head<H, true, false>), HeadLds<H>::TOTAL);
-    SET_LDS((k_head<H, false, true>), HeadLds<H>::TOTAL);
-    SET_LDS((k_head<H, true, true>), HeadLds<H>::TOTAL);
+    SET_LDS((k_mlp<H, true, true, false>), MlpCfg<H>::total(msets, true, false));
+    SET_LDS((k_mlp<H, false, true, false>), MlpCfg<H>::total(msets, false, false));
+    SET_LDS((k_mlp<H, true, false, false>), MlpCfg<H>::total(msets, true, false));
+    SET_LDS((k_mlp<H, false, false, false>), MlpCfg<H>::total(msets, false, false));
+    SET_LDS((k_mlp<H, true, false, true>), MlpCfg<H>::total(msets, true, true));
+    SET_LDS((k_mlp<H, true, true, true>), MlpCfg<H>::total(msets, true, true));
+    SET_LDS((k_mlp<H, false, false, true>), MlpCfg<H>::total(msets, false, true));
+    SET_LDS((k_mlp<H, false, true, true>), MlpCfg<H>::total(msets, false, true));
+    SET_LDS((k_qkv<H, false>), QkvCfg<H>::total(sets, false));
+    SET_LDS((k_qkv<H, true>), QkvCfg<H>::total(sets, true));
+    SET_LDS((k_head<H, false, false>), HeadLds<H>::total(false));
+    SET_LDS((k_head<H, true, false>), HeadLds<H>::total(true));
+    SET_LDS((k_head<H, false, true>), HeadLds<H>::total(false));
+    SET_LDS((k_head<H, true, true>), HeadLds<H>::total(true));
     return hipSuccess;
 }
 template <int HD, int CT>

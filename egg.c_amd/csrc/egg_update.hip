@@ -299,7 +299,7 @@ __global__ void k_scale_by_norm(float *x, const float *norm, int n) {
 // w, w + 4, ...); within a block, MFMA e multiplies the k pair {8c + e, 8c + 4 + e}.  The partial tiles are added in wave
 // order in LDS, so the summation order is fixed and results are reproducible; wave q writes rows 8q + 4g + e of the
 // tile.  mode 0: C = alpha * acc.  mode 1: C = (i == j ? 3 : 0) - acc  (3I - G, muon_internal.cuh:91-109).
-typedef float v4f __attribute__((ext_vector_type(4)));
+
 template <bool AK, bool BK>
 __global__ void __launch_bounds__(EGG_THREADS) k_sgemm(const float *A, long lda, long batch_a, const float *B, long ldb, long batch_b,
                                                       float *C, int M, int N, int K, float alpha, int mode) {
