@@ -176,7 +176,7 @@ __global__ void __launch_bounds__(EGG_THREADS, MlpCfg<H>::occ(ADAPT)) k_mlp(MlpP
     // pointer instead, every read carries an extra add of that (zero) base.
     typedef const __attribute__((address_space(3))) uint8_t *lds_u8_ptr;
     typedef const __attribute__((address_space(3))) int8_t *lds_i8_ptr;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, g = lane >> 5, j = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const FwdCommon &c = p.c;
     const int T = c.T;
     const TileMap tm = tile_map<CS>(c.tn, wave, blockIdx.x);

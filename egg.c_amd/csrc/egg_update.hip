@@ -352,10 +352,26 @@ __global__ void __launch_bounds__(EGG_THREADS) k_sgemm(const float *A, long lda,
 // reads of four consecutive k, a 2-way bank conflict at most); the other kind as [k][row] with k rows TILE + 8 floats
 // apart (4-byte reads; the two lane halves, four k rows apart, fall on different banks).
 // Within a block of eight k, MFMA e multiplies the pair {8c + e, 8c + 4 + e}, blocks in ascending order, whatever WT
-// is: the two tile sizes give bit-identical results, so the host may pick by the size of the grid.  Epilogues as above.
-template <bool AK, bool BK, int WT>
-__global__ void __launch_bounds__(EGG_THREADS, 2) k_sgemm_lds(const float *A, long lda, long batch_a, const float *B, long ldb, long batch_b,
-                                                             float *C, int M, int N, int K, float alpha, int mode) {
+// is: the two tile sizes give bit-identical results, so the host may pick by the size of the grid.
+// SYM: C is symmetric; only tiles on and above the diagonal are computed, elements above it are stored twice (36 of 64 tiles
+// at 512 columns).
+// A launch may multiply two left sides with the same B (blockIdx.z).  Epilogues, v the sum over k, e0 and e1 elements of
+// other matrices at the same place:
+enum { NS_SCALE, NS_B, NS_GRAM, NS_STEP, NS_FACTOR };
+struct SgemmJob {
+    const float *A; long batch_a; float *C; const float *e0, *e1; float *C2; int mode; float alpha;
+};
+struct SgemmJobs { SgemmJob j[2]; };
+__device__ __forceinline__ float ns_epilogue(const SgemmJob &job, float v, bool diag, size_t at) {
+    switch (job.mode) {
+        case NS_B: return (diag ? 3.0f : 0.0f) - v;                       // 3I - G (muon_internal.cuh:91-109)
+        case NS_STEP: return 0.25f * ((9.0f * job.e0[at] - 6.0f * job.e1[at]) + v);      // G (3I - G)^2 / 4 from G, G^2, G^3
+        case NS_FACTOR: return 0.5f * (3.0f * job.e0[at] - v);            // P (3I - G) / 2
+        default: return job.alpha * v;
+    }
+}
+template <bool AK, bool BK, int WT, bool SYM>
+__global__ void __launch_bounds__(EGG_THREADS, WT == 1 ? 4 : 2) k_sgemm_lds(SgemmJobs jobs, long lda, const float *B, long ldb, long batch_b, int M, int N, int K) {
     constexpr int TILE = 64 * WT, KC = 32, LDK = 36, LDI = TILE + 8, PIECES = TILE * KC / 4 / EGG_THREADS;
     constexpr int ASZ = AK ? TILE * LDK : KC * LDI, BSZ = BK ? TILE * LDK : KC * LDI;
     constexpr int RPI = TILE / 4;                 // 16-byte pieces per k row of an [k][row] chunk
@@ -363,9 +379,18 @@ __global__ void __launch_bounds__(EGG_THREADS, 2) k_sgemm_lds(const float *A, lo
     __shared__ __align__(16) float Bs[BSZ];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 5, j = lane & 31, tid = threadIdx.x;
     const int wm = wave >> 1, wn = wave & 1;
-    const int tiles_n = N / TILE, tile = blockIdx.x;
-    const int i0 = (tile / tiles_n) * TILE, j0 = (tile % tiles_n) * TILE;
-    A += (long)blockIdx.y * batch_a; B += (long)blockIdx.y * batch_b; C += (size_t)blockIdx.y * M * N;
+    const int tiles_n = N / TILE;
+    int ti = blockIdx.x / tiles_n, tj = blockIdx.x % tiles_n;
+    if (SYM) {
+        ti = 0; tj = blockIdx.x;
+        while (tj >= tiles_n - ti) { tj -= tiles_n - ti; ti++; }
+        tj += ti;
+    }
+    const int i0 = ti * TILE, j0 = tj * TILE;
+    const SgemmJob job = jobs.j[blockIdx.z];
+    const float *const A = job.A + (long)blockIdx.y * job.batch_a;
+    B += (long)blockIdx.y * batch_b;
+    const size_t out = (size_t)blockIdx.y * M * N;
     v16f acc[WT][WT];
 #pragma unroll
     for (int a = 0; a < WT; a++)
@@ -433,20 +458,41 @@ __global__ void __launch_bounds__(EGG_THREADS, 2) k_sgemm_lds(const float *A, lo
 #pragma unroll
         for (int tb = 0; tb < WT; tb++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int i = i0 + 32 * WT * wm + 32 * ta + 8 * (r >> 2) + 4 * g + (r & 3), jj = j0 + 32 * WT * wn + 32 * tb + j;
-                const float v = acc[ta][tb][r];
-                C[(size_t)i * N + jj] = (mode == 1) ? ((i == jj ? 3.0f : 0.0f) - v) : alpha * v;
+            for (int q = 0; q < 4; q++) {
+                const int i = i0 + 32 * WT * wm + 32 * ta + 8 * q + 4 * g, jj = j0 + 32 * WT * wn + 32 * tb + j;
+                v4f v;
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const size_t at = out + (size_t)(i + e) * N + jj;
+                    v[e] = ns_epilogue(job, acc[ta][tb][4 * q + e], i + e == jj, at);
+                    if (!SYM || i + e <= jj) {
+                        job.C[at] = v[e];
+                        if (SYM && job.mode == NS_GRAM) job.C2[at] = (i + e == jj ? 1.5f : 0.0f) - 0.5f * v[e];
+                    }
+                }
+                if (SYM) {
+                    const size_t at = out + (size_t)jj * N + i;
+                    if (ti < tj) {
+                        *reinterpret_cast<v4f *>(job.C + at) = v;
+                        if (job.mode == NS_GRAM) *reinterpret_cast<v4f *>(job.C2 + at) = -0.5f * v;
+                    } else
+#pragma unroll
+                        for (int e = 0; e < 4; e++)
+                            if (i + e < jj) {
+                                job.C[at + e] = v[e];
+                                if (job.mode == NS_GRAM) job.C2[at + e] = -0.5f * v[e];
+                            }
+                }
             }
 }
-template <int WT>
-static hipError_t sgemm_lds(bool ak, bool bk, const float *A, long lda, long batch_a, const float *B, long ldb, long batch_b, float *C,
-                            int M, int N, int K, float alpha, int mode, int batch, hipStream_t s) {
-    const dim3 grid((M / (64 * WT)) * (N / (64 * WT)), batch), block(EGG_THREADS);
-    if (ak && bk) hipLaunchKernelGGL((k_sgemm_lds<true, true, WT>), grid, block, 0, s, A, lda, batch_a, B, ldb, batch_b, C, M, N, K, alpha, mode);
-    else if (ak) hipLaunchKernelGGL((k_sgemm_lds<true, false, WT>), grid, block, 0, s, A, lda, batch_a, B, ldb, batch_b, C, M, N, K, alpha, mode);
-    else if (bk) hipLaunchKernelGGL((k_sgemm_lds<false, true, WT>), grid, block, 0, s, A, lda, batch_a, B, ldb, batch_b, C, M, N, K, alpha, mode);
-    else hipLaunchKernelGGL((k_sgemm_lds<false, false, WT>), grid, block, 0, s, A, lda, batch_a, B, ldb, batch_b, C, M, N, K, alpha, mode);
+template <int WT, bool SYM>
+static hipError_t sgemm_lds(bool ak, bool bk, const SgemmJobs &jobs, int n_jobs, long lda, const float *B, long ldb, long batch_b, int M, int N, int K, int batch, hipStream_t s) {
+    const int tm = M / (64 * WT), tn = N / (64 * WT);
+    const dim3 grid(SYM ? tn * (tn + 1) / 2 : tm * tn, batch, n_jobs), block(EGG_THREADS);
+    if (ak && bk) hipLaunchKernelGGL((k_sgemm_lds<true, true, WT, SYM>), grid, block, 0, s, jobs, lda, B, ldb, batch_b, M, N, K);
+    else if (ak) hipLaunchKernelGGL((k_sgemm_lds<true, false, WT, SYM>), grid, block, 0, s, jobs, lda, B, ldb, batch_b, M, N, K);
+    else if (bk) hipLaunchKernelGGL((k_sgemm_lds<false, true, WT, SYM>), grid, block, 0, s, jobs, lda, B, ldb, batch_b, M, N, K);
+    else hipLaunchKernelGGL((k_sgemm_lds<false, false, WT, SYM>), grid, block, 0, s, jobs, lda, B, ldb, batch_b, M, N, K);
     return hipGetLastError();
 }
 static int egg_update_cu_count() {
@@ -459,27 +505,33 @@ static int egg_update_cu_count() {
     return n;
 }
 // A(i,k) at A[i * sa_i + k * sa_k], B(k,j) at B[k * sb_k + j * sb_j]; one stride of each pair must be 1 and the other a
-// multiple of 4 (16-byte loads)
-static hipError_t sgemm(const float *A, long sa_i, long sa_k, long batch_a, const float *B, long sb_k, long sb_j, long batch_b, float *C, int M, int N, int K,
-                        float alpha, int mode, int batch, hipStream_t s) {
+// multiple of 4 (16-byte loads).  sym: the result is symmetric.
+static hipError_t sgemm(const SgemmJobs &jobs, int n_jobs, long sa_i, long sa_k, const float *B, long sb_k, long sb_j, long batch_b, int M, int N, int K,
+                        bool sym, int batch, hipStream_t s) {
     const bool ak = sa_k == 1, bk = sb_k == 1;
     if ((!ak && sa_i != 1) || (!bk && sb_j != 1) || M % 32 || N % 32 || K % 32) return hipErrorInvalidValue;
     const long lda = ak ? sa_i : sa_k, ldb = bk ? sb_j : sb_k;
-    if (lda % 4 || ldb % 4 || batch_a % 4 || batch_b % 4) return hipErrorInvalidValue;
+    if (lda % 4 || ldb % 4 || jobs.j[0].batch_a % 4 || batch_b % 4) return hipErrorInvalidValue;
     // The LDS-staged kernel where the shape allows it: 128 x 128 tiles when they still fill the GPU, 64 x 64 tiles otherwise
     // (bit-identical results, so the choice may depend on the batch)
     if (M % 64 == 0 && N % 64 == 0) {
-        const bool big = M % 128 == 0 && N % 128 == 0 && (long)(M / 128) * (N / 128) * batch >= 2 * egg_update_cu_count();
-        return big ? sgemm_lds<2>(ak, bk, A, lda, batch_a, B, ldb, batch_b, C, M, N, K, alpha, mode, batch, s)
-                   : sgemm_lds<1>(ak, bk, A, lda, batch_a, B, ldb, batch_b, C, M, N, K, alpha, mode, batch, s);
+        const long tiles = sym ? (long)(N / 128) * (N / 128 + 1) / 2 : (long)(M / 128) * (N / 128);
+        const bool big = M % 128 == 0 && N % 128 == 0 && tiles * batch * n_jobs >= 2 * egg_update_cu_count();
+        if (sym) return big ? sgemm_lds<2, true>(ak, bk, jobs, n_jobs, lda, B, ldb, batch_b, M, N, K, batch, s)
+                            : sgemm_lds<1, true>(ak, bk, jobs, n_jobs, lda, B, ldb, batch_b, M, N, K, batch, s);
+        return big ? sgemm_lds<2, false>(ak, bk, jobs, n_jobs, lda, B, ldb, batch_b, M, N, K, batch, s)
+                   : sgemm_lds<1, false>(ak, bk, jobs, n_jobs, lda, B, ldb, batch_b, M, N, K, batch, s);
     }
+    const SgemmJob &j = jobs.j[0];
+    if (n_jobs != 1 || j.mode > NS_B) return hipErrorInvalidValue;
     const dim3 grid((M / 32) * (N / 32), batch), block(EGG_THREADS);
-    if (ak && bk) hipLaunchKernelGGL((k_sgemm<true, true>), grid, block, 0, s, A, lda, batch_a, B, ldb, batch_b, C, M, N, K, alpha, mode);
-    else if (ak) hipLaunchKernelGGL((k_sgemm<true, false>), grid, block, 0, s, A, lda, batch_a, B, ldb, batch_b, C, M, N, K, alpha, mode);
-    else if (bk) hipLaunchKernelGGL((k_sgemm<false, true>), grid, block, 0, s, A, lda, batch_a, B, ldb, batch_b, C, M, N, K, alpha, mode);
-    else hipLaunchKernelGGL((k_sgemm<false, false>), grid, block, 0, s, A, lda, batch_a, B, ldb, batch_b, C, M, N, K, alpha, mode);
+    if (ak && bk) hipLaunchKernelGGL((k_sgemm<true, true>), grid, block, 0, s, j.A, lda, j.batch_a, B, ldb, batch_b, j.C, M, N, K, j.alpha, j.mode);
+    else if (ak) hipLaunchKernelGGL((k_sgemm<true, false>), grid, block, 0, s, j.A, lda, j.batch_a, B, ldb, batch_b, j.C, M, N, K, j.alpha, j.mode);
+    else if (bk) hipLaunchKernelGGL((k_sgemm<false, true>), grid, block, 0, s, j.A, lda, j.batch_a, B, ldb, batch_b, j.C, M, N, K, j.alpha, j.mode);
+    else hipLaunchKernelGGL((k_sgemm<false, false>), grid, block, 0, s, j.A, lda, j.batch_a, B, ldb, batch_b, j.C, M, N, K, j.alpha, j.mode);
     return hipGetLastError();
 }
+static SgemmJobs one_job(const float *A, long batch_a, float *C, int mode, float alpha = 1.f) { return SgemmJobs{{{A, batch_a, C, nullptr, nullptr, nullptr, mode, alpha}, {}}}; }
 __global__ void k_copy_f32(float *dst, const float *src, size_t n) {
     size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) dst[i] = src[i];
@@ -499,15 +551,54 @@ hipError_t egg_launch_newton_schulz_batched(const MuonWork &w, int rows, int col
     hipLaunchKernelGGL(k_scale_by_norm, dim3((n + 255) / 256, batch), dim3(256), 0, s, w.x, w.norm, n);
     float *cur = w.x, *nxt = w.swap;          // ping-pong instead of copying back after every iteration
     hipError_t e = hipSuccess;
+    // The Gram form.  An iteration X <- X (3I - G) / 2 with G = X^T X changes G to G (3I - G)^2 / 4, so the factors of all
+    // iterations can be multiplied up among short x short matrices and X once with their product: with k = the short side
+    // and r = long / short, 3/2 r + 6 products of k^3 for five iterations where each one on X itself takes 15/2 r (counting
+    // a symmetric product as half).  Used from r = 4 on, which is also where the second matrix buffer holds the four
+    // k x k matrices it needs; r = 1, the other shape of the models, would gain nothing.  In float32 it is closer to the
+    // exact iteration than that on X (relative error 3e-7 against 6e-7 for random matrices, 1.4e-6 against 4.3e-6 at rank
+    // one); but G is not computed from X again, and an eigenvalue that should be 0 grows 9/4-fold an iteration, so it is kept to
+    // eight iterations.  9 matrices of 512 x 2048, 5 iterations: 1.23 -> %GRAM% ms.
+    if (K % 64 == 0 && iters >= 1 && iters <= 8 && (long)rows * cols >= 4 * kk) {
+        float *G = w.swap, *S = w.swap + kk * batch, *next = w.swap + 2 * kk * batch;
+        float *P = iters & 1 ? w.bterm : w.swap + 3 * kk * batch, *Pn = iters & 1 ? w.swap + 3 * kk * batch : w.bterm;      // the last one in bterm
+        SgemmJobs gram = one_job(cur, n, G, NS_GRAM);
+        gram.j[0].C2 = P;
+        e = use_rows ? sgemm(gram, 1, cols, 1, cur, 1, cols, n, K, K, cols, true, batch, s)
+                     : sgemm(gram, 1, 1, cols, cur, cols, 1, n, K, K, rows, true, batch, s);
+        for (int it = 1; it < iters && e == hipSuccess; it++) {
+            // G^2, and the factor of this iteration onto P (the first is its P as it stands)
+            SgemmJobs square = one_job(G, kk, S, NS_SCALE);
+            if (it > 1) {
+                square.j[1] = SgemmJob{P, kk, Pn, P, nullptr, nullptr, NS_FACTOR, 0.f};
+                float *t = P; P = Pn; Pn = t;
+            }
+            e = sgemm(square, it > 1 ? 2 : 1, K, 1, G, 1, K, kk, K, K, K, true, batch, s);
+            if (e != hipSuccess) break;
+            const SgemmJobs step = {{{S, kk, next, G, S, nullptr, NS_STEP, 0.f}, {}}};
+            e = sgemm(step, 1, K, 1, G, 1, K, kk, K, K, K, true, batch, s);
+            float *t = G; G = next; next = t;
+        }
+        if (e == hipSuccess && iters > 1) {
+            const SgemmJobs last = {{{P, kk, Pn, P, nullptr, nullptr, NS_FACTOR, 0.f}, {}}};
+            e = sgemm(last, 1, K, 1, G, 1, K, kk, K, K, K, true, batch, s);
+            P = Pn;
+        }
+        if (e == hipSuccess && P != w.bterm) e = hipErrorUnknown;
+        if (e == hipSuccess) e = use_rows ? sgemm(one_job(P, kk, nxt, NS_SCALE), 1, K, 1, cur, cols, 1, n, rows, cols, K, false, batch, s)
+                                          : sgemm(one_job(cur, n, nxt, NS_SCALE), 1, cols, 1, P, 1, K, kk, rows, cols, K, false, batch, s);
+        cur = nxt;
+    } else
     for (int it = 0; it < iters && e == hipSuccess; it++) {
+        const bool sym = K % 64 == 0;
         if (use_rows) {
             // G = X X^T (rows x rows); X <- 0.5 (3I - G) X
-            e = sgemm(cur, cols, 1, n, cur, 1, cols, n, w.bterm, K, K, cols, 1.f, 1, batch, s);
-            if (e == hipSuccess) e = sgemm(w.bterm, K, 1, kk, cur, cols, 1, n, nxt, rows, cols, K, 0.5f, 0, batch, s);
+            e = sgemm(one_job(cur, n, w.bterm, NS_B), 1, cols, 1, cur, 1, cols, n, K, K, cols, sym, batch, s);
+            if (e == hipSuccess) e = sgemm(one_job(w.bterm, kk, nxt, NS_SCALE, 0.5f), 1, K, 1, cur, cols, 1, n, rows, cols, K, false, batch, s);
         } else {
             // G = X^T X (cols x cols); X <- 0.5 X (3I - G)
-            e = sgemm(cur, 1, cols, n, cur, cols, 1, n, w.bterm, K, K, rows, 1.f, 1, batch, s);
-            if (e == hipSuccess) e = sgemm(cur, cols, 1, n, w.bterm, K, 1, kk, nxt, rows, cols, K, 0.5f, 0, batch, s);
+            e = sgemm(one_job(cur, n, w.bterm, NS_B), 1, 1, cols, cur, cols, 1, n, K, K, rows, sym, batch, s);
+            if (e == hipSuccess) e = sgemm(one_job(cur, n, nxt, NS_SCALE, 0.5f), 1, cols, 1, w.bterm, K, 1, kk, rows, cols, K, false, batch, s);
         }
         float *t = cur; cur = nxt; nxt = t;
     }
