@@ -65,7 +65,7 @@ struct egg_ctx {
     int32_t *h_fit() { return h_loss() + cfg.population; }
     Scalars *d_scal = nullptr;
     // votes and optimizer step (egg_votes.hip): the noise table, and the matrices' descriptors in lists that one launch walks
-    NoiseTable noise = {nullptr, 0, 0, nullptr, nullptr, 0, nullptr};
+    NoiseTable noise = {nullptr, 0, 0, nullptr, nullptr, 0, 0, nullptr};
     struct MatList { int first, count, tiles; };
     MatDesc *d_mat = nullptr;
     MatList mat_all, mat_adam; std::vector<MatList> mat_muon, mat_one;     // every matrix; the AdamW ones; each Muon batch; each on its own (by tensor id)
@@ -458,9 +458,10 @@ extern "C" int egg_ctx_create(const egg_config *cfg, egg_ctx **out) {
     // noise table: the rows of the widest side of any matrix (4 * hidden, or the embedding's vocabulary), every layer's seeds
     ctx->noise.pairs_pad = ((c.population / 2) + 127) / 128 * 128;
     ctx->noise.rows = std::max(4 * c.hidden, c.vocab);
-    ctx->noise.ld = (size_t)(noise_entries(c, ctx->noise.pairs_pad) + 127) / 128 * 128;
+    ctx->noise.ld = egg_noise_ld(noise_entries(c, ctx->noise.pairs_pad)); ctx->noise.mask_ld = egg_noise_mask_ld(ctx->noise.pairs_pad);
     CR(hipMalloc(&ctx->noise.table, ctx->noise.rows * ctx->noise.ld));
-    CR(hipMalloc(&ctx->noise.neg, ctx->noise.pairs_pad)); CR(hipMalloc(&ctx->noise.nonzero, ctx->noise.pairs_pad));
+    CR(hipMalloc(&ctx->noise.neg, 4 * ctx->noise.mask_ld)); CR(hipMalloc(&ctx->noise.nonzero, 4 * ctx->noise.mask_ld));
+    CR(hipMemset(ctx->noise.neg, 0, 4 * ctx->noise.mask_ld)); CR(hipMemset(ctx->noise.nonzero, 0, 4 * ctx->noise.mask_ld));
     CR(hipMalloc(&ctx->noise.general, sizeof(int)));
     {
         const std::vector<MatDesc> md = matrix_descs(ctx);
@@ -858,7 +859,7 @@ extern "C" int egg_fitness(egg_ctx *ctx, const int32_t *d_loss, int32_t *d_fit, 
 static UpdLaunch make_upd(egg_ctx *ctx, const egg_ctx::MatList &l, const int32_t *d_fit, const float *d_lr) {
     const egg_config &c = ctx->cfg;
     UpdLaunch p; memset(&p, 0, sizeof(p));
-    p.mat = ctx->d_mat + l.first; p.n_mat = l.count; p.tiles = l.tiles;
+    p.mat = ctx->d_mat + l.first; p.n_mat = l.count; p.tiles = l.tiles; p.wide = c.hidden % 128 == 0 && c.vocab % 128 == 0;
     p.noise = ctx->noise; p.fit = d_fit; p.pairs = c.population / 2; p.d_lr = d_lr;
     p.beta1 = c.adam_beta1; p.beta2 = c.adam_beta2; p.eps = c.adam_eps; p.wd = c.adam_weight_decay; p.muon_momentum = c.muon_momentum;
     p.counter = ctx->d_counter; p.h_counter = ctx->h_result;
@@ -877,7 +878,7 @@ extern "C" int egg_update_tensor(egg_ctx *ctx, int id, const int32_t *d_fit, con
     const egg_tensor_info &t = ctx->tensors[id];
     UpdLaunch p = make_upd(ctx, ctx->mat_one[id], d_fit, d_lr);
     if (!t.is_matrix) { p.vec = ctx->d_vec_desc + ctx->vec_one[id]; p.n_vec = 1; p.vec_total = t.cols; }
-    p.count_of = egg_update_blocks(p);
+    p.count_of = t.is_matrix && t.muon && ctx->cfg.use_muon ? p.tiles : egg_update_blocks(p);
     SpanScope span(ctx, t.is_matrix ? EGG_K_UPDATE_MATRIX : EGG_K_UPDATE_VECTOR);
     int rc = table_of_tensor(ctx, id, d_fit, d_seed);
     if (rc) return rc;

@@ -46,9 +46,13 @@ hipError_t egg_launch_sample_deggs(const int32_t *logits, const int32_t *exp_lut
 // the noise of every tensor as shifted windows of one table, see egg_votes.hip
 #define EGG_MODEL_SEEDS 920        // seed offsets of the tensors outside the layers and of layer 0 lie below this
 #define EGG_LAYER_SEEDS 416        // those of a layer's tensors, above its 1000 * layer
+#define EGG_NOISE_FRONT 16         // a row's entry t lies at byte EGG_NOISE_FRONT + t
 struct NoiseTable {
-    int8_t *table; size_t ld; int rows;        // [rows][ld]
-    int8_t *neg, *nonzero; int pairs_pad;      // [pairs_pad] each (a multiple of 128): 0xff where the fitness is -1 / is not 0
+    int8_t *table; size_t ld; int rows;        // [rows][ld], ld a multiple of 128
+    // masks by pair (pairs_pad, a multiple of 128, of them): 0xff where the fitness is -1 / is not 0, zeros in front and behind.
+    // Copy k of four, mask_ld bytes apart, has pair p at byte EGG_NOISE_FRONT + k + p, so that any shift of the pairs finds
+    // its masks on a dword.
+    int8_t *neg, *nonzero; size_t mask_ld; int pairs_pad;
     int *general;                              // 1: some fitness lies outside {-1, 0, 1}
 };
 // what a whole step does between its forward and its update: losses and fitness from the loss sums, which go back to
@@ -71,6 +75,7 @@ struct MatDesc {
 struct VecDesc { int8_t *W; float *state; int n, first, off_a, off_b, seed_base; float lr_scale; int8_t *flags; };
 struct UpdLaunch {
     const MatDesc *mat; int n_mat, tiles;          // device array and its number of 64 x 64 tiles
+    bool wide;                                     // all sides are multiples of 128
     const VecDesc *vec; int n_vec, vec_total;      // device array; may be empty
     NoiseTable noise;
     const int32_t *fit; int pairs;
@@ -82,6 +87,8 @@ struct UpdLaunch {
                                        // cols, set to 1 where a weight changed (de/include/optimizer/adam.cuh:77-83)
 };
 int egg_update_blocks(const UpdLaunch &p);             // its workgroups
+size_t egg_noise_ld(int entries);                      // bytes of a table row that holds so many entries
+size_t egg_noise_mask_ld(int pairs_pad);
 hipError_t egg_launch_update(const UpdLaunch &p, hipStream_t s);
 hipError_t egg_launch_muon_apply(const UpdLaunch &p, float wd, hipStream_t s);
 hipError_t egg_launch_frag(const MatDesc *d_mat, int n_mat, int tiles, hipStream_t s);

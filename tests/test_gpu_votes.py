@@ -37,3 +37,28 @@ def test_votes_and_update_at_chunk_edges(pkg, orc, dev, pairs, values):
         assert np.array_equal(ctx.opt_state_download().view(np.int32), state.view(np.int32))
         assert ctx.last_update_count() == n_ref
     ctx.close()
+
+
+@pytest.mark.parametrize("values", [(-1, 0, 1), (-3, 2, 5)], ids=["ternary", "any"])
+@pytest.mark.parametrize("pairs", [1, 129])
+def test_update_in_wide_tiles(pkg, orc, dev, pairs, values):
+    """The same in the 128 x 128 tiles that a model of this size takes."""
+    import torch
+    kw = dict(hidden=512, head_dim=32, n_layers=1, seq_len=32, population=2 * pairs)
+    ocfg = orc.config(**kw)
+    ctx = pkg.Context(pkg.default_config(**kw))
+    model = orc.init_model(ocfg, 42)
+    state = np.zeros(model.size, orc.ADAM_DTYPE)
+    ctx.model_upload(model)
+    fit = np.random.default_rng(pairs).choice(np.array(values, np.int32), pairs)
+    seed, lr = 0x12345678, 5.0
+    d_fit = torch.from_numpy(fit).to(dev)
+    d_seed = torch.tensor([seed], dtype=torch.int32, device=dev)
+    d_lr = torch.tensor([lr], dtype=torch.float32, device=dev)
+    for _ in range(2):
+        ctx.es_update(d_fit.data_ptr(), d_seed.data_ptr(), d_lr.data_ptr())
+        n_ref = orc.es_update_adam(ocfg, model, state, fit, seed, lr)
+        assert np.array_equal(ctx.model_download(), model)
+        assert np.array_equal(ctx.opt_state_download().view(np.int32), state.view(np.int32))
+        assert ctx.last_update_count() == n_ref
+    ctx.close()
