@@ -706,6 +706,7 @@ static FwdCommon make_common(egg_ctx *ctx, const uint8_t *d_data, int64_t len, c
     f.t0 = 0; f.tn = c.seq_len;
     f.sigma = c.fixed_point + c.sigma_shift; f.sigma_vec = c.sigma_shift_vector;
     f.mask = ctx->mask_override >= 0 ? ctx->mask_override : noise_word(c);
+    egg_rank1_shifts(f.mask, f.sigma, &f.sb_shift, &f.a_shift);
     f.shift_attn = c.shift_attn; f.shift_out = c.shift_out; f.shift_logit = c.shift_logit;
     f.shift_mlp_up = c.shift_mlp_up; f.shift_mlp_down = c.shift_mlp_down;
     f.softmax_scale_bit = c.softmax_scale_bit; f.rope_scale_bit = c.rope_scale_bit;

@@ -343,15 +343,15 @@ __device__ __forceinline__ TileMap tile_map(int T, int wave, int block) {
 }
 static inline int tile_map_sets(int T, int cs) { int tpm = T / 32, tpw = EGG_WAVES / cs; return tpm >= tpw ? 1 : tpw / tpm; }
 
-// Combine a per-token value over the CS waves sharing a tile.  `site` is an LDS area of EGG_WAVES*64 ints that no
+// Combine a per-token value (the same in both halves) over the CS waves sharing a tile.  `site` is an LDS area of EGG_WAVES*32 ints that no
 // other exchange uses until every wave has passed another barrier.  Every wave of the workgroup must call it.
 // (xput and xget: its two halves, for a caller that passes a barrier of its own between them)
-__device__ __forceinline__ void xput(int v, int *site, int CS, const TileMap &tm, int lane) { site[(tm.tslot * CS + tm.cs) * 64 + lane] = v; }
+__device__ __forceinline__ void xput(int v, int *site, int CS, const TileMap &tm, int lane) { site[(tm.tslot * CS + tm.cs) * 32 + (lane & 31)] = v; }
 template <int CS, bool IS_MAX>
 __device__ __forceinline__ int xget(const int *site, const TileMap &tm, int lane) {
-    int r = site[(tm.tslot * CS) * 64 + lane];
+    int r = site[(tm.tslot * CS) * 32 + (lane & 31)];
 #pragma unroll
-    for (int c = 1; c < CS; c++) { int o = site[(tm.tslot * CS + c) * 64 + lane]; r = IS_MAX ? max(r, o) : r + o; }
+    for (int c = 1; c < CS; c++) { int o = site[(tm.tslot * CS + c) * 32 + (lane & 31)]; r = IS_MAX ? max(r, o) : r + o; }
     return r;
 }
 template <int CS, bool IS_MAX>

@@ -28,53 +28,27 @@ __device__ __forceinline__ int token_at(const FwdCommon &c, int64_t i) {
     return c.token_bytes == 4 ? (int)reinterpret_cast<const uint32_t *>(c.data)[i] : (int)c.data[i];
 }
 
-// acc[nt][r] += (sb * At[n]) >> sigma for NT column groups starting at table offset n_off
+// acc[nt][r] += (sb * A[n]) >> sigma for NT column groups starting at table offset n_off; the table holds A << a_shift, and sb
+// comes shifted by sb_shift (egg_rank1_shifts).  Two instructions an element where multiply, shift and add were three: k_qkv
+// 5.55 -> 5.47 ms at hidden 256 and 40,960 members, 1.52 -> 1.47 ms at hidden 512.
 template <int NT>
-__device__ __forceinline__ void add_perturb(v16i *acc, int sb, const int *At, int n_off, int sigma, int g) {
+__device__ __forceinline__ void add_perturb(v16i *acc, int sb, const int *At, int n_off, int g) {
 #pragma unroll
     for (int nt = 0; nt < NT; nt++)
 #pragma unroll
         for (int q = 0; q < 4; q++) {
             v4i a4 = *reinterpret_cast<const v4i *>(At + n_off + 32 * nt + 8 * q + 4 * g);
 #pragma unroll
-            for (int e = 0; e < 4; e++) acc[nt][4 * q + e] += mul24(sb, a4[e]) >> sigma;
+            for (int e = 0; e < 4; e++) acc[nt][4 * q + e] += __mulhi(sb, a4[e]);
         }
 }
-
-// same with the output-side noise kept as int8, already multiplied by the member's sign
 template <int NT>
-__device__ __forceinline__ void add_perturb8(v16i *acc, int sb, const int8_t *At, int n_off, int sigma, int g) {
+__device__ __forceinline__ void perturb_shift_groups(v16i *acc, int sb, const int *At, int n_off, int shift, int g) {
+    add_perturb<NT>(acc, sb, At, n_off, g);
 #pragma unroll
     for (int nt = 0; nt < NT; nt++)
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-            int a4 = *reinterpret_cast<const int *>(At + n_off + 32 * nt + 8 * q + 4 * g);
-#pragma unroll
-            for (int e = 0; e < 4; e++) acc[nt][4 * q + e] += mul24(sb, sx8(a4, e)) >> sigma;
-        }
-}
-
-// (acc + ((sb * a) >> sigma)) >> shift.  With FUSE it is evaluated as ((acc << sigma) + sb * a) >> (sigma + shift):
-// floor(floor(y / 2^sigma + acc) / 2^shift) == floor((y + acc * 2^sigma) / 2^(sigma + shift)) for integers, one
-// instruction less.  The host selects FUSE only when |acc| * 2^sigma + |sb * a| < 2^31 for the GEMM depth in question.
-template <bool FUSE>
-__device__ __forceinline__ int perturb_shift(int acc, int sb, int a, int sigma, int shift) {
-    // (measured: forcing the multiply apart from the add -- v_mul_i32_i24 with a byte operand select plus
-    // v_lshl_add_u32, one instruction less per element -- runs 2 % slower than the multiply-add the compiler picks)
-    if (FUSE) return (int)(((unsigned)acc << sigma) + (unsigned)mul24(sb, a)) >> (sigma + shift);
-    return (acc + (mul24(sb, a) >> sigma)) >> shift;
-}
-// acc[nt][r] = perturb_shift(acc[nt][r], sb, At[n], ...) for NT column groups starting at table offset n_off
-template <int NT, bool FUSE>
-__device__ __forceinline__ void perturb_shift_groups(v16i *acc, int sb, const int8_t *At, int n_off, int sigma, int shift, int g) {
-#pragma unroll
-    for (int nt = 0; nt < NT; nt++)
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            int a4 = *reinterpret_cast<const int *>(At + n_off + 32 * nt + 8 * q + 4 * g);
-#pragma unroll
-            for (int e = 0; e < 4; e++) acc[nt][4 * q + e] = perturb_shift<FUSE>(acc[nt][4 * q + e], sb, sx8(a4, e), sigma, shift);
-        }
+        for (int r = 0; r < 16; r++) acc[nt][r] >>= shift;
 }
 
 // exchange of packed 32-column groups between the waves sharing a tile: group k of tile slot ts, 16 bytes per lane
@@ -128,16 +102,17 @@ struct MlpCfg {
     static constexpr int UNIT = 16 * cmax(PRO * H, cmax(PRUP * SC, PRDN * H));
     static constexpr int WBYTES = 2 * UNIT;
     static constexpr int I32 = 9 * H;        // ex0[H] ex1[H] lnw[H] lnb[H] bup[4H] bdn[H]
-    static constexpr int I8 = 11 * H;        // exB[H] upB[H] dnB[4H] upA[4H] dnA[H]   (A noise already times the sign)
-    // The blocks behind the first one keep the up projection's output noise as int32 (UPA32): the GELU epilogue then
-    // multiplies by a table word as it stands instead of extracting a byte per element.  The first block has no room
-    // for it at three workgroups per CU (its value-rank tables take the space) and keeps the bytes.
+    static constexpr int I8 = 14 * H;        // exB[H] upB[H] dnB[4H] upA[4H] dnA[int32 H]   (A noise already times the sign)
+    // The up projection's output noise is kept as int32: the GELU epilogue then multiplies by a table word as it stands
+    // instead of extracting a byte per element.  Only the first block of hidden 256 has no room for it at three workgroups
+    // per CU (its value-rank tables take the space) and keeps the bytes.
+    static constexpr bool up32(bool first) { return !first || H != 256; }
     static constexpr int UPA32 = 3 * 4 * H;  // extra bytes of the int32 form: upA occupies 16H instead of 4H
     static constexpr int PER_SET = I32 * 4 + I8;
     // The normalised input is exchanged through whichever W buffer is idle at that point (TPW*32*H <= UNIT bytes);
     // the intermediate slices have their own small area because both W buffers are busy inside the sub-chunk loop.
     static constexpr int XCHG = CS > 1 ? TPW * 32 * SC : 0;
-    static constexpr int SITE = EGG_WAVES * 64;                       // ints per reduction site
+    static constexpr int SITE = EGG_WAVES * 32;                       // ints per reduction site
     static constexpr int RED = CS > 1 ? 2 * SITE * 4 : 0;             // two reduction sites used alternately
     static constexpr int OCC = H == 256 ? 3 : 2;                      // workgroups per CU the kernel is built for
     // first block only: rank of every byte value among the values present in the member's window [256], wave counts
@@ -148,24 +123,26 @@ struct MlpCfg {
     // (behind the first block ex1 does not exist: 4H bytes less.  At hidden 256 the total stays at 52 KB: the LDS is
     // handed out in granules, three workgroups of 53 KB no longer share a CU, and the kernel then runs 9 % slower.)
     // The overlay's variants hold the input-side noise as floats: exB, upB and dnB take four times their bytes.
-    static constexpr int per_set(bool first, bool adapt) { return PER_SET + (first ? 0 : UPA32 - 4 * H) + (adapt ? 3 * 6 * H : 0); }
+    static constexpr int per_set(bool first, bool adapt) { return PER_SET + (up32(first) ? UPA32 : 0) - (first ? 0 : 4 * H) + (adapt ? 3 * 6 * H : 0); }
     static int total(int sets, bool first, bool adapt) { return WBYTES + ACT + sets * per_set(first, adapt) + XCHG + RED + (first ? DEDUP : 0); }
     // the overlay's variants need the registers of two workgroups per CU
     static constexpr int occ(bool adapt) { return adapt && OCC > 2 ? 2 : OCC; }
 };
 
-// FUSE: the host has checked sigma <= 7 and |noise| <= 15, which bounds |acc| * 2^sigma + |sb * a| below 2^31 for
-// GEMM depths up to 1024 (depth * 127 * 127 * 128 + depth * 127 * 225), and the same bound for the up accumulator
-// with its bias seed (egg_mlp_up_acc_bound); the down projection (depth 4H) uses the fused form only for 4H <= 1024.
+// SEED: the down accumulator starts from (residual + bias) << shift_mlp_down instead of zero; the host has checked that its
+// range allows that (egg_mlp_down_acc_bound).  The residual then needs no register and no memory across the
+// sub-chunk loop -- without it it is parked in the x buffer and read again, 2 of 5 bytes that the kernel moves -- and the
+// epilogue neither extracts nor adds it.  Hidden 256, 40,960 members x 256
+// tokens: 9.33 -> 8.97 ms a launch, hidden 512, 2,048 x 512: 3.12 -> 3.05 ms (the residual stays in registers until the
+// accumulator is live: seeded in front of the norm, hidden 512 spills and takes 3.85 ms).
 // ADAPT: the d-eggs adaptive noise overlay is on (de/include/model/layers.cuh:215-296, :432-438,
 // de/src/kernels.cu:139-158); see k_qkv.  The down projection's input-side sum follows the reference thread of a
 // hidden unit, which adds its four terms (k = unit, unit + H, ...) into an int one float addition at a time; the
 // sub-chunks are therefore visited so that those four are consecutive.  At hidden 256, 2048 members x 256 tokens the overlay's
 // kernel took 0.91 ms with integer terms, spilling at three workgroups per CU; 0.63 ms as it is (0.47 without the overlay).
-template <int H, bool FIRST, bool FUSE, bool ADAPT>
+template <int H, bool FIRST, bool SEED, bool ADAPT>
 __global__ void __launch_bounds__(EGG_THREADS, MlpCfg<H>::occ(ADAPT)) k_mlp(MlpParams p) {
     typedef MlpCfg<H> M;
-    constexpr bool FUSE_DN = FUSE && 4 * H <= 1024;
     constexpr int CS = M::CS, KS = M::KS, NTS = M::NTS, HS = M::HS, NTU = M::NTU, SC = M::SC;
     // fragments read ahead of their MFMAs: at hidden 512 the accumulators and operands leave room for four
     constexpr int MAXF = H == 512 ? 4 : 8;
@@ -182,14 +159,14 @@ __global__ void __launch_bounds__(EGG_THREADS, MlpCfg<H>::occ(ADAPT)) k_mlp(MlpP
     const TileMap tm = tile_map<CS>(c.tn, wave, blockIdx.x);
     const int col0 = tm.cs * HS;                      // first output column of this wave's slice
     constexpr int PSET = M::per_set(FIRST, ADAPT), WB = ADAPT ? 4 : 1;        // WB: bytes of an input-side noise entry
-    constexpr bool UPA32 = !FIRST;
+    constexpr bool UPA32 = M::up32(FIRST);
     int8_t *tb = act + M::ACT + tm.set * PSET;
-    int *ex0 = reinterpret_cast<int *>(tb);           // FIRST: emb_bias + noise   | else: O-proj A noise * ns as int8
+    int *ex0 = reinterpret_cast<int *>(tb);           // FIRST: emb_bias + noise   | else: O-proj A noise
     int *ex1 = ex0 + H;                               // FIRST: b_dim noise * ns    | else: absent
     int *lnw = ex1 + (FIRST ? H : 0), *lnb = lnw + H, *bup = lnb + H, *bdn = bup + 4 * H;
     int8_t *exB = reinterpret_cast<int8_t *>(bdn + H);   // O-proj B noise
     int8_t *upB = exB + WB * H, *dnB = upB + WB * H, *upA = dnB + 4 * WB * H, *dnA = upA + (UPA32 ? 16 : 4) * H;
-    const int8_t *oA = reinterpret_cast<const int8_t *>(ex0);
+    const int *oA = ex0, *dnA32 = reinterpret_cast<const int *>(dnA);
     int8_t *xch = act + M::ACT + tm.sets * PSET;
     int *red = reinterpret_cast<int *>(xch + M::XCHG);
     int rsite = 0;          // the two reduction sites take turns, call by call (the same sequence in every wave)
@@ -233,16 +210,16 @@ __global__ void __launch_bounds__(EGG_THREADS, MlpCfg<H>::occ(ADAPT)) k_mlp(MlpP
                 // b_dim * q(hidden) * ns, not yet divided: the token's factor joins before the truncation
                 for (int i = tid; i < H; i += EGG_THREADS) e1[i] = noise_from_hash(pseed + OFF_EMB + H, i, c.mask) * p.q_emb[i] * nsx;
             } else {
-                fill_noise_i8_ov(reinterpret_cast<int8_t *>(e0), sbx + OFF_O_A, H, c.mask, tid, EGG_THREADS, nsx, p.q_o + H);
+                fill_noise_i32_ov(e0, sbx + OFF_O_A, H, c.mask, nsx << c.a_shift, tid, EGG_THREADS, p.q_o + H);
                 fill_noise_f32_ov(reinterpret_cast<float *>(eB), sbx + OFF_O_B, H, c.mask, tid, EGG_THREADS, p.q_o);
             }
             fill_vec_i32_ov(lw, p.ln_w, sbx + p.off_ln_a, sbx + p.off_ln_b, H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS, 2, p.q_ln_w);
             fill_vec_i32_ov(lb, p.ln_b, sbx + p.off_lnb_a, sbx + p.off_lnb_b, H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS, 0, p.q_ln_b);
-            if (UPA32) fill_noise_i32_ov(reinterpret_cast<int *>(uA), sbx + p.off_up_a, 4 * H, c.mask, nsx, tid, EGG_THREADS, p.q_up + H);
+            if (UPA32) fill_noise_i32_ov(reinterpret_cast<int *>(uA), sbx + p.off_up_a, 4 * H, c.mask, nsx << c.a_shift, tid, EGG_THREADS, p.q_up + H);
             else fill_noise_i8_ov(uA, sbx + p.off_up_a, 4 * H, c.mask, tid, EGG_THREADS, nsx, p.q_up + H);
             fill_vec_i32_ov(bu, p.b_up, sbx + p.off_bup_a, sbx + p.off_bup_b, 4 * H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS, c.shift_mlp_up, p.q_b_up, 128);
-            fill_noise_i8_ov(dA, sbx + p.off_dn_a, H, c.mask, tid, EGG_THREADS, nsx, p.q_dn + 4 * H);
-            fill_vec_i32_ov(bd, p.b_dn, sbx + p.off_bdn_a, sbx + p.off_bdn_b, H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS, 0, p.q_b_dn);
+            fill_noise_i32_ov(reinterpret_cast<int *>(dA), sbx + p.off_dn_a, H, c.mask, nsx << c.a_shift, tid, EGG_THREADS, p.q_dn + 4 * H);
+            fill_vec_i32_ov(bd, p.b_dn, sbx + p.off_bdn_a, sbx + p.off_bdn_b, H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS, SEED ? c.shift_mlp_down : 0, p.q_b_dn);
             fill_noise_f32_ov(reinterpret_cast<float *>(uB), sbx + p.off_up_b, H, c.mask, tid, EGG_THREADS, p.q_up);
             fill_noise_f32_ov(reinterpret_cast<float *>(dB), sbx + p.off_dn_b, 4 * H, c.mask, tid, EGG_THREADS, p.q_dn);
             continue;
@@ -251,18 +228,18 @@ __global__ void __launch_bounds__(EGG_THREADS, MlpCfg<H>::occ(ADAPT)) k_mlp(MlpP
             fill_vec_i32(e0, p.emb_bias, pseed + OFF_EMB_BIAS_A, pseed + OFF_EMB_BIAS_B, H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS);
             fill_noise_i32(e1, pseed + OFF_EMB + H, H, c.mask, nsx, tid, EGG_THREADS);
         } else {
-            fill_noise_i8(reinterpret_cast<int8_t *>(e0), sbx + OFF_O_A, H, c.mask, tid, EGG_THREADS, nsx);
+            fill_noise_i32(e0, sbx + OFF_O_A, H, c.mask, nsx << c.a_shift, tid, EGG_THREADS);
             fill_noise_i8(eB, sbx + OFF_O_B, H, c.mask, tid, EGG_THREADS);
         }
         fill_vec_i32(lw, p.ln_w, sbx + p.off_ln_a, sbx + p.off_ln_b, H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS, 2);     // 4 * gain, see standard_scale
         fill_vec_i32(lb, p.ln_b, sbx + p.off_lnb_a, sbx + p.off_lnb_b, H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS);
-        if (UPA32) fill_noise_i32(reinterpret_cast<int *>(uA), sbx + p.off_up_a, 4 * H, c.mask, nsx, tid, EGG_THREADS);
+        if (UPA32) fill_noise_i32(reinterpret_cast<int *>(uA), sbx + p.off_up_a, 4 * H, c.mask, nsx << c.a_shift, tid, EGG_THREADS);
         else fill_noise_i8(uA, sbx + p.off_up_a, 4 * H, c.mask, tid, EGG_THREADS, nsx);
         // the up bias is stored as (b + 128) << shift_mlp_up and seeds the up accumulator: ((a + (b << s)) >> s) == (a >> s) + b;
         // the 128 makes the clamped result (1..255) the GELU table's index
         fill_vec_i32(bu, p.b_up, sbx + p.off_bup_a, sbx + p.off_bup_b, 4 * H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS, c.shift_mlp_up, 128);
-        fill_noise_i8(dA, sbx + p.off_dn_a, H, c.mask, tid, EGG_THREADS, nsx);
-        fill_vec_i32(bd, p.b_dn, sbx + p.off_bdn_a, sbx + p.off_bdn_b, H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS);
+        fill_noise_i32(reinterpret_cast<int *>(dA), sbx + p.off_dn_a, H, c.mask, nsx << c.a_shift, tid, EGG_THREADS);
+        fill_vec_i32(bd, p.b_dn, sbx + p.off_bdn_a, sbx + p.off_bdn_b, H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS, SEED ? c.shift_mlp_down : 0);
         fill_noise_i8(uB, sbx + p.off_up_b, H, c.mask, tid, EGG_THREADS);
         fill_noise_i8(dB, sbx + p.off_dn_b, 4 * H, c.mask, tid, EGG_THREADS);
     }
@@ -371,7 +348,7 @@ __global__ void __launch_bounds__(EGG_THREADS, MlpCfg<H>::occ(ADAPT)) k_mlp(MlpP
                 }
                 if (ADAPT && CS > 1) sbo = xget<CS, false>(site, tm, laneA);
             }
-            perturb_shift_groups<NTS, FUSE>(acc, sbo, oA, col0, c.sigma, c.shift_out, gA);
+            perturb_shift_groups<NTS>(acc, sbo << c.sb_shift, oA, col0, c.shift_out, gA);
 #pragma unroll
             for (int nt = 0; nt < NTS; nt++) {
                 v4i xr = load_op(xrow, nt, gA);
@@ -387,7 +364,7 @@ __global__ void __launch_bounds__(EGG_THREADS, MlpCfg<H>::occ(ADAPT)) k_mlp(MlpP
         // park the residual (this wave owns the slice; invalid padding waves only recompute, and so do the rows of the
         // value table beyond the number of distinct values: nothing reads them, so nothing of them is written)
         const bool keep = valid && (!(FIRST && dedup) || t < nrows);
-        if (keep)
+        if (keep && !SEED)
 #pragma unroll
             for (int nt = 0; nt < NTS; nt++) store_op(xrow, nt, gA, xs[nt]);
 
@@ -416,8 +393,18 @@ __global__ void __launch_bounds__(EGG_THREADS, MlpCfg<H>::occ(ADAPT)) k_mlp(MlpP
         }
         if (ADAPT && CS == 1) dot_noise_ov<KS, 1>(nrm, reinterpret_cast<const float *>(upB), 0, gA, &sbu);
         if (!ADAPT) sbu = dot_noise<KS, false>(nrm, upB, 0, gA);
+        sbu <<= c.sb_shift;
         v16i accd[NTS];
-        zero_acc<NTS>(accd);
+        if (SEED) {
+#pragma unroll
+            for (int nt = 0; nt < NTS; nt++)
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const v4i b4 = *reinterpret_cast<const v4i *>(bdn + col0 + 32 * nt + 8 * q + 4 * gA);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) accd[nt][4 * q + e] = (sx8(xs[nt][q], e) << c.shift_mlp_down) + b4[e];
+                }
+        } else zero_acc<NTS>(accd);
         int sbd = 0;
         // ADAPT: running sums of the reference threads this lane stands in for; whole numbers and, with a term added, six
         // fraction bits below 4 * 127 * 127: exact in float32
@@ -467,7 +454,7 @@ __global__ void __launch_bounds__(EGG_THREADS, MlpCfg<H>::occ(ADAPT)) k_mlp(MlpP
                         for (int e = 0; e < 4; e++) {
                             // the accumulator carries + 128 (see the bias table): clamping to 1..255 is the clamp to +-127,
                             // and the result is the table index as it stands
-                            const int idx = min(255, max(1, perturb_shift<FUSE>(au[nt][4 * q + e], sbu, UPA32 ? a32[e] : sx8(a4, e), c.sigma, c.shift_mlp_up)));
+                            const int idx = min(255, max(1, (au[nt][4 * q + e] + __mulhi(sbu, UPA32 ? a32[e] : sx8(a4, e) << c.a_shift)) >> c.shift_mlp_up));
                             r4[e] = ADAPT ? (uint32_t)(int)reinterpret_cast<lds_i8_ptr>((uintptr_t)(uint32_t)idx)[M::WBYTES]
                                           : reinterpret_cast<lds_u8_ptr>((uintptr_t)(uint32_t)idx)[M::WBYTES];
                         }
@@ -513,7 +500,8 @@ __global__ void __launch_bounds__(EGG_THREADS, MlpCfg<H>::occ(ADAPT)) k_mlp(MlpP
         const int gB = laneB >> 5;
         sbd = sum_halves(sbd);
         sbd = xreduce<CS, false>(sbd, next_site(), tm, laneB);
-        perturb_shift_groups<NTS, FUSE_DN>(accd, sbd, dnA, col0, c.sigma, c.shift_mlp_down, gB);
+        perturb_shift_groups<NTS>(accd, sbd << c.sb_shift, dnA32, col0, c.shift_mlp_down, gB);
+        if (!SEED)
 #pragma unroll
         for (int nt = 0; nt < NTS; nt++) {
             v4i xr = load_op(xrow, nt, gB);          // the parked residual (for a padding wave: someone else's row, unused)
@@ -558,7 +546,7 @@ struct QkvCfg {
     // lnw lnb (int32) | qA kA vA (int32, times the sign: an operand of the multiply without a byte extraction) | qB kB vB (int8)
     static constexpr int PER_SET = 5 * H * 4 + 3 * H;
     static constexpr int XCHG = 0;             // the normalised input is exchanged through the idle W buffer
-    static constexpr int SITE = EGG_WAVES * 64;
+    static constexpr int SITE = EGG_WAVES * 32;
     static constexpr int RED = CS > 1 ? 2 * SITE * 4 : 0;       // two reduction sites used alternately (overlay: and one for each input-side sum)
     static constexpr int OCC = H == 256 ? 3 : 2;               // workgroups per CU the kernel is built for
     static constexpr int per_set(bool adapt) { return PER_SET + (adapt ? 3 * 3 * H : 0); }        // the overlay's qB kB vB are floats
@@ -633,9 +621,9 @@ __global__ void __launch_bounds__(EGG_THREADS, QkvCfg<H>::OCC) k_qkv(QkvParams p
         if (ADAPT) {
             fill_vec_i32_ov(lw, p.ln_w, sbx + OFF_LN_1_A, sbx + OFF_LN_1_B, H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS, 2, p.q_ln_w);
             fill_vec_i32_ov(lb, p.ln_b, sbx + OFF_LN_1_BIAS_A, sbx + OFF_LN_1_BIAS_B, H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS, 0, p.q_ln_b);
-            fill_noise_i32_ov(a0, sbx + OFF_Q_A, H, c.mask, nsx, tid, EGG_THREADS, p.q_wq + H);
-            fill_noise_i32_ov(a1, sbx + OFF_K_A, H, c.mask, nsx, tid, EGG_THREADS, p.q_wk + H);
-            fill_noise_i32_ov(a2, sbx + OFF_V_A, H, c.mask, nsx, tid, EGG_THREADS, p.q_wv + H);
+            fill_noise_i32_ov(a0, sbx + OFF_Q_A, H, c.mask, nsx << c.a_shift, tid, EGG_THREADS, p.q_wq + H);
+            fill_noise_i32_ov(a1, sbx + OFF_K_A, H, c.mask, nsx << c.a_shift, tid, EGG_THREADS, p.q_wk + H);
+            fill_noise_i32_ov(a2, sbx + OFF_V_A, H, c.mask, nsx << c.a_shift, tid, EGG_THREADS, p.q_wv + H);
             float *f0 = reinterpret_cast<float *>(b0);
             fill_noise_f32_ov(f0, sbx + OFF_Q_B, H, c.mask, tid, EGG_THREADS, p.q_wq);
             fill_noise_f32_ov(f0 + H, sbx + OFF_K_B, H, c.mask, tid, EGG_THREADS, p.q_wk);
@@ -643,9 +631,9 @@ __global__ void __launch_bounds__(EGG_THREADS, QkvCfg<H>::OCC) k_qkv(QkvParams p
         } else {
             fill_vec_i32(lw, p.ln_w, sbx + OFF_LN_1_A, sbx + OFF_LN_1_B, H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS, 2);     // 4 * gain, see standard_scale
             fill_vec_i32(lb, p.ln_b, sbx + OFF_LN_1_BIAS_A, sbx + OFF_LN_1_BIAS_B, H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS);
-            fill_noise_i32(a0, sbx + OFF_Q_A, H, c.mask, nsx, tid, EGG_THREADS);
-            fill_noise_i32(a1, sbx + OFF_K_A, H, c.mask, nsx, tid, EGG_THREADS);
-            fill_noise_i32(a2, sbx + OFF_V_A, H, c.mask, nsx, tid, EGG_THREADS);
+            fill_noise_i32(a0, sbx + OFF_Q_A, H, c.mask, nsx << c.a_shift, tid, EGG_THREADS);
+            fill_noise_i32(a1, sbx + OFF_K_A, H, c.mask, nsx << c.a_shift, tid, EGG_THREADS);
+            fill_noise_i32(a2, sbx + OFF_V_A, H, c.mask, nsx << c.a_shift, tid, EGG_THREADS);
             fill_noise_i8(b0, sbx + OFF_Q_B, H, c.mask, tid, EGG_THREADS);
             fill_noise_i8(b1, sbx + OFF_K_B, H, c.mask, tid, EGG_THREADS);
             fill_noise_i8(b2, sbx + OFF_V_B, H, c.mask, tid, EGG_THREADS);
@@ -701,7 +689,7 @@ __global__ void __launch_bounds__(EGG_THREADS, QkvCfg<H>::OCC) k_qkv(QkvParams p
                 else if (nw) pf(nw, 0);
                 mfma_cols<Q::PR / 2, NTS>(acc, nrm + u * (Q::PR / 2), cur, H, col0, lane);
             }
-            add_perturb<NTS>(acc, sb, An, col0, c.sigma, g);
+            add_perturb<NTS>(acc, sb << c.sb_shift, An, col0, g);
             if (which < 2) rope_inplace<NTS>(acc, c.rope_lut + (size_t)t * c.head_dim, c.head_dim, g, c.rope_scale_bit);
             const int mx = xreduce<CS, true>(absmax_to_float_groups<NTS>(acc), red + ((1 + which) & 1) * Q::SITE, tm, lane);
             v4i o[NTS];
@@ -1179,8 +1167,8 @@ __global__ void __launch_bounds__(EGG_THREADS, (H > 256 ? 1 : 2)) k_head(HeadPar
         fill_vec_i32(lnb, p.ln_b, pair_seed + OFF_LN_F_BIAS_A, pair_seed + OFF_LN_F_BIAS_B, H, c.mask, ns, c.sigma_vec, lane);
     }
     if (single) {
-        if (ADAPT) fill_noise_i32_ov(hA, pair_seed + OFF_EMB, 256, c.mask, ns, lane, 64, p.q_emb + H);
-        else fill_noise_i32(hA, pair_seed + OFF_EMB, 256, c.mask, ns, lane);
+        if (ADAPT) fill_noise_i32_ov(hA, pair_seed + OFF_EMB, 256, c.mask, ns << c.a_shift, lane, 64, p.q_emb + H);
+        else fill_noise_i32(hA, pair_seed + OFF_EMB, 256, c.mask, ns << c.a_shift, lane);
     }
     if (ADAPT) fill_noise_f32_ov(reinterpret_cast<float *>(hB), pair_seed + OFF_EMB + H, H, c.mask, lane, 64, p.q_emb);
     else fill_noise_i8(hB, pair_seed + OFF_EMB + H, H, c.mask, lane);
@@ -1199,6 +1187,7 @@ __global__ void __launch_bounds__(EGG_THREADS, (H > 256 ? 1 : 2)) k_head(HeadPar
         int sbh;
         if (ADAPT) dot_noise_ov<KS, 1>(nf, reinterpret_cast<const float *>(hB), 0, g, &sbh);
         else sbh = dot_noise<KS, false>(nf, hB, 0, g);
+        sbh <<= c.sb_shift;
         int gmax = INT_MIN, target;
         long long sum_ex; int tl;
         // two-pass softmax statistics (mgpu.cu:969-1009)
@@ -1206,7 +1195,7 @@ __global__ void __launch_bounds__(EGG_THREADS, (H > 256 ? 1 : 2)) k_head(HeadPar
             v16i acc[NV];
             zero_acc<NV>(acc);
             gemm_stream<H, 256, BLK>(acc, nf, p.embedding_frag, 256, 0, 0, ws, (pass + 1 < pass_end) ? w_unit_ptr<BLK>(p.embedding_frag, 256, 0, 0, 0) : nullptr, lane);
-            add_perturb<NV>(acc, sbh, hA, 0, c.sigma, g);
+            add_perturb<NV>(acc, sbh, hA, 0, g);
 #pragma unroll
             for (int nt = 0; nt < NV; nt++)
 #pragma unroll
@@ -1243,8 +1232,8 @@ __global__ void __launch_bounds__(EGG_THREADS, (H > 256 ? 1 : 2)) k_head(HeadPar
                 for (int vb = 0; vb < nvb; vb++) {
                     {                                   // read behind the barriers of the product below, by this wave only
                         const uint32_t seed = pair_seed + OFF_EMB + (uint32_t)(vb * 256) * 0x9e3779b9u;
-                        if (ADAPT) fill_noise_i32_ov(hA, seed, 256, c.mask, ns, lane, 64, p.q_emb + H + vb * 256);
-                        else fill_noise_i32(hA, seed, 256, c.mask, ns, lane);
+                        if (ADAPT) fill_noise_i32_ov(hA, seed, 256, c.mask, ns << c.a_shift, lane, 64, p.q_emb + H + vb * 256);
+                        else fill_noise_i32(hA, seed, 256, c.mask, ns << c.a_shift, lane);
                     }
                     const bool last = vb + 1 == nvb && phase == 1;
                     const int8_t *next = !last ? w_unit_ptr<BLK>(p.embedding_frag, V, 0, (vb + 1 == nvb ? 0 : vb + 1) * 256, 0)
@@ -1252,7 +1241,7 @@ __global__ void __launch_bounds__(EGG_THREADS, (H > 256 ? 1 : 2)) k_head(HeadPar
                     v16i acc[NV];
                     zero_acc<NV>(acc);
                     gemm_stream<H, 256, BLK>(acc, nf, p.embedding_frag, V, 0, vb * 256, ws, next, lane);
-                    add_perturb<NV>(acc, sbh, hA, 0, c.sigma, g);
+                    add_perturb<NV>(acc, sbh, hA, 0, g);
                     if (phase == 0) {
 #pragma unroll
                         for (int nt = 0; nt < NV; nt++)
@@ -1308,20 +1297,16 @@ static hipError_t launch_mlp_h(const MlpParams &p, bool first, hipStream_t s) {
     const int sets = tile_map_sets(p.c.tn, MlpCfg<H>::CS);
     dim3 grid((p.c.n_members + sets - 1) / sets), block(EGG_THREADS);
     size_t lds = MlpCfg<H>::total(sets, first, p.q_ln_w != nullptr);
-    // The up accumulator is seeded with (bias + 128 + noise) << shift_mlp_up (see the bias table), so its range is the
-    // GEMM's plus that seed; the fused perturb-and-shift needs |acc| * 2^sigma + |sb * a| below 2^31 for it as well.
-    const long long mag = egg_noise_magnitude(p.c.mask);
     const long long up_acc = egg_mlp_up_acc_bound(H, p.c.mask, p.c.sigma_vec, p.c.shift_mlp_up);
-    const bool up_fits = p.c.sigma >= 0 && p.c.sigma < 31 && (up_acc << p.c.sigma) + (long long)H * 127 * mag * mag < (1LL << 31);
-    const bool fuse = p.c.sigma <= 7 && mag <= 15 && up_fits;
     if (up_acc >= (1LL << 31)) return hipErrorInvalidValue;      // egg_ctx_create refuses such shifts
+    const bool seed = egg_mlp_down_acc_bound(H, p.c.mask, p.c.sigma_vec, p.c.shift_mlp_down) < (1LL << 31);
     if (p.q_ln_w) {      // adaptive noise overlay: its factors are at most 1, so the same bounds hold
-        if (first) { if (fuse) hipLaunchKernelGGL((k_mlp<H, true, true, true>), grid, block, lds, s, p); else hipLaunchKernelGGL((k_mlp<H, true, false, true>), grid, block, lds, s, p); }
-        else { if (fuse) hipLaunchKernelGGL((k_mlp<H, false, true, true>), grid, block, lds, s, p); else hipLaunchKernelGGL((k_mlp<H, false, false, true>), grid, block, lds, s, p); }
+        if (first) { if (seed) hipLaunchKernelGGL((k_mlp<H, true, true, true>), grid, block, lds, s, p); else hipLaunchKernelGGL((k_mlp<H, true, false, true>), grid, block, lds, s, p); }
+        else { if (seed) hipLaunchKernelGGL((k_mlp<H, false, true, true>), grid, block, lds, s, p); else hipLaunchKernelGGL((k_mlp<H, false, false, true>), grid, block, lds, s, p); }
         return hipGetLastError();
     }
-    if (first) { if (fuse) hipLaunchKernelGGL((k_mlp<H, true, true, false>), grid, block, lds, s, p); else hipLaunchKernelGGL((k_mlp<H, true, false, false>), grid, block, lds, s, p); }
-    else { if (fuse) hipLaunchKernelGGL((k_mlp<H, false, true, false>), grid, block, lds, s, p); else hipLaunchKernelGGL((k_mlp<H, false, false, false>), grid, block, lds, s, p); }
+    if (first) { if (seed) hipLaunchKernelGGL((k_mlp<H, true, true, false>), grid, block, lds, s, p); else hipLaunchKernelGGL((k_mlp<H, true, false, false>), grid, block, lds, s, p); }
+    else { if (seed) hipLaunchKernelGGL((k_mlp<H, false, true, false>), grid, block, lds, s, p); else hipLaunchKernelGGL((k_mlp<H, false, false, false>), grid, block, lds, s, p); }
     return hipGetLastError();
 }
 hipError_t egg_launch_mlp(const MlpParams &p, bool first, hipStream_t s) {

@@ -33,6 +33,22 @@ static inline long long egg_mlp_up_acc_bound(int hidden, int mask, int sigma_vec
     const long long seed = 127 + 128 + ((mag * mag) >> sigma_vec) + 1;
     return (long long)hidden * 127 * 127 + (seed << shift_mlp_up);
 }
+// The down projection's accumulator with (residual + bias + noise) << shift_mlp_down in it, plus the rank-one term: |sb * a| is at
+// most the depth times 127 times the squared magnitude.
+static inline long long egg_mlp_down_acc_bound(int hidden, int mask, int sigma_vec, int shift_mlp_down) {
+    const long long mag = egg_noise_magnitude(mask);
+    const long long seed = 127 + 127 + ((mag * mag) >> sigma_vec) + 1;
+    return 4LL * hidden * 127 * (127 + mag * mag) + (seed << shift_mlp_down);
+}
+
+// (sb * a) >> sigma of a rank-one term is the high word of (sb << sb_shift) * (a << a_shift), one instruction where the output
+// side's table holds the shifted noise: sb_shift + a_shift = 32 - sigma, with as little on sb as keeps a below 2^31 (sb has
+// 24 bits, the magnitude at most 7: at most 8 more are ever needed).
+static inline void egg_rank1_shifts(int mask, int sigma, int *sb_shift, int *a_shift) {
+    int t = 0;
+    while (sigma + t < 32 && egg_noise_magnitude(mask) >= (1LL << (sigma + t)) / 2) t++;
+    *sb_shift = t; *a_shift = 32 - sigma - t;
+}
 
 // what every forward kernel needs to know about the run
 struct FwdCommon {
@@ -49,6 +65,7 @@ struct FwdCommon {
     int t0, tn;                  // token positions [t0, t0 + tn) of every member are evaluated (multiples of 32; the whole window: 0, T);
                                  // attention still reads the K / V rows of every position in front of them
     int sigma;                   // fixed_point + sigma_shift
+    int sb_shift, a_shift;       // egg_rank1_shifts of it
     int sigma_vec;               // sigma_shift_vector
     int mask;                    // noise magnitude mask
     int shift_attn, shift_out, shift_logit, shift_mlp_up, shift_mlp_down;
