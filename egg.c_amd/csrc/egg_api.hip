@@ -57,6 +57,7 @@ struct egg_ctx {
     int8_t *d_x = nullptr, *d_q = nullptr, *d_k = nullptr, *d_v = nullptr, *d_ao = nullptr;
     unsigned long long *d_loss_acc = nullptr, *d_counter = nullptr;
     int32_t *d_loss = nullptr, *d_fit = nullptr;
+    int exp_last = 0;               // the last entry of the exponential's table that is not zero
     bool acc_dirty = false;         // the loss sums may hold something (a forward ended early): the next one clears them
     // what the host reads after a step, written by the step itself: changed weights | losses | fitness
     unsigned long long *h_result = nullptr;
@@ -396,6 +397,7 @@ extern "C" int egg_ctx_create(const egg_config *cfg, egg_ctx **out) {
     for (int i = 0; i < 256; i++) {
         double val = exp(-(double)i / c.softmax_exp_scale) * (double)(1 << c.softmax_scale_bit);
         ex[i] = (val >= 1.0) ? (int32_t)round(val) : 0;
+        if (ex[i]) ctx->exp_last = i;
         int8_t input = (int8_t)i;
         double x = (double)input / (1 << c.fixed_point);
         double y = 0.5 * x * (1.0 + erf(x / 1.41421356));
@@ -799,7 +801,7 @@ static int forward_chunk(egg_ctx *ctx, const uint8_t *d_data, int64_t len, const
     }
     {
         HeadParams p; memset(&p, 0, sizeof(p)); p.c = f;
-        p.ln_w = M + L.ln_f; p.ln_b = M + L.ln_f_bias; p.embedding_frag = F + L.embedding; p.x = ctx->d_x;
+        p.ln_w = M + L.ln_f; p.ln_b = M + L.ln_f_bias; p.embedding_frag = F + L.embedding; p.x = ctx->d_x; p.exp_last = ctx->exp_last;
         p.loss_acc = ctx->logits_override ? ctx->d_counter + 1 : ctx->d_loss_acc; p.logits_tap = ctx->logits_override ? ctx->logits_override : (taps ? ctx->d_tap_logits : nullptr);
         if (Q) { p.q_ln_w = Q + L.ln_f; p.q_ln_b = Q + L.ln_f_bias; p.q_emb = Q + L.embedding; }
         { SpanScope span(ctx, EGG_K_HEAD); HIP_TRY(egg_launch_head(p, s)); }

@@ -1129,7 +1129,7 @@ struct HeadLds {
 
 // ADAPT: adaptive noise overlay; the tied head takes the embedding's per-hidden q values on its input side and the
 // per-token values on its output side (de/src/kernels.cu:200-240)
-// BIG: a vocabulary of more than 256 entries
+// BIG: a vocabulary of more than 256 entries with an exponential's table that k_head_big has too few counters for
 template <int H, bool ADAPT, bool BIG>
 __global__ void __launch_bounds__(EGG_THREADS, (H > 256 ? 1 : 2)) k_head(HeadParams p) {
     constexpr int KS = H / 32, NV = 256 / 32, BLK = H < 256 ? H : 256;
@@ -1291,6 +1291,200 @@ __global__ void __launch_bounds__(EGG_THREADS, (H > 256 ? 1 : 2)) k_head(HeadPar
     if (lane == 0 && valid) atomicAdd(p.loss_acc + member, (unsigned long long)wave_loss);
 }
 
+// The head for a vocabulary of more than 256 entries, with one pass over it.  The reference goes over the logits twice, for
+// their maximum and for the sum of exp_lut[min(255, maximum - logit)] (de/src/kernels.cu:233-272); k_head does the same and
+// multiplies twice.  But the sum only depends on how many logits lie 0, 1, ... `exp_last` below the maximum (behind that the
+// table is zero), so the logits are counted as they come: a token has a counter in LDS for each distance from a ceiling
+// that lies above the maximum of its first block, and a last one for everything further down.  A later maximum above the
+// ceiling (once or twice in a long vocabulary) has the wave move that token's counters.  The target's logit is a product of its own (4 H operations).
+// A logit then costs about six vector instructions and one LDS atomic instead of 16, a gather and a second MFMA share.
+// Blocks of 128 columns (64 accumulator registers) leave room for two waves per SIMD where k_head<512> has one; the four
+// waves share one member's tables (four members' at fewer than four tiles) and take a tile each.  Eight waves sharing a ring of
+// four units of W fetch half as much but take their vector and matrix phases together: 776 us where two workgroups of four
+// take 751.
+// Hidden 512, vocabulary 8,192, 510 members x 256 tokens: 3.1 -> 0.68 ms.
+// (160 counters: what two workgroups of four waves leave of a CU's LDS.  The default table ends at 75, which puts the ceiling
+// 83 above the first block; with 39 and the counters moved one after the other by a token's own lanes this was half of
+// the kernel's time.)
+constexpr int HEAD_BINS = 160, HEAD_LAST = HEAD_BINS - 32;      // the table has to end at an index below HEAD_LAST
+template <int H>
+struct BigHead {
+    static constexpr int BLK = H < 256 ? H : 256, COLS = H < 128 ? H : 128, NV = COLS / 32, KS = H / 32;
+    static constexpr int PR = (H / 16) < 8 ? (H / 16) : 8, NU = (H / 16) / PR, UNIT = 16 * PR * COLS;
+    static constexpr int per_set(bool adapt) { return (2 * H + 2 * COLS) * 4 + (adapt ? 4 : 1) * H; }      // lnw lnb hA[2][COLS] + hB (overlay: floats)
+    static constexpr int hist(bool wide) { return HEAD_BINS * (wide ? 128 : 64); }      // of one wave
+    static constexpr int total(int sets, bool adapt, bool wide) { return 2 * UNIT + 1024 + sets * per_set(adapt) + EGG_WAVES * hist(wide); }
+};
+// WIDE: counters of 32 bits, for vocabularies that could overflow 16
+template <int H, bool ADAPT, bool WIDE>
+__global__ void __launch_bounds__(EGG_THREADS, 2) k_head_big(HeadParams p) {
+    typedef BigHead<H> B;
+    constexpr int KS = B::KS, NV = B::NV, COLS = B::COLS, BLK = B::BLK, PSET = B::per_set(ADAPT);
+    typedef typename std::conditional<WIDE, uint32_t, uint16_t>::type count_t;
+    extern __shared__ __align__(16) int8_t smem[];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, g = lane >> 5, j = lane & 31;
+    const FwdCommon &c = p.c;
+    const int T = c.T, V = c.vocab, nvb = V / COLS;
+    const TileMap tm = tile_map<1>(c.tn, wave, blockIdx.x);
+    int *lut = reinterpret_cast<int *>(smem + 2 * B::UNIT);
+    int8_t *sets = smem + 2 * B::UNIT + 1024, *tb = sets + tm.set * PSET;
+    int *lnw = reinterpret_cast<int *>(tb), *lnb = lnw + H, *hA = lnb + H;
+    int8_t *hB = reinterpret_cast<int8_t *>(hA + 2 * COLS);
+    int8_t *hist = sets + tm.sets * PSET + wave * B::hist(WIDE);
+    // this lane's token: its counter of row r, and what to add to the dword it lies in
+    count_t *cell = reinterpret_cast<count_t *>(hist) + (WIDE ? j : 2 * (j & 15) + (j >> 4));
+    const uint32_t one = WIDE || j < 16 ? 1u : 65536u;
+    uint32_t *cell_dword = reinterpret_cast<uint32_t *>(hist) + (WIDE ? j : (j & 15));
+
+    // (read once: the copies below are opaque to the compiler, and a load behind them would wait for them as well)
+    const uint32_t step_seed = __builtin_amdgcn_readfirstlane(*c.d_step_seed);
+    WStream ws; wstream_init(ws, smem, B::UNIT);
+    const DmaPlan<B::PR, COLS> plan = dma_plan<B::PR, COLS>(BLK);
+    auto pf = [&](int vb, int u) {
+        const int pr = u * B::PR, n = vb * COLS;               // first p-row and column of the unit
+        w_prefetch2<B::PR, COLS>(ws, p.embedding_frag + ((size_t)(pr / (BLK / 16)) * (V / BLK) + n / BLK) * (BLK * BLK) +
+                                     ((size_t)(pr % (BLK / 16)) * BLK + n % BLK) * 16, plan);
+    };
+    pf(0, 0);
+    auto member_of = [&](int s) { const int m = (int)blockIdx.x * tm.sets + s; return c.pop_offset + (m < c.n_members ? m : c.n_members - 1); };
+    auto fill_out_noise = [&](int vb) {                        // columns of block vb, every member of the workgroup
+        for (int s = 0; s < tm.sets; s++) {
+            const int mem = member_of(s);
+            const uint32_t seed = step_seed + (uint32_t)(mem / 2) + OFF_EMB + (uint32_t)(vb * COLS) * 0x9e3779b9u;
+            int *dst = reinterpret_cast<int *>(sets + s * PSET) + 2 * H + (vb & 1) * COLS;
+            const int mult = ((mem & 1) ? -1 : 1) << c.a_shift;
+            if (ADAPT) fill_noise_i32_ov(dst, seed, COLS, c.mask, mult, threadIdx.x, EGG_THREADS, p.q_emb + H + vb * COLS);
+            else fill_noise_i32(dst, seed, COLS, c.mask, mult, threadIdx.x, EGG_THREADS);
+        }
+    };
+    for (int i = threadIdx.x; i < 256; i += EGG_THREADS) lut[i] = c.exp_lut[i];
+    for (int s = 0; s < tm.sets; s++) {
+        const int mem = member_of(s), nsx = (mem & 1) ? -1 : 1;
+        const uint32_t ps = step_seed + (uint32_t)(mem / 2);
+        int *w = reinterpret_cast<int *>(sets + s * PSET), *b = w + H;
+        int8_t *in = reinterpret_cast<int8_t *>(b + H + 2 * COLS);
+        if (ADAPT) {
+            fill_vec_i32_ov(w, p.ln_w, ps + OFF_LN_F_A, ps + OFF_LN_F_B, H, c.mask, nsx, c.sigma_vec, threadIdx.x, EGG_THREADS, 2, p.q_ln_w);
+            fill_vec_i32_ov(b, p.ln_b, ps + OFF_LN_F_BIAS_A, ps + OFF_LN_F_BIAS_B, H, c.mask, nsx, c.sigma_vec, threadIdx.x, EGG_THREADS, 0, p.q_ln_b);
+            fill_noise_f32_ov(reinterpret_cast<float *>(in), ps + OFF_EMB + H, H, c.mask, threadIdx.x, EGG_THREADS, p.q_emb);
+        } else {
+            fill_vec_i32(w, p.ln_w, ps + OFF_LN_F_A, ps + OFF_LN_F_B, H, c.mask, nsx, c.sigma_vec, threadIdx.x, EGG_THREADS, 2);   // 4 * gain, see standard_scale
+            fill_vec_i32(b, p.ln_b, ps + OFF_LN_F_BIAS_A, ps + OFF_LN_F_BIAS_B, H, c.mask, nsx, c.sigma_vec, threadIdx.x, EGG_THREADS);
+            fill_noise_i8(in, ps + OFF_EMB + H, H, c.mask, threadIdx.x, EGG_THREADS);
+        }
+    }
+    fill_out_noise(0);
+    for (int i = lane; i < B::hist(WIDE) / 16; i += 64) reinterpret_cast<v4i *>(hist)[i] = v4i{0, 0, 0, 0};
+    __syncthreads();
+
+    int mloc = tm.mloc;
+    const bool valid = mloc < c.n_members;
+    if (!valid) mloc = c.n_members - 1;
+    const int member = c.pop_offset + mloc;
+    const uint32_t pair_seed = step_seed + (uint32_t)(member / 2);
+    const int t = c.t0 + (tm.tile0 + EGG_WAVES * (int)blockIdx.y) * 32 + j;
+    v4i nf[KS];
+    {
+        v4i x[KS];
+        const size_t row = ((size_t)mloc * T + t) * H;
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) x[ks] = load_op(p.x + row, ks, g);
+        standard_norm<KS>(x, nf, lnw, lnb, g);
+    }
+    int sbh;
+    if (ADAPT) dot_noise_ov<KS, 1>(nf, reinterpret_cast<const float *>(hB), 0, g, &sbh);
+    else sbh = dot_noise<KS, false>(nf, hB, 0, g);
+    sbh <<= c.sb_shift;
+    // the target's logit: its column of the fragment-major embedding holds 16 bytes per k-step and half, in operand order
+    int target_logit;
+    {
+        const int target = token_at(c, stream_pos_of(c, member) + t + 1);
+        int dot = 0;
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+            const v4i w = *reinterpret_cast<const v4i *>(p.embedding_frag + ((size_t)(ks / (BLK / 32)) * (V / BLK) + target / BLK) * (BLK * BLK) +
+                                                         ((size_t)(2 * (ks % (BLK / 32)) + g) * BLK + target % BLK) * 16);
+#pragma unroll
+            for (int q = 0; q < 4; q++) dot = dot4(w[q], nf[ks][q], dot);
+        }
+        dot = sum_halves(dot);
+        int a = noise_from_hash(pair_seed + OFF_EMB, (uint32_t)target, c.mask);
+        if (ADAPT) a = overlay_scaled(a, p.q_emb[H + target]);
+        target_logit = (dot + __mulhi(sbh, a * ((member & 1) ? -1 : 1) << c.a_shift)) >> c.shift_logit;
+    }
+    const int room = HEAD_BINS - 2 - p.exp_last;
+    int gmax = 0, top = 0;
+#pragma unroll 1
+    for (int vb = 0; vb < nvb; vb++) {
+        v16i acc[NV];
+        zero_acc<NV>(acc);
+#pragma unroll
+        for (int u = 0; u < B::NU; u++) {
+            const int8_t *cur = w_acquire(ws);
+            if (u + 1 < B::NU) pf(vb, u + 1); else if (vb + 1 < nvb) pf(vb + 1, 0);
+            if (u == 0 && vb + 1 < nvb) fill_out_noise(vb + 1);      // everyone has left block vb - 1, whose table this is
+            mfma_cols<B::PR / 2, NV>(acc, nf + u * (B::PR / 2), cur, COLS, 0, lane);
+        }
+        add_perturb<NV>(acc, sbh, hA + (vb & 1) * COLS, 0, g);
+        int most = INT_MIN;
+#pragma unroll
+        for (int nt = 0; nt < NV; nt++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) { acc[nt][r] >>= c.shift_logit; most = max(most, acc[nt][r]); }
+        most = max_halves(most);
+        if (p.logits_tap && valid)
+#pragma unroll
+            for (int nt = 0; nt < NV; nt++)
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    v4i o4;
+#pragma unroll
+                    for (int e = 0; e < 4; e++) o4[e] = acc[nt][4 * q + e];
+                    *reinterpret_cast<v4i *>(p.logits_tap + ((size_t)mloc * T + t) * V + vb * COLS + 32 * nt + 8 * q + 4 * g) = o4;
+                }
+        if (vb == 0) { gmax = most; top = most + room; }
+        gmax = max(gmax, most);
+        if (__any(gmax > top)) {
+            const int by = gmax > top ? gmax + room - top : 0;
+            for (uint32_t need = (uint32_t)__ballot(by != 0); need; need &= need - 1) {
+                const int tok = __builtin_ctz(need), d = __builtin_amdgcn_readlane(by, tok);
+                count_t *const of = reinterpret_cast<count_t *>(hist) + (WIDE ? tok : 2 * (tok & 15) + (tok >> 4));
+                count_t v[(HEAD_BINS + 63) / 64];
+#pragma unroll
+                for (int k = 0; k < (HEAD_BINS + 63) / 64; k++) { const int r = lane + 64 * k; v[k] = r >= d && r < HEAD_BINS - 1 ? of[(r - d) * 32] : 0; }
+#pragma unroll
+                for (int k = 0; k < (HEAD_BINS + 63) / 64; k++) { const int r = lane + 64 * k; if (r < HEAD_BINS - 1) of[r * 32] = v[k]; }
+                wave_lds_fence();
+            }
+            top += by;
+            wave_lds_fence();
+        }
+#pragma unroll
+        for (int nt = 0; nt < NV; nt++)
+#pragma unroll
+            for (int r = 0; r < 16; r++)
+                __hip_atomic_fetch_add(cell_dword + min((uint32_t)(top - acc[nt][r]), (uint32_t)(HEAD_BINS - 1)) * (WIDE ? 32u : 16u), one, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+    }
+    wave_lds_fence();
+    long long sum_ex = 0;
+    for (int i = g; i <= p.exp_last; i += 2) sum_ex += (long long)(uint32_t)cell[(i + top - gmax) * 32] * lut[i];
+    sum_ex = sum_halves64(sum_ex);
+    // loss (mgpu.cu:1012-1024)
+    long long log_sum = 0;
+    if (sum_ex > 0) {
+        const int pos = 63 - __clzll((unsigned long long)sum_ex);
+        log_sum = ((long long)pos << 4) - ((long long)c.softmax_scale_bit << 4);
+    }
+    long long wave_loss = g == 0 ? (log_sum >> 1) + gmax - target_logit : 0;
+#pragma unroll
+    for (int off = 16; off > 0; off >>= 1) {
+        const int lo = __shfl_xor((int)(wave_loss & 0xffffffffll), off, 64);
+        const int hi = __shfl_xor((int)(wave_loss >> 32), off, 64);
+        wave_loss += ((long long)hi << 32) | (unsigned int)lo;
+    }
+    if (lane == 0 && valid) atomicAdd(p.loss_acc + member, (unsigned long long)wave_loss);
+}
+
 // ============================================================================ host launchers
 template <int H>
 static hipError_t launch_mlp_h(const MlpParams &p, bool first, hipStream_t s) {
@@ -1370,12 +1564,25 @@ hipError_t egg_launch_attn(const AttnParams &p, hipStream_t s) {
     }
 }
 
+template <int H, bool ADAPT>
+static hipError_t launch_head_big(const HeadParams &p, hipStream_t s) {
+    const int sets = tile_map_sets(p.c.tn, 1), tiles = p.c.tn / 32;
+    const bool wide = p.c.vocab > 32768;
+    const dim3 grid((p.c.n_members + sets - 1) / sets, tiles > EGG_WAVES ? tiles / EGG_WAVES : 1), block(EGG_THREADS);
+    const size_t lds = BigHead<H>::total(sets, ADAPT, wide);
+    if (wide) hipLaunchKernelGGL((k_head_big<H, ADAPT, true>), grid, block, lds, s, p);
+    else hipLaunchKernelGGL((k_head_big<H, ADAPT, false>), grid, block, lds, s, p);
+    return hipGetLastError();
+}
 template <int H>
 static hipError_t launch_head_h(const HeadParams &p, hipStream_t s) {
     dim3 grid((p.c.n_members + EGG_WAVES - 1) / EGG_WAVES), block(EGG_THREADS);
     size_t lds = HeadLds<H>::total(p.q_ln_w != nullptr);
     if (p.c.vocab < 256 || p.c.vocab % 256) return hipErrorInvalidValue;
-    if (p.c.vocab > 256) {
+    if (p.c.vocab > 256 && p.exp_last < HEAD_LAST) {
+        if (p.q_ln_w) return launch_head_big<H, true>(p, s);
+        return launch_head_big<H, false>(p, s);
+    } else if (p.c.vocab > 256) {
         if (p.q_ln_w) hipLaunchKernelGGL((k_head<H, true, true>), grid, block, lds, s, p);
         else hipLaunchKernelGGL((k_head<H, false, true>), grid, block, lds, s, p);
     } else if (p.q_ln_w) hipLaunchKernelGGL((k_head<H, true, false>), grid, block, lds, s, p);
@@ -1428,6 +1635,11 @@ static hipError_t prepare_h(int T) {
     SET_LDS((k_head<H, true, false>), HeadLds<H>::total(true));
     SET_LDS((k_head<H, false, true>), HeadLds<H>::total(false));
     SET_LDS((k_head<H, true, true>), HeadLds<H>::total(true));
+    const int hsets = std::max(tile_map_sets(T, 1), tile_map_sets(32, 1));
+    SET_LDS((k_head_big<H, false, false>), BigHead<H>::total(hsets, false, false));
+    SET_LDS((k_head_big<H, true, false>), BigHead<H>::total(hsets, true, false));
+    SET_LDS((k_head_big<H, false, true>), BigHead<H>::total(hsets, false, true));
+    SET_LDS((k_head_big<H, true, true>), BigHead<H>::total(hsets, true, true));
     return hipSuccess;
 }
 template <int HD, int CT>

@@ -121,4 +121,5 @@ struct HeadParams {
     unsigned long long *loss_acc; // [population] two's-complement int64 accumulators
     int32_t *logits_tap;          // optional [n_members][T][vocab] natural order (may be null)
     const int8_t *q_ln_w, *q_ln_b, *q_emb;   // adaptive noise overlay q values (embedding: H per-hidden, then vocab per-token), or null
+    int exp_last;                 // the last entry of exp_lut that is not zero
 };
