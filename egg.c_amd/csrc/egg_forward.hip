@@ -1127,6 +1127,26 @@ struct HeadLds {
     static constexpr int total(bool adapt) { return WBLOCK + 1024 + EGG_WAVES * per_wave(adapt); }
 };
 
+// One logit of a token: the entry's column of the fragment-major embedding holds 16 bytes per k-step and half, in operand order.
+// (Picking it out of the accumulators took two instructions for every logit.)
+template <int H, bool ADAPT>
+__device__ __forceinline__ int logit_of(const HeadParams &p, const v4i *nf, int sbh, uint32_t pair_seed, int member, int entry, int g) {
+    constexpr int BLK = H < 256 ? H : 256;
+    const FwdCommon &c = p.c;
+    int dot = 0;
+#pragma unroll
+    for (int ks = 0; ks < H / 32; ks++) {
+        const v4i w = *reinterpret_cast<const v4i *>(p.embedding_frag + ((size_t)(ks / (BLK / 32)) * (c.vocab / BLK) + entry / BLK) * (BLK * BLK) +
+                                                     ((size_t)(2 * (ks % (BLK / 32)) + g) * BLK + entry % BLK) * 16);
+#pragma unroll
+        for (int q = 0; q < 4; q++) dot = dot4(w[q], nf[ks][q], dot);
+    }
+    dot = sum_halves(dot);
+    int a = noise_from_hash(pair_seed + OFF_EMB, (uint32_t)entry, c.mask);
+    if (ADAPT) a = overlay_scaled(a, p.q_emb[H + entry]);
+    return (dot + __mulhi(sbh, a * ((member & 1) ? -1 : 1) << c.a_shift)) >> c.shift_logit;
+}
+
 // ADAPT: adaptive noise overlay; the tied head takes the embedding's per-hidden q values on its input side and the
 // per-token values on its output side (de/src/kernels.cu:200-240)
 // BIG: a vocabulary of more than 256 entries with an exponential's table that k_head_big has too few counters for
@@ -1188,10 +1208,11 @@ __global__ void __launch_bounds__(EGG_THREADS, (H > 256 ? 1 : 2)) k_head(HeadPar
         if (ADAPT) dot_noise_ov<KS, 1>(nf, reinterpret_cast<const float *>(hB), 0, g, &sbh);
         else sbh = dot_noise<KS, false>(nf, hB, 0, g);
         sbh <<= c.sb_shift;
-        int gmax = INT_MIN, target;
-        long long sum_ex; int tl;
+        int gmax = INT_MIN, tl;
+        long long sum_ex;
         // two-pass softmax statistics (mgpu.cu:969-1009)
         if constexpr (single) {
+            tl = logit_of<H, ADAPT>(p, nf, sbh, pair_seed, member, c.data[spos + t + 1], g);
             v16i acc[NV];
             zero_acc<NV>(acc);
             gemm_stream<H, 256, BLK>(acc, nf, p.embedding_frag, 256, 0, 0, ws, (pass + 1 < pass_end) ? w_unit_ptr<BLK>(p.embedding_frag, 256, 0, 0, 0) : nullptr, lane);
@@ -1201,18 +1222,12 @@ __global__ void __launch_bounds__(EGG_THREADS, (H > 256 ? 1 : 2)) k_head(HeadPar
 #pragma unroll
                 for (int r = 0; r < 16; r++) { acc[nt][r] >>= c.shift_logit; gmax = max(gmax, acc[nt][r]); }
             gmax = max_halves(gmax);
-            target = c.data[spos + t + 1];
-            sum_ex = 0; tl = 0;
+            uint32_t sum = 0;                              // 128 table entries below 2^21
 #pragma unroll
             for (int nt = 0; nt < NV; nt++)
 #pragma unroll
-                for (int r = 0; r < 16; r++) {
-                    int idx = min(255, max(0, gmax - acc[nt][r]));
-                    sum_ex += lut[idx];
-                    if (col_of(nt, r, g) == target) tl = acc[nt][r];
-                }
-            sum_ex = sum_halves64(sum_ex);
-            tl = sum_halves(tl);
+                for (int r = 0; r < 16; r++) sum += (uint32_t)lut[min(255, max(0, gmax - acc[nt][r]))];
+            sum_ex = sum_halves64((long long)sum);
             if (p.logits_tap && valid)
 #pragma unroll
                 for (int nt = 0; nt < NV; nt++)
@@ -1224,7 +1239,7 @@ __global__ void __launch_bounds__(EGG_THREADS, (H > 256 ? 1 : 2)) k_head(HeadPar
                         *reinterpret_cast<v4i *>(p.logits_tap + ((size_t)mloc * T + t) * 256 + 32 * nt + 8 * q + 4 * g) = o4;
                     }
         } else {
-            target = token_at(c, spos + t + 1);
+            const int target = token_at(c, spos + t + 1);
             sum_ex = 0; tl = 0;
 #pragma unroll 1
             for (int phase = 0; phase < 2; phase++) {
@@ -1395,23 +1410,7 @@ __global__ void __launch_bounds__(EGG_THREADS, 2) k_head_big(HeadParams p) {
     if (ADAPT) dot_noise_ov<KS, 1>(nf, reinterpret_cast<const float *>(hB), 0, g, &sbh);
     else sbh = dot_noise<KS, false>(nf, hB, 0, g);
     sbh <<= c.sb_shift;
-    // the target's logit: its column of the fragment-major embedding holds 16 bytes per k-step and half, in operand order
-    int target_logit;
-    {
-        const int target = token_at(c, stream_pos_of(c, member) + t + 1);
-        int dot = 0;
-#pragma unroll
-        for (int ks = 0; ks < KS; ks++) {
-            const v4i w = *reinterpret_cast<const v4i *>(p.embedding_frag + ((size_t)(ks / (BLK / 32)) * (V / BLK) + target / BLK) * (BLK * BLK) +
-                                                         ((size_t)(2 * (ks % (BLK / 32)) + g) * BLK + target % BLK) * 16);
-#pragma unroll
-            for (int q = 0; q < 4; q++) dot = dot4(w[q], nf[ks][q], dot);
-        }
-        dot = sum_halves(dot);
-        int a = noise_from_hash(pair_seed + OFF_EMB, (uint32_t)target, c.mask);
-        if (ADAPT) a = overlay_scaled(a, p.q_emb[H + target]);
-        target_logit = (dot + __mulhi(sbh, a * ((member & 1) ? -1 : 1) << c.a_shift)) >> c.shift_logit;
-    }
+    const int target_logit = logit_of<H, ADAPT>(p, nf, sbh, pair_seed, member, token_at(c, stream_pos_of(c, member) + t + 1), g);
     const int room = HEAD_BINS - 2 - p.exp_last;
     int gmax = 0, top = 0;
 #pragma unroll 1
