@@ -83,12 +83,17 @@ __device__ __forceinline__ void exchange_operand(int8_t *buf, const TileMap &tm,
 // of the down GEMM), so only the down accumulator of the wave's column slice, the normalised input and one
 // sub-chunk accumulator are live.  W streams through two LDS buffers in units of at most 16 KB.  The residual is
 // parked in the x buffer and re-read at the end.
-template <int H>
+// Column slices of k_mlp and k_qkv, i.e. waves that share a token tile: as few as the registers allow where there are tiles
+// enough (hidden 512 with two, not four: twice the MFMAs per staged unit and half the exchanges outweigh the registers
+// of the 256-column accumulator; k_qkv 2.05 -> 1.57 ms per 2048 members x 512 tokens), twice as many where there
+// would be at most one wave to a SIMD: each then has half the work.  Forward of 64 members x 32 tokens, 2 layers: 74 -> 58 us at hidden
+// 64, 113 -> 83 at 128, 134 -> 99 at 256, 373 -> 317 at 512; at two waves to a SIMD it loses 4 to 28 %.
+template <int H> constexpr int few_slices() { return H == 512 ? 2 : Shape<H>::CS; }
+template <int H> constexpr int many_slices() { return 2 * few_slices<H>(); }
+template <int H> static bool use_many_slices(const FwdCommon &c) { return (long long)c.n_members * (c.tn / 32) * few_slices<H>() <= 1024; }     // 1024 SIMDs
+template <int H, int CSV>
 struct MlpCfg {
-    typedef Shape<H> S;
-    // hidden 512 runs the MLP with two column slices (not four): twice the MFMAs per staged unit and half the
-    // exchanges outweigh the register spills of the 256-column accumulator
-    static constexpr int CS = H == 512 ? 2 : S::CS;
+    static constexpr int CS = CSV;
     static constexpr int TPW = EGG_WAVES / CS, HS = H / CS, NTS = HS / 32, KS = H / 32;
     static constexpr int NTU = CS == 1 ? 2 : 1;          // up-GEMM column groups per wave and sub-chunk
     static constexpr int SC = 32 * CS * NTU;             // intermediate columns per sub-chunk
@@ -140,9 +145,9 @@ struct MlpCfg {
 // hidden unit, which adds its four terms (k = unit, unit + H, ...) into an int one float addition at a time; the
 // sub-chunks are therefore visited so that those four are consecutive.  At hidden 256, 2048 members x 256 tokens the overlay's
 // kernel took 0.91 ms with integer terms, spilling at three workgroups per CU; 0.63 ms as it is (0.47 without the overlay).
-template <int H, bool FIRST, bool SEED, bool ADAPT>
-__global__ void __launch_bounds__(EGG_THREADS, MlpCfg<H>::occ(ADAPT)) k_mlp(MlpParams p) {
-    typedef MlpCfg<H> M;
+template <int H, bool FIRST, bool SEED, bool ADAPT, int CSV>
+__global__ void __launch_bounds__(EGG_THREADS, (MlpCfg<H, CSV>::occ(ADAPT))) k_mlp(MlpParams p) {
+    typedef MlpCfg<H, CSV> M;
     constexpr int CS = M::CS, KS = M::KS, NTS = M::NTS, HS = M::HS, NTU = M::NTU, SC = M::SC;
     // fragments read ahead of their MFMAs: at hidden 512 the accumulators and operands leave room for four
     constexpr int MAXF = H == 512 ? 4 : 8;
@@ -255,8 +260,9 @@ __global__ void __launch_bounds__(EGG_THREADS, MlpCfg<H>::occ(ADAPT)) k_mlp(MlpP
     // The first block (embedding, norm, MLP, residual, adaptive norm) has no attention in front of it: its result is a
     // function of the member and the byte value alone.  It is therefore evaluated once per distinct byte value of the
     // member's window -- row r of `p.tab` belongs to the r-th smallest value present -- and copied to every position
-    // that holds the value at the end.  (A workgroup that serves several members keeps the per-position form.)
-    const bool dedup = FIRST && p.tab != nullptr && tm.sets == 1;
+    // that holds the value at the end.  (A workgroup that serves several members, or takes a window in one pass, keeps the
+    // per-position form.)
+    const bool dedup = FIRST && p.tab != nullptr && tm.sets == 1 && tm.passes > 1;
     uint8_t *rnk = reinterpret_cast<uint8_t *>(red) + M::RED;
     int *wcnt = reinterpret_cast<int *>(rnk + 256);
     uint8_t *uniq = H < 256 ? rnk + 272 : reinterpret_cast<uint8_t *>(exB);
@@ -534,12 +540,10 @@ __global__ void __launch_bounds__(EGG_THREADS, MlpCfg<H>::occ(ADAPT)) k_mlp(MlpP
 }
 
 // ============================================================================ QKV
-template <int H>
+template <int H, int CSV>
 struct QkvCfg {
-    typedef Shape<H> S;
-    // hidden 512: two column slices, as in the MLP (2.05 -> 1.57 ms per 2048 members x 512 tokens against four)
-    static constexpr int CS = H == 512 ? 2 : S::CS;
-    static constexpr int TPW = EGG_WAVES / CS, HS = H / CS, NTS = HS / 32, KS = S::KS;
+    static constexpr int CS = CSV;
+    static constexpr int TPW = EGG_WAVES / CS, HS = H / CS, NTS = HS / 32, KS = H / 32;
     static constexpr int PR = (H / 16) < (1024 / H) ? (H / 16) : (1024 / H), NU = (H / 16) / PR;   // p-rows per unit, units per matrix
     static constexpr int UNIT = 16 * PR * H;
     static constexpr int WBYTES = 2 * UNIT;
@@ -557,7 +561,7 @@ struct QkvCfg {
 // head, so a lane needs only the head_dim/32 * 8 pairs of its own slots.
 // The reference evaluates (ve*c -+ vo*s + 2^(bit-1)) >> bit in int64, and so does this code: 64-bit multiply-adds
 // (v_mad_i64_i32, full rate on gfx950); the shifted result fits 32 bits like the reference's AccumType.
-// The NT column groups must start at a head boundary.  The
+// The NT column groups must start at a head boundary, or be one group (rope_row then starts at it).  The
 // pairs are read where they are used (one 16-byte load per two pairs, cache hits): holding a token's 16 pairs in
 // registers across the three projections costs the 32 registers that separate two from three workgroups per CU.
 template <int NT>
@@ -586,9 +590,9 @@ __device__ __forceinline__ void rope_inplace(v16i *acc, const int32_t *rope_row,
 // noise are scaled when the per-member tables are filled, the input-side sums are taken term by term (dot_noise_ov), each
 // wave of a tile over its own column slice, and added up with the exchange of the normalised input.  Hidden 256, 2048
 // members x 256 tokens: 0.49 -> 0.32 ms with that and the float terms; without the overlay 0.29.
-template <int H, bool ADAPT>
-__global__ void __launch_bounds__(EGG_THREADS, QkvCfg<H>::OCC) k_qkv(QkvParams p) {
-    typedef QkvCfg<H> Q;
+template <int H, bool ADAPT, int CSV>
+__global__ void __launch_bounds__(EGG_THREADS, (QkvCfg<H, CSV>::OCC)) k_qkv(QkvParams p) {
+    typedef QkvCfg<H, CSV> Q;
     constexpr int CS = Q::CS, KS = Q::KS, NTS = Q::NTS, HS = Q::HS;
     extern __shared__ __align__(16) int8_t smem[];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, g = lane >> 5, j = lane & 31;
@@ -690,7 +694,7 @@ __global__ void __launch_bounds__(EGG_THREADS, QkvCfg<H>::OCC) k_qkv(QkvParams p
                 mfma_cols<Q::PR / 2, NTS>(acc, nrm + u * (Q::PR / 2), cur, H, col0, lane);
             }
             add_perturb<NTS>(acc, sb << c.sb_shift, An, col0, g);
-            if (which < 2) rope_inplace<NTS>(acc, c.rope_lut + (size_t)t * c.head_dim, c.head_dim, g, c.rope_scale_bit);
+            if (which < 2) rope_inplace<NTS>(acc, c.rope_lut + (size_t)t * c.head_dim + col0 % c.head_dim, c.head_dim, g, c.rope_scale_bit);
             const int mx = xreduce<CS, true>(absmax_to_float_groups<NTS>(acc), red + ((1 + which) & 1) * Q::SITE, tm, lane);
             v4i o[NTS];
             adaptive_scale_floats<NTS>(acc, mx, o);
@@ -1485,22 +1489,22 @@ __global__ void __launch_bounds__(EGG_THREADS, 2) k_head_big(HeadParams p) {
 }
 
 // ============================================================================ host launchers
+template <int H, bool ADAPT, int CSV>
+static hipError_t launch_mlp_cs(const MlpParams &p, bool first, hipStream_t s) {
+    const int sets = tile_map_sets(p.c.tn, CSV);
+    const dim3 grid((p.c.n_members + sets - 1) / sets), block(EGG_THREADS);
+    const size_t lds = MlpCfg<H, CSV>::total(sets, first, ADAPT);
+    const bool seed = egg_mlp_down_acc_bound(H, p.c.mask, p.c.sigma_vec, p.c.shift_mlp_down) < (1LL << 31);
+    if (first) { if (seed) hipLaunchKernelGGL((k_mlp<H, true, true, ADAPT, CSV>), grid, block, lds, s, p); else hipLaunchKernelGGL((k_mlp<H, true, false, ADAPT, CSV>), grid, block, lds, s, p); }
+    else { if (seed) hipLaunchKernelGGL((k_mlp<H, false, true, ADAPT, CSV>), grid, block, lds, s, p); else hipLaunchKernelGGL((k_mlp<H, false, false, ADAPT, CSV>), grid, block, lds, s, p); }
+    return hipGetLastError();
+}
 template <int H>
 static hipError_t launch_mlp_h(const MlpParams &p, bool first, hipStream_t s) {
-    const int sets = tile_map_sets(p.c.tn, MlpCfg<H>::CS);
-    dim3 grid((p.c.n_members + sets - 1) / sets), block(EGG_THREADS);
-    size_t lds = MlpCfg<H>::total(sets, first, p.q_ln_w != nullptr);
-    const long long up_acc = egg_mlp_up_acc_bound(H, p.c.mask, p.c.sigma_vec, p.c.shift_mlp_up);
-    if (up_acc >= (1LL << 31)) return hipErrorInvalidValue;      // egg_ctx_create refuses such shifts
-    const bool seed = egg_mlp_down_acc_bound(H, p.c.mask, p.c.sigma_vec, p.c.shift_mlp_down) < (1LL << 31);
-    if (p.q_ln_w) {      // adaptive noise overlay: its factors are at most 1, so the same bounds hold
-        if (first) { if (seed) hipLaunchKernelGGL((k_mlp<H, true, true, true>), grid, block, lds, s, p); else hipLaunchKernelGGL((k_mlp<H, true, false, true>), grid, block, lds, s, p); }
-        else { if (seed) hipLaunchKernelGGL((k_mlp<H, false, true, true>), grid, block, lds, s, p); else hipLaunchKernelGGL((k_mlp<H, false, false, true>), grid, block, lds, s, p); }
-        return hipGetLastError();
-    }
-    if (first) { if (seed) hipLaunchKernelGGL((k_mlp<H, true, true, false>), grid, block, lds, s, p); else hipLaunchKernelGGL((k_mlp<H, true, false, false>), grid, block, lds, s, p); }
-    else { if (seed) hipLaunchKernelGGL((k_mlp<H, false, true, false>), grid, block, lds, s, p); else hipLaunchKernelGGL((k_mlp<H, false, false, false>), grid, block, lds, s, p); }
-    return hipGetLastError();
+    if (egg_mlp_up_acc_bound(H, p.c.mask, p.c.sigma_vec, p.c.shift_mlp_up) >= (1LL << 31)) return hipErrorInvalidValue;      // egg_ctx_create refuses such shifts
+    if (p.q_ln_w) return launch_mlp_cs<H, true, few_slices<H>()>(p, first, s);       // the adaptive overlay has this form only
+    if (use_many_slices<H>(p.c)) return launch_mlp_cs<H, false, many_slices<H>()>(p, first, s);
+    return launch_mlp_cs<H, false, few_slices<H>()>(p, first, s);
 }
 hipError_t egg_launch_mlp(const MlpParams &p, bool first, hipStream_t s) {
     switch (p.c.H) {
@@ -1512,14 +1516,17 @@ hipError_t egg_launch_mlp(const MlpParams &p, bool first, hipStream_t s) {
     }
 }
 
+template <int H, bool ADAPT, int CSV>
+static hipError_t launch_qkv_cs(const QkvParams &p, hipStream_t s) {
+    const int sets = tile_map_sets(p.c.tn, CSV);
+    hipLaunchKernelGGL((k_qkv<H, ADAPT, CSV>), dim3((p.c.n_members + sets - 1) / sets), dim3(EGG_THREADS), (QkvCfg<H, CSV>::total(sets, ADAPT)), s, p);
+    return hipGetLastError();
+}
 template <int H>
 static hipError_t launch_qkv_h(const QkvParams &p, hipStream_t s) {
-    const int sets = tile_map_sets(p.c.tn, QkvCfg<H>::CS);
-    dim3 grid((p.c.n_members + sets - 1) / sets), block(EGG_THREADS);
-    size_t lds = QkvCfg<H>::total(sets, p.q_ln_w != nullptr);
-    if (p.q_ln_w) hipLaunchKernelGGL((k_qkv<H, true>), grid, block, lds, s, p);
-    else hipLaunchKernelGGL((k_qkv<H, false>), grid, block, lds, s, p);
-    return hipGetLastError();
+    if (p.q_ln_w) return launch_qkv_cs<H, true, few_slices<H>()>(p, s);
+    if (use_many_slices<H>(p.c)) return launch_qkv_cs<H, false, many_slices<H>()>(p, s);
+    return launch_qkv_cs<H, false, few_slices<H>()>(p, s);
 }
 hipError_t egg_launch_qkv(const QkvParams &p, hipStream_t s) {
     switch (p.c.H) {
@@ -1610,26 +1617,24 @@ static hipError_t no_static_lds(K kern) {
     if (e != hipSuccess) return e;
     return a.sharedSizeBytes == 0 ? hipSuccess : hipErrorInvalidConfiguration;
 }
+template <int H, bool ADAPT, int CSV>
+static hipError_t prepare_cs(int T) {
+    // table sets per workgroup: the whole window's, or a single tile's (a prompt's first tiles may be evaluated alone)
+    const int sets = std::max(tile_map_sets(T, CSV), tile_map_sets(32, CSV));
+    for (hipError_t e : {no_static_lds(&k_mlp<H, true, true, ADAPT, CSV>), no_static_lds(&k_mlp<H, false, true, ADAPT, CSV>),
+                         no_static_lds(&k_mlp<H, true, false, ADAPT, CSV>), no_static_lds(&k_mlp<H, false, false, ADAPT, CSV>)})
+        if (e != hipSuccess) return e;
+    SET_LDS((k_mlp<H, true, true, ADAPT, CSV>), (MlpCfg<H, CSV>::total(sets, true, ADAPT)));
+    SET_LDS((k_mlp<H, true, false, ADAPT, CSV>), (MlpCfg<H, CSV>::total(sets, true, ADAPT)));
+    SET_LDS((k_mlp<H, false, true, ADAPT, CSV>), (MlpCfg<H, CSV>::total(sets, false, ADAPT)));
+    SET_LDS((k_mlp<H, false, false, ADAPT, CSV>), (MlpCfg<H, CSV>::total(sets, false, ADAPT)));
+    SET_LDS((k_qkv<H, ADAPT, CSV>), (QkvCfg<H, CSV>::total(sets, ADAPT)));
+    return hipSuccess;
+}
 template <int H>
 static hipError_t prepare_h(int T) {
-    // table sets per workgroup: the whole window's, or a single tile's (egg_generate evaluates one tile per new token)
-    const int sets = std::max(tile_map_sets(T, QkvCfg<H>::CS), tile_map_sets(32, QkvCfg<H>::CS));
-    const int msets = std::max(tile_map_sets(T, MlpCfg<H>::CS), tile_map_sets(32, MlpCfg<H>::CS));
-    for (hipError_t e : {no_static_lds(&k_mlp<H, true, true, false>), no_static_lds(&k_mlp<H, false, true, false>),
-                         no_static_lds(&k_mlp<H, true, false, false>), no_static_lds(&k_mlp<H, false, false, false>),
-                         no_static_lds(&k_mlp<H, true, true, true>), no_static_lds(&k_mlp<H, false, true, true>),
-                         no_static_lds(&k_mlp<H, true, false, true>), no_static_lds(&k_mlp<H, false, false, true>)})
+    for (hipError_t e : {prepare_cs<H, true, few_slices<H>()>(T), prepare_cs<H, false, few_slices<H>()>(T), prepare_cs<H, false, many_slices<H>()>(T)})
         if (e != hipSuccess) return e;
-    SET_LDS((k_mlp<H, true, true, false>), MlpCfg<H>::total(msets, true, false));
-    SET_LDS((k_mlp<H, false, true, false>), MlpCfg<H>::total(msets, false, false));
-    SET_LDS((k_mlp<H, true, false, false>), MlpCfg<H>::total(msets, true, false));
-    SET_LDS((k_mlp<H, false, false, false>), MlpCfg<H>::total(msets, false, false));
-    SET_LDS((k_mlp<H, true, false, true>), MlpCfg<H>::total(msets, true, true));
-    SET_LDS((k_mlp<H, true, true, true>), MlpCfg<H>::total(msets, true, true));
-    SET_LDS((k_mlp<H, false, false, true>), MlpCfg<H>::total(msets, false, true));
-    SET_LDS((k_mlp<H, false, true, true>), MlpCfg<H>::total(msets, false, true));
-    SET_LDS((k_qkv<H, false>), QkvCfg<H>::total(sets, false));
-    SET_LDS((k_qkv<H, true>), QkvCfg<H>::total(sets, true));
     SET_LDS((k_head<H, false, false>), HeadLds<H>::total(false));
     SET_LDS((k_head<H, true, false>), HeadLds<H>::total(true));
     SET_LDS((k_head<H, false, true>), HeadLds<H>::total(false));
