@@ -456,7 +456,6 @@ extern "C" int egg_ctx_create(const egg_config *cfg, egg_ctx **out) {
     CR(hipMalloc(&ctx->d_scal, sizeof(Scalars)));
     CR(hipHostMalloc(reinterpret_cast<void **>(&ctx->h_result), 16 + (size_t)c.population * 4 + (size_t)(c.population / 2) * 4, hipHostMallocCoherent));
     memset(ctx->h_result, 0, 16 + (size_t)c.population * 4 + (size_t)(c.population / 2) * 4);
-    CR(egg_host_out_create(&ctx->out, (size_t)std::max<int64_t>(ctx->L.total, ctx->state_bytes)));
     // noise table: the rows of the widest side of any matrix (4 * hidden, or the embedding's vocabulary), every layer's seeds
     ctx->noise.pairs_pad = ((c.population / 2) + 127) / 128 * 128;
     ctx->noise.rows = std::max(4 * c.hidden, c.vocab);
@@ -504,6 +503,12 @@ extern "C" int egg_sync(egg_ctx *ctx) {
 
 extern "C" int64_t egg_model_bytes(const egg_ctx *ctx) { return ctx ? ctx->L.total : 0; }
 
+// The pinned slots of downloads, made with the first model (or the first download): a context for the linear layer alone
+// needs none.
+static int host_out_ready(egg_ctx *ctx) {
+    if (!ctx->out.mem) HIP_TRY(egg_host_out_create(&ctx->out, (size_t)std::max<int64_t>(ctx->L.total, ctx->state_bytes)));
+    return EGG_OK;
+}
 // ------------------------------------------------------------------ init_model (mgpu.cu:428-519)
 static inline uint32_t xorshift32_host(uint32_t *st) { uint32_t x = *st; x ^= x << 13; x ^= x >> 17; x ^= x << 5; *st = x; return x; }
 static inline int8_t gen_noise_host(uint32_t *rng, int mask, int gaussian) {
@@ -540,16 +545,19 @@ extern "C" int egg_model_init(egg_ctx *ctx, uint32_t seed) {
     for (int i = 0; i < H; i++) m[L.ln_f + i] = 16;
     HIP_TRY(hipStreamSynchronize(ctx->stream));
     HIP_TRY(hipMemcpy(ctx->d_model, m.data(), m.size(), hipMemcpyHostToDevice));
+    if (int rc = host_out_ready(ctx)) return rc;
     return refresh_frag(ctx);
 }
 extern "C" int egg_model_upload(egg_ctx *ctx, const void *h, size_t bytes) {
     if (!ctx || !h || (int64_t)bytes != ctx->L.total) return fail(ctx, EGG_E_INVALID, "model size mismatch");
     HIP_TRY(hipStreamSynchronize(ctx->stream));
     HIP_TRY(hipMemcpy(ctx->d_model, h, bytes, hipMemcpyHostToDevice));
+    if (int rc = host_out_ready(ctx)) return rc;
     return refresh_frag(ctx);
 }
 extern "C" int egg_model_download(egg_ctx *ctx, void *h, size_t bytes) {
     if (!ctx || !h || (int64_t)bytes != ctx->L.total) return fail(ctx, EGG_E_INVALID, "model size mismatch");
+    if (int rc = host_out_ready(ctx)) return rc;
     HIP_TRY(egg_host_out(ctx->out, h, ctx->d_model, bytes, ctx->stream));
     return EGG_OK;
 }
@@ -629,6 +637,7 @@ extern "C" int egg_opt_state_upload(egg_ctx *ctx, const void *h, size_t bytes) {
 }
 extern "C" int egg_opt_state_download(egg_ctx *ctx, void *h, size_t bytes) {
     if (!ctx || !h || (int64_t)bytes != ctx->state_bytes) return fail(ctx, EGG_E_INVALID, "state size mismatch");
+    if (int rc = host_out_ready(ctx)) return rc;
     HIP_TRY(egg_host_out(ctx->out, h, ctx->d_state, bytes, ctx->stream));
     return EGG_OK;
 }
@@ -677,8 +686,9 @@ static int linear_impl(egg_ctx *ctx, const int8_t *d_X, const int8_t *d_W, int m
     if (!ctx || !d_X || !d_W || members < 1 || T < 32 || T % 32 || (!d_Y32 && !d_Y8) || shift < 0 || shift > 31)
         return fail(ctx, EGG_E_INVALID, "egg_perturbed_linear arguments");
     if (K < 64 || N < 64 || K % 64 || N % 64) return fail(ctx, EGG_E_INVALID, "egg_perturbed_linear: K and N must be multiples of 64");
-    const bool ws = egg_plinear_ws_shape(K, N) && !ctx->plin_no_ws;
-    if (!ws && (size_t)K * N > ctx->plin_frag_bytes) {
+    // kernels that read the canonical W (egg_ctx_linear_kernel turns both off)
+    const bool direct = !ctx->plin_no_ws && (egg_plinear_ws_shape(K, N) || egg_plinear_small(members, T, K, N));
+    if (!direct && (size_t)K * N > ctx->plin_frag_bytes) {
         HIP_TRY(hipStreamSynchronize(ctx->stream));
         if (ctx->d_plin_frag) (void)hipFree(ctx->d_plin_frag);
         ctx->d_plin_frag = nullptr; ctx->plin_frag_bytes = 0;
@@ -686,9 +696,9 @@ static int linear_impl(egg_ctx *ctx, const int8_t *d_X, const int8_t *d_W, int m
         ctx->plin_frag_bytes = (size_t)K * N;
     }
     PlinParams p = {d_X, ctx->d_plin_frag, members, T, K, N, seed, off_a, off_b, shift, ctx->cfg.fixed_point + ctx->cfg.sigma_shift,
-                    noise_word(ctx->cfg), d_Y32, d_Y8, plain, own_noise, ws ? d_W : nullptr};
+                    noise_word(ctx->cfg), d_Y32, d_Y8, plain, own_noise, direct ? d_W : nullptr};
     span_begin(ctx, EGG_K_PLINEAR);
-    hipError_t e = ws ? hipSuccess : egg_launch_plinear_swizzle(d_W, ctx->d_plin_frag, T, K, N, ctx->stream);
+    hipError_t e = direct ? hipSuccess : egg_launch_plinear_swizzle(d_W, ctx->d_plin_frag, T, K, N, ctx->stream);
     if (e == hipSuccess) e = egg_launch_plinear(p, ctx->stream);
     span_end(ctx);
     if (e == hipErrorInvalidValue) return fail(ctx, EGG_E_INVALID, "egg_perturbed_linear: unsupported (K, N)");
@@ -997,6 +1007,7 @@ extern "C" int egg_overlay_upload(egg_ctx *ctx, const void *h, size_t bytes) {
 extern "C" int egg_overlay_download(egg_ctx *ctx, void *h, size_t bytes) {
     if (!ctx || !h || (int64_t)bytes != ctx->L.total) return fail(ctx, EGG_E_INVALID, "overlay size mismatch");
     if (!ctx->adaptive) return fail(ctx, EGG_E_STATE, "egg_adaptive_enable has not been called");
+    if (int rc = host_out_ready(ctx)) return rc;
     HIP_TRY(egg_host_out(ctx->out, h, ctx->d_overlay, bytes, ctx->stream));
     return EGG_OK;
 }

@@ -31,18 +31,18 @@ __global__ void __launch_bounds__(256) k_out(v4i *dst, const v4i *src, size_t by
 
 }  // namespace
 
-hipError_t egg_host_out_create(HostOut *o, size_t largest) {
-    o->slot = std::max<size_t>(4096, std::min(SLOT_MAX, ((largest + SLOTS - 1) / SLOTS + 4095) & ~(size_t)4095));
-    hipError_t e = hipHostMalloc(reinterpret_cast<void **>(&o->mem), SLOTS * o->slot, hipHostMallocCoherent);
-    for (int i = 0; i < SLOTS && e == hipSuccess; i++) e = hipEventCreateWithFlags(&o->done[i], hipEventDisableTiming | hipEventReleaseToSystem);
-    return e;
-}
 void egg_host_out_destroy(HostOut *o) {
     for (hipEvent_t &d : o->done) if (d) { (void)hipEventDestroy(d); d = nullptr; }
     if (o->mem) (void)hipHostFree(o->mem);
     o->mem = nullptr;
 }
-
+hipError_t egg_host_out_create(HostOut *o, size_t largest) {
+    o->slot = std::max<size_t>(4096, std::min(SLOT_MAX, ((largest + SLOTS - 1) / SLOTS + 4095) & ~(size_t)4095));
+    hipError_t e = hipHostMalloc(reinterpret_cast<void **>(&o->mem), SLOTS * o->slot, hipHostMallocCoherent);
+    for (int i = 0; i < SLOTS && e == hipSuccess; i++) e = hipEventCreateWithFlags(&o->done[i], hipEventDisableTiming | hipEventReleaseToSystem);
+    if (e != hipSuccess) egg_host_out_destroy(o);
+    return e;
+}
 hipError_t egg_host_out(HostOut &o, void *dst, const void *src, size_t bytes, hipStream_t s) {
     if (!o.mem || (reinterpret_cast<uintptr_t>(src) & 15)) return hipErrorInvalidValue;
     // a short piece goes as a whole, through as many slots as it covers: splitting it would cost more events than it overlaps

@@ -23,6 +23,7 @@ struct PlinParams {
                             // W-stationary kernel, which needs no fragment-major copy
 };
 bool egg_plinear_ws_shape(int K, int N);
+bool egg_plinear_small(int members, int T, int K, int N);                 // one launch on the canonical W (egg_linear.hip)
 hipError_t egg_launch_plinear_ws(const PlinParams &p, hipStream_t s);      // egg_linear_ws.hip
 hipError_t egg_launch_plinear(const PlinParams &p, hipStream_t s);
 int egg_plinear_block(int K, int N);

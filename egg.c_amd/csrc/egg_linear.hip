@@ -450,6 +450,56 @@ static hipError_t launch_two(const PlinParams &p, hipStream_t s) {
     return hipGetLastError();
 }
 
+// Few rows: one launch that reads the canonical W, where the kernels above need a rearranged copy of it first.  A call of a few
+// thousand rows is bound by its launches (8 us for two), not by what they do.  A workgroup takes a token tile and 128
+// columns, a wave 32 of them: its fragment of a k-step is four coalesced dwords a lane of W's rows of four, straight from L2,
+// all of them requested at once.  Every tile reads its columns of W again, so it is used while that is cheap (egg_plinear_small).  128 tokens: 256 x 448
+// 33 -> 4.5 us, 512 x 384 42 -> 5 us, 512 x 512 11 -> 5 us.
+template <int K>
+__global__ void __launch_bounds__(EGG_THREADS) k_plinear_small(PlinParams p) {
+    constexpr int KS = K / 32;
+    __shared__ __align__(16) int8_t Bt[K];
+    __shared__ __align__(16) int At[128];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, g = lane >> 5, j = lane & 31, N = p.N;
+    const int first = (int)blockIdx.y * 128, n0 = first + 32 * wave;
+    const bool any = n0 < N;
+    const size_t row = (size_t)blockIdx.x * 32 + j;
+    const int member = (int)((size_t)blockIdx.x * 32 / p.T);
+    v4i x[KS], w[KS];
+    if (any) {
+        const int *W = reinterpret_cast<const int *>(p.Wblocked) + n0 + j;
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+            x[ks] = load_op(p.X + row * K, ks, g);
+#pragma unroll
+            for (int q = 0; q < 4; q++) w[ks][q] = W[(size_t)(8 * ks + 4 * g + q) * N];
+        }
+    }
+    if (!p.plain) {
+        const uint32_t ps = p.seed + (uint32_t)(p.own_noise ? member : member / 2);
+        const int ns = (!p.own_noise && (member & 1)) ? -1 : 1;
+        fill_noise_i8(Bt, ps + p.off_b, K, p.mask, threadIdx.x, EGG_THREADS);
+        for (int i = threadIdx.x; i < 128; i += EGG_THREADS) At[i] = noise_from_hash(ps + p.off_a, (uint32_t)(first + i), p.mask) * ns;
+        __syncthreads();
+    }
+    if (!any) return;
+    const int sb = p.plain ? 0 : dot_noise<KS, true>(x, Bt, 0, g);
+    v16i acc;
+#pragma unroll
+    for (int r = 0; r < 16; r++) acc[r] = 0;
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(w[ks], x[ks], acc, 0, 0, 0);
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        v4i a4 = {0, 0, 0, 0}, o;
+        if (!p.plain) a4 = *reinterpret_cast<const v4i *>(At + 32 * wave + 8 * q + 4 * g);
+#pragma unroll
+        for (int e = 0; e < 4; e++) o[e] = p.plain ? acc[4 * q + e] >> p.shift : perturbed<false>(acc[4 * q + e], sb, a4[e], p.sigma, p.shift);
+        if (p.Y32) *reinterpret_cast<v4i *>(p.Y32 + row * N + n0 + 8 * q + 4 * g) = o;
+        if (p.Y8) *reinterpret_cast<int *>(p.Y8 + row * N + n0 + 8 * q + 4 * g) = pack4(clip127(o[0]), clip127(o[1]), clip127(o[2]), clip127(o[3]));
+    }
+}
+
 template <int K, int N, bool OUT32, bool FUSE>
 static hipError_t launch_one(const PlinParams &p, hipStream_t s) {
     dim3 grid((p.members + EGG_WAVES - 1) / EGG_WAVES), block(EGG_THREADS);
@@ -503,6 +553,25 @@ static hipError_t launch_two_k(const PlinParams &p, hipStream_t s) {
     return e;
 }
 
+bool egg_plinear_small(int members, int T, int K, int N) {
+    if (!(two_tile_shape(T, K, N) || one_tile_case(K, N) || egg_plinear_ws_shape(K, N)) || (K != 64 && K != 128 && K != 256 && K != 512 && K != 1024)) return false;
+    // workgroups times K: up to 2^20 against the kernels that need a rearranged W (at 2^20, 512 x 128: 25 us both; 256 x 448: 16
+    // against 34), up to 2^18 against the W-stationary one (512 x 512: 8 us against 12, twice that: 14 against 12)
+    return (long long)members * (T / 32) * ((N + 127) / 128) * K <= (egg_plinear_ws_shape(K, N) ? 1 << 18 : 1 << 20);
+}
+static hipError_t launch_small(const PlinParams &p, hipStream_t s) {
+    const dim3 grid((unsigned)((long long)p.members * (p.T / 32)), (p.N + 127) / 128), block(EGG_THREADS);
+    switch (p.K) {
+        case 64: hipLaunchKernelGGL(k_plinear_small<64>, grid, block, 0, s, p); break;
+        case 128: hipLaunchKernelGGL(k_plinear_small<128>, grid, block, 0, s, p); break;
+        case 256: hipLaunchKernelGGL(k_plinear_small<256>, grid, block, 0, s, p); break;
+        case 512: hipLaunchKernelGGL(k_plinear_small<512>, grid, block, 0, s, p); break;
+        case 1024: hipLaunchKernelGGL(k_plinear_small<1024>, grid, block, 0, s, p); break;
+        default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
 hipError_t egg_launch_plinear_swizzle(const int8_t *W, int8_t *Wf, int T, int K, int N, hipStream_t s) {
     if (two_tile_shape(T, K, N)) {
         const int chunks = K * N / 16;
@@ -517,6 +586,7 @@ hipError_t egg_launch_plinear_swizzle(const int8_t *W, int8_t *Wf, int T, int K,
 
 hipError_t egg_launch_plinear(const PlinParams &p, hipStream_t s) {
     if (p.T % 32 || p.T < 32 || p.members < 1) return hipErrorInvalidValue;
+    if (p.Wblocked && egg_plinear_small(p.members, p.T, p.K, p.N)) return launch_small(p, s);
     if (p.Wblocked && egg_plinear_ws_shape(p.K, p.N)) return egg_launch_plinear_ws(p, s);
     if (two_tile_shape(p.T, p.K, p.N)) return p.K == 256 ? launch_two_k<256>(p, s) : launch_two_k<512>(p, s);
 #define CASE(K_, N_) if (p.K == K_ && p.N == N_) return launch_kn<K_, N_>(p, s);
