@@ -52,7 +52,7 @@ EXPORTS = [
     "egg_checkpoint_save", "egg_checkpoint_load", "egg_eggc_save", "egg_eggc_load_latest",
     "egg_learning_rate", "egg_learning_rate_deggs", "egg_model_info_save", "egg_next_seed", "egg_ctx_enable_taps", "egg_ctx_first_block_dedup", "egg_tap_download",
     "egg_ctx_enable_timing", "egg_timing_reset", "egg_timing_get",
-    "egg_opt_state_bytes", "egg_tensor_state_offset", "egg_newton_schulz", "egg_describe_layout", "egg_muon_plan", "egg_ctx_generate_kv_cache", "egg_newton_schulz_static",
+    "egg_opt_state_bytes", "egg_tensor_state_offset", "egg_newton_schulz", "egg_describe_layout", "egg_muon_plan", "egg_ctx_generate_kv_cache", "egg_ctx_generate_wait_limit", "egg_newton_schulz_static",
     "egg_gru_default_config", "egg_gru_create", "egg_gru_destroy", "egg_gru_last_error", "egg_gru_model_bytes",
     "egg_gru_model_init", "egg_gru_model_upload", "egg_gru_model_download", "egg_gru_state_reset",
     "egg_gru_state_download", "egg_gru_step", "egg_gru_losses", "egg_gru_forward_mode",
@@ -127,6 +127,7 @@ def lib():
         L.egg_step_launch.argtypes = [vp, i64, u32, C.c_float]
         L.egg_step_losses.argtypes = [vp, vp, vp]
         L.egg_generate.argtypes = [vp, vp, i32, i32, u32]
+        L.egg_ctx_generate_wait_limit.argtypes = [vp, i32]
         L.egg_generate_deggs.argtypes = [vp, vp, i32, i32, u32, C.c_float, C.c_float, C.c_float]
         L.egg_deggs_sampling_constants.argtypes = [vp, C.c_float, C.c_float, C.POINTER(C.c_int32), C.POINTER(C.c_int32)]
         L.egg_shape_fitness.argtypes = [vp, i32, i32, C.c_double, i32, C.c_double, vp, vp]
@@ -434,6 +435,10 @@ class Context:
         """The same with d-eggs' sampler: temperature, min-p filter and presence penalty (its defaults)."""
         self._ck(lib().egg_generate_deggs(self._h, C.c_void_p(d_buffer), seed_len, gen_len, seed & 0xFFFFFFFF, temp, min_p, penalty),
                  "egg_generate_deggs")
+
+    def generate_wait_limit(self, polls):
+        """Polls after which a wait of the persistent generation launch is given up (0: at once, one workgroup does it all)."""
+        self._ck(lib().egg_ctx_generate_wait_limit(self._h, polls), "egg_ctx_generate_wait_limit")
 
     def generate_kv_cache(self, on=True):
         """egg_generate / egg_generate_deggs with (default) or without the per-layer K / V cache; same tokens either way."""

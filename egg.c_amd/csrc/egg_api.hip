@@ -80,7 +80,8 @@ struct egg_ctx {
     // generation (egg_generate): token buffer [T + 1], logits of one member [T][vocab], a zero start index / seed
     uint8_t *d_gen_tok = nullptr; int32_t *d_gen_logits = nullptr, *d_gen_ws = nullptr; Scalars *d_gen_scal = nullptr;
     int8_t *d_gen_kv = nullptr; bool gen_kv_cache = true;      // per-layer K / V rows of the prompt (egg_ctx_generate_kv_cache)
-    int8_t *d_dec_kv = nullptr; unsigned long long *d_dec_slots = nullptr; uint32_t *d_dec_epoch = nullptr; int *h_dec_fail = nullptr;    // egg_decode.hip
+    int8_t *d_dec_kv = nullptr; unsigned long long *d_dec_slots = nullptr; uint32_t *d_dec_epoch = nullptr;    // egg_decode.hip; behind the epoch its flag
+    int dec_wait_limit = 1 << 23;   // polls of one wait, some seconds (egg_ctx_generate_wait_limit)
     int mask_override = -1; int32_t *logits_override = nullptr;
     bool first_dedup = true;        // first block once per distinct byte value of a member's window (egg_ctx_first_block_dedup)
     VecDesc *d_vec_desc = nullptr; int n_vec = 0, vec_total = 0;       // all vector tensors, then each on its own
@@ -275,7 +276,6 @@ static void free_all(egg_ctx *ctx) {
                     ctx->noise.neg, ctx->noise.nonzero, ctx->noise.general, ctx->d_mat, ctx->d_tap, ctx->d_tap_logits, ctx->d_gen_tok, ctx->d_gen_logits, ctx->d_gen_ws, ctx->d_gen_scal, ctx->d_gen_kv, ctx->d_dec_kv, ctx->d_dec_slots, ctx->d_dec_epoch, ctx->d_vec_desc,
                     ctx->d_overlay, ctx->d_overlay_q, ctx->d_flags, ctx->d_ov_segs};
     for (void *p : ptrs) if (p) (void)hipFree(p);
-    if (ctx->h_dec_fail) (void)hipHostFree(ctx->h_dec_fail);
     if (ctx->h_result) (void)hipHostFree(ctx->h_result);
     egg_host_out_destroy(&ctx->out);
     for (auto &sp : ctx->spans) { (void)hipEventDestroy(sp.a); (void)hipEventDestroy(sp.b); }
@@ -497,7 +497,6 @@ extern "C" int egg_ctx_set_stream(egg_ctx *ctx, void *s) {
 extern "C" int egg_sync(egg_ctx *ctx) {
     if (!ctx) return EGG_E_INVALID;
     HIP_TRY(hipStreamSynchronize(ctx->stream));
-    if (ctx->h_dec_fail && *(volatile int *)ctx->h_dec_fail) return fail(ctx, EGG_E_HIP, "a generation did not finish: its workgroups were not on the GPU together");
     return EGG_OK;
 }
 
@@ -1144,23 +1143,16 @@ extern "C" uint32_t egg_next_seed(uint32_t seed, uint64_t step) {
 // by token (egg_decode.hip).  With the cache switched off (egg_ctx_generate_kv_cache) every new token runs the forward
 // over the whole window instead and is sampled by a launch of its own; the tokens are the same.
 struct DeggsSampling { float temp; int min_p_limit, penalty_int; };
-// the persistent launch's buffers; a launch that gave up leaves them in no defined state
+// the persistent launch's buffers
 static int decode_buffers(egg_ctx *ctx) {
     const egg_config &c = ctx->cfg; const size_t strips = c.hidden / 16, slots = (size_t)egg_decode_slots(c.hidden) * 8;
-    if (!ctx->h_dec_fail) {
-        HIP_TRY(egg_prepare_decode(c.hidden, c.vocab));
-        HIP_TRY(hipMalloc(&ctx->d_dec_kv, strips * c.n_layers * c.seq_len * (c.head_dim + 16)));
-        HIP_TRY(hipMalloc(&ctx->d_dec_slots, slots)); HIP_TRY(hipMalloc(&ctx->d_dec_epoch, 4));
-        HIP_TRY(hipMemset(ctx->d_dec_slots, 0, slots)); HIP_TRY(hipMemset(ctx->d_dec_epoch, 0, 4));
-        HIP_TRY(hipHostMalloc(&ctx->h_dec_fail, sizeof(int)));
-        *ctx->h_dec_fail = 0;
-    }
-    if (*(volatile int *)ctx->h_dec_fail) {
-        HIP_TRY(hipStreamSynchronize(ctx->stream));
-        HIP_TRY(hipMemset(ctx->d_dec_slots, 0, slots)); HIP_TRY(hipMemset(ctx->d_dec_epoch, 0, 4));
-        *ctx->h_dec_fail = 0;
-        return fail(ctx, EGG_E_HIP, "the generation before this one did not finish: its workgroups were not on the GPU together");
-    }
+    if (ctx->d_dec_epoch) return EGG_OK;
+    HIP_TRY(egg_prepare_decode(c.hidden, c.vocab));
+    if (!ctx->d_dec_kv) HIP_TRY(hipMalloc(&ctx->d_dec_kv, strips * c.n_layers * c.seq_len * (c.head_dim + 16)));
+    if (!ctx->d_dec_slots) HIP_TRY(hipMalloc(&ctx->d_dec_slots, slots));
+    HIP_TRY(hipMemset(ctx->d_dec_slots, 0, slots));
+    HIP_TRY(hipMalloc(&ctx->d_dec_epoch, 8));
+    HIP_TRY(hipMemset(ctx->d_dec_epoch, 0, 8));
     return EGG_OK;
 }
 static int generate_impl(egg_ctx *ctx, uint8_t *d_buffer, int seed_len, int gen_len, uint32_t seed, const DeggsSampling *de) {
@@ -1213,8 +1205,9 @@ static int generate_impl(egg_ctx *ctx, uint8_t *d_buffer, int seed_len, int gen_
             p.shift_attn = c.shift_attn; p.shift_out = c.shift_out; p.shift_logit = c.shift_logit; p.shift_up = c.shift_mlp_up; p.shift_dn = c.shift_mlp_down;
             p.rope_bit = c.rope_scale_bit;
             p.tokens = d_buffer; p.out = d_buffer; p.token_bytes = tb; p.t_first = seed_len - 1; p.count = gen_len;
-            p.prompt_kv = ctx->d_gen_kv; p.kcache = ctx->d_dec_kv; p.vcache = ctx->d_dec_kv + (size_t)(c.hidden / 16) * c.n_layers * T * c.head_dim;
-            p.slots = ctx->d_dec_slots; p.epoch = ctx->d_dec_epoch; p.fail = ctx->h_dec_fail;
+            p.kv = ctx->d_gen_kv; p.logits = ctx->d_gen_ws; p.kcache = ctx->d_dec_kv; p.vcache = ctx->d_dec_kv + (size_t)(c.hidden / 16) * c.n_layers * T * c.head_dim;
+            p.slots = ctx->d_dec_slots; p.epoch = ctx->d_dec_epoch;
+            p.fail = reinterpret_cast<int *>(ctx->d_dec_epoch + 1); p.wait_limit = ctx->dec_wait_limit;
             p.seed = seed; p.deggs = de != nullptr; p.temp = de ? de->temp : 1.f; p.min_p_limit = de ? de->min_p_limit : 0; p.penalty_int = de ? de->penalty_int : 0;
             const hipError_t e = egg_launch_decode(p, c.hidden, s);
             if (e != hipSuccess) rc = fail(ctx, EGG_E_HIP, "egg_launch_decode", e);
@@ -1240,6 +1233,11 @@ static int generate_impl(egg_ctx *ctx, uint8_t *d_buffer, int seed_len, int gen_
 extern "C" int egg_ctx_generate_kv_cache(egg_ctx *ctx, int enable) {
     if (!ctx) return EGG_E_INVALID;
     ctx->gen_kv_cache = enable != 0;
+    return EGG_OK;
+}
+extern "C" int egg_ctx_generate_wait_limit(egg_ctx *ctx, int polls) {
+    if (!ctx || polls < 0) return fail(ctx, EGG_E_INVALID, "egg_ctx_generate_wait_limit arguments");
+    ctx->dec_wait_limit = polls;
     return EGG_OK;
 }
 extern "C" int egg_generate(egg_ctx *ctx, uint8_t *d_buffer, int seed_len, int gen_len, uint32_t seed) {

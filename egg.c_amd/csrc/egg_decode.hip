@@ -4,21 +4,25 @@
 // A token of the unperturbed model is a chain of small matrix-vector products: what bounds it is not the weights (29 MB at
 // hidden 512, 8 layers: 6 us at the memory's rate) but how fast one stage's result reaches the next stage's workgroups.
 // As launches over one 32-token tile (one workgroup each, 2 L + 2 of them streaming whole matrices through one CU) a
-// token took 1.76 ms at that size and 93 us at hidden 256, 4 layers.  Here H / 16 workgroups stay for the whole
+// token took 1.76 ms at that size (vocabulary 8192) and 93 us at hidden 256, 4 layers, vocabulary 256.  Here H / 16 workgroups stay for the whole
 // continuation; workgroup w owns 16 columns of every H-wide product (48 of Q | K | V, 64 of the MLP's up projection, V / 16
 // tiles of the head dealt round) and they exchange results through tagged messages: 8 bytes, the value and the number
 // of the exchange, written and polled with device-scope accesses, so the data is its own arrival flag and an exchange costs
 // one store-to-load trip (0.6 us on one XCD, 1.0 us across them) instead of a launch.  Everything every workgroup needs
 // whole -- the residual row, the norms -- each computes for itself.  The weights of a stage are requested in front of the
-// wait for its input.  Measured: 96 and 39 us a token at the two sizes; an exchange takes 0.8 to 1.5 us with the waits for
-// the slowest workgroup, the short dependent computations between two of them 0.3 to 1 us.  All workgroups on one XCD
+// wait for its input.  Measured: 97 and 47 us a token at the two sizes for one continuation on its own (64 tokens behind
+// a prompt of 32: 7.0 and 3.1 ms); contexts that generate at the same time share the chip, three of them finish one each 2.7 and
+// 1.1 ms.  An exchange takes 0.8 to 1.5 us with the waits for the slowest workgroup, the short dependent computations between
+// two of them 0.3 to 1 us.  All workgroups on one XCD
 // were 5 % faster at hidden 256 and 8 % slower at 512 (the weights do not fit its L2), and several such launches would
 // share that XCD.
 //
 // A message slot is written again one exchange of the same kind later.  Every workgroup sends in every exchange of a layer
 // and takes in all it needs of an exchange before it sends in the next, so a slot is only written again when its last
 // reader is past it.  Workgroups hold few resources (256 threads, two to a CU by their registers) and need not start together, only be
-// resident together in the end; a wait that is not answered within its bound ends the launch and raises `fail`.
+// resident together in the end.  A wait that is not answered within its bound raises `fail` and ends the launch; the launch
+// behind it (k_decode_alone) then does the whole continuation with one workgroup, which waits for nobody, and clears the
+// messages.  So a continuation always arrives, in stream order, and what is queued behind it finds everything in its initial state.
 #include "egg_device.h"
 #include "egg_launch.h"
 
@@ -27,7 +31,6 @@
 namespace {
 
 constexpr int THREADS = 256;
-constexpr int MAX_POLLS = 1 << 23;             // some seconds
 typedef unsigned long long u64;
 
 // ---- messages
@@ -35,10 +38,12 @@ typedef unsigned long long u64;
 __device__ __forceinline__ void send(u64 *slots, uint32_t i, uint32_t tag, int value) {
     __hip_atomic_store(slots + i, ((u64)tag << 32) | (uint32_t)value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-// N slots `stride` apart, all wanted with the same tag; slots from `count` on are not waited for
+// N slots `stride` apart, all wanted with the same tag; slots from `count` on are not waited for.  false: not within `limit` polls
 template <int N>
-__device__ __forceinline__ bool receive(int (&out)[N], const u64 *slots, uint32_t first, uint32_t stride, int count, uint32_t tag) {
-    for (int polls = 0; polls < MAX_POLLS; polls++) {
+__device__ __forceinline__ bool receive(int (&out)[N], const u64 *slots, uint32_t first, uint32_t stride, int count, uint32_t tag, int limit) {
+#pragma unroll
+    for (int i = 0; i < N; i++) out[i] = 0;
+    for (int polls = 0; polls < limit; polls++) {
         u64 m[N];
 #pragma unroll
         for (int i = 0; i < N; i++) m[i] = __hip_atomic_load(slots + (i < count ? first + i * stride : 0u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -179,11 +184,11 @@ struct Norm {                                   // gains and biases of a standar
 
 // the residual values of an exchange: adaptive norm (egg_adaptive_normalize.h:10-103) -> new residual row, in x and in s.x
 template <int H>
-__device__ __forceinline__ bool take_residual(Lds &s, const u64 *slots, uint32_t tag, int (&x)[Norm<H>::NE]) {
+__device__ __forceinline__ bool take_residual(Lds &s, const u64 *slots, uint32_t tag, int (&x)[Norm<H>::NE], int limit) {
     constexpr int NE = Norm<H>::NE;
     const int tid = threadIdx.x;
     int v[NE];
-    if (!receive<NE>(v, slots, tid, 256, tid < H ? NE : 0, tag)) s.dead = 1;
+    if (!receive<NE>(v, slots, tid, 256, tid < H ? NE : 0, tag, limit)) s.dead = 1;
     int mx = 0;
 #pragma unroll
     for (int i = 0; i < NE; i++) { if (tid >= H) v[i] = 0; mx = max(mx, abs(v[i])); }
@@ -211,9 +216,9 @@ __device__ __forceinline__ int exp_of(const Lds &s, const DecodeParams &p, int l
     return s.lut[idx < 0 ? 0 : (idx > 255 ? 255 : idx)];
 }
 
-// a wait ran into its bound: say so in host memory and leave (the others run into theirs)
+// a wait ran into its bound: say so and leave (the others run into theirs, and who has not started yet does not begin)
 __device__ void give_up(const DecodeParams &p) {
-    if (threadIdx.x == 0) __hip_atomic_store(p.fail, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (threadIdx.x == 0) __hip_atomic_store(p.fail, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // The sampler (mgpu.cu:1212-1283, d-eggs/src/kernels.cu:382-478): maximum, table weights, threshold hash_rng(seed + 555 t, 0)
@@ -239,7 +244,7 @@ __device__ bool sample(Lds &s, int *logit, int count, const DecodeParams &p, int
     if (tid == 0) send(m_max, wg, tag, mx);
     if (wave == 0) {
         int got[1];
-        if (!receive<1>(got, m_max, lane & 31, 0, (lane & 31) < G ? 1 : 0, tag)) s.dead = 1;
+        if (!receive<1>(got, m_max, lane & 31, 0, (lane & 31) < G ? 1 : 0, tag, p.wait_limit)) s.dead = 1;
         mx = row_pair_reduce<true>(row_reduce<true>((lane & 31) < G ? got[0] : INT_MIN));
         if (lane == 0) s.smax[0] = mx;
     }
@@ -256,7 +261,7 @@ __device__ bool sample(Lds &s, int *logit, int count, const DecodeParams &p, int
         const long long upto16 = scan64(lane < 16 ? mine : 0), all = lane64(upto16, 63);
         if (lane < 2) send(m_sum, 2 * wg + lane, tag, (int)(lane ? all >> 32 : all));
         int got[2];
-        if (!receive<2>(got, m_sum, 2 * (lane & 31), 1, (lane & 31) < G ? 2 : 0, tag)) s.dead = 1;
+        if (!receive<2>(got, m_sum, 2 * (lane & 31), 1, (lane & 31) < G ? 2 : 0, tag, p.wait_limit)) s.dead = 1;
         const long long theirs = lane < G ? ((long long)got[1] << 32) | (uint32_t)got[0] : 0;
         const long long upto = scan64(theirs), total = lane64(upto, 63);
         const uint32_t r = hash_rng(p.seed + (uint32_t)t * 555u, 0);
@@ -285,7 +290,7 @@ __device__ bool sample(Lds &s, int *logit, int count, const DecodeParams &p, int
                 else reinterpret_cast<uint8_t *>(p.out)[t + 1] = (uint8_t)sel;
             }
         }
-        if (lane == 0) { if (receive<1>(got1, m_tok, 0, 0, 1, tag)) s.tok[t + 1] = got1[0]; else s.dead = 1; }
+        if (lane == 0) { if (receive<1>(got1, m_tok, 0, 0, 1, tag, p.wait_limit)) s.tok[t + 1] = got1[0]; else s.dead = 1; }
     }
     __syncthreads();
     return !s.dead;
@@ -309,7 +314,7 @@ __global__ void __launch_bounds__(THREADS) k_decode(DecodeParams p) {
     for (int i = tid; i <= p.t_first; i += THREADS) s.tok[i] = p.token_bytes == 4 ? (int)reinterpret_cast<const uint32_t *>(p.tokens)[i] : (int)p.tokens[i];
     // the prompt's K / V rows (slot order, [layer][K, V][T][H]) -> this workgroup's own copies: its head's keys, its strip's values
     for (int l = 0; l < p.n_layers; l++) {
-        const int8_t *K = p.prompt_kv + (size_t)(2 * l) * T * H, *Vv = K + (size_t)T * H;
+        const int8_t *K = p.kv + (size_t)(2 * l) * T * H, *Vv = K + (size_t)T * H;
         const int kd = hd / 4;
         for (int i = tid; i < p.t_first * kd; i += THREADS) {
             const int row = i / kd, d = i % kd;
@@ -320,7 +325,9 @@ __global__ void __launch_bounds__(THREADS) k_decode(DecodeParams p) {
             *reinterpret_cast<int *>(vc + ((size_t)l * T + row) * 16 + 4 * d) = *reinterpret_cast<const int *>(Vv + (size_t)row * H + slot_of(c0 + 4 * d));
         }
     }
+    if (tid == 0 && __hip_atomic_load(p.fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) s.dead = 1;
     __syncthreads();
+    if (s.dead) return;
     const uint32_t steps = (uint32_t)p.n_layers + 2u;
     for (int t = p.t_first; t < p.t_first + p.count; t++, tag += steps) {
         // ---- embedding (mgpu.cu:901-934, ns = 0)
@@ -344,7 +351,7 @@ __global__ void __launch_bounds__(THREADS) k_decode(DecodeParams p) {
                 const int row = (tid >> 4) & 3, n = tid & 15;
                 const int rope_at = t * hd + ((c0 + n) % hd & ~1);
                 const int cs = p.rope_lut[rope_at], sn = p.rope_lut[rope_at + 1];
-                if (!take_residual<H>(s, m_dn, tg - 1, x)) return give_up(p);
+                if (!take_residual<H>(s, m_dn, tg - 1, x, p.wait_limit)) return give_up(p);
                 ln.apply(s, x);
                 const int acc = qkv.finish(s);
                 v4i kr[2][4]; int vr[8];
@@ -374,7 +381,7 @@ __global__ void __launch_bounds__(THREADS) k_decode(DecodeParams p) {
                 const bool head_thread = tid >= 128 && lane < hd, max_thread = tid < 96 && (tid & 31) < G;
                 int got[1];
                 if (!receive<1>(got, m_qkv, head_thread ? (head * strips + lane / 16) * 64 + (tid < 192 ? 0 : 16) + (lane & 15) : (tid & 31) * 64 + 48 + (tid >> 5), 0,
-                                head_thread || max_thread ? 1 : 0, tg)) s.dead = 1;
+                                head_thread || max_thread ? 1 : 0, tg, p.wait_limit)) s.dead = 1;
                 const int mx32 = row_pair_reduce<true>(row_reduce<true>(max_thread ? got[0] : 0));
                 if (tid < 96 && (tid & 31) == 0) s.smax[tid >> 5] = mx32;
                 __syncthreads();
@@ -446,7 +453,7 @@ __global__ void __launch_bounds__(THREADS) k_decode(DecodeParams p) {
                 // ---- output projection of the strip, residual
                 {
                     int a[1];
-                    if (!receive<1>(a, m_ao, tid, 0, tid < H / 4 ? 1 : 0, tg)) s.dead = 1;
+                    if (!receive<1>(a, m_ao, tid, 0, tid < H / 4 ? 1 : 0, tg, p.wait_limit)) s.dead = 1;
                     if (tid < H / 4) *reinterpret_cast<int *>(s.op + slot_of(4 * tid)) = a[0];
                     const int o = wo.finish(s);
                     if (s.dead) return give_up(p);
@@ -461,7 +468,7 @@ __global__ void __launch_bounds__(THREADS) k_decode(DecodeParams p) {
             const int bu = tid < 64 ? b_up[(uint32_t)(64 * wg + tid)] : 0;
             if (l >= 0) {
                 ln.load(M + (p.ln_2 + l * (uint32_t)H), M + (p.ln_2_bias + l * (uint32_t)H));
-                if (!take_residual<H>(s, m_res, tg, x)) return give_up(p);
+                if (!take_residual<H>(s, m_res, tg, x, p.wait_limit)) return give_up(p);
             }
             ln.apply(s, x);
             {
@@ -477,7 +484,7 @@ __global__ void __launch_bounds__(THREADS) k_decode(DecodeParams p) {
             const int bd = tid < 16 ? b_dn[(uint32_t)(c0 + tid)] : 0;
             {
                 int a[NE];
-                if (!receive<NE>(a, m_up, tid, 256, tid < H ? NE : 0, tg)) s.dead = 1;
+                if (!receive<NE>(a, m_up, tid, 256, tid < H ? NE : 0, tg, p.wait_limit)) s.dead = 1;
 #pragma unroll
                 for (int i = 0; i < NE; i++)
                     if (tid < H) *reinterpret_cast<int *>(s.op + slot_of(4 * (tid + 256 * i))) = a[i];
@@ -492,7 +499,7 @@ __global__ void __launch_bounds__(THREADS) k_decode(DecodeParams p) {
         // ---- head: tiles of 16 columns dealt round, four at a time
         const uint32_t tg = tag + (uint32_t)p.n_layers + 1u;
         constexpr int BLOCK = H > 256 ? 256 : H;
-        if (!take_residual<H>(s, m_dn, tg - 1, x)) return give_up(p);
+        if (!take_residual<H>(s, m_dn, tg - 1, x, p.wait_limit)) return give_up(p);
         ln.apply(s, x);
         int count = 0;                          // logits of this workgroup
         for (int t0 = wg; t0 < V / 16; t0 += 4 * G) {
@@ -517,17 +524,176 @@ __global__ void __launch_bounds__(THREADS) k_decode(DecodeParams p) {
     if (wg == 0 && tid == 0) *p.epoch = tag;
 }
 
+// The same continuation by one workgroup, if the launch in front gave up: no exchange, nothing to wait for.  It reads the canonical
+// weights (a thread a column), keeps the K / V rows behind the prompt's and the logits in memory, and then puts messages, epoch
+// and flag back to what a first launch finds.  Written to be right, not fast (0.2 ms a token at hidden 256, 4 layers,
+// 2.1 ms at hidden 512, 8 layers, vocabulary 8192); with nothing to do its launch does not show in a continuation's time.
+struct Alone {
+    int8_t q[512], ao[512];                     // slot order
+    int wide[3 * 512];                          // results of a product, by column
+    long long tsum[512];
+    int tok;
+};
+__device__ __forceinline__ int column(const Lds &s, const int8_t *W, int K, int N, int n) {
+    const int *w = reinterpret_cast<const int *>(W) + n;
+    int acc = 0;
+    for (int k = 0; k < K / 4; k++) acc = dot4(w[(size_t)k * N], *reinterpret_cast<const int *>(s.op + slot_of(4 * k)), acc);
+    return acc;
+}
+template <int H>
+__global__ void __launch_bounds__(THREADS) k_decode_alone(DecodeParams p) {
+    constexpr int NE = Norm<H>::NE;
+    __shared__ Lds s;
+    __shared__ Alone a;
+    if (!*p.fail) return;
+    const int tid = threadIdx.x, T = p.T, V = p.vocab, hd = p.head_dim;
+    const int8_t *const M = p.model;
+    const size_t hh = (size_t)H * H;
+    s.lut[tid] = p.exp_lut[tid]; s.act[tid] = p.act_lut[tid];
+    for (int i = tid; i <= p.t_first; i += THREADS) s.tok[i] = p.token_bytes == 4 ? (int)reinterpret_cast<const uint32_t *>(p.tokens)[i] : (int)p.tokens[i];
+    __syncthreads();
+    int x[NE];
+    Norm<H> ln;
+    auto byte_of = [](int k) { return slot_of(k & ~3) + (k & 3); };
+    // adaptive norm of H values of a.wide (egg_adaptive_normalize.h:10-103) -> out(k, value)
+    auto adapt = [&](const int *v, auto out) {
+        __syncthreads();
+        int mx = 0;
+        for (int k = tid; k < H; k += THREADS) mx = max(mx, abs(v[k]));
+        mx = wg_reduce<true>(mx, s.redm);
+        const float scale = 127.0f / ((float)mx + 1e-9f);
+        for (int k = tid; k < H; k += THREADS) out(k, round_half_away((float)v[k] * scale));
+        __syncthreads();
+    };
+    auto residual = [&] {                       // a.wide -> the residual row
+        adapt(a.wide, [&](int k, int v) { s.x[k] = (int8_t)v; });
+#pragma unroll
+        for (int i = 0; i < NE; i++) { const int k = tid + 256 * i; x[i] = k < H ? (int)s.x[k] : 0; }
+    };
+    auto norm = [&](uint32_t w, uint32_t b) { ln.load(M + w, M + b); ln.apply(s, x); __syncthreads(); };
+    for (int t = p.t_first; t < p.t_first + p.count; t++) {
+        const int token = s.tok[t];
+#pragma unroll
+        for (int i = 0; i < NE; i++) {
+            const int k = tid + 256 * i;
+            x[i] = k < H ? clip127((int)(M + p.embedding)[((size_t)(k >> 2) * V + token) * 4 + (k & 3)] + (int)(M + p.emb_bias)[k]) : 0;
+            if (k < H) s.x[k] = (int8_t)x[i];
+        }
+        for (int l = -1; l < p.n_layers; l++) {
+            if (l >= 0) {
+                norm(p.ln_1 + l * (uint32_t)H, p.ln_1_bias + l * (uint32_t)H);
+                for (int n = tid; n < H; n += THREADS) {
+                    a.wide[n] = column(s, M + p.w_q + l * hh, H, H, n);
+                    a.wide[H + n] = column(s, M + p.w_k + l * hh, H, H, n);
+                    a.wide[2 * H + n] = column(s, M + p.w_v + l * hh, H, H, n);
+                }
+                __syncthreads();
+                for (int i = tid; i < H; i += THREADS) {          // RoPE of the pairs of Q, then of K
+                    int *v = a.wide + 2 * i;
+                    const int at = t * hd + 2 * i % H % hd;
+                    const long long c = p.rope_lut[at], sn = p.rope_lut[at + 1], half = 1ll << (p.rope_bit - 1), v0 = v[0], v1 = v[1];
+                    v[0] = (int)((v0 * c - v1 * sn + half) >> p.rope_bit);
+                    v[1] = (int)((v0 * sn + v1 * c + half) >> p.rope_bit);
+                }
+                int8_t *const K = p.kv + (size_t)(2 * l) * T * H, *const Vv = K + (size_t)T * H;
+                adapt(a.wide, [&](int k, int v) { a.q[byte_of(k)] = (int8_t)v; });
+                adapt(a.wide + H, [&](int k, int v) { K[(size_t)t * H + byte_of(k)] = (int8_t)v; });
+                adapt(a.wide + 2 * H, [&](int k, int v) { Vv[(size_t)t * H + byte_of(k)] = (int8_t)v; });
+                for (int c0 = 0; c0 < H; c0 += hd) {              // a head
+                    int mx = INT_MIN;
+                    for (int at = tid; at <= t; at += THREADS) {
+                        int d = 0;
+                        for (int i = 0; i < hd / 4; i++)
+                            d = dot4(*reinterpret_cast<const int *>(K + (size_t)at * H + c0 + 4 * i), *reinterpret_cast<const int *>(a.q + c0 + 4 * i), d);
+                        s.w[at] = d >> p.shift_attn;
+                        mx = max(mx, s.w[at]);
+                    }
+                    mx = wg_reduce<true>(mx, s.smax);
+                    for (int at = tid; at <= t; at += THREADS) s.w[at] = s.lut[min(mx - s.w[at], 255)];
+                    __syncthreads();
+                    if (tid < hd) {
+                        const int at0 = byte_of(c0 + tid);
+                        long long num = 0, den = 0;
+                        for (int at = 0; at <= t; at++) { num += (long long)s.w[at] * Vv[(size_t)at * H + at0]; den += s.w[at]; }
+                        a.ao[at0] = (int8_t)(num / (den ? den : 1));
+                    }
+                    __syncthreads();
+                }
+                for (int k = tid; k < H / 4; k += THREADS) reinterpret_cast<int *>(s.op)[k] = reinterpret_cast<const int *>(a.ao)[k];
+                __syncthreads();
+                for (int n = tid; n < H; n += THREADS) a.wide[n] = (int)s.x[n] + (column(s, M + p.w_o + l * hh, H, H, n) >> p.shift_out);
+                residual();
+                norm(p.ln_2 + l * (uint32_t)H, p.ln_2_bias + l * (uint32_t)H);
+            } else
+                norm(p.ln_init, p.ln_init_bias);
+            const int8_t *up = M + (l < 0 ? p.w_up_init : p.w_up + 4 * l * hh), *b_up = M + (l < 0 ? p.b_up_init : p.b_up + l * (size_t)(4 * H));
+            const int8_t *dn = M + (l < 0 ? p.w_dn_init : p.w_dn + 4 * l * hh), *b_dn = M + (l < 0 ? p.b_dn_init : p.b_dn + l * (size_t)H);
+            int g[4 * NE];
+#pragma unroll
+            for (int i = 0; i < 4 * NE; i++) {
+                const int n = tid + 256 * i;
+                g[i] = n < 4 * H ? s.act[(uint8_t)clip127((column(s, up, H, 4 * H, n) >> p.shift_up) + b_up[n])] : 0;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < 4 * NE; i++) { const int n = tid + 256 * i; if (n < 4 * H) s.op[byte_of(n)] = (int8_t)g[i]; }
+            __syncthreads();
+            for (int n = tid; n < H; n += THREADS) a.wide[n] = (int)s.x[n] + (column(s, dn, 4 * H, H, n) >> p.shift_dn) + b_dn[n];
+            residual();
+        }
+        norm(p.ln_f, p.ln_f_bias);
+        int mx = INT_MIN;
+        for (int v = tid; v < V; v += THREADS) {
+            int lg = column(s, M + p.embedding, H, V, v) >> p.shift_logit;
+            if (p.deggs && p.penalty_int) {
+                uint32_t count = 0;
+                for (int i = 0; i <= t; i++) count += s.tok[i] == v;
+                lg = (int)((uint32_t)lg - count * (uint32_t)p.penalty_int);
+            }
+            p.logits[v] = lg;
+            mx = max(mx, lg);
+        }
+        mx = wg_reduce<true>(mx, s.redm);
+        // the order of the reference's H threads: thread r owns v = r, r + H, ... (see sample)
+        for (int r = tid; r < H; r += THREADS) {
+            long long sum = 0;
+            for (int v = r; v < V; v += H) sum += exp_of(s, p, p.logits[v], mx);
+            a.tsum[r] = sum;
+        }
+        __syncthreads();
+        if (tid == 0) {
+            long long total = 0, running = 0;
+            for (int r = 0; r < H; r++) total += a.tsum[r];
+            const long long thresh = total > 0 ? (long long)hash_rng(p.seed + (uint32_t)t * 555u, 0) % total : 0;
+            int r = 0, sel = 0;
+            while (r < H && running + a.tsum[r] <= thresh) running += a.tsum[r++];
+            for (int v = r; r < H && v < V; v += H) {
+                running += exp_of(s, p, p.logits[v], mx);
+                if (running > thresh) { sel = v; break; }
+            }
+            s.tok[t + 1] = sel;
+            if (p.token_bytes == 4) reinterpret_cast<uint32_t *>(p.out)[t + 1] = (uint32_t)sel;
+            else reinterpret_cast<uint8_t *>(p.out)[t + 1] = (uint8_t)sel;
+        }
+        __syncthreads();
+    }
+    for (int64_t i = tid; i < egg_decode_slots(H); i += THREADS) p.slots[i] = 0;
+    if (tid == 0) { *p.epoch = 0; *p.fail = 0; }
+}
+
 // the logits that the workgroup with the most head tiles keeps
 int logit_bytes(int H, int vocab) { return (vocab / 16 + H / 16 - 1) / (H / 16) * 16 * (int)sizeof(int); }
 template <int H>
 hipError_t launch(const DecodeParams &p, hipStream_t s) {
     hipLaunchKernelGGL(k_decode<H>, dim3(H / 16), dim3(THREADS), logit_bytes(H, p.vocab), s, p);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_decode_alone<H>, dim3(1), dim3(THREADS), 0, s, p);
     return hipGetLastError();
 }
 
 }  // namespace
 
-int64_t egg_decode_slots(int H) { return (int64_t)(H / 16) * 67 + 4 * H + 8; }
 hipError_t egg_prepare_decode(int H, int vocab) {
     const int bytes = logit_bytes(H, vocab);
     if (bytes + (int)sizeof(Lds) <= 64 * 1024) return hipSuccess;

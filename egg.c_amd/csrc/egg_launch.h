@@ -111,14 +111,15 @@ struct DecodeParams {
     const uint8_t *tokens;             // the prompt: tokens 0..t_first of token_bytes each
     void *out; int token_bytes;        // token t + 1 goes to out[t + 1]
     int t_first, count;                // positions t_first .. t_first + count - 1 are evaluated and sampled from
-    const int8_t *prompt_kv;           // [layer][K, V][T][H] slot order: the rows of the positions in front of t_first
+    int8_t *kv;                        // [layer][K, V][T][H] slot order: the rows of the positions in front of t_first
     int8_t *kcache, *vcache;           // [H / 16][layer][T][head_dim], [H / 16][layer][T][16]
-    unsigned long long *slots;         // egg_decode_slots, zero before the first launch
-    uint32_t *epoch;                   // number of the last exchange, zero before the first launch
-    int *fail;                         // host memory: set when a wait ran into its bound
+    int32_t *logits;                   // vocab of them, scratch
+    // zero before the first launch: egg_decode_slots messages, the number of the last exchange, and the flag that a wait ran
+    // into its bound of wait_limit polls
+    unsigned long long *slots; uint32_t *epoch; int *fail; int wait_limit;
     uint32_t seed; int deggs; float temp; int min_p_limit, penalty_int;
 };
-int64_t egg_decode_slots(int H);
+constexpr int64_t egg_decode_slots(int H) { return (int64_t)(H / 16) * 67 + 4 * H + 8; }
 hipError_t egg_prepare_decode(int H, int vocab);      // before the first launch
 hipError_t egg_launch_decode(const DecodeParams &p, int H, hipStream_t s);
 

@@ -240,11 +240,17 @@ uint32_t egg_next_seed(uint32_t seed, uint64_t step);
  * followed by room for gen_len more (seed_len + gen_len <= seq_len); the unperturbed model continues the prompt with
  * the reference's three-pass LUT sampling, threshold hash_rng(seed + t*555, 0) % sum.  Enqueued on the stream.
  * Like the reference (d_gen_kv, mgpu.cu:1160-1170, :1199-1202) it keeps every layer's K / V rows of the sequence: the
- * prompt is evaluated once, each new token costs one 32-token tile.  egg_ctx_generate_kv_cache(ctx, 0) makes every new
- * token re-evaluate the whole window instead (same tokens; for checks).  With a vocabulary above 256 the buffer holds
- * uint32 tokens (d-eggs' TokenType), here and in egg_generate_deggs; the lengths count tokens. */
+ * prompt is evaluated once over its 32-token tiles, and one persistent launch of hidden / 16 workgroups, which exchange
+ * results through memory, evaluates and samples the new tokens.  Those workgroups must all get a place on the GPU; if a
+ * wait among them is not answered within egg_ctx_generate_wait_limit polls (default 2^23, some seconds) the launch ends
+ * and the one behind it repeats the continuation with a single workgroup, slower and with the same tokens, so the call
+ * completes in stream order either way and nothing about it is reported later.  egg_ctx_generate_kv_cache(ctx, 0) makes
+ * every new token re-evaluate the whole window instead (same tokens; for checks).  With a vocabulary above 256 the buffer
+ * holds uint32 tokens (d-eggs' TokenType), here and in egg_generate_deggs; the lengths count tokens.  The first call on a
+ * context allocates its buffers; later ones can be captured. */
 int  egg_generate(egg_ctx *ctx, uint8_t *d_buffer, int seed_len, int gen_len, uint32_t seed);
 int  egg_ctx_generate_kv_cache(egg_ctx *ctx, int enable);
+int  egg_ctx_generate_wait_limit(egg_ctx *ctx, int polls);      /* 0: the single workgroup does every continuation */
 /* d-eggs' generate_sequence_kernel (d-eggs/src/kernels.cu:307-490, call site d-eggs/src/worker.cu:563-571): the same
  * continuation with its sampler -- every earlier occurrence of a byte lowers that byte's logit by
  * (int)(penalty * 2^shift_logit) (:398-402), differences to the maximum are divided by `temp` in float and truncated

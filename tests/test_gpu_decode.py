@@ -87,3 +87,22 @@ def test_decode_on_two_streams_and_replayed(pkg, dev):
         assert np.array_equal(bufs[0].cpu().numpy(), want[0])
     for ctx in ctxs:
         ctx.close()
+
+
+@pytest.mark.parametrize("hidden,head_dim,layers,seq,vocab,lengths", SHAPES, ids=["h%d_v%d_t%d" % (s[0], s[4], s[3]) for s in SHAPES])
+def test_unanswered_waits_cost_time_only(pkg, dev, hidden, head_dim, layers, seq, vocab, lengths):
+    """Waits that run into their bound (here: at once, or after a few polls, somewhere in the middle) leave the continuation
+    to one workgroup: the tokens are the same in stream order, and the launches queued behind it are not disturbed."""
+    ctx = _context(pkg, dev, hidden, head_dim, layers, seq, vocab)
+    for n, new in lengths[-2:]:
+        for generate in (ctx.generate, ctx.generate_deggs):
+            if generate == ctx.generate_deggs and (n + new > 256 or n > hidden):
+                continue
+            bufs = [_prompt(dev, vocab, n, n + new) for _ in range(6)]
+            for b, limit in zip(bufs, (1 << 23, 0, 1 << 23, 3, 20, 1 << 23)):
+                ctx.generate_wait_limit(limit)
+                generate(b.data_ptr(), n, new, 77)
+            ctx.model_download()                         # any call that waits for the stream, no error
+            got = [b.cpu().numpy() for b in bufs]
+            assert all(np.array_equal(g, got[0]) for g in got), (n, new)
+    ctx.close()
