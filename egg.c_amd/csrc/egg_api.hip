@@ -1155,6 +1155,11 @@ static int decode_buffers(egg_ctx *ctx) {
     HIP_TRY(hipMemset(ctx->d_dec_epoch, 0, 8));
     return EGG_OK;
 }
+// logits of every position of the window: only a whole-window forward reaches the head
+static int window_logits(egg_ctx *ctx) {
+    if (!ctx->d_gen_logits) HIP_TRY(hipMalloc(&ctx->d_gen_logits, (size_t)ctx->cfg.seq_len * ctx->cfg.vocab * 4));
+    return EGG_OK;
+}
 static int generate_impl(egg_ctx *ctx, uint8_t *d_buffer, int seed_len, int gen_len, uint32_t seed, const DeggsSampling *de) {
     if (!ctx || !d_buffer) return EGG_E_INVALID;
     const egg_config &c = ctx->cfg; const int T = c.seq_len, total = seed_len + gen_len;
@@ -1163,23 +1168,23 @@ static int generate_impl(egg_ctx *ctx, uint8_t *d_buffer, int seed_len, int gen_
     if (gen_len == 0) return EGG_OK;
     const int tb = c.vocab > 256 ? 4 : 1;          // bytes per token of the buffer
     hipStream_t s = ctx->stream;
-    if (!ctx->d_gen_tok) {
-        HIP_TRY(hipMalloc(&ctx->d_gen_tok, ((size_t)T + 16) * tb));
-        HIP_TRY(hipMalloc(&ctx->d_gen_ws, (size_t)2 * c.vocab * 4));
-        HIP_TRY(hipMalloc(&ctx->d_gen_logits, (size_t)T * c.vocab * 4));
+    const bool cached = ctx->gen_kv_cache && ctx->L.total < ((int64_t)1 << 32);        // the persistent launch addresses the blob with 32 bits
+    if (!ctx->d_gen_scal) {
+        if (!ctx->d_gen_tok) HIP_TRY(hipMalloc(&ctx->d_gen_tok, ((size_t)T + 16) * tb));
+        if (!ctx->d_gen_ws) HIP_TRY(hipMalloc(&ctx->d_gen_ws, (size_t)2 * c.vocab * 4));
+        if (!ctx->d_gen_kv) HIP_TRY(hipMalloc(&ctx->d_gen_kv, (size_t)c.n_layers * 2 * T * c.hidden));
         HIP_TRY(hipMalloc(&ctx->d_gen_scal, sizeof(Scalars)));
         HIP_TRY(hipMemset(ctx->d_gen_scal, 0, sizeof(Scalars)));
-        HIP_TRY(hipMalloc(&ctx->d_gen_kv, (size_t)c.n_layers * 2 * T * c.hidden));
     }
     int rc = decode_buffers(ctx);
+    if (!rc && !cached) rc = window_logits(ctx);
     if (rc) return rc;
-    const bool cached = ctx->gen_kv_cache && ctx->L.total < ((int64_t)1 << 32);        // the persistent launch addresses the blob with 32 bits
     if (!cached || seed_len > 1) {
         HIP_TRY(egg_launch_zero_u64(reinterpret_cast<unsigned long long *>(ctx->d_gen_tok), (T + 16) * tb / 8, s));   // a fill kernel, not a memset node: a caller may be capturing this stream
         HIP_TRY(hipMemcpyAsync(ctx->d_gen_tok, d_buffer, (size_t)seed_len * tb, hipMemcpyDeviceToDevice, s));
     }
     const bool taps = ctx->taps; ctx->taps = false;
-    ctx->mask_override = 0; ctx->logits_override = ctx->d_gen_logits;
+    ctx->mask_override = 0; ctx->logits_override = cached ? nullptr : ctx->d_gen_logits;
     // data_len = T + 1 puts the member's stream position at 0 (mgpu.cu:864-870 with len - T == 1)
     auto forward = [&](const FwdRange *range) {
         return forward_chunk(ctx, ctx->d_gen_tok, (int64_t)T + 1, &ctx->d_gen_scal->start, &ctx->d_gen_scal->seed, 0, 1, range);
@@ -1233,7 +1238,7 @@ static int generate_impl(egg_ctx *ctx, uint8_t *d_buffer, int seed_len, int gen_
 extern "C" int egg_ctx_generate_kv_cache(egg_ctx *ctx, int enable) {
     if (!ctx) return EGG_E_INVALID;
     ctx->gen_kv_cache = enable != 0;
-    return EGG_OK;
+    return enable ? EGG_OK : window_logits(ctx);      // here, so that a generation may be captured from its second call on
 }
 extern "C" int egg_ctx_generate_wait_limit(egg_ctx *ctx, int polls) {
     if (!ctx || polls < 0) return fail(ctx, EGG_E_INVALID, "egg_ctx_generate_wait_limit arguments");

@@ -247,7 +247,8 @@ uint32_t egg_next_seed(uint32_t seed, uint64_t step);
  * completes in stream order either way and nothing about it is reported later.  egg_ctx_generate_kv_cache(ctx, 0) makes
  * every new token re-evaluate the whole window instead (same tokens; for checks).  With a vocabulary above 256 the buffer
  * holds uint32 tokens (d-eggs' TokenType), here and in egg_generate_deggs; the lengths count tokens.  The first call on a
- * context allocates its buffers; later ones can be captured. */
+ * context allocates its buffers (egg_ctx_generate_kv_cache(ctx, 0) the logits of the whole window), later ones can be
+ * captured. */
 int  egg_generate(egg_ctx *ctx, uint8_t *d_buffer, int seed_len, int gen_len, uint32_t seed);
 int  egg_ctx_generate_kv_cache(egg_ctx *ctx, int enable);
 int  egg_ctx_generate_wait_limit(egg_ctx *ctx, int polls);      /* 0: the single workgroup does every continuation */
