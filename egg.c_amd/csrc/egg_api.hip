@@ -66,7 +66,7 @@ struct egg_ctx {
     int32_t *h_fit() { return h_loss() + cfg.population; }
     Scalars *d_scal = nullptr;
     // votes and optimizer step (egg_votes.hip): the noise table, and the matrices' descriptors in lists that one launch walks
-    NoiseTable noise = {nullptr, 0, 0, nullptr, nullptr, 0, 0, nullptr};
+    NoiseTable noise = {};
     struct MatList { int first, count, tiles; };
     MatDesc *d_mat = nullptr;
     MatList mat_all, mat_adam; std::vector<MatList> mat_muon, mat_one;     // every matrix; the AdamW ones; each Muon batch; each on its own (by tensor id)
@@ -456,11 +456,18 @@ extern "C" int egg_ctx_create(const egg_config *cfg, egg_ctx **out) {
     CR(hipMalloc(&ctx->d_scal, sizeof(Scalars)));
     CR(hipHostMalloc(reinterpret_cast<void **>(&ctx->h_result), 16 + (size_t)c.population * 4 + (size_t)(c.population / 2) * 4, hipHostMallocCoherent));
     memset(ctx->h_result, 0, 16 + (size_t)c.population * 4 + (size_t)(c.population / 2) * 4);
-    // noise table: the rows of the widest side of any matrix (4 * hidden, or the embedding's vocabulary), every layer's seeds
+    // noise table: the rows of the widest side of any layer's matrix (4 * hidden) with every layer's seeds, and rows for the
+    // rest of the embedding's columns, several to a place
     ctx->noise.pairs_pad = ((c.population / 2) + 127) / 128 * 128;
-    ctx->noise.rows = std::max(4 * c.hidden, c.vocab);
-    ctx->noise.ld = egg_noise_ld(noise_entries(c, ctx->noise.pairs_pad)); ctx->noise.mask_ld = egg_noise_mask_ld(ctx->noise.pairs_pad);
-    CR(hipMalloc(&ctx->noise.table, ctx->noise.rows * ctx->noise.ld));
+    ctx->noise.layer_rows = 4 * c.hidden; ctx->noise.rows = std::max(4 * c.hidden, c.vocab);
+    ctx->noise.emb_t = OFF_EMB + ctx->noise.pairs_pad + 16;
+    ctx->noise.ld = egg_noise_ld(noise_entries(c, ctx->noise.pairs_pad)); ctx->noise.emb_ld = egg_noise_ld(ctx->noise.emb_t);
+    {
+        const int more = ctx->noise.rows - ctx->noise.layer_rows, share = (int)(ctx->noise.ld / ctx->noise.emb_ld);
+        ctx->noise.emb_rows = ((more + share - 1) / share + 127) / 128 * 128;
+    }
+    ctx->noise.mask_ld = egg_noise_mask_ld(ctx->noise.pairs_pad);
+    CR(hipMalloc(&ctx->noise.table, (size_t)(ctx->noise.layer_rows + ctx->noise.emb_rows) * ctx->noise.ld));
     CR(hipMalloc(&ctx->noise.neg, 4 * ctx->noise.mask_ld)); CR(hipMalloc(&ctx->noise.nonzero, 4 * ctx->noise.mask_ld));
     CR(hipMemset(ctx->noise.neg, 0, 4 * ctx->noise.mask_ld)); CR(hipMemset(ctx->noise.nonzero, 0, 4 * ctx->noise.mask_ld));
     CR(hipMalloc(&ctx->noise.general, sizeof(int)));
@@ -882,7 +889,7 @@ static int table_of_tensor(egg_ctx *ctx, int id, const int32_t *d_fit, const uin
     const egg_config &c = ctx->cfg; const egg_tensor_info &t = ctx->tensors[id];
     const int lo = t.seed_base + std::min(t.off_a, t.off_b), hi = t.seed_base + std::max(t.off_a, t.off_b) + ctx->noise.pairs_pad;
     HIP_TRY(egg_launch_noise_table(ctx->noise, d_seed, d_fit, StepEnd{}, c.population / 2, noise_word(c), t.is_matrix ? std::max(t.rows, t.cols) : t.cols,
-                                   4 * c.hidden, lo, hi, t.off_a + ctx->noise.pairs_pad + 16, c.n_layers, nullptr, ctx->stream));
+                                   lo, hi, c.n_layers, nullptr, ctx->stream));
     return EGG_OK;
 }
 extern "C" int egg_update_tensor(egg_ctx *ctx, int id, const int32_t *d_fit, const uint32_t *d_seed, const float *d_lr) {
@@ -925,8 +932,8 @@ static int es_update(egg_ctx *ctx, const int32_t *d_fit, const StepEnd &end, con
     adam.count_of = count_of;
     {
         SpanScope span(ctx, EGG_K_UPDATE_MATRIX);
-        HIP_TRY(egg_launch_noise_table(ctx->noise, d_seed, d_fit, end, c.population / 2, noise_word(c), ctx->noise.rows, 4 * c.hidden, 0,
-                                       noise_entries(c, ctx->noise.pairs_pad), ctx->noise.pairs_pad + 16, c.n_layers, ctx->d_counter, ctx->stream));
+        HIP_TRY(egg_launch_noise_table(ctx->noise, d_seed, d_fit, end, c.population / 2, noise_word(c), ctx->noise.rows, 0,
+                                       noise_entries(c, ctx->noise.pairs_pad), c.n_layers, ctx->d_counter, ctx->stream));
         HIP_TRY(egg_launch_update(adam, ctx->stream));
     }
     // Muon matrices (LAUNCH_ADAM_MATRIX under USE_MUON, mgpu.cu:1587-1595), a batch of one shape at a time: momentum of

@@ -49,7 +49,11 @@ hipError_t egg_launch_sample_deggs(const int32_t *logits, const int32_t *exp_lut
 #define EGG_LAYER_SEEDS 416        // those of a layer's tensors, above its 1000 * layer
 #define EGG_NOISE_FRONT 16         // a row's entry t lies at byte EGG_NOISE_FRONT + t
 struct NoiseTable {
-    int8_t *table; size_t ld; int rows;        // [rows][ld], ld a multiple of 128
+    // Rows [0, layer_rows) of ld bytes (a multiple of 128).  Rows from there on belong to the embedding's columns alone, whose
+    // window ends in front of entry emb_t: they need emb_ld bytes (a multiple of 128), and as many of them as fit ld share one
+    // place -- emb_rows places (a multiple of 128) hold rows layer_rows + i, + emb_rows, + 2 emb_rows ... of place i side by
+    // side, so that the rows of a tile of 64 or 128 lie ld apart like all others.
+    int8_t *table; size_t ld, emb_ld; int rows, layer_rows, emb_rows, emb_t;
     // masks by pair (pairs_pad, a multiple of 128, of them): 0xff where the fitness is -1 / is not 0, zeros in front and behind.
     // Copy k of four, mask_ld bytes apart, has pair p at byte EGG_NOISE_FRONT + k + p, so that any shift of the pairs finds
     // its masks on a dword.
@@ -62,7 +66,7 @@ struct StepEnd { unsigned long long *acc; int32_t *loss, *fit, *h_loss, *h_fit; 
 // rows [0, rows) of the entries [t_lo, t_hi) (rows from layer_rows on only below emb_t), the fitness masks, and *counter = 0
 // unless it is null
 hipError_t egg_launch_noise_table(const NoiseTable &nt, const uint32_t *d_seed, const int32_t *d_fit, const StepEnd &end, int pairs, int mask, int rows,
-                                  int layer_rows, int t_lo, int t_hi, int emb_t, int n_layers, unsigned long long *counter, hipStream_t s);
+                                  int t_lo, int t_hi, int n_layers, unsigned long long *counter, hipStream_t s);
 struct MatDesc {
     int8_t *W, *frag; float *state;    // canonical weights, their fragment-major copy, optimizer state ({m,v,acc} or Muon's {m,acc})
     float *muon_x;                     // Muon: the matrix's [rows][cols] slot of the workspace, else null

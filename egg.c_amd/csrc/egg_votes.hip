@@ -6,8 +6,8 @@
 // The reference draws two noise values per (weight, pair).  Which value a tensor draws for pair p and row or column i is
 // hash_rng(seed + p + seed_base + off, i): tensors differ in a shift of the pair index only.  So ONE table
 //     N[i][t] = noise_from_hash(seed + t, i)
-// holds every tensor's noise, a tensor's row i being N[i][seed_base + off ...].  It has max(4 hidden, vocab) rows of
-// pairs + 1000 layers entries -- 25 million hashes at hidden 256, 4 layers, 20,480 pairs, where panels of one tensor
+// holds every tensor's noise, a tensor's row i being N[i][seed_base + off ...].  It has 4 hidden rows of pairs + 1000 layers
+// entries and, for the columns of the embedding, vocab - 4 hidden more rows of pairs entries -- 25 million hashes at hidden 256, 4 layers, 20,480 pairs, where panels of one tensor
 // after the other were 440 million -- and the vote matrices  sum_p fit_p A_p[n] B_p[k]  of all tensors are int8 matrix
 // products over shifted windows of it.
 #include "egg_device.h"
@@ -18,13 +18,19 @@
 
 // ---------------------------------------------------------------- noise table
 // Thread: 16 consecutive entries of one row, one 16-byte store.  Bound by the hash (about 15 vector instructions an entry);
-// entries no tensor reads are left out: rows past `layer_rows` belong to the embedding alone (layer 0 offsets below
-// emb_t), and between the layers' windows there are gaps while there are fewer pairs than a layer's 1000 seeds.
+// entries no tensor reads are left out: rows past `layer_rows` belong to the embedding alone (and share the space of one:
+// 28 MB instead of 0.5 GB at vocabulary 65,536, hidden 64, 8 layers), and between the layers' windows there are gaps
+// while there are fewer pairs than a layer's 1000 seeds.
 // The first workgroups turn the fitness into byte masks and clear the update counter (when it is to be cleared).  In a whole
 // step (end.acc) they do what stands between the forward and the update as well, four pairs a thread: losses and
 // fitness, in device memory and in the host's copy, and the loss sums set back to zero: three launches less, and no copies
 // when the host asks (a step of hidden 64, 2 layers, 64 members with its results read: 207 -> 146 us).
 typedef int int_any __attribute__((aligned(1)));
+__device__ __forceinline__ int8_t *noise_row(const NoiseTable &nt, int r) {
+    if (r < nt.layer_rows) return nt.table + (size_t)r * nt.ld;
+    const unsigned at = (unsigned)(r - nt.layer_rows), slot = at / (unsigned)nt.emb_rows;
+    return nt.table + (size_t)(r - (int)slot * nt.emb_rows) * nt.ld + slot * nt.emb_ld;
+}
 __device__ __forceinline__ void store_masks(const NoiseTable &nt, int pair, int neg, int nz) {
 #pragma unroll
     for (int k = 0; k < 4; k++) {
@@ -77,8 +83,7 @@ __device__ __forceinline__ void end_of_step(const NoiseTable &nt, const StepEnd 
     store_masks(nt, 4 * c, n4, z4);
 }
 __global__ void __launch_bounds__(256) k_noise_table(NoiseTable nt, const uint32_t *d_seed, const int32_t *fit, StepEnd end, int first, int pairs,
-                                                     int mask, int rows, int layer_rows, int t_lo, int t_hi, int emb_t,
-                                                     int n_layers, unsigned long long *counter) {
+                                                     int mask, int rows, int t_lo, int t_hi, int n_layers, unsigned long long *counter) {
     if ((int)blockIdx.x < first) {
         if (blockIdx.x == 0 && threadIdx.x == 0 && counter) *counter = 0ull;
         if (end.acc) end_of_step(nt, end, pairs); else masks_of_fitness(nt, fit, pairs);
@@ -87,7 +92,7 @@ __global__ void __launch_bounds__(256) k_noise_table(NoiseTable nt, const uint32
     const int per_row = (t_hi - t_lo + 15) / 16;
     const int64_t i = (int64_t)((int)blockIdx.x - first) * 256 + threadIdx.x;
     const int r = (int)(i / per_row), t0 = t_lo + 16 * (int)(i % per_row);
-    if (r >= rows || (r >= layer_rows && t0 >= emb_t)) return;
+    if (r >= rows || (r >= nt.layer_rows && t0 >= nt.emb_t)) return;
     if (pairs < 512) {
         const int l = min(t0 / 1000, n_layers - 1), rel = t0 - 1000 * l;
         if (rel >= (l ? EGG_LAYER_SEEDS : EGG_MODEL_SEEDS) + nt.pairs_pad + 16) return;
@@ -101,20 +106,21 @@ __global__ void __launch_bounds__(256) k_noise_table(NoiseTable nt, const uint32
         for (int e = 0; e < 4; e++) v[e] = noise_from_hash(s + (uint32_t)(4 * q + e), (uint32_t)r, mask);
         o[q] = pack4(v[0], v[1], v[2], v[3]);
     }
-    *reinterpret_cast<v4i *>(nt.table + (size_t)r * nt.ld + EGG_NOISE_FRONT + t0) = o;
+    *reinterpret_cast<v4i *>(noise_row(nt, r) + EGG_NOISE_FRONT + t0) = o;
 }
 // the last window ends with the entries; it is read in whole chunks of 128 from 15 bytes in front of it on
 size_t egg_noise_ld(int entries) { return ((size_t)EGG_NOISE_FRONT + entries + 128 + 32 + 127) / 128 * 128; }
 size_t egg_noise_mask_ld(int pairs_pad) { return (size_t)EGG_NOISE_FRONT + pairs_pad + 128 + 16; }
 hipError_t egg_launch_noise_table(const NoiseTable &nt, const uint32_t *d_seed, const int32_t *d_fit, const StepEnd &end, int pairs, int mask, int rows,
-                                  int layer_rows, int t_lo, int t_hi, int emb_t, int n_layers, unsigned long long *counter, hipStream_t s) {
+                                  int t_lo, int t_hi, int n_layers, unsigned long long *counter, hipStream_t s) {
     t_lo &= ~15;
     t_hi = (t_hi + 15) & ~15;
-    if (rows < 1 || rows > nt.rows || t_lo < 0 || (size_t)t_hi + EGG_NOISE_FRONT > nt.ld) return hipErrorInvalidValue;
+    if (rows < 1 || rows > nt.rows || t_lo < 0 || (size_t)t_hi + EGG_NOISE_FRONT > nt.ld || (size_t)nt.emb_t + 16 + EGG_NOISE_FRONT > nt.emb_ld)
+        return hipErrorInvalidValue;
     const int64_t items = (int64_t)rows * ((t_hi - t_lo) / 16);
     const int first = end.acc ? (nt.pairs_pad / 4 + 255) / 256 : 1;
     hipLaunchKernelGGL(k_noise_table, dim3((unsigned)((items + 255) / 256 + first)), dim3(256), 0, s, nt, d_seed, d_fit, end, first, pairs, mask, rows,
-                       layer_rows, t_lo, t_hi, emb_t, n_layers, counter);
+                       t_lo, t_hi, n_layers, counter);
     return hipGetLastError();
 }
 
@@ -239,7 +245,7 @@ __device__ __forceinline__ int vector_elements(const UpdLaunch &p, int gi) {
     const int d = find_last(p.n_vec, gi, [&](int i) { return p.vec[i].first; });
     const VecDesc t = p.vec[d];
     const int idx = gi - t.first;
-    const int8_t *row = p.noise.table + (size_t)idx * p.noise.ld;
+    const int8_t *row = p.noise.table + (size_t)idx * p.noise.ld;          // vector tensors have at most layer_rows elements
     float *const st = t.state + (size_t)(idx + lane) * 3;
     float m = 0.f, v = 0.f, acc = 0.f;
     int w = 0;
@@ -389,8 +395,8 @@ __global__ void __launch_bounds__(EGG_THREADS, WT == 1 ? 3 : 2) k_update(UpdLaun
     const int k0 = (tile / tiles_n) * ROWS, n0 = (tile % tiles_n) * ROWS;
     const int c = threadIdx.x & 7, r = threadIdx.x >> 3;
     const Windows w(p.noise, t.t_a, t.t_b);
-    const size_t down = 32 * p.noise.ld;
-    const int8_t *pa = p.noise.table + (size_t)(n0 + r) * p.noise.ld + w.a + 16 * c;
+    const size_t down = 32 * p.noise.ld;                     // a tile's rows lie ld apart wherever they start (see NoiseTable)
+    const int8_t *pa = noise_row(p.noise, n0) + (size_t)r * p.noise.ld + w.a + 16 * c;
     const int8_t *pb = p.noise.table + (size_t)(k0 + r) * p.noise.ld + w.b + 16 * c;
     const int general = *p.noise.general, length = w.length(p.pairs);
     v4i a[PARTS], b[PARTS], neg, nz;
@@ -519,7 +525,7 @@ int egg_update_blocks(const UpdLaunch &p) { return (wide_tiles(p) ? p.tiles / 4 
 hipError_t egg_launch_update(const UpdLaunch &p, hipStream_t s) {
     const int blocks = egg_update_blocks(p);
     if (blocks < 1) return hipSuccess;
-    if (p.noise.pairs_pad % 128 || p.vec_total % VEC || (p.tiles && p.n_mat < 1) || (p.vec_total && p.n_vec < 1)) return hipErrorInvalidValue;
+    if (p.noise.pairs_pad % 128 || p.noise.layer_rows % 128 || p.noise.emb_rows % 128 || p.vec_total % VEC || (p.tiles && p.n_mat < 1) || (p.vec_total && p.n_vec < 1)) return hipErrorInvalidValue;
     if (wide_tiles(p)) hipLaunchKernelGGL(k_update<2>, dim3(blocks), dim3(EGG_THREADS), 0, s, p);
     else hipLaunchKernelGGL(k_update<1>, dim3(blocks), dim3(EGG_THREADS), 0, s, p);
     return hipGetLastError();

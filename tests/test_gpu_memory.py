@@ -32,3 +32,13 @@ def test_first_generation_takes_no_logits_of_the_whole_window(pkg, dev):
     assert before - _free(dev) >= 96 << 20 and torch.equal(b.cpu(), want)
     ctx.close()
     warm.close()
+
+
+def test_context_of_a_large_vocabulary(pkg, dev):
+    """The noise table takes the embedding's columns by their own windows (about 25 MB), not with every layer's seeds (0.5 GB)."""
+    warm = pkg.Context(pkg.default_config(hidden=64, head_dim=32, n_layers=1, seq_len=32, population=2))
+    before = _free(dev)
+    ctx = pkg.Context(pkg.default_config(hidden=64, head_dim=32, n_layers=8, seq_len=32, vocab=65536, population=2))
+    assert before - _free(dev) < 160 << 20               # 9 MB of weights, 54 MB of optimizer state, the table
+    ctx.close()
+    warm.close()

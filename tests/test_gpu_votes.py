@@ -62,3 +62,31 @@ def test_update_in_wide_tiles(pkg, orc, dev, pairs, values):
         assert np.array_equal(ctx.opt_state_download().view(np.int32), state.view(np.int32))
         assert ctx.last_update_count() == n_ref
     ctx.close()
+
+
+@pytest.mark.parametrize("pairs", [1, 129])
+@pytest.mark.parametrize("hidden,vocab", [(64, 768), (128, 16384)], ids=["64_tiles", "128_tiles"])
+def test_embedding_columns_behind_the_layers_rows(pkg, orc, dev, hidden, vocab, pairs):
+    """The noise table's rows from 4 hidden on are shorter ones, for the columns of the embedding alone."""
+    import torch
+    kw = dict(hidden=hidden, head_dim=32, n_layers=2, seq_len=32, vocab=vocab, population=2 * pairs)
+    ocfg = orc.config(**kw)
+    ctx = pkg.Context(pkg.default_config(**kw))
+    fit = np.random.default_rng(pairs).choice(np.array([-1, 1], np.int32), pairs)
+    seed, d_fit = 0xFFFFFFF0, torch.from_numpy(fit).to(dev)
+    d_seed = torch.from_numpy(np.array([seed], np.uint32).view(np.int32)).to(dev)
+    t = next(t for t in ctx.tensors() if t["name"] == "embedding")
+    ref = np.zeros(t["rows"] * t["cols"], np.int32)
+    orc.lib().orc_matrix_votes(C.byref(ocfg), t["rows"], t["cols"], t["off_a"], t["off_b"], t["seed_base"],
+                               fit.ctypes.data_as(C.c_void_p), pairs, C.c_uint32(seed), ref.ctypes.data_as(C.c_void_p))
+    d_votes = torch.zeros(ref.size, dtype=torch.int32, device=dev)
+    ctx.matrix_votes(t["id"], d_fit.data_ptr(), d_seed.data_ptr(), d_votes.data_ptr())
+    ctx.sync()
+    assert np.array_equal(d_votes.cpu().numpy(), ref)
+    # and in the launch of a whole update: the first moment of an untouched state is (1 - beta1) * -vote
+    d_lr = torch.zeros(1, dtype=torch.float32, device=dev)
+    ctx.es_update(d_fit.data_ptr(), d_seed.data_ptr(), d_lr.data_ptr())
+    at = ctx.tensor_state_offset(t["id"]) // 4
+    m = ctx.opt_state_download()[at:at + 3 * ref.size:3]
+    assert np.array_equal(m, (np.float32(1) - np.float32(ctx.cfg.adam_beta1)) * -ref.astype(np.float32))
+    ctx.close()
