@@ -934,6 +934,13 @@ static int es_update(egg_ctx *ctx, const int32_t *d_fit, const StepEnd &end, con
         SpanScope span(ctx, EGG_K_UPDATE_MATRIX);
         HIP_TRY(egg_launch_noise_table(ctx->noise, d_seed, d_fit, end, c.population / 2, noise_word(c), ctx->noise.rows, 0,
                                        noise_entries(c, ctx->noise.pairs_pad), c.n_layers, ctx->d_counter, ctx->stream));
+        // (timed, they go apart, so that each class has its time; a matrix's and a vector's results do not depend on it)
+        if (ctx->timing) adam.vec_total = 0;
+        HIP_TRY(egg_launch_update(adam, ctx->stream));
+    }
+    if (ctx->timing) {
+        SpanScope span(ctx, EGG_K_UPDATE_VECTOR);
+        adam.n_mat = adam.tiles = 0; adam.vec_total = ctx->vec_total;
         HIP_TRY(egg_launch_update(adam, ctx->stream));
     }
     // Muon matrices (LAUNCH_ADAM_MATRIX under USE_MUON, mgpu.cu:1587-1595), a batch of one shape at a time: momentum of

@@ -344,7 +344,8 @@ int  egg_gru_losses(egg_gru_ctx *ctx, int32_t *host_loss, int32_t *host_fit);  /
 int  egg_gru_forward_mode(egg_gru_ctx *ctx, int staged);
 
 /* per-kernel-class timing with hipEvent pairs recorded on the context's stream around each launch (the
- * reference only splits Fwd/Host/Upd wall time, full_cuda_train_egg.cu:1116-1126).  Not usable while capturing. */
+ * reference only splits Fwd/Host/Upd wall time, full_cuda_train_egg.cu:1116-1126).  Not usable while capturing.  An
+ * untimed update takes the vector tensors in the launch of the matrices; timed, they have one of their own. */
 enum { EGG_K_MLP_FIRST = 0, EGG_K_QKV = 1, EGG_K_ATTN = 2, EGG_K_MLP = 3, EGG_K_HEAD = 4,
        EGG_K_UPDATE_MATRIX = 5, EGG_K_UPDATE_VECTOR = 6, EGG_K_PLINEAR = 7,
        EGG_K_MUON_NS = 8 /* the Newton-Schulz chain of a Muon batch; votes, momentum and apply count as UPDATE_MATRIX */,

@@ -90,3 +90,23 @@ def test_embedding_columns_behind_the_layers_rows(pkg, orc, dev, hidden, vocab, 
     m = ctx.opt_state_download()[at:at + 3 * ref.size:3]
     assert np.array_equal(m, (np.float32(1) - np.float32(ctx.cfg.adam_beta1)) * -ref.astype(np.float32))
     ctx.close()
+
+
+@pytest.mark.parametrize("muon", [0, 1])
+def test_timed_update_has_both_classes_and_the_same_results(pkg, dev, muon):
+    import torch
+    got = []
+    for timed in (False, True):
+        ctx = pkg.Context(pkg.default_config(hidden=64, head_dim=32, n_layers=2, seq_len=32, population=40, use_muon=muon))
+        ctx.model_init(42)
+        fit = torch.from_numpy(np.random.default_rng(1).integers(-1, 2, 20).astype(np.int32)).to(dev)
+        seed, lr = torch.tensor([5], dtype=torch.int32, device=dev), torch.tensor([5.0], device=dev)
+        ctx.enable_timing(timed)
+        for _ in range(2):
+            ctx.es_update(fit.data_ptr(), seed.data_ptr(), lr.data_ptr())
+        got.append((ctx.model_download(), ctx.opt_state_download(), ctx.last_update_count()))
+        if timed:
+            launches = {k: v[0] for k, v in ctx.timing().items()}
+            assert launches["update_vector"] == 2 and launches["update_matrix"] >= 2, launches
+        ctx.close()
+    assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1]) and got[0][2] == got[1][2] > 0
