@@ -260,8 +260,8 @@ def main():
         gru = {"value": gcfg.population * gcfg.seq_len / sec, "unit": "member-tokens/s", "ms_per_step": sec * 1e3,
                "workload": "full_trained_egg.c defaults, one full step (forward of %d members x %d tokens + update)" % (gcfg.population, gcfg.seq_len),
                "note": "the bit-exact GPU twin of the CPU baseline's program: 128 members of 4096 strictly sequential tokens, walked as a "
-                       "pipeline over the layers with one launch per tick (2 T + 6 L + 1 launches); a tick is bound by streaming the "
-                       "tick's weights into the L2s again, which do not keep them across launches"}
+                       "pipeline over layers and chunks of 32 tokens, one launch a tick (T / 32 + 4 L of them); bound by the recurrence, "
+                       "T steps one after the other that a CU takes with its weights in registers and LDS"}
         gctx.close()
     except Exception as e:
         gru = {"error": str(e)}
@@ -307,9 +307,14 @@ def main():
         ops_tok = {"mlp_first": 2.0 * 8 * H5 * H5, "qkv": 2.0 * 3 * H5 * H5, "attn": 2.0 * 2 * H5 * (T5 + 1) / 2,
                    "mlp": 2.0 * 9 * H5 * H5, "head": 2.0 * H5 * 256}
         launches = {"mlp_first": 1, "qkv": L5, "attn": L5, "mlp": L5, "head": 1}
-        # Newton-Schulz: 5 x (Gram K x K x L, then L x K x K) = 20 K^2 L flops per matrix, K = min, L = max dimension
+        # Newton-Schulz, five iterations, in products of k^3 (2 k^3 flops), k the short side and r = long / short, symmetric
+        # products counted as half: 3/2 r + 6 in Gram form (r >= 4: the iterations on short x short matrices, the long one
+        # multiplied twice), 15/2 r on the matrix itself
         groups, _, _ = pkg.muon_plan(c5ctx.cfg)
-        ns_flops = sum(20.0 * min(g["rows"], g["cols"]) ** 2 * max(g["rows"], g["cols"]) * g["members"] for g in groups)
+        ns_flops = 0.0
+        for g in groups:
+            k, r = min(g["rows"], g["cols"]), max(g["rows"], g["cols"]) / min(g["rows"], g["cols"])
+            ns_flops += g["members"] * 2.0 * k ** 3 * (1.5 * r + 6 if r >= 4 else 7.5 * r)
         ns_ms = tm["muon_ns"][1]
         c5 = {"value": toks / sec, "unit": "member-tokens/s", "ms_per_step": sec * 1e3, "forward_ms": fwd_ms, "update_ms": upd_ms,
               "population": P5,
@@ -326,8 +331,8 @@ def main():
               "workload": f"hidden {H5}, 8 heads, seq {T5}, {L5} layers, ternary-packed weights (unpacked on upload, weight limit 1), "
                           f"population {P5} in one launch per kernel, one full step: forward + fitness + votes + Muon"}
         c5ctx.close()
-        # the same shape with d-eggs' default vocabulary (VOCAB_SIZE 8192, uint32 tokens): the head then costs 2 x 2 H V
-        # ops per token (the projection runs twice, like the reference's) beside the layers' 2 x 12 H^2 each
+        # the same shape with d-eggs' default vocabulary (VOCAB_SIZE 8192, uint32 tokens): the head then costs 2 H V ops per
+        # token (one pass over the vocabulary) beside the layers' 2 x 12 H^2 each
         try:
             PV = min(P5, 4096)
             raw = d_data[: 1 << 23].to(torch.int32)
@@ -345,7 +350,7 @@ def main():
             vtm = vctx.timing()
             c5["vocab_8192"] = {"value": PV * T5 / vsec, "unit": "member-tokens/s", "ms_per_step": vsec * 1e3, "population": PV,
                                 "kernel_ms_per_step": {k: round(vtm[k][1], 3) for k in fwd if vtm[k][0]},
-                                "head_frac_mfma": round(2 * 2.0 * H5 * 8192 * PV * T5 / (vtm["head"][1] * 1e-3) / PEAK_INT8_OPS, 4) if vtm["head"][1] > 0 else None,
+                                "head_frac_mfma": round(2.0 * H5 * 8192 * PV * T5 / (vtm["head"][1] * 1e-3) / PEAK_INT8_OPS, 4) if vtm["head"][1] > 0 else None,
                                 "workload": f"as above with vocabulary 8192 and uint32 tokens, population {PV}, int8 weights from the reference initialisation"}
             vctx.close()
             del d_tok, raw

@@ -135,11 +135,13 @@ struct MlpCfg {
 };
 
 // SEED: the down accumulator starts from (residual + bias) << shift_mlp_down instead of zero; the host has checked that its
-// range allows that (egg_mlp_down_acc_bound).  The residual then needs no register and no memory across the
-// sub-chunk loop -- without it it is parked in the x buffer and read again, 2 of 5 bytes that the kernel moves -- and the
-// epilogue neither extracts nor adds it.  Hidden 256, 40,960 members x 256
-// tokens: 9.33 -> 8.97 ms a launch, hidden 512, 2,048 x 512: 3.12 -> 3.05 ms (the residual stays in registers until the
-// accumulator is live: seeded in front of the norm, hidden 512 spills and takes 3.85 ms).
+// range allows that (egg_mlp_down_acc_bound: with the default noise up to a shift of 22; the other form serves 23 and 24).
+// The residual then needs no register and no memory across the sub-chunk loop -- without it it is parked in the x buffer and
+// read again, 2 of 5 bytes that the kernel moves -- and the epilogue neither extracts nor adds it.  Hidden 256, 40,960
+// members x 256 tokens: 9.33 -> 8.97 ms a launch, hidden 512, 2,048 x 512: 3.12 -> 3.05 ms (the residual stays in
+// registers until the accumulator is live: seeded in front of the norm, hidden 512 spills in its sub-chunk loop and takes
+// 3.85 ms.  As it is, hidden 512 still keeps 6 registers -- the first block 21 -- in scratch across a pass: 7 and 30 accesses a
+// pass, none in the sub-chunk loop; without SEED it keeps none).
 // ADAPT: the d-eggs adaptive noise overlay is on (de/include/model/layers.cuh:215-296, :432-438,
 // de/src/kernels.cu:139-158); see k_qkv.  The down projection's input-side sum follows the reference thread of a
 // hidden unit, which adds its four terms (k = unit, unit + H, ...) into an int one float addition at a time; the

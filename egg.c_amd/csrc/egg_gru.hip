@@ -1,7 +1,8 @@
 // egg_gru.hip -- the reference's CPU program (full_trained_egg.c, "egg.c": GRU-style recurrent byte LM with
 // sequential-xorshift rank-1 noise and the +-1 threshold update) on gfx950.
 //
-// The model is recurrent, so tokens are serial; the GEMM's free dimension is the population.  A workgroup of 16
+// Noise, update and the C ABI, and the simpler of two ways to evaluate the forward (egg_gru_forward_mode(ctx, 0); the default is
+// the pipeline of egg_gru_pipe.hip): tokens are serial, the GEMM's free dimension is the population.  A workgroup of 16
 // waves owns 32 members (16 antithetic pairs): every perturbed matmul (egg.c:108-177) is one
 // v_mfma_i32_32x32x32_i8 strip per wave (A operand = 32 output rows of W read straight from the fragment-major
 // copy in L2, B operand = the 32 members' input vectors in LDS), output rows are split over the waves and the

@@ -17,12 +17,14 @@
 // v_mfma_i32_16x16x64_i8 with a barrier behind each.  The 16 columns hold the 8 members twice: lanes of the first copy finish
 // strips 0 and 2, lanes of the second strips 1 and 3, so the elementwise arithmetic -- more than the products -- uses every
 // lane.  What bounds a token (2.35 us at hidden 512) is one wave per SIMD issuing, one behind the other, the reads of operand and
-// LDS fragments, 64 MFMAs and about 300 vector instructions; the order between them changed nothing.  "Pipe order" (egg_gru.h) of a row is the order in which those lanes hold 64 rows' results, so what a wave stores is
-// operand for the next product as it stands.
+// LDS fragments, 64 MFMAs and about 300 vector instructions; the order between them changed nothing.
+// "Pipe order" (egg_gru.h) of a row is the order in which those lanes hold 64 rows' results, so what a wave stores is operand
+// for the next product as it stands.
 //
 // A, E, D, head: a workgroup of eight waves takes 8 members; a wave has 32 tokens of one member as the columns of
 // v_mfma_i32_32x32x32_i8 (one member: its noise vectors are wave-uniform), the weights go by in blocks of 64 output columns
-// through two LDS buffers that all eight waves read.
+// through two LDS buffers that all eight waves read.  (At hidden 512 D reloads 9 registers from scratch for each block of 64
+// columns and 128 MFMAs; the recurrence and the other stages use none.)
 #include "egg_gru.h"
 
 #pragma clang fp contract(off)

@@ -74,7 +74,8 @@ def main():
     print("%-60s %5s %5s %12s %10s %10s %7s %12s %7s" % ("kernel", "VGPR", "AGPR", "scratch B/ln", "waves/SIMD", "VGPR spill", "LDS B", "scratch@loop", "deepest"))
     seen = set()
     for r, n in zip(rows, names):
-        n = re.sub(r"\(.*", "", n).replace("void ", "")
+        # the arguments go, an anonymous namespace in front of the name too
+        n = re.sub(r"\(.*", "", n.replace("(anonymous namespace)::", "")).replace("void ", "")
         key = (n, r.get("VGPRs"), r.get(KEYS[2]))
         if key in seen:
             continue

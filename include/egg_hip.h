@@ -118,10 +118,12 @@ int  egg_perturbed_linear_own_noise(egg_ctx *ctx, const int8_t *d_X, const int8_
 int  egg_shared_linear(egg_ctx *ctx, const int8_t *d_X, const int8_t *d_W_blocked,
                        int members, int T, int K, int N, int shift, int32_t *d_Y32, int8_t *d_Y8);
 
-/* No counterpart in the reference.  For K = 512 or 256 with N = 512 the three calls above run a W-stationary kernel
- * (one persistent workgroup per CU keeps the whole of W in its registers and streams the activations through LDS);
- * w_stationary = 0 makes them use the W-streaming kernels instead, which serve every other shape.  Results are
- * identical; the switch exists so that both can be measured and compared. */
+/* No counterpart in the reference.  The three calls above choose between three kinds of kernel: few rows (members *
+ * T / 32 * ceil(N / 128) * K up to 2^20, or 2^18 where the next kind serves the shape) run one launch that reads the matrix
+ * as it is given; for K = 512 or 256 with N = 512 a W-stationary kernel (one persistent workgroup per CU keeps the whole
+ * of W in its registers and streams the activations through LDS) does the same; everything else runs W-streaming kernels on
+ * a rearranged copy of the matrix that each call makes in a buffer of the context.  w_stationary = 0 sends every call to
+ * the W-streaming kernels.  Results are identical; the switch exists so that they can be measured and compared. */
 int  egg_ctx_linear_kernel(egg_ctx *ctx, int w_stationary);
 
 /* train_sequence_kernel<<<batch,...>>> (mgpu.cu:847-1029, launch :1531): evaluates members
@@ -314,7 +316,7 @@ int  egg_tap_download(egg_ctx *ctx, const char *name, int member, void *host_out
 typedef struct egg_gru_ctx egg_gru_ctx;
 typedef struct egg_gru_config {
     int hidden;            /* HIDDEN_DIM 512 (64, 128, 256 or 512)          full_trained_egg.c:12 */
-    int n_layers;          /* N_LAYERS 4                                    :13 */
+    int n_layers;          /* N_LAYERS 4 (at most 8)                        :13 */
     int seq_len;           /* SEQ_LEN 4096                                  :14 */
     int vocab;             /* VOCAB_SIZE 256                                :11 */
     int population;        /* POPULATION_SIZE 128 (multiple of 32)          :15 */
@@ -337,10 +339,10 @@ int  egg_gru_state_download(egg_gru_ctx *ctx, void *host_states, size_t bytes);
 int  egg_gru_step(egg_gru_ctx *ctx, const uint8_t *d_data, int64_t data_len, int64_t start_idx, uint32_t step_seed, int do_update);
 int  egg_gru_losses(egg_gru_ctx *ctx, int32_t *host_loss, int32_t *host_fit);  /* synchronises */
 /* How egg_gru_step evaluates forward_pass (full_trained_egg.c:213-296) -- same results either way.  1 (default): the
- * stages of a layer's token (norm, gate products, state update, norm, expand, project; for the head norm, logits,
- * loss) are spread over the GPU by output strip and member tile, and the sequence is walked as a pipeline over the
- * layers with one launch per tick that carries every stage that is ready (2 T + 6 L + 1 launches, 64 to a hipGraph);
- * 0: one persistent workgroup per 32 members for the whole sequence. */
+ * sequence in chunks of 32 tokens, walked as a pipeline over the layers: per layer and chunk the products that do not
+ * depend on the layer's state, the recurrence, the MLP's two halves, each in a tick of its own; one launch a tick carries
+ * every stage of every layer and the head (seq_len / 32 + 4 n_layers ticks for up to 512 members at a time).  0: one
+ * persistent workgroup per 32 members for the whole sequence. */
 int  egg_gru_forward_mode(egg_gru_ctx *ctx, int staged);
 
 /* per-kernel-class timing with hipEvent pairs recorded on the context's stream around each launch (the
