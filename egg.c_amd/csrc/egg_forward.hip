@@ -81,8 +81,8 @@ __device__ __forceinline__ void exchange_operand(int8_t *buf, const TileMap &tm,
 // ============================================================================ MLP block
 // The 4H-wide intermediate is produced SC columns at a time (up GEMM, GELU epilogue, immediately consumed as k-steps
 // of the down GEMM), so only the down accumulator of the wave's column slice, the normalised input and one
-// sub-chunk accumulator are live.  W streams through two LDS buffers in units of at most 16 KB.  The residual is
-// parked in the x buffer and re-read at the end.
+// sub-chunk accumulator are live.  W streams through two LDS buffers in units of at most 16 KB.  The residual starts the
+// down accumulator (SEED below), or is parked in the x buffer and re-read at the end.
 // Column slices of k_mlp and k_qkv, i.e. waves that share a token tile: as few as the registers allow where there are tiles
 // enough (hidden 512 with two, not four: twice the MFMAs per staged unit and half the exchanges outweigh the registers
 // of the 256-column accumulator; k_qkv 2.05 -> 1.57 ms per 2048 members x 512 tokens), twice as many where there
