@@ -4,7 +4,7 @@
 // A token of the unperturbed model is a chain of small matrix-vector products: what bounds it is not the weights (29 MB at
 // hidden 512, 8 layers: 6 us at the memory's rate) but how fast one stage's result reaches the next stage's workgroups.
 // As launches over one 32-token tile (one workgroup each, 2 L + 2 of them streaming whole matrices through one CU) a
-// token took 1.76 ms at that size (vocabulary 8192) and 93 us at hidden 256, 4 layers, vocabulary 256.  Here H / 16 workgroups stay for the whole
+// token took 1.76 ms at that size (vocabulary 8192) and 0.25 ms at hidden 256, 4 layers, vocabulary 256.  Here H / 16 workgroups stay for the whole
 // continuation; workgroup w owns 16 columns of every H-wide product (48 of Q | K | V, 64 of the MLP's up projection, V / 16
 // tiles of the head dealt round) and they exchange results through tagged messages: 8 bytes, the value and the number
 // of the exchange, written and polled with device-scope accesses, so the data is its own arrival flag and an exchange costs
