@@ -511,44 +511,13 @@ __device__ __forceinline__ void standard_norm(const v4i *x, v4i *out, const int 
     standard_scale<KS>(x, out, mn, wt, bt, 0, g);
 }
 
-// adaptive_*_normalize (egg_adaptive_normalize.h:10-103), also in two parts: max |val| over NT column groups
-// (both lane halves of the token combined), then the scaling.  The reference's final clamp to +-127 never binds:
-// |val| <= mx, so (float)val * (127.0f / (float)mx) <= 127 * (1 + 2^-23) and rounds to at most 127.
-template <int NT>
-__device__ __forceinline__ int absmax_groups(const v16i *val) {
-    int hi = 0, lo = 0;
-#pragma unroll
-    for (int nt = 0; nt < NT; nt++)
-#pragma unroll
-        for (int r = 0; r < 16; r += 2) {
-            hi = max(max(hi, val[nt][r]), val[nt][r + 1]);
-            lo = min(min(lo, val[nt][r]), val[nt][r + 1]);
-        }
-    int mx = max(hi, -lo);
-    return max_halves(mx);
-}
-template <int NT>
-__device__ __forceinline__ void adaptive_scale(const v16i *val, int mx, v4i *out) {
-    const float scale = 127.0f / ((float)mx + 1e-9f);
-#pragma unroll
-    for (int nt = 0; nt < NT; nt++)
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            int o[4];
-#pragma unroll
-            for (int e = 0; e < 4; e++) o[e] = round_half_away((float)val[nt][4 * q + e] * scale);
-            out[nt][q] = pack4(o[0], o[1], o[2], o[3]);
-        }
-}
-template <int NT>
-__device__ __forceinline__ void adaptive_norm(const v16i *val, v4i *out) {
-    adaptive_scale<NT>(val, absmax_groups<NT>(val), out);
-}
-
-// The same two parts with the conversion to float first: (float) is monotonic, so the largest |(float)val| is the
-// float of the largest |val| the reference converts, and |.| is an operand modifier of the float maximum (one
-// three-operand maximum per two values instead of a maximum and a minimum).  The values are left as floats (bit
-// patterns) for the scaling; the result is the maximum's bit pattern, which orders like the float since it is not negative.
+// adaptive_*_normalize (egg_adaptive_normalize.h:10-103), also in two parts: max |val| over NT column groups (both lane halves of the
+// token combined), then the scaling.  The reference's final clamp to +-127 never binds: |val| <= mx, so
+// (float)val * (127.0f / (float)mx) <= 127 * (1 + 2^-23) and rounds to at most 127.
+// The conversion to float comes first: (float) is monotonic, so the largest |(float)val| is the float of the largest |val| the
+// reference converts, and |.| is an operand modifier of the float maximum (one three-operand maximum per two values instead of a
+// maximum and a minimum).  The values are left as floats (bit patterns) for the scaling; the result is the maximum's bit
+// pattern, which orders like the float since it is not negative.
 template <int NT>
 __device__ __forceinline__ int absmax_to_float_groups(v16i *val) {
     float m0 = 0.0f, m1 = 0.0f;
@@ -564,16 +533,40 @@ __device__ __forceinline__ int absmax_to_float_groups(v16i *val) {
         }
     return max_halves(__float_as_int(fmaxf(m0, m1)));
 }
+// The reference rounds the float product val * s, s = 127 / mx, half away from zero.  val and mx are whole numbers, so 127 val / mx lies on a
+// tie or at least 1 / (2 mx) away from one, and while that is more than the two roundings can move a product (mx < 33157 =
+// 2^23 / 253) only true ties depend on them: 63.5 (val = mx / 2), and where 254 divides mx every k + 0.5.  Elsewhere
+// fma(val, s, 1.5 * 2^23) rounds to the same integer, with its two's complement byte at the bottom of the sum: one instruction
+// where product, half with the sign, sum and conversion were four.  At 63.5 the fused sum goes up like the reference if the
+// scale does not lie below 127 / mx, so where the reference's product reaches 63.5 the next float above serves.  What is left,
+// mx from 33157 on and multiples of 254 from 10414 = 41 * 254 on (15 of them do differ), takes the reference's own steps; a
+// wave decides for all of its tokens.  All mx below 33157 with all val were compared on the CPU.
+__device__ __forceinline__ float adaptive_fused_scale(float mx, float s, bool *exact) {
+    const float tie = (mx * 0.5f) * s;
+    const float nearest = __builtin_rintf(mx * (1.0f / 254.0f));
+    *exact = mx < 10414.0f || (mx < 33157.0f && __builtin_fmaf(nearest, -254.0f, mx) != 0.0f);
+    return tie >= 63.5f && __builtin_fmaf(mx, s, -127.0f) <= 0.0f ? __int_as_float(__float_as_int(s) + 1) : s;
+}
+// (in place, so that the uncommon case costs no registers: it leaves whole numbers for the fused sum)
 template <int NT>
-__device__ __forceinline__ void adaptive_scale_floats(const v16i *valf, int mx_bits, v4i *out) {
-    const float scale = 127.0f / (__int_as_float(mx_bits) + 1e-9f);
+__device__ __forceinline__ void adaptive_scale_floats(v16i *valf, int mx_bits, v4i *out) {
+    const float mx = __int_as_float(mx_bits), scale = 127.0f / (mx + 1e-9f);
+    bool exact;
+    float fused = adaptive_fused_scale(mx, scale, &exact);
+    if (!__all(exact)) {
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) valf[nt][r] = __float_as_int((float)round_half_away(__int_as_float(valf[nt][r]) * scale));
+        fused = 1.0f;
+    }
 #pragma unroll
     for (int nt = 0; nt < NT; nt++)
 #pragma unroll
         for (int q = 0; q < 4; q++) {
             int o[4];
 #pragma unroll
-            for (int e = 0; e < 4; e++) o[e] = round_half_away(__int_as_float(valf[nt][4 * q + e]) * scale);
+            for (int e = 0; e < 4; e++) o[e] = __float_as_int(__builtin_fmaf(__int_as_float(valf[nt][4 * q + e]), fused, 12582912.0f));
             out[nt][q] = pack4(o[0], o[1], o[2], o[3]);
         }
 }
