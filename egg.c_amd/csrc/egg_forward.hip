@@ -28,9 +28,20 @@ __device__ __forceinline__ int token_at(const FwdCommon &c, int64_t i) {
     return c.token_bytes == 4 ? (int)reinterpret_cast<const uint32_t *>(c.data)[i] : (int)c.data[i];
 }
 
-// acc[nt][r] += (sb * A[n]) >> sigma for NT column groups starting at table offset n_off; the table holds A << a_shift, and sb
-// comes shifted by sb_shift (egg_rank1_shifts).  Two instructions an element where multiply, shift and add were three: k_qkv
-// 5.55 -> 5.47 ms at hidden 256 and 40,960 members, 1.52 -> 1.47 ms at hidden 512.
+// (sb * A[n]) >> sigma for NT column groups starting at table offset n_off, where an accumulator starts from it (start_perturb: the
+// sum on the input side is known before the product; one instruction an element) or is added to it (add_perturb: two).  The
+// table holds A << a_shift, and sb comes shifted by sb_shift (egg_rank1_shifts).
+template <int NT>
+__device__ __forceinline__ void start_perturb(v16i *acc, int sb, const int *At, int n_off, int g) {
+#pragma unroll
+    for (int nt = 0; nt < NT; nt++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            v4i a4 = *reinterpret_cast<const v4i *>(At + n_off + 32 * nt + 8 * q + 4 * g);
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc[nt][4 * q + e] = __mulhi(sb, a4[e]);
+        }
+}
 template <int NT>
 __device__ __forceinline__ void add_perturb(v16i *acc, int sb, const int *At, int n_off, int g) {
 #pragma unroll
@@ -327,12 +338,14 @@ __global__ void __launch_bounds__(EGG_THREADS, (MlpCfg<H, CSV>::occ(ADAPT))) k_m
         } else {
             // attention output projection + residual + adaptive norm (mgpu.cu:827-831)
             v16i acc[NTS];
-            zero_acc<NTS>(acc);
-            int sbo;
             {
+                int sbo;
                 v4i aop[KS];
 #pragma unroll
                 for (int ks = 0; ks < KS; ks++) aop[ks] = load_op(p.ao + row, ks, gA);
+                if (SEED)
+#pragma unroll
+                    for (int nt = 0; nt < NTS; nt++) xs[nt] = load_op(xrow, nt, gA);
                 int *const site = ADAPT && CS > 1 ? next_site() : nullptr;
                 if (ADAPT) {
                     // the waves of a tile take a column slice of the row each
@@ -348,20 +361,30 @@ __global__ void __launch_bounds__(EGG_THREADS, (MlpCfg<H, CSV>::occ(ADAPT))) k_m
                     dot_noise_ov<NTS, 1>(own, reinterpret_cast<const float *>(exB) + col0, 0, gA, &sbo);
                     if (CS > 1) xput(sbo, site, CS, tm, laneA);
                 } else sbo = dot_noise<KS, false>(aop, exB, 0, gA);
+                constexpr bool LATE = ADAPT && CS > 1;        // the sum comes with the exchange behind the first barrier
+                if (LATE) zero_acc<NTS>(acc); else start_perturb<NTS>(acc, sbo << c.sb_shift, oA, col0, gA);
+                if (SEED)
+#pragma unroll
+                    for (int nt = 0; nt < NTS; nt++)
+#pragma unroll
+                        for (int r = 0; r < 16; r++) acc[nt][r] += sx8(xs[nt][r >> 2], r & 3) << c.shift_out;
 #pragma unroll
                 for (int u = 0; u < M::OU; u++) {
                     const int8_t *cur = w_acquire(ws);
                     if (u + 1 < M::OU) pf_o(u + 1); else pf_up(0, 0);
                     mfma_cols<M::PRO / 2, NTS, MAXF>(acc, aop + u * (M::PRO / 2), cur, H, col0, laneA);
                 }
-                if (ADAPT && CS > 1) sbo = xget<CS, false>(site, tm, laneA);
+                if (LATE) add_perturb<NTS>(acc, xget<CS, false>(site, tm, laneA) << c.sb_shift, oA, col0, gA);
             }
-            perturb_shift_groups<NTS>(acc, sbo << c.sb_shift, oA, col0, c.shift_out, gA);
 #pragma unroll
             for (int nt = 0; nt < NTS; nt++) {
-                v4i xr = load_op(xrow, nt, gA);
 #pragma unroll
-                for (int r = 0; r < 16; r++) acc[nt][r] += sx8(xr[r >> 2], r & 3);
+                for (int r = 0; r < 16; r++) acc[nt][r] >>= c.shift_out;
+                if (!SEED) {
+                    v4i xr = load_op(xrow, nt, gA);
+#pragma unroll
+                    for (int r = 0; r < 16; r++) acc[nt][r] += sx8(xr[r >> 2], r & 3);
+                }
             }
             const int mx = xreduce<CS, true>(absmax_to_float_groups<NTS>(acc), next_site(), tm, laneA);
             adaptive_scale_floats<NTS>(acc, mx, xs);
@@ -687,7 +710,7 @@ __global__ void __launch_bounds__(EGG_THREADS, (QkvCfg<H, CSV>::OCC)) k_qkv(QkvP
             const int sb = !ADAPT ? dot_noise<KS, false>(nrm, Bn, 0, g) : CS > 1 ? xget<CS, false>(red + (2 + which) * Q::SITE, tm, lane)
                                   : which == 0 ? sb3[0] : which == 1 ? sb3[1] : sb3[2];
             v16i acc[NTS];
-            zero_acc<NTS>(acc);
+            start_perturb<NTS>(acc, sb << c.sb_shift, An, col0, g);
 #pragma unroll
             for (int u = 0; u < Q::NU; u++) {
                 const int8_t *cur = w_acquire(ws);
@@ -695,7 +718,6 @@ __global__ void __launch_bounds__(EGG_THREADS, (QkvCfg<H, CSV>::OCC)) k_qkv(QkvP
                 else if (nw) pf(nw, 0);
                 mfma_cols<Q::PR / 2, NTS>(acc, nrm + u * (Q::PR / 2), cur, H, col0, lane);
             }
-            add_perturb<NTS>(acc, sb << c.sb_shift, An, col0, g);
             if (which < 2) rope_inplace<NTS>(acc, c.rope_lut + (size_t)t * c.head_dim + col0 % c.head_dim, c.head_dim, g, c.rope_scale_bit);
             const int mx = xreduce<CS, true>(absmax_to_float_groups<NTS>(acc), red + ((1 + which) & 1) * Q::SITE, tm, lane);
             v4i o[NTS];
@@ -1220,9 +1242,8 @@ __global__ void __launch_bounds__(EGG_THREADS, (H > 256 ? 1 : 2)) k_head(HeadPar
         if constexpr (single) {
             tl = logit_of<H, ADAPT>(p, nf, sbh, pair_seed, member, c.data[spos + t + 1], g);
             v16i acc[NV];
-            zero_acc<NV>(acc);
+            start_perturb<NV>(acc, sbh, hA, 0, g);
             gemm_stream<H, 256, BLK>(acc, nf, p.embedding_frag, 256, 0, 0, ws, (pass + 1 < pass_end) ? w_unit_ptr<BLK>(p.embedding_frag, 256, 0, 0, 0) : nullptr, lane);
-            add_perturb<NV>(acc, sbh, hA, 0, g);
 #pragma unroll
             for (int nt = 0; nt < NV; nt++)
 #pragma unroll
@@ -1251,7 +1272,7 @@ __global__ void __launch_bounds__(EGG_THREADS, (H > 256 ? 1 : 2)) k_head(HeadPar
             for (int phase = 0; phase < 2; phase++) {
 #pragma unroll 1
                 for (int vb = 0; vb < nvb; vb++) {
-                    {                                   // read behind the barriers of the product below, by this wave only
+                    {                                   // the wave's own table
                         const uint32_t seed = pair_seed + OFF_EMB + (uint32_t)(vb * 256) * 0x9e3779b9u;
                         if (ADAPT) fill_noise_i32_ov(hA, seed, 256, c.mask, ns << c.a_shift, lane, 64, p.q_emb + H + vb * 256);
                         else fill_noise_i32(hA, seed, 256, c.mask, ns << c.a_shift, lane);
@@ -1260,9 +1281,9 @@ __global__ void __launch_bounds__(EGG_THREADS, (H > 256 ? 1 : 2)) k_head(HeadPar
                     const int8_t *next = !last ? w_unit_ptr<BLK>(p.embedding_frag, V, 0, (vb + 1 == nvb ? 0 : vb + 1) * 256, 0)
                                                : ((pass + 1 < pass_end) ? w_unit_ptr<BLK>(p.embedding_frag, V, 0, 0, 0) : nullptr);
                     v16i acc[NV];
-                    zero_acc<NV>(acc);
+                    wave_lds_fence();
+                    start_perturb<NV>(acc, sbh, hA, 0, g);
                     gemm_stream<H, 256, BLK>(acc, nf, p.embedding_frag, V, 0, vb * 256, ws, next, lane);
-                    add_perturb<NV>(acc, sbh, hA, 0, g);
                     if (phase == 0) {
 #pragma unroll
                         for (int nt = 0; nt < NV; nt++)
@@ -1422,7 +1443,10 @@ __global__ void __launch_bounds__(EGG_THREADS, 2) k_head_big(HeadParams p) {
 #pragma unroll 1
     for (int vb = 0; vb < nvb; vb++) {
         v16i acc[NV];
-        zero_acc<NV>(acc);
+        // (a block's table is written behind the first barrier of the block in front of it: with one unit a block no barrier lies
+        // between that and here)
+        if (B::NU > 1) start_perturb<NV>(acc, sbh, hA + (vb & 1) * COLS, 0, g);
+        else zero_acc<NV>(acc);
 #pragma unroll
         for (int u = 0; u < B::NU; u++) {
             const int8_t *cur = w_acquire(ws);
@@ -1430,7 +1454,7 @@ __global__ void __launch_bounds__(EGG_THREADS, 2) k_head_big(HeadParams p) {
             if (u == 0 && vb + 1 < nvb) fill_out_noise(vb + 1);      // everyone has left block vb - 1, whose table this is
             mfma_cols<B::PR / 2, NV>(acc, nf + u * (B::PR / 2), cur, COLS, 0, lane);
         }
-        add_perturb<NV>(acc, sbh, hA + (vb & 1) * COLS, 0, g);
+        if (B::NU == 1) add_perturb<NV>(acc, sbh, hA + (vb & 1) * COLS, 0, g);
         int most = INT_MIN;
 #pragma unroll
         for (int nt = 0; nt < NV; nt++)
@@ -1496,7 +1520,8 @@ static hipError_t launch_mlp_cs(const MlpParams &p, bool first, hipStream_t s) {
     const int sets = tile_map_sets(p.c.tn, CSV);
     const dim3 grid((p.c.n_members + sets - 1) / sets), block(EGG_THREADS);
     const size_t lds = MlpCfg<H, CSV>::total(sets, first, ADAPT);
-    const bool seed = egg_mlp_down_acc_bound(H, p.c.mask, p.c.sigma_vec, p.c.shift_mlp_down) < (1LL << 31);
+    const bool seed = egg_mlp_down_acc_bound(H, p.c.mask, p.c.sigma_vec, p.c.shift_mlp_down) < (1LL << 31) &&
+                      (first || egg_out_acc_bound(H, p.c.mask, p.c.shift_out) < (1LL << 31));
     if (first) { if (seed) hipLaunchKernelGGL((k_mlp<H, true, true, ADAPT, CSV>), grid, block, lds, s, p); else hipLaunchKernelGGL((k_mlp<H, true, false, ADAPT, CSV>), grid, block, lds, s, p); }
     else { if (seed) hipLaunchKernelGGL((k_mlp<H, false, true, ADAPT, CSV>), grid, block, lds, s, p); else hipLaunchKernelGGL((k_mlp<H, false, false, ADAPT, CSV>), grid, block, lds, s, p); }
     return hipGetLastError();

@@ -41,6 +41,12 @@ static inline long long egg_mlp_down_acc_bound(int hidden, int mask, int sigma_v
     return 4LL * hidden * 127 * (127 + mag * mag) + (seed << shift_mlp_down);
 }
 
+// The attention output projection's accumulator with residual << shift_out in it, likewise.
+static inline long long egg_out_acc_bound(int hidden, int mask, int shift_out) {
+    const long long mag = egg_noise_magnitude(mask);
+    return (long long)hidden * 127 * (127 + mag * mag) + (127LL << shift_out);
+}
+
 // (sb * a) >> sigma of a rank-one term is the high word of (sb << sb_shift) * (a << a_shift), one instruction where the output
 // side's table holds the shifted noise: sb_shift + a_shift = 32 - sigma, with as little on sb as keeps a below 2^31 (sb has
 // 24 bits, the magnitude at most 7: at most 8 more are ever needed).
