@@ -102,6 +102,15 @@ __device__ __forceinline__ void exchange_operand(int8_t *buf, const TileMap &tm,
 template <int H> constexpr int few_slices() { return H == 512 ? 2 : Shape<H>::CS; }
 template <int H> constexpr int many_slices() { return 2 * few_slices<H>(); }
 template <int H> static bool use_many_slices(const FwdCommon &c) { return (long long)c.n_members * (c.tn / 32) * few_slices<H>() <= 1024; }     // 1024 SIMDs
+// One slice at hidden 256, where a wave holds the whole 256-column accumulator: two workgroups to a CU instead of three, but twice the tokens share
+// each staged unit of W, no operand is exchanged, and a unit's barrier comes half as often per token.  8,192 members x 256 tokens:
+// k_mlp 1.74 -> 1.60 ms, k_qkv 1.02 -> 0.90, the overlay's k_qkv (2,048 members) 0.28 -> 0.26; 192 members: 93 -> 76 and 54 -> 44 us.  (The overlay's
+// k_mlp spills 26 registers and takes 0.64 instead of 0.58 ms.)  From 1,536 tiles on; at 1,024 tiles of 32-token windows two slices win, 27 to 30 us.
+constexpr int ONE_SLICE_TILES = 1536;
+static bool use_one_slice_qkv(const FwdCommon &c) { return (long long)c.n_members * (c.tn / 32) >= ONE_SLICE_TILES; }
+// (k_mlp with windows of one tile would hold the tables of four members, one workgroup to a CU: 83 -> 96 us at 2,048 members.  A first block that
+// is evaluated once per byte value needs more than one pass over the window, which four tiles are not with one slice: 356 -> 417 us.)
+static bool use_one_slice_mlp(const FwdCommon &c, bool by_value) { return c.tn >= 64 && use_one_slice_qkv(c) && !(by_value && c.tn == 128); }
 template <int H, int CSV>
 struct MlpCfg {
     static constexpr int CS = CSV;
@@ -122,7 +131,7 @@ struct MlpCfg {
     // The up projection's output noise is kept as int32: the GELU epilogue then multiplies by a table word as it stands
     // instead of extracting a byte per element.  Only the first block of hidden 256 has no room for it at three workgroups
     // per CU (its value-rank tables take the space) and keeps the bytes.
-    static constexpr bool up32(bool first) { return !first || H != 256; }
+    static constexpr bool up32(bool first) { return !first || H != 256 || CS == 1; }
     static constexpr int UPA32 = 3 * 4 * H;  // extra bytes of the int32 form: upA occupies 16H instead of 4H
     static constexpr int PER_SET = I32 * 4 + I8;
     // The normalised input is exchanged through whichever W buffer is idle at that point (TPW*32*H <= UNIT bytes);
@@ -130,7 +139,7 @@ struct MlpCfg {
     static constexpr int XCHG = CS > 1 ? TPW * 32 * SC : 0;
     static constexpr int SITE = EGG_WAVES * 32;                       // ints per reduction site
     static constexpr int RED = CS > 1 ? 2 * SITE * 4 : 0;             // two reduction sites used alternately
-    static constexpr int OCC = H == 256 ? 3 : 2;                      // workgroups per CU the kernel is built for
+    static constexpr int OCC = H == 256 && CS > 1 ? 3 : 2;             // workgroups per CU the kernel is built for
     // first block only: rank of every byte value among the values present in the member's window [256], wave counts
     // [4 ints], and below hidden 256 the list of present values [256] (from hidden 256 on it lives in the table slot
     // of the O projection's noise, which the first block does not use)
@@ -577,7 +586,7 @@ struct QkvCfg {
     static constexpr int XCHG = 0;             // the normalised input is exchanged through the idle W buffer
     static constexpr int SITE = EGG_WAVES * 32;
     static constexpr int RED = CS > 1 ? 2 * SITE * 4 : 0;       // two reduction sites used alternately (overlay: and one for each input-side sum)
-    static constexpr int OCC = H == 256 ? 3 : 2;               // workgroups per CU the kernel is built for
+    static constexpr int OCC = H == 256 && CS > 1 ? 3 : 2;      // workgroups per CU the kernel is built for
     static constexpr int per_set(bool adapt) { return PER_SET + (adapt ? 3 * 3 * H : 0); }        // the overlay's qB kB vB are floats
     static int total(int sets, bool adapt) { return WBYTES + sets * per_set(adapt) + XCHG + RED + (adapt && CS > 1 ? 3 * SITE * 4 : 0); }
 };
@@ -1531,6 +1540,7 @@ static hipError_t launch_mlp_h(const MlpParams &p, bool first, hipStream_t s) {
     if (egg_mlp_up_acc_bound(H, p.c.mask, p.c.sigma_vec, p.c.shift_mlp_up) >= (1LL << 31)) return hipErrorInvalidValue;      // egg_ctx_create refuses such shifts
     if (p.q_ln_w) return launch_mlp_cs<H, true, few_slices<H>()>(p, first, s);       // the adaptive overlay has this form only
     if (use_many_slices<H>(p.c)) return launch_mlp_cs<H, false, many_slices<H>()>(p, first, s);
+    if constexpr (H == 256) if (use_one_slice_mlp(p.c, first && p.tab)) return launch_mlp_cs<H, false, 1>(p, first, s);
     return launch_mlp_cs<H, false, few_slices<H>()>(p, first, s);
 }
 hipError_t egg_launch_mlp(const MlpParams &p, bool first, hipStream_t s) {
@@ -1551,6 +1561,7 @@ static hipError_t launch_qkv_cs(const QkvParams &p, hipStream_t s) {
 }
 template <int H>
 static hipError_t launch_qkv_h(const QkvParams &p, hipStream_t s) {
+    if constexpr (H == 256) if (use_one_slice_qkv(p.c)) return p.q_ln_w ? launch_qkv_cs<H, true, 1>(p, s) : launch_qkv_cs<H, false, 1>(p, s);
     if (p.q_ln_w) return launch_qkv_cs<H, true, few_slices<H>()>(p, s);
     if (use_many_slices<H>(p.c)) return launch_qkv_cs<H, false, many_slices<H>()>(p, s);
     return launch_qkv_cs<H, false, few_slices<H>()>(p, s);
@@ -1645,6 +1656,12 @@ static hipError_t no_static_lds(K kern) {
     return a.sharedSizeBytes == 0 ? hipSuccess : hipErrorInvalidConfiguration;
 }
 template <int H, bool ADAPT, int CSV>
+static hipError_t prepare_qkv(int T) {
+    const int sets = std::max(tile_map_sets(T, CSV), tile_map_sets(32, CSV));
+    SET_LDS((k_qkv<H, ADAPT, CSV>), (QkvCfg<H, CSV>::total(sets, ADAPT)));
+    return hipSuccess;
+}
+template <int H, bool ADAPT, int CSV>
 static hipError_t prepare_cs(int T) {
     // table sets per workgroup: the whole window's, or a single tile's (a prompt's first tiles may be evaluated alone)
     const int sets = std::max(tile_map_sets(T, CSV), tile_map_sets(32, CSV));
@@ -1655,13 +1672,15 @@ static hipError_t prepare_cs(int T) {
     SET_LDS((k_mlp<H, true, false, ADAPT, CSV>), (MlpCfg<H, CSV>::total(sets, true, ADAPT)));
     SET_LDS((k_mlp<H, false, true, ADAPT, CSV>), (MlpCfg<H, CSV>::total(sets, false, ADAPT)));
     SET_LDS((k_mlp<H, false, false, ADAPT, CSV>), (MlpCfg<H, CSV>::total(sets, false, ADAPT)));
-    SET_LDS((k_qkv<H, ADAPT, CSV>), (QkvCfg<H, CSV>::total(sets, ADAPT)));
-    return hipSuccess;
+    return prepare_qkv<H, ADAPT, CSV>(T);
 }
 template <int H>
 static hipError_t prepare_h(int T) {
     for (hipError_t e : {prepare_cs<H, true, few_slices<H>()>(T), prepare_cs<H, false, few_slices<H>()>(T), prepare_cs<H, false, many_slices<H>()>(T)})
         if (e != hipSuccess) return e;
+    if constexpr (H == 256)
+        for (hipError_t e : {prepare_cs<H, false, 1>(T), prepare_qkv<H, true, 1>(T)})
+            if (e != hipSuccess) return e;
     SET_LDS((k_head<H, false, false>), HeadLds<H>::total(false));
     SET_LDS((k_head<H, true, false>), HeadLds<H>::total(true));
     SET_LDS((k_head<H, false, true>), HeadLds<H>::total(false));
