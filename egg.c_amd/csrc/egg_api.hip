@@ -905,7 +905,7 @@ extern "C" int egg_update_tensor(egg_ctx *ctx, int id, const int32_t *d_fit, con
     if (t.is_matrix && t.muon && ctx->cfg.use_muon) {
         // LAUNCH_ADAM_MATRIX under USE_MUON (mgpu.cu:1587-1595)
         HIP_TRY(egg_launch_newton_schulz(ctx->muon, t.rows, t.cols, 5, ctx->stream));
-        HIP_TRY(egg_launch_muon_apply(p, ctx->cfg.adam_weight_decay, ctx->stream));
+        HIP_TRY(egg_launch_muon_apply(p, ctx->cfg.adam_weight_decay, 0, ctx->stream));
     }
     return EGG_OK;
 }
@@ -958,8 +958,9 @@ static int es_update(egg_ctx *ctx, const int32_t *d_fit, const StepEnd &end, con
             UpdLaunch p = make_upd(ctx, ctx->mat_muon[batch], d_fit, d_lr);
             p.count_of = count_of;
             { SpanScope span(ctx, EGG_K_UPDATE_MATRIX); HIP_TRY(egg_launch_update(p, ctx->stream)); }
-            { SpanScope span(ctx, EGG_K_MUON_NS); HIP_TRY(egg_launch_newton_schulz_batched(ctx->muon, t0.rows, t0.cols, 5, p.n_mat, ctx->stream)); }
-            { SpanScope span(ctx, EGG_K_UPDATE_MATRIX); HIP_TRY(egg_launch_muon_apply(p, c.adam_weight_decay, ctx->stream)); }
+            const float *result = ctx->muon.x;
+            { SpanScope span(ctx, EGG_K_MUON_NS); HIP_TRY(egg_launch_newton_schulz_batched(ctx->muon, t0.rows, t0.cols, 5, p.n_mat, ctx->stream, &result)); }
+            { SpanScope span(ctx, EGG_K_UPDATE_MATRIX); HIP_TRY(egg_launch_muon_apply(p, c.adam_weight_decay, result - ctx->muon.x, ctx->stream)); }
         }
     }
     // d-eggs runs the overlay rule after each tensor's update (de/src/worker.cu:446-523); tensors and their overlay

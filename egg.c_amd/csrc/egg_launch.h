@@ -95,7 +95,7 @@ int egg_update_blocks(const UpdLaunch &p);             // its workgroups
 size_t egg_noise_ld(int entries);                      // bytes of a table row that holds so many entries
 size_t egg_noise_mask_ld(int pairs_pad);
 hipError_t egg_launch_update(const UpdLaunch &p, hipStream_t s);
-hipError_t egg_launch_muon_apply(const UpdLaunch &p, float wd, hipStream_t s);
+hipError_t egg_launch_muon_apply(const UpdLaunch &p, float wd, ptrdiff_t moved, hipStream_t s);      // moved: from MatDesc::muon_x to the orthogonalised matrix, in floats
 hipError_t egg_launch_frag(const MatDesc *d_mat, int n_mat, int tiles, hipStream_t s);
 
 // adaptive noise overlay (de/src/kernels.cu:61-77): for every entry of every segment, +inc where the flag is set, -dec
@@ -135,7 +135,7 @@ hipError_t egg_launch_ternary_pack(const int8_t *src, uint8_t *packed, int n_ele
 // 5 Newton-Schulz iterations on fp32 MFMA, quantised apply (egg_launch_muon_apply).
 struct MuonWork { float *x, *swap, *gram, *bterm, *partials, *norm; };   // x/swap: rows*cols, gram/bterm: K*K, partials: 1024
 hipError_t egg_launch_newton_schulz(const MuonWork &w, int rows, int cols, int iters, hipStream_t s);
-hipError_t egg_launch_newton_schulz_batched(const MuonWork &w, int rows, int cols, int iters, int batch, hipStream_t s);
+hipError_t egg_launch_newton_schulz_batched(const MuonWork &w, int rows, int cols, int iters, int batch, hipStream_t s, const float **result);
 // ---- device memory to the caller's memory (egg_hostout.hip)
 struct HostOut { int8_t *mem = nullptr; size_t slot = 0; hipEvent_t done[8] = {}; };
 hipError_t egg_host_out_create(HostOut *o, size_t largest);       // largest: the longest piece that is usually asked for

@@ -8,6 +8,7 @@
 #include "egg_launch.h"
 #include <mutex>
 #include <string>
+#include <type_traits>
 
 #pragma clang fp contract(off)
 
@@ -347,12 +348,20 @@ __global__ void __launch_bounds__(EGG_THREADS) k_sgemm(const float *A, long lda,
 // output element summed by one wave over the whole of K (no partial tiles to add up).  A workgroup owns a TILE x TILE
 // block of C, TILE = 64 WT: wave (wm, wn) owns the 32 WT x 32 WT quarter as WT x WT MFMA tiles.  A TILE x 32 chunk of A
 // and a 32 x TILE chunk of B go global -> registers -> LDS (the next chunk's loads are in flight while the MFMAs of the
-// current one run); with WT = 2 every value read from LDS feeds two MFMAs and the L2 traffic per flop is a quarter of
-// the 32 x 32 kernel's.  An operand whose k stride is 1 sits in LDS as [row][k] with rows 36 floats apart (16-byte
-// reads of four consecutive k, a 2-way bank conflict at most); the other kind as [k][row] with k rows TILE + 8 floats
-// apart (4-byte reads; the two lane halves, four k rows apart, fall on different banks).
-// Within a block of eight k, MFMA e multiplies the pair {8c + e, 8c + 4 + e}, blocks in ascending order, whatever WT
-// is: the two tile sizes give bit-identical results, so the host may pick by the size of the grid.
+// current one run, and those of the one behind it).
+// The float32 matrix instruction does 64 multiplications a clock and SIMD, the bf16 one 1,024, so every operand is taken apart on its
+// way into LDS: x = x0 + x1 + x2, each the nearest bf16 of what is left (8 + 8 + 8 bits: 24, the float's own), and a product is
+// the six partial products of at least 2^-18 of it: x0 y0, x0 y1, x1 y0, x1 y1, x0 y2, x2 y0.  They are exact, what is left out is below 2^-26 of
+// the product, a quarter of the rounding of one float32 addition; they are added in float32, the smallest first.  Five iterations
+// against 64 bits are nearer than with the float32 instruction: relative error of random matrices 9.1e-7 -> 6.0e-7 at 512 x 512, 4.2e-7 -> 2.7e-7 at
+// 512 x 2048, 3.3e-7 -> 2.6e-7 at 64 x 64, rank one 6.2e-6 -> 4.0e-6 (rows scaled over e^4 4.2e-7 -> 4.3e-7 and 9.7e-7 -> 6.8e-7).  Times: G (upper half) of 32
+// matrices of 512 x 512 63 -> 60 us, X B of them 89 -> 64, 2048 x 512 x 512 of nine 127 -> 82, and the products of nine 512 x 512 38 -> 26.5:
+// those are 16 chunks one after the other, at one to three workgroups a CU.
+// An operand sits in LDS as three planes [row][k] of bf16 with rows 80 bytes apart (a lane reads eight consecutive k of its row as 16
+// bytes; 16 such rows fall on all banks once).  One whose k stride is not 1 is turned over on the way: a thread
+// takes four rows at two consecutive k.
+// What an output element is summed from, and in which order, does not depend on WT: the two tile sizes give bit-identical
+// results, so the host may pick by the size of the grid.
 // SYM: C is symmetric; only tiles on and above the diagonal are computed, elements above it are stored twice (36 of 64 tiles
 // at 512 columns).
 // A launch may multiply two left sides with the same B (blockIdx.z).  Epilogues, v the sum over k, e0 and e1 elements of
@@ -362,21 +371,45 @@ struct SgemmJob {
     const float *A; long batch_a; float *C; const float *e0, *e1; float *C2; int mode; float alpha;
 };
 struct SgemmJobs { SgemmJob j[2]; };
-__device__ __forceinline__ float ns_epilogue(const SgemmJob &job, float v, bool diag, size_t at) {
-    switch (job.mode) {
-        case NS_B: return (diag ? 3.0f : 0.0f) - v;                       // 3I - G (muon_internal.cuh:91-109)
-        case NS_STEP: return 0.25f * ((9.0f * job.e0[at] - 6.0f * job.e1[at]) + v);      // G (3I - G)^2 / 4 from G, G^2, G^3
-        case NS_FACTOR: return 0.5f * (3.0f * job.e0[at] - v);            // P (3I - G) / 2
-        default: return job.alpha * v;
+// v of the 16 elements (i + 8q + e, jj) of a lane (at: the first one's place) -> what is stored.  All reads of the other matrices come first: left
+// between the stores, which may alias them as far as the compiler knows, each would be waited for by itself.
+__device__ __forceinline__ void ns_epilogue(const SgemmJob &job, v16f &v, int i, int jj, size_t at, int N) {
+    v16f x, y;
+    if (job.mode == NS_STEP || job.mode == NS_FACTOR)
+#pragma unroll
+        for (int r = 0; r < 16; r++) x[r] = job.e0[at + (size_t)(8 * (r >> 2) + (r & 3)) * N];
+    if (job.mode == NS_STEP)
+#pragma unroll
+        for (int r = 0; r < 16; r++) y[r] = job.e1[at + (size_t)(8 * (r >> 2) + (r & 3)) * N];
+#pragma unroll
+    for (int r = 0; r < 16; r++)
+        switch (job.mode) {
+            case NS_B: v[r] = (i + 8 * (r >> 2) + (r & 3) == jj ? 3.0f : 0.0f) - v[r]; break;       // 3I - G (muon_internal.cuh:91-109)
+            case NS_STEP: v[r] = 0.25f * ((9.0f * x[r] - 6.0f * y[r]) + v[r]); break;               // G (3I - G)^2 / 4 from G, G^2, G^3
+            case NS_FACTOR: v[r] = 0.5f * (3.0f * x[r] - v[r]); break;                              // P (3I - G) / 2
+            default: v[r] = job.alpha * v[r];
+        }
+}
+typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+typedef float v2f __attribute__((ext_vector_type(2)));
+constexpr int NS_PLANES = 3;
+// two values as NS_PLANES pairs of bf16
+__device__ __forceinline__ void split_bf16(float a, float b, uint32_t *pl) {
+#pragma unroll
+    for (int p = 0; p < NS_PLANES; p++) {
+        const v2f x = {a, b};
+        pl[p] = __builtin_bit_cast(uint32_t, __builtin_convertvector(x, v2bf));
+        a -= __uint_as_float(pl[p] << 16);
+        b -= __uint_as_float(pl[p] & 0xffff0000u);
     }
 }
 template <bool AK, bool BK, int WT, bool SYM>
-__global__ void __launch_bounds__(EGG_THREADS, WT == 1 ? 4 : 2) k_sgemm_lds(SgemmJobs jobs, long lda, const float *B, long ldb, long batch_b, int M, int N, int K) {
-    constexpr int TILE = 64 * WT, KC = 32, LDK = 36, LDI = TILE + 8, PIECES = TILE * KC / 4 / EGG_THREADS;
-    constexpr int ASZ = AK ? TILE * LDK : KC * LDI, BSZ = BK ? TILE * LDK : KC * LDI;
-    constexpr int RPI = TILE / 4;                 // 16-byte pieces per k row of an [k][row] chunk
-    __shared__ __align__(16) float As[ASZ];
-    __shared__ __align__(16) float Bs[BSZ];
+__global__ void __launch_bounds__(EGG_THREADS, WT == 1 ? 3 : 2) k_sgemm_lds(SgemmJobs jobs, long lda, const float *B, long ldb, long batch_b, int M, int N, int K) {
+    constexpr int TILE = 64 * WT, KC = 32, ROW = 80, PLANE = TILE * ROW, PIECES = TILE * KC / 4 / EGG_THREADS;
+    constexpr int AHEAD = 2;
+    __shared__ __align__(16) int8_t As[NS_PLANES * PLANE];
+    __shared__ __align__(16) int8_t Bs[NS_PLANES * PLANE];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 5, j = lane & 31, tid = threadIdx.x;
     const int wm = wave >> 1, wn = wave & 1;
     const int tiles_n = N / TILE;
@@ -398,73 +431,103 @@ __global__ void __launch_bounds__(EGG_THREADS, WT == 1 ? 4 : 2) k_sgemm_lds(Sgem
         for (int b = 0; b < WT; b++)
 #pragma unroll
             for (int r = 0; r < 16; r++) acc[a][b][r] = 0.f;
-    // global -> registers: PIECES 16-byte pieces of each operand's chunk per thread
-    v4f ra[PIECES], rb[PIECES];
-    auto load_chunk = [&](int k0) {
+    // global -> registers: PIECES 16-byte pieces of each operand's chunk per thread, AHEAD chunks early.  k stride 1: four k of a row a piece; otherwise four rows at k, and the next piece at
+    // k + 1, sixteen such pairs of k in sixteen lanes (their writes fall on different banks).
+    v4f ra[AHEAD][PIECES], rb[AHEAD][PIECES];
+    auto load_operand = [&](auto kone, const float *X, long ld, int x0, int k0, v4f *r) {
 #pragma unroll
         for (int p = 0; p < PIECES; p++) {
-            const int idx = tid + EGG_THREADS * p;
-            if (AK) ra[p] = *reinterpret_cast<const v4f *>(A + (long)(i0 + (idx >> 3)) * lda + k0 + 4 * (idx & 7));
-            else ra[p] = *reinterpret_cast<const v4f *>(A + (long)(k0 + idx / RPI) * lda + i0 + 4 * (idx % RPI));
-            if (BK) rb[p] = *reinterpret_cast<const v4f *>(B + (long)(j0 + (idx >> 3)) * ldb + k0 + 4 * (idx & 7));
-            else rb[p] = *reinterpret_cast<const v4f *>(B + (long)(k0 + idx / RPI) * ldb + j0 + 4 * (idx % RPI));
+            constexpr bool KONE = decltype(kone)::value;
+            const int idx = tid + EGG_THREADS * (KONE ? p : p >> 1);
+            r[p] = KONE ? *reinterpret_cast<const v4f *>(X + (long)(x0 + (idx >> 3)) * ld + k0 + 4 * (idx & 7))
+                        : *reinterpret_cast<const v4f *>(X + (long)(k0 + 2 * (idx & 15) + (p & 1)) * ld + x0 + 4 * (idx >> 4));
         }
     };
-    auto store_chunk = [&]() {
+    auto store_operand = [&](auto kone, int8_t *X, const v4f *r) {
+        constexpr bool KONE = decltype(kone)::value;
+        if constexpr (KONE) {
 #pragma unroll
-        for (int p = 0; p < PIECES; p++) {
-            const int idx = tid + EGG_THREADS * p;
-            if (AK) *reinterpret_cast<v4f *>(As + (idx >> 3) * LDK + 4 * (idx & 7)) = ra[p];
-            else *reinterpret_cast<v4f *>(As + (idx / RPI) * LDI + 4 * (idx % RPI)) = ra[p];
-            if (BK) *reinterpret_cast<v4f *>(Bs + (idx >> 3) * LDK + 4 * (idx & 7)) = rb[p];
-            else *reinterpret_cast<v4f *>(Bs + (idx / RPI) * LDI + 4 * (idx % RPI)) = rb[p];
-        }
-    };
-    load_chunk(0);
-    for (int k0 = 0; k0 < K; k0 += KC) {
-        __syncthreads();                    // every wave has finished reading the previous chunk
-        store_chunk();
-        __syncthreads();
-        if (k0 + KC < K) load_chunk(k0 + KC);
+            for (int p = 0; p < PIECES; p++) {
+                const int idx = tid + EGG_THREADS * p;
+                uint32_t lo[NS_PLANES], hi[NS_PLANES];
+                split_bf16(r[p][0], r[p][1], lo);
+                split_bf16(r[p][2], r[p][3], hi);
 #pragma unroll
-        for (int c = 0; c < KC / 8; c++) {
-            v4f a4[WT], b4[WT];
+                for (int pl = 0; pl < NS_PLANES; pl++)
+                    *reinterpret_cast<uint64_t *>(X + pl * PLANE + (idx >> 3) * ROW + 8 * (idx & 7)) = (uint64_t)hi[pl] << 32 | lo[pl];
+            }
+        } else {
 #pragma unroll
-            for (int t = 0; t < WT; t++) {
-                const int row = 32 * WT * wm + 32 * t + j, col = 32 * WT * wn + 32 * t + j;
-                if (AK) a4[t] = *reinterpret_cast<const v4f *>(As + row * LDK + 8 * c + 4 * g);
-                else {
+            for (int p = 0; p < PIECES; p += 2) {
+                const int idx = tid + EGG_THREADS * (p >> 1);
 #pragma unroll
-                    for (int e = 0; e < 4; e++) a4[t][e] = As[(8 * c + 4 * g + e) * LDI + row];
-                }
-                if (BK) b4[t] = *reinterpret_cast<const v4f *>(Bs + col * LDK + 8 * c + 4 * g);
-                else {
+                for (int e = 0; e < 4; e++) {
+                    uint32_t w[NS_PLANES];
+                    split_bf16(r[p][e], r[p + 1][e], w);
 #pragma unroll
-                    for (int e = 0; e < 4; e++) b4[t][e] = Bs[(8 * c + 4 * g + e) * LDI + col];
+                    for (int pl = 0; pl < NS_PLANES; pl++) *reinterpret_cast<uint32_t *>(X + pl * PLANE + (4 * (idx >> 4) + e) * ROW + 4 * (idx & 15)) = w[pl];
                 }
             }
+        }
+    };
+    const std::integral_constant<bool, AK> a_kone{};
+    const std::integral_constant<bool, BK> b_kone{};
+    // (loads behind the last chunk ask for it again: with a load on one path only, the compiler's wait for a chunk would count on none in flight)
+    auto load_chunk = [&](int n, int k0) {
+        const int k = min(k0, K - KC);
+        load_operand(a_kone, A, lda, i0, k, ra[n]);
+        load_operand(b_kone, B, ldb, j0, k, rb[n]);
+    };
+    auto chunk = [&](int n, int k0) {
+        __syncthreads();                    // every wave has finished reading the previous chunk
+        store_operand(a_kone, As, ra[n]);
+        store_operand(b_kone, Bs, rb[n]);
+        __syncthreads();
+        load_chunk(n, k0 + AHEAD * KC);
 #pragma unroll
-            for (int e = 0; e < 4; e++)
+        for (int c = 0; c < KC / 16; c++) {
+            v8bf a[WT][NS_PLANES], b[WT][NS_PLANES];
+#pragma unroll
+            for (int t = 0; t < WT; t++)
+#pragma unroll
+                for (int pl = 0; pl < NS_PLANES; pl++) {
+                    a[t][pl] = *reinterpret_cast<const v8bf *>(As + pl * PLANE + (32 * WT * wm + 32 * t + j) * ROW + 32 * c + 16 * g);
+                    b[t][pl] = *reinterpret_cast<const v8bf *>(Bs + pl * PLANE + (32 * WT * wn + 32 * t + j) * ROW + 32 * c + 16 * g);
+                }
+            constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+            for (int m = 0; m < 6; m++)
 #pragma unroll
                 for (int ta = 0; ta < WT; ta++)
 #pragma unroll
                     for (int tb = 0; tb < WT; tb++)
-                        acc[ta][tb] = __builtin_amdgcn_mfma_f32_32x32x2f32(a4[ta][e], b4[tb][e], acc[ta][tb], 0, 0, 0);
+                        acc[ta][tb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[ta][PA[m]], b[tb][PB[m]], acc[ta][tb], 0, 0, 0);
         }
-    }
+    };
+#pragma unroll
+    for (int n = 0; n < AHEAD; n++) load_chunk(n, n * KC);
+    int k0 = 0;
+    for (; k0 + AHEAD * KC <= K; k0 += AHEAD * KC)
+#pragma unroll
+        for (int n = 0; n < AHEAD; n++) chunk(n, k0 + n * KC);
+#pragma unroll
+    for (int n = 0; n < AHEAD - 1; n++)
+        if (k0 + n * KC < K) chunk(n, k0 + n * KC);
     // accumulator register r of lane (j, g) is row 8 (r / 4) + 4 g + r % 4, column j of its 32 x 32 tile
 #pragma unroll
     for (int ta = 0; ta < WT; ta++)
 #pragma unroll
-        for (int tb = 0; tb < WT; tb++)
+        for (int tb = 0; tb < WT; tb++) {
+            const int i1 = i0 + 32 * WT * wm + 32 * ta + 4 * g, jj = j0 + 32 * WT * wn + 32 * tb + j;
+            ns_epilogue(job, acc[ta][tb], i1, jj, out + (size_t)i1 * N + jj, N);
 #pragma unroll
             for (int q = 0; q < 4; q++) {
-                const int i = i0 + 32 * WT * wm + 32 * ta + 8 * q + 4 * g, jj = j0 + 32 * WT * wn + 32 * tb + j;
+                const int i = i1 + 8 * q;
                 v4f v;
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
                     const size_t at = out + (size_t)(i + e) * N + jj;
-                    v[e] = ns_epilogue(job, acc[ta][tb][4 * q + e], i + e == jj, at);
+                    v[e] = acc[ta][tb][4 * q + e];
                     if (!SYM || i + e <= jj) {
                         job.C[at] = v[e];
                         if (SYM && job.mode == NS_GRAM) job.C2[at] = (i + e == jj ? 1.5f : 0.0f) - 0.5f * v[e];
@@ -484,6 +547,7 @@ __global__ void __launch_bounds__(EGG_THREADS, WT == 1 ? 4 : 2) k_sgemm_lds(Sgem
                             }
                 }
             }
+        }
 }
 template <int WT, bool SYM>
 static hipError_t sgemm_lds(bool ak, bool bk, const SgemmJobs &jobs, int n_jobs, long lda, const float *B, long ldb, long batch_b, int M, int N, int K, int batch, hipStream_t s) {
@@ -538,8 +602,9 @@ __global__ void k_copy_f32(float *dst, const float *src, size_t n) {
 }
 
 // `batch` matrices of rows x cols, matrix b at w.x + b * rows * cols (w.swap likewise), its 3I - G term at
-// w.bterm + b * K * K (K = min(rows, cols)), its 256 norm partials at w.partials + 256 b, its norm at w.norm + b
-hipError_t egg_launch_newton_schulz_batched(const MuonWork &w, int rows, int cols, int iters, int batch, hipStream_t s) {
+// w.bterm + b * K * K (K = min(rows, cols)), its 256 norm partials at w.partials + 256 b, its norm at w.norm + b.  The result goes back to
+// w.x, or stays where it is, in w.x or w.swap, and *result says where.
+hipError_t egg_launch_newton_schulz_batched(const MuonWork &w, int rows, int cols, int iters, int batch, hipStream_t s, const float **result) {
     if (rows % 32 || cols % 32 || batch < 1 || batch > 65535) return hipErrorInvalidValue;
     if ((reinterpret_cast<uintptr_t>(w.x) | reinterpret_cast<uintptr_t>(w.swap) | reinterpret_cast<uintptr_t>(w.bterm)) & 15) return hipErrorInvalidValue;   // 16-byte loads
     const int n = rows * cols;
@@ -605,11 +670,12 @@ hipError_t egg_launch_newton_schulz_batched(const MuonWork &w, int rows, int col
     }
     if (e != hipSuccess) return e;
     const size_t total = (size_t)n * batch;
+    if (result) { *result = cur; return hipGetLastError(); }
     if (cur != w.x) hipLaunchKernelGGL(k_copy_f32, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, w.x, cur, total);
     return hipGetLastError();
 }
 hipError_t egg_launch_newton_schulz(const MuonWork &w, int rows, int cols, int iters, hipStream_t s) {
-    return egg_launch_newton_schulz_batched(w, rows, cols, iters, 1, s);
+    return egg_launch_newton_schulz_batched(w, rows, cols, iters, 1, s, nullptr);
 }
 
 // ---------------------------------------------------------------- Newton-Schulz for callers that cannot allocate

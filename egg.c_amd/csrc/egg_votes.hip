@@ -534,7 +534,7 @@ hipError_t egg_launch_update(const UpdLaunch &p, hipStream_t s) {
 // muon_apply_update_kernel (muon_internal.cuh:112-170) for every matrix of a list: a thread takes one 16-byte unit of the
 // fragment-major copy (16 rows of one column), so neighbouring lanes read and write neighbouring columns throughout.
 // Bound by memory (22 bytes an element).
-__global__ void __launch_bounds__(256) k_muon_apply(UpdLaunch p, float wd) {
+__global__ void __launch_bounds__(256) k_muon_apply(UpdLaunch p, float wd, ptrdiff_t moved) {
     __shared__ int sums[EGG_WAVES];
     const MatDesc t = p.mat[find_last(p.n_mat, blockIdx.x, [&](int i) { return p.mat[i].tile_first; })];
     const int u = ((int)blockIdx.x - t.tile_first) * 256 + (int)threadIdx.x;       // 256 units to a 64 x 64 tile
@@ -542,37 +542,47 @@ __global__ void __launch_bounds__(256) k_muon_apply(UpdLaunch p, float wd) {
     const float lr = (*p.d_lr) * t.lr_scale;
     int changes = 0;
     v4i unit;
+    // (all reads first: each would otherwise wait for the stores in front of it)
+    int w4[4];
+    float4 s0[4], s1[4];
+    float x[4][4];
 #pragma unroll
     for (int q = 0; q < 4; q++) {
         const int kr = 32 * ks + 8 * q + 4 * g;
         const size_t idx = ((size_t)(kr >> 2) * t.cols + n) * 4;
-        const int w4 = *reinterpret_cast<const int *>(t.W + idx);
-        float4 *sp = reinterpret_cast<float4 *>(t.state + idx * 2);
-        const float4 s0 = sp[0], s1 = sp[1];
-        float acc[4] = {s0.y, s0.w, s1.y, s1.w};
+        const float4 *sp = reinterpret_cast<const float4 *>(t.state + idx * 2);
+        w4[q] = *reinterpret_cast<const int *>(t.W + idx);
+        s0[q] = sp[0]; s1[q] = sp[1];
+#pragma unroll
+        for (int e = 0; e < 4; e++) x[q][e] = (t.muon_x + moved)[(size_t)(kr + e) * t.cols + n];
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const size_t idx = ((size_t)((32 * ks + 8 * q + 4 * g) >> 2) * t.cols + n) * 4;
+        float acc[4] = {s0[q].y, s0[q].w, s1[q].y, s1[q].w};
         int wv[4];
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-            wv[e] = sx8(w4, e);
-            const float x = t.muon_x[(size_t)(kr + e) * t.cols + n];
+            wv[e] = sx8(w4[q], e);
             const float wdw = wd * (float)wv[e];
-            const float step = (-lr) * (x + wdw);
+            const float step = (-lr) * (x[q][e] + wdw);
             acc[e] += step;
             changes += threshold_apply(acc[e], wv[e], t.limit);
         }
         unit[q] = pack4(wv[0], wv[1], wv[2], wv[3]);
         *reinterpret_cast<int *>(t.W + idx) = unit[q];
-        sp[0] = make_float4(s0.x, acc[0], s0.z, acc[1]);
-        sp[1] = make_float4(s1.x, acc[2], s1.z, acc[3]);
+        float4 *sp = reinterpret_cast<float4 *>(t.state + idx * 2);
+        sp[0] = make_float4(s0[q].x, acc[0], s0[q].z, acc[1]);
+        sp[1] = make_float4(s1[q].x, acc[2], s1[q].z, acc[3]);
     }
     *frag_unit(t, ks, g, n) = unit;
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) changes += __shfl_xor(changes, off, 64);
     count_changes(p, changes, sums);
 }
-hipError_t egg_launch_muon_apply(const UpdLaunch &p, float wd, hipStream_t s) {
+hipError_t egg_launch_muon_apply(const UpdLaunch &p, float wd, ptrdiff_t moved, hipStream_t s) {
     if (p.tiles < 1) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_muon_apply, dim3(p.tiles), dim3(256), 0, s, p, wd);
+    hipLaunchKernelGGL(k_muon_apply, dim3(p.tiles), dim3(256), 0, s, p, wd, moved);
     return hipGetLastError();
 }
 
