@@ -468,6 +468,38 @@ __device__ __forceinline__ void dot_noise_ov(const v4i *xop, const float *tab, i
     for (int i = 0; i < NB; i++) sb[i] = sum_halves((int)s[i]);
 }
 
+// ---------------------------------------------------------------- the rank-one term as one more k-step of a product
+// (sb * a) >> sigma, sb = hi * 2^sigma + lo, is hi * a + ((lo * a) >> sigma), and a is one of 31 values (|a| <= 15).  The column side of the k-step
+// holds, for a = r - 15, a one in one of thirty places and a and 8 a in the last place of each half (row r of a table in LDS, the halves 512 bytes apart,
+// from which the columns gather: their neighbours' rows fall on different banks); the token side the thirty values ((lo * v) >> sigma) and the
+// digits of hi = d0 + 8 d1.  All are bytes and the sum is exact: a matrix instruction for 32 columns of a tile instead of two or three vector
+// instructions an element.  A token whose hi does not fit (|d1| > 127: its row follows the noise's signs) has d1 + 8 d2 = hi >> 3, and 8 more
+// k-steps add 8 d2 alone.  egg_rank1_kstep says for which noise this serves.
+__device__ __forceinline__ void fill_rank1_rows(int8_t *rows, int tid, int nthr) {
+    for (int n = tid; n < 1024; n += nthr) {
+        const int half = n >> 9, a = ((n >> 4) & 31) - 15, k = n & 15;
+        rows[n] = (int8_t)(k == 15 ? (half ? 8 * a : a) : a == (half ? -1 - k : k + 1) ? 1 : 0);
+    }
+}
+__device__ __forceinline__ int rank1_row(int a) { return (a + 15) * 16; }            // its place in a half
+// word w of the token's operand: four of the thirty values, or three and a digit
+__device__ __forceinline__ int rank1_word(int w, int s, int sigma, int digit) {
+    int v[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) v[e] = w == 3 && e == 3 ? digit : mul24(s, 4 * w + e + 1) >> sigma;
+    return pack4(v[0], v[1], v[2], v[3]);
+}
+struct Rank1Token { int s, digit, far; bool wide; };        // far: 8 d2 in place (upper half), wide: some token of the wave has one
+__device__ __forceinline__ Rank1Token rank1_token(int sb, int sigma, int g) {
+    const int lo = sb & ((1 << sigma) - 1), hi = sb >> sigma;
+    int d1 = hi >> 3, d2 = 0;
+    Rank1Token t;
+    t.wide = __any(d1 > 127 || d1 < -127);
+    if (t.wide) { d2 = (d1 * 7282) >> 16; d1 -= 8 * d2; }          // a ninth
+    t.s = g ? -lo : lo; t.digit = g ? d1 : (hi & 7); t.far = g ? (int)((unsigned)d2 << 24) : 0;
+    return t;
+}
+
 // ---------------------------------------------------------------- norms on a token held as a packed operand
 // apply_standard_norm (mgpu.cu:646-678) in two parts so that the row sum can be combined across waves:
 // sum of |x| over N column groups (this lane's half only), then the scaling of N groups whose first column is col0.

@@ -42,7 +42,8 @@ struct PlinWS {
     static constexpr int OFF_A = OFF_B + NTAB * K;                // A noise * sign, int32 [wave][NTAB][NW]
     static constexpr int OFF_SB = OFF_A + NTAB * N * 4;           // partial noise dots, int32 [tile parity][wave][32 tokens]
     static constexpr int OFF_STAGE = OFF_SB + 2 * EGG_WAVES * 32 * 4;
-    static constexpr int TOTAL = OFF_STAGE + EGG_WAVES * STAGE;
+    static constexpr int OFF_ROWS = OFF_STAGE + EGG_WAVES * STAGE; // rows of the rank-one k-step
+    static constexpr int TOTAL = OFF_ROWS + 1024;
     static_assert(NW % 32 == 0 && K % 128 == 0 && KS % EGG_WAVES == 0, "shape");
     static_assert(K * NW <= 65536, "a wave's slice of W must fit 256 registers");
     static_assert(SLICES % KS == 0 || KS % SLICES == 0, "slices spread evenly over the k-steps");
@@ -82,12 +83,18 @@ __device__ __forceinline__ void wait_vmcnt_upto(int n) {
 // MODE: 0 = the shared-weight product alone (no rank-1 term), 1 = perturbed, 2 = perturbed with the fused shift,
 // 3 = the shared-weight product alone with int8 results and a shift of exactly 8: the accumulator is clamped where it
 // stands (to [-127 * 256, 127 * 256 + 255]) and the result is its second byte, which the pack's byte permute picks,
-// so the shift costs no instruction
+// so the shift costs no instruction; 4 and 5 = perturbed, with the rank-one term as one more k-step (rank1_token) and the epilogues of 0
+// and 3: a tile's x.B are known in the middle of its own k-loop, so the term joins the accumulators while they are still in the matrix pipe.  Four
+// matrix instructions more a tile and about 45 vector ones for the token's operand, in place of three a result.  8,192 members x 128 tokens x 512 x 512,
+// int8:
+// 347 -> 334 us and, a noise of its own for every member, 329 -> 320; K = 256 218 -> 208 (at the power limit: 2.2 vector instructions a result fewer, of 5.4).
+// int32 results do not gain, 516 -> 522 us, and keep the vector epilogue
 template <int K, int N, bool OUT32, int MODE>
 __global__ void __launch_bounds__(EGG_THREADS, 1) k_plinear_ws(PlinParams p) {
     typedef PlinWS<K, N> P;
-    constexpr bool PLAIN = MODE == 0 || MODE == 3, FUSE = MODE == 2, BYTE1 = MODE == 3;
-    static_assert(!(BYTE1 && OUT32), "the byte-pick form packs int8 results");
+    constexpr bool PLAIN = MODE == 0 || MODE == 3, FUSE = MODE == 2, BYTE1 = MODE == 3 || MODE == 5, RANK = MODE >= 4;
+    constexpr bool BARE = PLAIN || RANK;                          // nothing to add to a finished accumulator
+    static_assert(!((BYTE1 || RANK) && OUT32), "these forms have int8 results");
     constexpr int KS = P::KS, NCT = P::NCT, NW = P::NW, CB = P::CB, NSLOT = P::NSLOT, PF = P::PF, NTAB = P::NTAB;
     constexpr int STORES = OUT32 ? NCT * 4 : NCT;                 // global store instructions per tile and wave
     constexpr int MID = KS / 2;                                   // k-step in front of which the tile's barrier sits
@@ -97,7 +104,9 @@ __global__ void __launch_bounds__(EGG_THREADS, 1) k_plinear_ws(PlinParams p) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, g = lane >> 5, j = lane & 31;
     int8_t *Btab = smem + P::OFF_B;
     int *Atab = reinterpret_cast<int *>(smem + P::OFF_A) + wave * NTAB * NW;
+    uint16_t *Rtab = reinterpret_cast<uint16_t *>(Atab);           // RANK: rank1_row of A instead, in the order of the W fragments' rows
     int *sbx = reinterpret_cast<int *>(smem + P::OFF_SB);          // [tile parity][token][wave]
+    if (RANK) fill_rank1_rows(smem + P::OFF_ROWS, threadIdx.x, EGG_THREADS);
     int8_t *stage = smem + P::OFF_STAGE + wave * P::STAGE;
 
     // Workgroup b takes members b, b + grid, b + 2 grid, ...: at any time the workgroups of the grid read and write one
@@ -193,7 +202,12 @@ __global__ void __launch_bounds__(EGG_THREADS, 1) k_plinear_ws(PlinParams p) {
         const int set = (member / grid) % NTAB;            // consecutive members of this workgroup rotate through the sets
         const int ns = (!p.own_noise && (member & 1)) ? -1 : 1;
         const uint32_t ps = p.seed + (uint32_t)(p.own_noise ? member : member / 2);
-        for (int i = lane; i < NW; i += 64) Atab[set * NW + i] = noise_from_hash(ps + p.off_a, wave * NW + i, p.mask) * ns;
+        for (int i = lane; i < NW; i += 64) {
+            if (RANK) {
+                const int r = i & 31, col = (i & ~31) + 16 * ((r >> 2) & 1) + 4 * (r >> 3) + (r & 3);
+                Rtab[set * NW + i] = (uint16_t)rank1_row(noise_from_hash(ps + p.off_a, wave * NW + col, p.mask) * ns);
+            } else Atab[set * NW + i] = noise_from_hash(ps + p.off_a, wave * NW + i, p.mask) * ns;
+        }
         for (int i = lane; i < K / EGG_WAVES; i += 64)
             Btab[set * K + wave * (K / EGG_WAVES) + i] = (int8_t)noise_from_hash(ps + p.off_b, wave * (K / EGG_WAVES) + i, p.mask);
     };
@@ -216,7 +230,7 @@ __global__ void __launch_bounds__(EGG_THREADS, 1) k_plinear_ws(PlinParams p) {
     // its fourth slice.
     auto ep_value = [&](int accv, int a, int sbv) -> int {
         if (BYTE1) return min(127 * 256 + 255, max(-127 * 256, accv));
-        const int o = PLAIN ? (accv >> p.shift) : ws_perturbed<FUSE>(accv, sbv, a, p.sigma, p.shift);
+        const int o = BARE ? (accv >> p.shift) : ws_perturbed<FUSE>(accv, sbv, a, p.sigma, p.shift);
         return OUT32 ? o : clip127(o);
     };
     int o8[4];                                   // int8: the packed results of the slices of one column tile
@@ -247,7 +261,7 @@ __global__ void __launch_bounds__(EGG_THREADS, 1) k_plinear_ws(PlinParams p) {
     auto ep_slice = [&](v16i (&acc)[NCT], int s, const int *Aset, int sbv, size_t row0) {
         const int ct = s >> 2, q = s & 3;
         v4i a4 = {0, 0, 0, 0};
-        if (!PLAIN) a4 = *reinterpret_cast<const v4i *>(Aset + 32 * ct + 16 * g + 4 * q);
+        if (!BARE) a4 = *reinterpret_cast<const v4i *>(Aset + 32 * ct + 16 * g + 4 * q);
         int o[4];
 #pragma unroll
         for (int e = 0; e < 4; e++) o[e] = ep_value(acc[ct][4 * q + e], a4[e], sbv);
@@ -265,7 +279,7 @@ __global__ void __launch_bounds__(EGG_THREADS, 1) k_plinear_ws(PlinParams p) {
         // for t = 0 the epilogue processes zeros and stores them to tile 0's rows, which the real epilogue of tile 0
         // overwrites later from the same wave
         const size_t prow0 = row_prev;
-        const int *Aprev = Atab + (PLAIN ? 0 : ((m_prev / grid) % NTAB) * NW);
+        const int *Aprev = Atab + (BARE ? 0 : ((m_prev / grid) % NTAB) * NW);
         const int8_t *Bcur = Btab + (PLAIN ? 0 : ((m_cur / grid) % NTAB) * K);
         int sbp = 0, sb_next = 0;
         constexpr int SPK = P::SLICES >= KS ? P::SLICES / KS : 1;           // epilogue slices per k-step
@@ -275,7 +289,7 @@ __global__ void __launch_bounds__(EGG_THREADS, 1) k_plinear_ws(PlinParams p) {
         for (int si = 0; si < SPK; si++) pre_a[si] = v4i{0, 0, 0, 0};
         auto load_small = [&](int ks) {          // A noise of the slices finished in k-step ks; fragment and B noise of the x.B share
             if (ks >= KS) return;
-            if (!PLAIN && ks % KPS == 0) {
+            if (!BARE && ks % KPS == 0) {
 #pragma unroll
                 for (int si = 0; si < SPK; si++) {
                     const int sl = (ks / KPS) * SPK + si;
@@ -288,6 +302,12 @@ __global__ void __launch_bounds__(EGG_THREADS, 1) k_plinear_ws(PlinParams p) {
             }
         };
         load_small(0);
+        // RANK: the token's operand is put together behind the matrix instructions of the k-steps that follow the exchange of x.B
+        const uint16_t *Rcur = Rtab + (RANK ? ((m_cur / grid) % NTAB) * NW : 0);
+        constexpr int WPK = 4 / (KS - MID - 2 < 4 ? KS - MID - 2 : 4);       // words of it per k-step
+        Rank1Token tk = {0, 0, 0, false};
+        v4i tok = {0, 0, 0, 0}, rows[NCT];
+        int at[NCT];
 #pragma unroll
         for (int ks = 0; ks < KS; ks++) {
             if (ks == MID) {
@@ -359,6 +379,16 @@ __global__ void __launch_bounds__(EGG_THREADS, 1) k_plinear_ws(PlinParams p) {
                     }
                 }
                 if (!PLAIN && ks < QS) sbp = dot4(xs[ct & 3], b4[ct & 3], sbp);
+                if (RANK) {
+                    if (ks == MID + 1 && ct == 1)
+#pragma unroll
+                        for (int c = 0; c < NCT; c++) at[c] = Rcur[32 * c + j];
+                    if (ks == MID + 2 && ct == 0) tk = rank1_token(sb_next, p.sigma, g);
+                    if (ks >= MID + 2 && ct < WPK && (ks - MID - 2) * WPK + ct < 4) tok[((ks - MID - 2) * WPK + ct) & 3] = rank1_word((ks - MID - 2) * WPK + ct, tk.s, p.sigma, tk.digit);
+                    if (ks == KS - 1 && ct == 0)
+#pragma unroll
+                        for (int c = 0; c < NCT; c++) rows[c] = *reinterpret_cast<const v4i *>(smem + P::OFF_ROWS + at[c] + g * 512);
+                }
                 if (ct == NCT - 1) {
                     if (ep_here) {
 #pragma unroll
@@ -376,6 +406,17 @@ __global__ void __launch_bounds__(EGG_THREADS, 1) k_plinear_ws(PlinParams p) {
                     }
                 }
                 __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        if (RANK) {
+#pragma unroll
+            for (int ct = 0; ct < NCT; ct++) cur[ct] = __builtin_amdgcn_mfma_i32_32x32x32_i8(rows[ct], tok, cur[ct], 0, 0, 0);
+            if (__builtin_expect(tk.wide, 0)) {
+                const v4i far = {0, 0, 0, tk.far};
+#pragma unroll 1
+                for (int x = 0; x < 8; x++)
+#pragma unroll
+                    for (int ct = 0; ct < NCT; ct++) cur[ct] = __builtin_amdgcn_mfma_i32_32x32x32_i8(rows[ct], far, cur[ct], 0, 0, 0);
             }
         }
         sb_prev = sb_next;
@@ -397,7 +438,7 @@ __global__ void __launch_bounds__(EGG_THREADS, 1) k_plinear_ws(PlinParams p) {
     // after the last step (m_prev, row_prev) is the last tile
     if (t < n_local) step(accA, accB, t);
     const size_t lrow0 = row_prev;
-    const int *Alast = Atab + (PLAIN ? 0 : ((m_prev / grid) % NTAB) * NW);
+    const int *Alast = Atab + (BARE ? 0 : ((m_prev / grid) % NTAB) * NW);
     if (t < n_local) {
 #pragma unroll
         for (int s = 0; s < P::SLICES; s++) ep_slice(accA, s, Alast, sb_prev, lrow0);
@@ -431,11 +472,15 @@ static hipError_t launch_ws_kn(const PlinParams &p, hipStream_t s) {
     const long long mag = egg_noise_magnitude(p.mask);
     const long long bound = ((long long)K * 128 * 128 << p.sigma) + (long long)K * 128 * mag * mag;
     const bool fuse = p.sigma >= 0 && p.sigma <= 12 && p.sigma + p.shift < 32 && bound < (1LL << 31);
-    const int mode = p.plain ? 0 : (fuse ? 2 : 1);
+    // int8 results: the k-step form where the noise and its sums fit it, else the vector epilogue
+    const bool rank = !p.plain && egg_rank1_kstep(K, p.mask, p.sigma);
+    const int mode = p.plain ? 0 : fuse ? 2 : 1;
+    const bool byte1 = p.shift == 8;
     hipError_t e = hipSuccess;
-    if (p.Y32) e = mode == 0 ? launch_ws<K, N, true, 0>(p, s) : (mode == 1 ? launch_ws<K, N, true, 1>(p, s) : launch_ws<K, N, true, 2>(p, s));
-    if (e == hipSuccess && p.Y8) e = mode == 0 ? (p.shift == 8 ? launch_ws<K, N, false, 3>(p, s) : launch_ws<K, N, false, 0>(p, s))
-                                               : (mode == 1 ? launch_ws<K, N, false, 1>(p, s) : launch_ws<K, N, false, 2>(p, s));
+    if (p.Y32) e = mode == 0 ? launch_ws<K, N, true, 0>(p, s) : mode == 1 ? launch_ws<K, N, true, 1>(p, s) : launch_ws<K, N, true, 2>(p, s);
+    if (e == hipSuccess && p.Y8) e = mode == 0 ? (byte1 ? launch_ws<K, N, false, 3>(p, s) : launch_ws<K, N, false, 0>(p, s))
+                                   : rank ? (byte1 ? launch_ws<K, N, false, 5>(p, s) : launch_ws<K, N, false, 4>(p, s))
+                                   : mode == 1 ? launch_ws<K, N, false, 1>(p, s) : launch_ws<K, N, false, 2>(p, s);
     return e;
 }
 // shapes the W-stationary kernel is built for

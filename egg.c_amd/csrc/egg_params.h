@@ -56,6 +56,13 @@ static inline void egg_rank1_shifts(int mask, int sigma, int *sb_shift, int *a_s
     *sb_shift = t; *a_shift = 32 - sigma - t;
 }
 
+// The rank-one term as one more k-step of the product (rank1_token): 31 noise values, lo * 15 in 24 bits, and a sum whose
+// high part fits the digits: with its ninth in d2, |d1| and |d2| stay below 128 up to |hi| >> 3 of 1,000.
+static inline bool egg_rank1_kstep(int depth, int mask, int sigma) {
+    const long long mag = egg_noise_magnitude(mask);
+    return mag <= 15 && sigma <= 16 && ((long long)depth * 128 * mag >> sigma) < 8 * 1000;
+}
+
 // what every forward kernel needs to know about the run
 struct FwdCommon {
     const uint8_t  *data;        // token stream (device): bytes, or uint32 tokens when token_bytes is 4
