@@ -23,8 +23,11 @@
 //
 // A, E, D, head: a workgroup of eight waves takes 8 members; a wave has 32 tokens of one member as the columns of
 // v_mfma_i32_32x32x32_i8 (one member: its noise vectors are wave-uniform), the weights go by in blocks of 64 output columns
-// through two LDS buffers that all eight waves read.  (At hidden 512 D reloads 9 registers from scratch for each block of 64
-// columns and 128 MFMAs; the recurrence and the other stages use none.)
+// through four LDS buffers that all eight waves read.
+//
+// A tick at hidden 512, 4 layers, 128 members (272 workgroups): R 90 us (the weights 15, 32 tokens of 2.3), E 71, D 61, A 45, the head 22 behind an A.
+// D was 106 and the tick's length: its input row came from memory once for every 64 output columns, and every stage's wait for a
+// small load of a block took the copy that had just been requested along.
 #include "egg_gru.h"
 
 #pragma clang fp contract(off)
@@ -91,13 +94,22 @@ __device__ __forceinline__ void stage_rec(const PipeParams &p, int l, int tile, 
     }
     const PipeMat m1 = p.m[6 * l + 1], m3 = p.m[6 * l + 3];
     v4i w1[4][KS], w3[4][KS];
+    // (straight to LDS what stays there: through registers the loads behind it waited for those stores.  Inline assembly for the reason given at
+    // dma_unit, egg_device.h; waited for in front of the token loop)
+    const uint32_t w3_lds = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(size_t)(const __attribute__((address_space(3))) int8_t *)lds) + wave * 18 * 1024;
+#pragma unroll
+    for (int s = 0; s < 4; s++)
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++)
+            if (R::in_lds(s, ks))
+                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                             : : "s"(w3_lds + R::lds_slot(s, ks) * 1024), "v"((uint32_t)lane * 16), "s"(p.frag + m3.w_off + ((4 * wave + s) * (uint32_t)KS + ks) * 1024u) : "memory", "m0");
 #pragma unroll
     for (int s = 0; s < 4; s++)
 #pragma unroll
         for (int ks = 0; ks < KS; ks++) {
             w1[s][ks] = rec_frag(p.frag + m1.w_off, 4 * wave + s, ks, KS, lane);
             if (!R::in_lds(s, ks)) w3[s][ks] = rec_frag(p.frag + m3.w_off, 4 * wave + s, ks, KS, lane);
-            else *reinterpret_cast<v4i *>(w3l + R::lds_slot(s, ks) * 1024) = rec_frag(p.frag + m3.w_off, 4 * wave + s, ks, KS, lane);
         }
     const uint32_t at = 64 * wave + 16 * g + (second ? 8 : 0);          // this lane's 8 bytes of a row: strips 0 and 2, or 1 and 3
     const long long pair = (p.first + local) >> 1;
@@ -210,27 +222,32 @@ __device__ __forceinline__ void fetch_block(int8_t *dst, const int8_t *src) {
     else asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\tglobal_load_lds_dwordx4 %1, %2 offset:1024\n\t"
                       "global_load_lds_dwordx4 %1, %2 offset:2048\n\tglobal_load_lds_dwordx4 %1, %2 offset:3072" : : "s"(m0v), "v"(v), "s"(sb) : "memory", "m0");
 }
-// the blocks of one or two matrices in turn, double buffered
+// The blocks of one or two matrices in turn, through a ring of four buffers: a block is requested three blocks ahead of its use.  A wave
+// waits for its own part of the oldest by counting the younger copies, so a request follows every take (past the end the last
+// block again, which no one reads), and other loads and stores in flight make the wait longer, never shorter.  The caller puts a
+// block's small loads in front of `request`: loads return in order, and the compiler, which does not see the copies, waits for
+// everything behind the last load that it knows of.
 template <int H>
 struct Blocks {
-    int8_t *fill, *other;
-    const int8_t *a, *b; int na, n, next;          // blocks 0 .. na - 1 at a, na .. n - 1 at b
+    static constexpr int BUFS = 4, SIZE = 64 * H, PER = H >= 128 ? H / 128 : 1;
+    int8_t *base;
+    const int8_t *a, *b; int na, n, next, used;    // blocks 0 .. na - 1 at a, na .. n - 1 at b
     __device__ __forceinline__ void begin(int8_t *lds, const int8_t *first, int n_first, const int8_t *second, int n_second) {
-        fill = lds; other = lds + 64 * H; a = first; b = second; na = n_first; n = n_first + n_second; next = 0;
-        request();
+        base = lds; a = first; b = second; na = n_first; n = n_first + n_second; next = used = 0;
     }
-    __device__ __forceinline__ void request() {
-        if (next < n) fetch_block<H>(fill, next < na ? a + (size_t)next * 64 * H : b + (size_t)(next - na) * 64 * H);
+    __device__ __forceinline__ void request(int i) {        // i: the block's place in its matrix
+        fetch_block<H>(base + (next & (BUFS - 1)) * SIZE, i < na ? a + (size_t)i * SIZE : b + (size_t)(i - na) * SIZE);
         next++;
     }
+    __device__ __forceinline__ void request() { request(min(next, n - 1)); }
     __device__ __forceinline__ const int8_t *take() {
-        __builtin_amdgcn_s_waitcnt(0x0F70);        // vmcnt(0)
+        static_assert((BUFS - 2) * PER < 16, "the wait's low field");
+        __builtin_amdgcn_s_waitcnt(0x0F70 | ((BUFS - 2) * PER));
         __syncthreads();
-        const int8_t *got = fill;
-        fill = other; other = const_cast<int8_t *>(got);
-        request();
-        return got;
+        return base + (used++ & (BUFS - 1)) * SIZE;
     }
+    // the copies that no one reads: a workgroup's LDS must not be written behind its end
+    __device__ __forceinline__ void drain() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 };
 template <int NK>
 __device__ __forceinline__ void multiply(v16i (&acc)[2], const v4i (&x)[NK], const int8_t *block, int lane) {
@@ -240,6 +257,18 @@ __device__ __forceinline__ void multiply(v16i (&acc)[2], const v4i (&x)[NK], con
         const v4i f0 = *reinterpret_cast<const v4i *>(f), f1 = *reinterpret_cast<const v4i *>(f + 512);
         acc[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(f0, x[ks], acc[0], 0, 0, 0);
         acc[1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(f1, x[ks], acc[1], 0, 0, 0);
+    }
+}
+// the same, and each k-step's operand gives way to the one at `ops` (load_ops) when it has been multiplied
+template <int NK>
+__device__ __forceinline__ void multiply_reload(v16i (&acc)[2], v4i (&x)[NK], const int8_t *block, const int8_t *ops, int lane) {
+#pragma unroll
+    for (int ks = 0; ks < NK; ks++) {
+        const int8_t *f = block + ((2 * ks + (lane >> 5)) * 64 + (lane & 31)) * 16;
+        const v4i f0 = *reinterpret_cast<const v4i *>(f), f1 = *reinterpret_cast<const v4i *>(f + 512);
+        acc[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(f0, x[ks], acc[0], 0, 0, 0);
+        acc[1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(f1, x[ks], acc[1], 0, 0, 0);
+        x[ks] = *reinterpret_cast<const v4i *>(ops + 1024 * ks + (uint32_t)lane * 16);
     }
 }
 template <int NK>
@@ -355,16 +384,21 @@ __device__ __forceinline__ void stage_a(const PipeParams &p, int l, int unit8, i
     norm<NK>(x, row_gain(p, H, l, 0), t.g);
     const int xb0 = t.ns * sum_halves(noise_dot<NK>(x, p.noise_pipe + m0.b_off + t.pair * H, t.g)),
               xb2 = t.ns * sum_halves(noise_dot<NK>(x, p.noise_pipe + m2.b_off + t.pair * H, t.g));
+    auto noise_of = [&](int b) { return p.noise_slot + (b >= NB ? m2.a_off : m0.a_off) + t.pair * H + 64 * (b >= NB ? b - NB : b) + 16 * t.g; };
+    v4i a0 = ld16(noise_of(0)), a1 = ld16(noise_of(0) + 32);
+    for (int i = 0; i < 3; i++) blocks.request();
     for (int b = 0; b < 2 * NB; b++) {
         const int which = b >= NB, nb = which ? b - NB : b;
-        const int8_t *a = p.noise_slot + (which ? m2.a_off : m0.a_off) + t.pair * H + 64 * nb + 16 * t.g;
-        const v4i a0 = ld16(a), a1 = ld16(a + 32);
         const int8_t *w = blocks.take();
         v16i acc[2];
         begin_block(acc, which ? xb2 : xb0, a0, a1, p.sigma);
+        const int8_t *a = noise_of(min(b + 1, 2 * NB - 1));
+        a0 = ld16(a); a1 = ld16(a + 32);
+        blocks.request();
         multiply<NK>(acc, x, w, t.lane);
         store_pieces(buf_g(p, H, l, which, chunk) + row + 64 * nb, finish_block(acc, 8), t.g);
     }
+    blocks.drain();
 }
 template <int H>
 __device__ __forceinline__ void stage_e(const PipeParams &p, int l, int unit8, int chunk, int8_t *lds) {
@@ -381,11 +415,16 @@ __device__ __forceinline__ void stage_e(const PipeParams &p, int l, int unit8, i
     const int8_t *a = p.noise_slot + m.a_off + t.pair * 4 * H + 16 * t.g, *bd = p.noise_pipe + p.m[6 * l + 5].b_off + t.pair * 4 * H + 16 * t.g;
     int8_t *out = buf_m(p, H, l, chunk) + (size_t)t.local * C * 4 * H + t.lane * 16;
     int xbd = 0;                                   // the projection's x . B, of the results as they leave
+    v4i a0 = ld16(a), a1 = ld16(a + 32), nn0 = ld16(bd), nn1 = ld16(bd + 32);
+    for (int i = 0; i < 3; i++) blocks.request();
     for (int b = 0; b < NB; b++) {
-        const v4i a0 = ld16(a + 64 * b), a1 = ld16(a + 64 * b + 32), n0 = ld16(bd + 64 * b), n1 = ld16(bd + 64 * b + 32);
         const int8_t *w = blocks.take();
         v16i acc[2];
         begin_block(acc, xb, a0, a1, p.sigma);
+        const v4i n0 = nn0, n1 = nn1;
+        const int ahead = 64 * min(b + 1, NB - 1);
+        a0 = ld16(a + ahead); a1 = ld16(a + ahead + 32); nn0 = ld16(bd + ahead); nn1 = ld16(bd + ahead + 32);
+        blocks.request();
         multiply<NK>(acc, x, w, t.lane);
         const Pieces o = finish_block(acc, 8);
 #pragma unroll
@@ -395,6 +434,7 @@ __device__ __forceinline__ void stage_e(const PipeParams &p, int l, int unit8, i
     }
     xbd = t.ns * sum_halves(xbd);
     if (t.g == 0) buf_xb(p, H, l, chunk)[row] = xbd;
+    blocks.drain();
 }
 template <int H>
 __device__ __forceinline__ void stage_d(const PipeParams &p, int l, int unit8, int chunk, int8_t *lds) {
@@ -409,27 +449,37 @@ __device__ __forceinline__ void stage_d(const PipeParams &p, int l, int unit8, i
                  *a = p.noise_slot + m.a_off + t.pair * H + 16 * t.g;
     int8_t *out = buf_x(p, H, l + 1, chunk) + row * H;
     const int xb = buf_xb(p, H, l, chunk)[row];
-    // a quarter of the input row at a time, the next one on its way while a block of weights is multiplied with this one
-    v4i x0[NK], x1[NK];
-    load_ops<NK>(x0, in, lane16);
-    for (int b = 0; b < NB; b++) {
-        const v4i a0 = ld16(a + 64 * b), a1 = ld16(a + 64 * b + 32), r0 = ld16(res + 64 * b), r1 = ld16(res + 64 * b + 32);
-        v16i acc[2];
-        begin_block(acc, xb, a0, a1, p.sigma);
+    // NBP blocks of 64 columns at a time, for which the input row goes by in quarters (with one block at a time it came from memory eight
+    // times, four times the weights' bytes); the next quarter replaces this one as the last block's products leave it.
+    constexpr int NBP = NB < 4 ? NB : 4;
+    auto place = [&](int n) { n = min(n, 4 * NB - 1); const int part = n / (4 * NBP), kc = n / NBP % 4, j = n % NBP; return (part * NBP + j) * 4 + kc; };
+    v4i x[NK];
+    load_ops<NK>(x, in, lane16);
+    for (int i = 0; i < 3; i++) blocks.request(place(i));
+#pragma unroll 1
+    for (int part = 0; part < NB / NBP; part++) {
+        v16i acc[NBP][2];
 #pragma unroll
-        for (int kc = 0; kc < 4; kc += 2) {
-            const int8_t *w = blocks.take();
-            load_ops<NK>(x1, in + (kc + 1) * NK * 1024, lane16);
-            multiply<NK>(acc, x0, w, t.lane);
-            w = blocks.take();
-            load_ops<NK>(x0, in + ((kc + 2) & 3) * NK * 1024, lane16);
-            multiply<NK>(acc, x1, w, t.lane);
+        for (int j = 0; j < NBP; j++) begin_block(acc[j], xb, ld16(a + 64 * (part * NBP + j)), ld16(a + 64 * (part * NBP + j) + 32), p.sigma);
+#pragma unroll 1
+        for (int kc = 0; kc < 4; kc++)
+#pragma unroll
+            for (int j = 0; j < NBP; j++) {
+                const int8_t *w = blocks.take();
+                blocks.request(place(blocks.next));
+                if (j + 1 < NBP) multiply<NK>(acc[j], x, w, t.lane);
+                else multiply_reload<NK>(acc[j], x, w, in + ((kc + 1) & 3) * NK * 1024, t.lane);
+            }
+#pragma unroll
+        for (int j = 0; j < NBP; j++) {
+            const int at = 64 * (part * NBP + j);
+            Pieces o = finish_block(acc[j], 9);
+            o.lo = cadd16(o.lo, ld16(res + at));
+            o.hi = cadd16(o.hi, ld16(res + at + 32));
+            store_pieces(out + at, o, t.g);
         }
-        Pieces o = finish_block(acc, 9);
-        o.lo = cadd16(o.lo, r0);
-        o.hi = cadd16(o.hi, r1);
-        store_pieces(out + 64 * b, o, t.g);
     }
+    blocks.drain();
 }
 // output norm, logits (egg.c:288-294), loss (egg.c:321-330)
 template <int H>
@@ -439,7 +489,7 @@ __device__ __forceinline__ void stage_head(const PipeParams &p, int unit8, int c
     const PipeMat m = p.m[6 * p.L];
     Blocks<H> blocks;
     blocks.begin(lds, p.frag + m.w_off, p.V / 64, nullptr, 0);
-    int *exp2 = reinterpret_cast<int *>(lds + 2 * 64 * H);
+    int *exp2 = reinterpret_cast<int *>(lds + Blocks<H>::BUFS * 64 * H);
     if (threadIdx.x < 256) exp2[threadIdx.x] = p.exp2[threadIdx.x];            // the first take() synchronises
     v4i x[NK];
     load_row<NK>(x, buf_x(p, H, p.L, chunk) + ((size_t)t.local * C + (t.lane & 31)) * H, t.g);
@@ -448,11 +498,15 @@ __device__ __forceinline__ void stage_head(const PipeParams &p, int unit8, int c
     const int8_t *a = p.noise_slot + m.a_off + t.pair * p.V + 16 * t.g;
     const int target = p.data[stream_pos(p, t.member) + t.token + 1];
     int sum_exp = 0, tl = 0;
+    v4i a0 = ld16(a), a1 = ld16(a + 32);
+    for (int i = 0; i < 3; i++) blocks.request();
     for (int b = 0; b < p.V / 64; b++) {
-        const v4i a0 = ld16(a + 64 * b), a1 = ld16(a + 64 * b + 32);
         const int8_t *w = blocks.take();
         v16i acc[2];
         begin_block(acc, xb, a0, a1, p.sigma);
+        const int ahead = 64 * min(b + 1, p.V / 64 - 1);
+        a0 = ld16(a + ahead); a1 = ld16(a + ahead + 32);
+        blocks.request();
         multiply<NK>(acc, x, w, t.lane);
 #pragma unroll
         for (int half = 0; half < 2; half++) {
@@ -467,6 +521,7 @@ __device__ __forceinline__ void stage_head(const PipeParams &p, int unit8, int c
                 }
         }
     }
+    blocks.drain();
     sum_exp = sum_halves(sum_exp); tl = sum_halves(tl);
     int lg2 = 0;                                   // log2_fixed (egg.c:309-319)
     if (sum_exp > 0) {
@@ -483,14 +538,17 @@ __device__ __forceinline__ void stage_head(const PipeParams &p, int unit8, int c
 template <int H>
 __global__ void __launch_bounds__(THREADS, 2) k_gru_tick(PipeParams p, int tick, int chunks) {
     extern __shared__ __align__(16) int8_t lds[];
-    const int n = p.members / 8, role = (int)blockIdx.x / (p.L * n), i = (int)blockIdx.x % (p.L * n), l = i / n, u = i % n;
+    // Workgroups go to the eight XCDs in turn; those of one XCD take consecutive units of a role, so that the tiles of a layer meet in one
+    // or two L2s and its weights (3 MB at hidden 512) stay there.
+    const int n = p.members / 8, units = p.L * n, role = (int)blockIdx.x / units, at = (int)blockIdx.x % units;
+    const int i = units & 7 ? at : (at & 7) * (units >> 3) + (at >> 3), l = i / n, u = i % n;
     auto chunk_at = [&](int layer, int stage) { const int c = tick - 4 * layer - stage; return c >= 0 && c < chunks ? c : -1; };
     int c;
     if (role == 0) { if ((c = chunk_at(l, 1)) >= 0) stage_rec<H>(p, l, u, c, lds); }
     else if (role == 1) { if ((c = chunk_at(l, 2)) >= 0) stage_e<H>(p, l, u, c, lds); }
     else if (role == 2) { if ((c = chunk_at(l, 3)) >= 0) stage_d<H>(p, l, u, c, lds); }
     else if (role == 3) { if ((c = chunk_at(l, 0)) >= 0) stage_a<H>(p, l, u, c, lds); }
-    else if ((c = chunk_at(p.L, 0)) >= 0) stage_head<H>(p, i, c, lds);
+    else if ((c = chunk_at(p.L, 0)) >= 0) stage_head<H>(p, at, c, lds);
 }
 
 // the state between its natural order, [member][L][H], and the pipe order of the ticks, [L][member][H]; zero losses
@@ -530,7 +588,7 @@ __global__ void k_gru_rows(const int8_t *model, int8_t *rows, int H, int L, int 
 }
 
 template <int H>
-constexpr int tick_lds() { return Rec<H>::LDS > 2 * 64 * H + 1024 ? Rec<H>::LDS : 2 * 64 * H + 1024; }
+constexpr int tick_lds() { return Rec<H>::LDS > Blocks<H>::BUFS * 64 * H + 1024 ? Rec<H>::LDS : Blocks<H>::BUFS * 64 * H + 1024; }
 template <int H>
 hipError_t forward(const PipeParams &p, hipStream_t s) {
     const int chunks = (p.T + C - 1) / C, n = p.members / 8, items = std::max(p.members, p.L * p.members * (H / 4));
