@@ -10,12 +10,19 @@
 // of the exchange, written and polled with device-scope accesses, so the data is its own arrival flag and an exchange costs
 // one store-to-load trip (0.6 us on one XCD, 1.0 us across them) instead of a launch.  Everything every workgroup needs
 // whole -- the residual row, the norms -- each computes for itself.  The weights of a stage are requested in front of the
-// wait for its input.  Measured: 97 and 47 us a token at the two sizes for one continuation on its own (64 tokens behind
-// a prompt of 32: 7.0 and 3.1 ms); contexts that generate at the same time share the chip, three of them finish one each 2.7 and
-// 1.1 ms.  An exchange takes 0.8 to 1.5 us with the waits for the slowest workgroup, the short dependent computations between
-// two of them 0.3 to 1 us.  All workgroups on one XCD
-// were 5 % faster at hidden 256 and 8 % slower at 512 (the weights do not fit its L2), and several such launches would
-// share that XCD.
+// wait for its input.
+//
+// An exchange takes 1.2 to 2.2 us with the waits for the slowest workgroup, the short dependent computations between
+// two of them 0.3 to 1.5 us, so their number counts.  Gathered, the attention's output and the MLP's intermediate are two exchanges a
+// layer, and what the product of each gives are two more.  Up to hidden 256 a workgroup multiplies its own strip of them with the rows
+// of the next matrix instead and the partial sums are exchanged (`Rows`): three exchanges a layer in place of five.
+// Measured, 64 tokens behind a prompt of 32, alone and with three contexts that generate at the same time (one each
+// finishes), five exchanges -> three: hidden 64, 2 layers 1.57 / 0.57 -> 1.22 / 0.43 ms; hidden 128, 4 layers 3.04 / 1.03 -> 2.29 / 0.78;
+// hidden 256, 4 layers 2.95 / 1.06 -> 2.66 / 0.96; hidden 256, 8 layers, vocabulary 8192 5.65 / 2.10 -> 5.09 / 1.89.  Each workgroup reads H * H / 4
+// bytes of messages for it, 16 KB at hidden 256 and 64 KB at 512, where such an exchange takes 2.5 to 3.2 us and the
+// two-column messages 350 registers: 7.02 -> 7.24 ms alone, so hidden 512 gathers (97 us a token).
+// All workgroups on one XCD were 5 % faster at hidden 256 and 8 % slower at 512 (the weights do not fit its L2), and several such
+// launches would share that XCD.
 //
 // A message slot is written again one exchange of the same kind later.  Every workgroup sends in every exchange of a layer
 // and takes in all it needs of an exchange before it sends in the next, so a slot is only written again when its last
@@ -102,6 +109,7 @@ struct Lds {
     int w[512];                                // attention weights
     int pv[64 * 17];                           // by group of positions: the strip's 16 weighted sums and the sum of the weights
     __align__(16) int8_t qs[64], ks[64], vs[16];      // the head's new query and key, the strip's new value
+    __align__(16) int8_t own[64];                     // the strip's attention output, its columns of the MLP's intermediate
     int lut[256]; int8_t act[256];
     long long tsum[64];
     int tok[512];                              // the sequence
@@ -119,7 +127,9 @@ struct Strip {
     __device__ __forceinline__ void load(int t, const int8_t *frag, int cols, int col) {
         const uint32_t wave = threadIdx.x >> 6, pl = (threadIdx.x >> 4) & 3, n = (uint32_t)col + (threadIdx.x & 15);
         // a uniform base and 32-bit offsets: no 64-bit address arithmetic, no address registers
-        const uint32_t at = n / B * (B * B) + n % B * 16;
+        uint32_t at = n / B * (B * B) + n % B * 16;
+        // computed here and not ahead of the loop over the layers, where the offsets of all loads take registers that the sums need
+        if constexpr (egg_decode_sums(K)) asm volatile("" : "+v"(at));
 #pragma unroll
         for (int i = 0; i < IT; i++) {
             const uint32_t p = 16 * i + 4 * wave + pl;
@@ -200,6 +210,81 @@ __device__ __forceinline__ bool take_residual(Lds &s, const u64 *slots, uint32_t
         if (tid < H) s.x[tid + 256 * i] = (int8_t)x[i];
     }
     return !s.dead;
+}
+
+// ---- products of a strip of rows, up to hidden 256: workgroup w multiplies its own R values (of the attention's output, of the MLP's
+// intermediate) with the R rows of the next matrix that belong to them, which lie together in the canonical blocked weights, and sends
+// the partial sums of every column; a receiver adds up the H / 16 of them.  They are exact integers, so the sums are
+// what a product of the gathered row gives, and the row itself is never exchanged.
+// A message holds two columns' sums of 21 bits (64 * 127 * 128 < 2^20) and 22 bits of the exchange's number: what a slot held before
+// is the exchange in front, so far fewer would tell them apart.
+constexpr uint32_t TAG22 = (1u << 22) - 1u;
+template <int H, int R>
+struct Rows {
+    static constexpr int D = R / 8;             // a thread's column pair and its half of the rows: the other half is 32 lanes away
+    int2 w[D];
+    static __device__ __forceinline__ int pair() { return (int)((threadIdx.x >> 6) * 32 + (threadIdx.x & 31)); }
+    static __device__ __forceinline__ int half() { return (int)((threadIdx.x >> 5) & 1); }
+    __device__ __forceinline__ void load(const int8_t *W, int row0) {           // W: uniform
+        if (pair() >= H / 2) return;
+        uint32_t at = half() * (D * H * 4) + 8 * pair();
+        asm volatile("" : "+v"(at));
+        W += (uint32_t)(row0 >> 2) * H * 4u;
+#pragma unroll
+        for (int i = 0; i < D; i++) w[i] = *reinterpret_cast<const int2 *>(W + (at + i * H * 4u));
+    }
+    __device__ __forceinline__ void send_sums(const int8_t *values, u64 *slots, int wg, uint32_t tag) const {
+        int a = 0, b = 0;
+        if (pair() < H / 2) {
+#pragma unroll
+            for (int i = 0; i < D; i++) {
+                const int v = *reinterpret_cast<const int *>(values + 4 * (half() * D + i));
+                a = dot4(w[i].x, v, a); b = dot4(w[i].y, v, b);
+            }
+        }
+        a = half_reduce<false>(a); b = half_reduce<false>(b);
+        if (pair() < H / 2 && half() == 0)
+            __hip_atomic_store(slots + (uint32_t)(wg * (H / 2) + pair()), ((u64)(tag & TAG22) << 42) | ((u64)((uint32_t)b & 0x1fffffu) << 21) | ((uint32_t)a & 0x1fffffu),
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+};
+// x + (sum >> shift) + bias of an exchange of partial sums, then the adaptive norm (egg_adaptive_normalize.h:10-103) -> new residual row
+// Thread k has column k; it takes half of the messages of its pair of columns, its neighbour the other half.
+template <int H>
+__device__ __forceinline__ bool take_sums(Lds &s, const u64 *slots, uint32_t tag, int shift, int bias, int &x, int limit) {
+    constexpr int M = H / 32;
+    const int tid = threadIdx.x;
+    int v = 0;
+    if (tid < H) {
+        bool all = false;
+        int lo = 0, hi = 0;
+        const u64 *from = slots + ((tid >> 1) + (tid & 1) * (M * (H / 2)));
+        asm volatile("" : "+v"(from));           // one address and offsets: M addresses for each exchange would be kept over the layers
+        for (int polls = 0; polls < limit && !all; polls++) {
+            u64 m[M];
+#pragma unroll
+            for (int g = 0; g < M; g++) m[g] = __hip_atomic_load(from + g * (H / 2), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            all = true;
+            lo = hi = 0;
+#pragma unroll
+            for (int g = 0; g < M; g++) {
+                all &= (uint32_t)(m[g] >> 42) == (tag & TAG22);
+                lo += (int)((uint32_t)m[g] << 11) >> 11;
+                hi += (int)((uint32_t)(m[g] >> 21) << 11) >> 11;
+            }
+        }
+        if (!all) s.dead = 1;
+        v = (tid & 1 ? hi : lo) + __builtin_amdgcn_update_dpp(0, tid & 1 ? lo : hi, 0xB1, 0xf, 0xf, false);
+        v = x + (v >> shift) + bias;
+    }
+    const int mx = wg_reduce<true>(abs(v), s.redm);
+    x = round_half_away((float)v * (127.0f / ((float)mx + 1e-9f)));
+    return !s.dead;
+}
+template <int H>
+__device__ __forceinline__ bool take(Lds &s, const u64 *slots, uint32_t tag, int shift, int bias, int (&x)[Norm<H>::NE], int limit) {
+    if constexpr (egg_decode_sums(H)) return take_sums<H>(s, slots, tag, shift, bias, x[0], limit);
+    else return take_residual<H>(s, slots, tag, x, limit);
 }
 
 __device__ __forceinline__ int exp_of(const Lds &s, const DecodeParams &p, int logit, int mx) {
@@ -296,15 +381,18 @@ __device__ bool sample(Lds &s, int *logit, int count, const DecodeParams &p, int
     return !s.dead;
 }
 
+// two workgroups to a CU, 256 registers; asked for at hidden 512, which has them anyway, the bound costs 1 % of its time
 template <int H>
-__global__ void __launch_bounds__(THREADS) k_decode(DecodeParams p) {
+__global__ void __launch_bounds__(THREADS, egg_decode_sums(H) ? 2 : 1) k_decode(DecodeParams p) {
     constexpr int G = H / 16, NE = Norm<H>::NE;
+    constexpr bool SUMS = egg_decode_sums(H);
     __shared__ Lds s;
     extern __shared__ int logit[];              // this workgroup's V / H logits of its 16 columns
     const int wg = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), c0 = 16 * wg;
     const int hd = p.head_dim, strips = hd / 16, head = wg / strips, T = p.T, V = p.vocab;
-    u64 *const m_qkv = p.slots, *const m_ao = m_qkv + G * 64, *const m_res = m_ao + H, *const m_up = m_res + H, *const m_dn = m_up + H,
-               *const m_max = m_dn + H, *const m_sum = m_max + G, *const m_tok = m_sum + 2 * G;
+    constexpr int N_AO = SUMS ? 0 : H, N_UP = SUMS ? 0 : H, N_RES = SUMS ? G * (H / 2) : H;
+    u64 *const m_qkv = p.slots, *const m_ao = m_qkv + G * 64, *const m_res = m_ao + N_AO, *const m_up = m_res + N_RES, *const m_dn = m_up + N_UP,
+               *const m_max = m_dn + N_RES, *const m_sum = m_max + G, *const m_tok = m_sum + 2 * G;
     int8_t *const kc = p.kcache + (size_t)wg * p.n_layers * T * hd, *const vc = p.vcache + (size_t)wg * p.n_layers * T * 16;
     const int8_t *const M = p.model, *const F = p.frag;
     const uint32_t hh = (uint32_t)H * H, h4 = 4u * H;
@@ -340,6 +428,7 @@ __global__ void __launch_bounds__(THREADS) k_decode(DecodeParams p) {
             x[i] = k < H ? clip127((int)(M + p.embedding)[((uint32_t)(k >> 2) * V + token) * 4 + (k & 3)] + (int)(M + p.emb_bias)[(uint32_t)k]) : 0;
             if (k < H) s.x[k] = (int8_t)x[i];
         }
+        int bd = 0;                            // of the down projection in front, where its sums are exchanged
         for (int l = -1; l < p.n_layers; l++) {
             const uint32_t tg = tag + (uint32_t)(l + 1);
             if (l >= 0) {
@@ -351,7 +440,7 @@ __global__ void __launch_bounds__(THREADS) k_decode(DecodeParams p) {
                 const int row = (tid >> 4) & 3, n = tid & 15;
                 const int rope_at = t * hd + ((c0 + n) % hd & ~1);
                 const int cs = p.rope_lut[rope_at], sn = p.rope_lut[rope_at + 1];
-                if (!take_residual<H>(s, m_dn, tg - 1, x, p.wait_limit)) return give_up(p);
+                if (!take<H>(s, m_dn, tg - 1, p.shift_dn, bd, x, p.wait_limit)) return give_up(p);
                 ln.apply(s, x);
                 const int acc = qkv.finish(s);
                 v4i kr[2][4]; int vr[8];
@@ -394,7 +483,8 @@ __global__ void __launch_bounds__(THREADS) k_decode(DecodeParams p) {
                 __syncthreads();
                 if (tid < hd / 4) *reinterpret_cast<int *>(kl + (uint32_t)(t * hd + 4 * tid)) = reinterpret_cast<const int *>(s.ks)[tid];
                 else if (tid >= 64 && tid < 68) *reinterpret_cast<int *>(vl + (uint32_t)(t * 16 + 4 * (tid - 64))) = reinterpret_cast<const int *>(s.vs)[tid - 64];
-                Strip<1, H> wo; wo.template load<H>(0, F + (p.w_o + l * hh), H, c0);
+                Rows<H, 16> wo_rows; Strip<1, H> wo;
+                if constexpr (SUMS) wo_rows.load(M + (p.w_o + l * hh), c0); else wo.template load<H>(0, F + (p.w_o + l * hh), H, c0);
                 int sc[2], mx = INT_MIN;
 #pragma unroll
                 for (int i = 0; i < 2; i++) {
@@ -448,10 +538,13 @@ __global__ void __launch_bounds__(THREADS) k_decode(DecodeParams p) {
                     quo += rest < 0 ? -1 : (rest >= den ? 1 : 0);
                     const int r = num < 0 ? -quo : quo;
                     const int packed = pack4(__builtin_amdgcn_readlane(r, 0), __builtin_amdgcn_readlane(r, 16), __builtin_amdgcn_readlane(r, 32), __builtin_amdgcn_readlane(r, 48));
-                    if ((tid & 63) == 0) send(m_ao, 4 * wg + wave, tg, packed);
+                    if ((tid & 63) == 0) { if constexpr (SUMS) reinterpret_cast<int *>(s.own)[wave] = packed; else send(m_ao, 4 * wg + wave, tg, packed); }
                 }
                 // ---- output projection of the strip, residual
-                {
+                if constexpr (SUMS) {
+                    __syncthreads();
+                    wo_rows.send_sums(s.own, m_res, wg, tg);
+                } else {
                     int a[1];
                     if (!receive<1>(a, m_ao, tid, 0, tid < H / 4 ? 1 : 0, tg, p.wait_limit)) s.dead = 1;
                     if (tid < H / 4) *reinterpret_cast<int *>(s.op + slot_of(4 * tid)) = a[0];
@@ -466,31 +559,35 @@ __global__ void __launch_bounds__(THREADS) k_decode(DecodeParams p) {
 #pragma unroll
             for (int i = 0; i < 4; i++) up.template load<H>(i, F + (l < 0 ? p.w_up_init : p.w_up + 4 * l * hh), 4 * H, 64 * wg + 16 * i);
             const int bu = tid < 64 ? b_up[(uint32_t)(64 * wg + tid)] : 0;
+            Rows<H, 64> dn_rows;
+            if constexpr (SUMS) dn_rows.load(M + (l < 0 ? p.w_dn_init : p.w_dn + 4 * l * hh), 64 * wg);
             if (l >= 0) {
                 ln.load(M + (p.ln_2 + l * (uint32_t)H), M + (p.ln_2_bias + l * (uint32_t)H));
-                if (!take_residual<H>(s, m_res, tg, x, p.wait_limit)) return give_up(p);
+                if (!take<H>(s, m_res, tg, p.shift_out, 0, x, p.wait_limit)) return give_up(p);
             }
             ln.apply(s, x);
-            {
-                const int a = up.finish(s);
+            const int a = up.finish(s), g = tid < 64 ? (int)s.act[(uint8_t)clip127((a >> p.shift_up) + bu)] : 0;
+            if constexpr (SUMS) {
+                if (tid < 64) s.own[tid] = (int8_t)g;
+                __syncthreads();
+                dn_rows.send_sums(s.own, m_dn, wg, tg);
+                bd = tid < H ? (int)b_dn[(uint32_t)tid] : 0;
+            } else {
                 if (tid < 64) {
-                    const int g = (uint8_t)s.act[(uint8_t)clip127((a >> p.shift_up) + bu)];
-                    const int g1 = __builtin_amdgcn_update_dpp(0, g, 0x55, 0xf, 0xf, false), g2 = __builtin_amdgcn_update_dpp(0, g, 0xAA, 0xf, 0xf, false),
-                              g3 = __builtin_amdgcn_update_dpp(0, g, 0xFF, 0xf, 0xf, false);     // lanes 1, 2, 3 of the quad
-                    if ((tid & 3) == 0) send(m_up, 16 * wg + (tid >> 2), tg, g | (g1 << 8) | (g2 << 16) | (g3 << 24));
+                    const int g0 = g & 255, g1 = __builtin_amdgcn_update_dpp(0, g0, 0x55, 0xf, 0xf, false), g2 = __builtin_amdgcn_update_dpp(0, g0, 0xAA, 0xf, 0xf, false),
+                              g3 = __builtin_amdgcn_update_dpp(0, g0, 0xFF, 0xf, 0xf, false);     // lanes 1, 2, 3 of the quad
+                    if ((tid & 3) == 0) send(m_up, 16 * wg + (tid >> 2), tg, g0 | (g1 << 8) | (g2 << 16) | (g3 << 24));
                 }
-            }
-            Strip<1, 4 * H> dn; dn.template load<H>(0, F + (l < 0 ? p.w_dn_init : p.w_dn + 4 * l * hh), H, c0);
-            const int bd = tid < 16 ? b_dn[(uint32_t)(c0 + tid)] : 0;
-            {
-                int a[NE];
-                if (!receive<NE>(a, m_up, tid, 256, tid < H ? NE : 0, tg, p.wait_limit)) s.dead = 1;
+                Strip<1, 4 * H> dn; dn.template load<H>(0, F + (l < 0 ? p.w_dn_init : p.w_dn + 4 * l * hh), H, c0);
+                const int b = tid < 16 ? b_dn[(uint32_t)(c0 + tid)] : 0;
+                int up4[NE];
+                if (!receive<NE>(up4, m_up, tid, 256, tid < H ? NE : 0, tg, p.wait_limit)) s.dead = 1;
 #pragma unroll
                 for (int i = 0; i < NE; i++)
-                    if (tid < H) *reinterpret_cast<int *>(s.op + slot_of(4 * (tid + 256 * i))) = a[i];
+                    if (tid < H) *reinterpret_cast<int *>(s.op + slot_of(4 * (tid + 256 * i))) = up4[i];
                 const int d = dn.finish(s);
                 if (s.dead) return give_up(p);
-                if (tid < 16) send(m_dn, c0 + tid, tg, (int)s.x[c0 + tid] + (d >> p.shift_dn) + bd);
+                if (tid < 16) send(m_dn, c0 + tid, tg, (int)s.x[c0 + tid] + (d >> p.shift_dn) + b);
             }
             // the next norm's gains: the next layer's first, or the last
             const bool last = l + 1 == p.n_layers;
@@ -499,7 +596,7 @@ __global__ void __launch_bounds__(THREADS) k_decode(DecodeParams p) {
         // ---- head: tiles of 16 columns dealt round, four at a time
         const uint32_t tg = tag + (uint32_t)p.n_layers + 1u;
         constexpr int BLOCK = H > 256 ? 256 : H;
-        if (!take_residual<H>(s, m_dn, tg - 1, x, p.wait_limit)) return give_up(p);
+        if (!take<H>(s, m_dn, tg - 1, p.shift_dn, bd, x, p.wait_limit)) return give_up(p);
         ln.apply(s, x);
         int count = 0;                          // logits of this workgroup
         for (int t0 = wg; t0 < V / 16; t0 += 4 * G) {

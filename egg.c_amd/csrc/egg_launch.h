@@ -123,7 +123,9 @@ struct DecodeParams {
     unsigned long long *slots; uint32_t *epoch; int *fail; int wait_limit;
     uint32_t seed; int deggs; float temp; int min_p_limit, penalty_int;
 };
-constexpr int64_t egg_decode_slots(int H) { return (int64_t)(H / 16) * 67 + 4 * H + 8; }
+// a layer's two matrices behind a strip exchange their products' partial sums (egg_decode.hip) instead of their inputs
+constexpr bool egg_decode_sums(int H) { return H <= 256; }
+constexpr int64_t egg_decode_slots(int H) { return (int64_t)(H / 16) * 67 + (egg_decode_sums(H) ? H / 16 * H : 4 * H) + 8; }
 hipError_t egg_prepare_decode(int H, int vocab);      // before the first launch
 hipError_t egg_launch_decode(const DecodeParams &p, int H, hipStream_t s);
 

@@ -53,6 +53,34 @@ def test_decode_equals_whole_window_evaluation(pkg, dev, hidden, head_dim, layer
     ctx.close()
 
 
+@pytest.mark.parametrize("hidden,head_dim", [(64, 32), (128, 64), (256, 64)])
+def test_decode_with_the_largest_partial_sums(pkg, dev, hidden, head_dim):
+    """Up to hidden 256 a strip's 64 intermediate and 16 attention values travel as partial sums of 21 bits.  Saturated
+    intermediates (bias and weights at the ends of int8) on matrices of -128 and 127 make the largest ones there are,
+    64 * 127 * 128, of both signs and in both halves of a message; two of every three columns stay random."""
+    ctx = _context(pkg, dev, hidden, head_dim, 2, 128, 256)
+    model, rng = ctx.model_download(), np.random.default_rng(3)
+    names = set()
+    for t in ctx.tensors():
+        n = t["rows"] * t["cols"]
+        if t["is_matrix"] and t["name"] in ("w_down", "w_o", "w_emb_mlp_down"):
+            names.add(t["name"])
+            block = model[t["offset"]:t["offset"] + n].reshape(-1, t["cols"], 4)      # four rows of a column together
+            block[:, ::6], block[:, 3::6] = -128, 127
+        elif not t["is_matrix"] and "up" in t["name"] and "bias" in t["name"]:
+            model[t["offset"]:t["offset"] + n] = rng.choice(np.array([-128, 127], np.int8), n, p=[0.1, 0.9])
+    ctx.model_upload(model)
+    got = []
+    for cached in (True, False):
+        ctx.generate_kv_cache(cached)
+        b = _prompt(dev, 256, 20, 84)
+        ctx.generate(b.data_ptr(), 20, 64, 11)
+        ctx.sync()
+        got.append(b.cpu().numpy())
+    assert len(names) == 3 and np.array_equal(got[0], got[1])
+    ctx.close()
+
+
 def test_decode_on_two_streams_and_replayed(pkg, dev):
     import torch
     ctxs = [_context(pkg, dev, h, 64, 2, 128, 256) for h in (256, 512)]
