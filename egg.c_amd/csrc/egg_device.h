@@ -371,8 +371,8 @@ __device__ __forceinline__ void zero_acc(v16i *acc) {
 }
 
 // ---------------------------------------------------------------- per-member noise tables (one wave fills its own)
-__device__ __forceinline__ void fill_noise_i8(int8_t *dst, uint32_t seed, int n, int mask, int lane, int nthr = 64, int mult = 1) {
-    for (int i = lane; i < n; i += nthr) dst[i] = (int8_t)(noise_from_hash(seed, i, mask) * mult);
+__device__ __forceinline__ void fill_noise_i8(int8_t *dst, uint32_t seed, int n, int mask, int lane, int nthr = 64, int mult = 1, int add = 0) {
+    for (int i = lane; i < n; i += nthr) dst[i] = (int8_t)(noise_from_hash(seed, i, mask) * mult + add);
 }
 // dst[i] = noise(seed, i) * mult
 __device__ __forceinline__ void fill_noise_i32(int *dst, uint32_t seed, int n, int mask, int mult, int lane, int nthr = 64) {

@@ -139,7 +139,7 @@ struct MlpCfg {
     static constexpr int XCHG = CS > 1 ? TPW * 32 * SC : 0;
     static constexpr int SITE = EGG_WAVES * 32;                       // ints per reduction site
     static constexpr int RED = CS > 1 ? 2 * SITE * 4 : 0;             // two reduction sites used alternately
-    static constexpr int OCC = H == 256 && CS > 1 ? 3 : 2;             // workgroups per CU the kernel is built for
+    static constexpr int OCC = (H == 256 && CS > 1) || (H == 128 && CS == 1) ? 3 : 2;             // workgroups per CU the kernel is built for
     // first block only: rank of every byte value among the values present in the member's window [256], wave counts
     // [4 ints], and below hidden 256 the list of present values [256] (from hidden 256 on it lives in the table slot
     // of the O projection's noise, which the first block does not use)
@@ -148,8 +148,17 @@ struct MlpCfg {
     // (behind the first block ex1 does not exist: 4H bytes less.  At hidden 256 the total stays at 52 KB: the LDS is
     // handed out in granules, three workgroups of 53 KB no longer share a CU, and the kernel then runs 9 % slower.)
     // The overlay's variants hold the input-side noise as floats: exB, upB and dnB take four times their bytes.
-    static constexpr int per_set(bool first, bool adapt) { return PER_SET + (up32(first) ? UPA32 : 0) - (first ? 0 : 4 * H) + (adapt ? 3 * 6 * H : 0); }
-    static int total(int sets, bool first, bool adapt) { return WBYTES + ACT + sets * per_set(first, adapt) + XCHG + RED + (first ? DEDUP : 0); }
+    static constexpr int per_set(bool first, bool adapt, bool rank) { return PER_SET + (!rank && up32(first) ? UPA32 : 0) - (first ? 0 : 4 * H) + (adapt ? 3 * 6 * H : 0); }
+    // The up projection's rank-one term as one more k-step (rank1_token) instead of a multiply, an add and a quarter of an LDS read an element, for
+    // the noise that egg_rank1_kstep allows.  It costs the registers of the token's operand and of a row: 8,192 members x 256 tokens at hidden 256
+    // 1.64 -> 1.58 ms, 2,048 x 512 at hidden 512 3.01 -> 2.96 (7 more registers in scratch across a pass), 16,384 x 128 at hidden 64 0.246 -> 0.235,
+    // 8,192 x 128 at hidden 128 0.296 -> 0.291 at three workgroups per CU as before (0.335 at two, which its 178 registers would give).  Hidden 256 with two
+    // slices would keep 8 registers in scratch: 80 -> 83 us for 2,048 members of 32 tokens, so it has the other form only.
+    static constexpr bool RANK1 = !(H == 256 && CS == 2);
+    static constexpr int ROWS = 1024;        // its table, last
+    static __host__ __device__ constexpr int total(int sets, bool first, bool adapt, bool rank) {
+        return WBYTES + ACT + sets * per_set(first, adapt, rank) + XCHG + RED + (first ? DEDUP : 0) + (rank ? ROWS : 0);
+    }
     // the overlay's variants need the registers of two workgroups per CU
     static constexpr int occ(bool adapt) { return adapt && OCC > 2 ? 2 : OCC; }
 };
@@ -167,7 +176,7 @@ struct MlpCfg {
 // hidden unit, which adds its four terms (k = unit, unit + H, ...) into an int one float addition at a time; the
 // sub-chunks are therefore visited so that those four are consecutive.  At hidden 256, 2048 members x 256 tokens the overlay's
 // kernel took 0.91 ms with integer terms, spilling at three workgroups per CU; 0.63 ms as it is (0.47 without the overlay).
-template <int H, bool FIRST, bool SEED, bool ADAPT, int CSV>
+template <int H, bool FIRST, bool SEED, bool ADAPT, int CSV, bool RANK>
 __global__ void __launch_bounds__(EGG_THREADS, (MlpCfg<H, CSV>::occ(ADAPT))) k_mlp(MlpParams p) {
     typedef MlpCfg<H, CSV> M;
     constexpr int CS = M::CS, KS = M::KS, NTS = M::NTS, HS = M::HS, NTU = M::NTU, SC = M::SC;
@@ -185,8 +194,8 @@ __global__ void __launch_bounds__(EGG_THREADS, (MlpCfg<H, CSV>::occ(ADAPT))) k_m
     const int T = c.T;
     const TileMap tm = tile_map<CS>(c.tn, wave, blockIdx.x);
     const int col0 = tm.cs * HS;                      // first output column of this wave's slice
-    constexpr int PSET = M::per_set(FIRST, ADAPT), WB = ADAPT ? 4 : 1;        // WB: bytes of an input-side noise entry
-    constexpr bool UPA32 = M::up32(FIRST);
+    constexpr int PSET = M::per_set(FIRST, ADAPT, RANK), WB = ADAPT ? 4 : 1;        // WB: bytes of an input-side noise entry
+    constexpr bool UPA32 = !RANK && M::up32(FIRST);
     int8_t *tb = act + M::ACT + tm.set * PSET;
     int *ex0 = reinterpret_cast<int *>(tb);           // FIRST: emb_bias + noise   | else: O-proj A noise
     int *ex1 = ex0 + H;                               // FIRST: b_dim noise * ns    | else: absent
@@ -195,6 +204,8 @@ __global__ void __launch_bounds__(EGG_THREADS, (MlpCfg<H, CSV>::occ(ADAPT))) k_m
     int8_t *upB = exB + WB * H, *dnB = upB + WB * H, *upA = dnB + 4 * WB * H, *dnA = upA + (UPA32 ? 16 : 4) * H;
     const int *oA = ex0, *dnA32 = reinterpret_cast<const int *>(dnA);
     int8_t *xch = act + M::ACT + tm.sets * PSET;
+    int8_t *rank_rows = smem + M::total(tm.sets, FIRST, ADAPT, RANK) - M::ROWS;
+    if (RANK) fill_rank1_rows(rank_rows, threadIdx.x, EGG_THREADS);
     int *red = reinterpret_cast<int *>(xch + M::XCHG);
     int rsite = 0;          // the two reduction sites take turns, call by call (the same sequence in every wave)
     auto next_site = [&]() { rsite ^= 1; return red + rsite * M::SITE; };
@@ -261,7 +272,7 @@ __global__ void __launch_bounds__(EGG_THREADS, (MlpCfg<H, CSV>::occ(ADAPT))) k_m
         fill_vec_i32(lw, p.ln_w, sbx + p.off_ln_a, sbx + p.off_ln_b, H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS, 2);     // 4 * gain, see standard_scale
         fill_vec_i32(lb, p.ln_b, sbx + p.off_lnb_a, sbx + p.off_lnb_b, H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS);
         if (UPA32) fill_noise_i32(reinterpret_cast<int *>(uA), sbx + p.off_up_a, 4 * H, c.mask, nsx << c.a_shift, tid, EGG_THREADS);
-        else fill_noise_i8(uA, sbx + p.off_up_a, 4 * H, c.mask, tid, EGG_THREADS, nsx);
+        else fill_noise_i8(uA, sbx + p.off_up_a, 4 * H, c.mask, tid, EGG_THREADS, nsx, RANK ? 15 : 0);       // RANK: the number of its row
         // the up bias is stored as (b + 128) << shift_mlp_up and seeds the up accumulator: ((a + (b << s)) >> s) == (a >> s) + b;
         // the 128 makes the clamped result (1..255) the GELU table's index
         fill_vec_i32(bu, p.b_up, sbx + p.off_bup_a, sbx + p.off_bup_b, 4 * H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS, c.shift_mlp_up, 128);
@@ -433,7 +444,13 @@ __global__ void __launch_bounds__(EGG_THREADS, (MlpCfg<H, CSV>::occ(ADAPT))) k_m
         }
         if (ADAPT && CS == 1) dot_noise_ov<KS, 1>(nrm, reinterpret_cast<const float *>(upB), 0, gA, &sbu);
         if (!ADAPT) sbu = dot_noise<KS, false>(nrm, upB, 0, gA);
-        sbu <<= c.sb_shift;
+        v4i tok; int far = 0; bool wide = false;
+        if (RANK) {
+            const Rank1Token tk = rank1_token(sbu, c.sigma, gA);
+#pragma unroll
+            for (int w = 0; w < 4; w++) tok[w] = rank1_word(w, tk.s, c.sigma, tk.digit);
+            far = tk.far; wide = tk.wide;
+        } else sbu <<= c.sb_shift;
         v16i accd[NTS];
         if (SEED) {
 #pragma unroll
@@ -462,6 +479,11 @@ __global__ void __launch_bounds__(EGG_THREADS, (MlpCfg<H, CSV>::occ(ADAPT))) k_m
         for (int it = 0; it < M::NSUB; it++) {
             const int s = sub_chunk(it);
             v16i au[NTU];
+            v4i rr[NTU];
+            if (RANK)
+#pragma unroll
+                for (int nt = 0; nt < NTU; nt++)
+                    rr[nt] = *reinterpret_cast<const v4i *>(rank_rows + gL * 512 + 16 * (int)reinterpret_cast<const uint8_t *>(upA)[s * SC + tm.cs * 32 * NTU + 32 * nt + (laneL & 31)]);
 #pragma unroll
             for (int nt = 0; nt < NTU; nt++)
 #pragma unroll
@@ -474,6 +496,17 @@ __global__ void __launch_bounds__(EGG_THREADS, (MlpCfg<H, CSV>::occ(ADAPT))) k_m
             for (int ku = 0; ku < M::UPU; ku++) {
                 const int8_t *cur = w_acquire(ws);
                 if (ku + 1 < M::UPU) pf_up(s, ku + 1); else pf_dn(s, 0);
+                if (RANK && ku == 0) {
+#pragma unroll
+                    for (int nt = 0; nt < NTU; nt++) au[nt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(rr[nt], tok, au[nt], 0, 0, 0);
+                    if (__builtin_expect(wide, 0)) {
+                        const v4i f = {0, 0, 0, far};
+#pragma unroll 1
+                        for (int i = 0; i < 8; i++)
+#pragma unroll
+                            for (int nt = 0; nt < NTU; nt++) au[nt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(rr[nt], f, au[nt], 0, 0, 0);
+                    }
+                }
                 mfma_cols<M::PRUP / 2, NTU, MAXF>(au, nrm + ku * (M::PRUP / 2), cur, SC, tm.cs * 32 * NTU, laneL);
             }
             v4i mid[CS * NTU];
@@ -488,13 +521,13 @@ __global__ void __launch_bounds__(EGG_THREADS, (MlpCfg<H, CSV>::occ(ADAPT))) k_m
                         int n0 = nb + 32 * nt + 8 * q + 4 * gL;
                         int a4 = 0; v4i a32 = {0, 0, 0, 0};
                         if (UPA32) a32 = *reinterpret_cast<const v4i *>(reinterpret_cast<const int *>(upA) + n0);
-                        else a4 = *reinterpret_cast<const int *>(upA + n0);
+                        else if (!RANK) a4 = *reinterpret_cast<const int *>(upA + n0);
                         uint32_t r4[4];          // byte 0: the activation of element e (ADAPT: sign-extended)
 #pragma unroll
                         for (int e = 0; e < 4; e++) {
                             // the accumulator carries + 128 (see the bias table): clamping to 1..255 is the clamp to +-127,
                             // and the result is the table index as it stands
-                            const int idx = min(255, max(1, (au[nt][4 * q + e] + __mulhi(sbu, UPA32 ? a32[e] : sx8(a4, e) << c.a_shift)) >> c.shift_mlp_up));
+                            const int idx = min(255, max(1, (RANK ? au[nt][4 * q + e] : au[nt][4 * q + e] + __mulhi(sbu, UPA32 ? a32[e] : sx8(a4, e) << c.a_shift)) >> c.shift_mlp_up));
                             r4[e] = ADAPT ? (uint32_t)(int)reinterpret_cast<lds_i8_ptr>((uintptr_t)(uint32_t)idx)[M::WBYTES]
                                           : reinterpret_cast<lds_u8_ptr>((uintptr_t)(uint32_t)idx)[M::WBYTES];
                         }
@@ -1524,16 +1557,21 @@ __global__ void __launch_bounds__(EGG_THREADS, 2) k_head_big(HeadParams p) {
 }
 
 // ============================================================================ host launchers
-template <int H, bool ADAPT, int CSV>
-static hipError_t launch_mlp_cs(const MlpParams &p, bool first, hipStream_t s) {
+template <int H, bool ADAPT, int CSV, bool RANK>
+static hipError_t launch_mlp_rank(const MlpParams &p, bool first, hipStream_t s) {
     const int sets = tile_map_sets(p.c.tn, CSV);
     const dim3 grid((p.c.n_members + sets - 1) / sets), block(EGG_THREADS);
-    const size_t lds = MlpCfg<H, CSV>::total(sets, first, ADAPT);
+    const size_t lds = MlpCfg<H, CSV>::total(sets, first, ADAPT, RANK);
     const bool seed = egg_mlp_down_acc_bound(H, p.c.mask, p.c.sigma_vec, p.c.shift_mlp_down) < (1LL << 31) &&
                       (first || egg_out_acc_bound(H, p.c.mask, p.c.shift_out) < (1LL << 31));
-    if (first) { if (seed) hipLaunchKernelGGL((k_mlp<H, true, true, ADAPT, CSV>), grid, block, lds, s, p); else hipLaunchKernelGGL((k_mlp<H, true, false, ADAPT, CSV>), grid, block, lds, s, p); }
-    else { if (seed) hipLaunchKernelGGL((k_mlp<H, false, true, ADAPT, CSV>), grid, block, lds, s, p); else hipLaunchKernelGGL((k_mlp<H, false, false, ADAPT, CSV>), grid, block, lds, s, p); }
+    if (first) { if (seed) hipLaunchKernelGGL((k_mlp<H, true, true, ADAPT, CSV, RANK>), grid, block, lds, s, p); else hipLaunchKernelGGL((k_mlp<H, true, false, ADAPT, CSV, RANK>), grid, block, lds, s, p); }
+    else { if (seed) hipLaunchKernelGGL((k_mlp<H, false, true, ADAPT, CSV, RANK>), grid, block, lds, s, p); else hipLaunchKernelGGL((k_mlp<H, false, false, ADAPT, CSV, RANK>), grid, block, lds, s, p); }
     return hipGetLastError();
+}
+template <int H, bool ADAPT, int CSV>
+static hipError_t launch_mlp_cs(const MlpParams &p, bool first, hipStream_t s) {
+    if constexpr (!ADAPT && MlpCfg<H, CSV>::RANK1) if (egg_rank1_kstep(H, p.c.mask, p.c.sigma)) return launch_mlp_rank<H, false, CSV, true>(p, first, s);
+    return launch_mlp_rank<H, ADAPT, CSV, false>(p, first, s);
 }
 template <int H>
 static hipError_t launch_mlp_h(const MlpParams &p, bool first, hipStream_t s) {
@@ -1661,18 +1699,24 @@ static hipError_t prepare_qkv(int T) {
     SET_LDS((k_qkv<H, ADAPT, CSV>), (QkvCfg<H, CSV>::total(sets, ADAPT)));
     return hipSuccess;
 }
-template <int H, bool ADAPT, int CSV>
-static hipError_t prepare_cs(int T) {
+template <int H, bool ADAPT, int CSV, bool RANK>
+static hipError_t prepare_mlp(int T) {
     // table sets per workgroup: the whole window's, or a single tile's (a prompt's first tiles may be evaluated alone)
     const int sets = std::max(tile_map_sets(T, CSV), tile_map_sets(32, CSV));
-    for (hipError_t e : {no_static_lds(&k_mlp<H, true, true, ADAPT, CSV>), no_static_lds(&k_mlp<H, false, true, ADAPT, CSV>),
-                         no_static_lds(&k_mlp<H, true, false, ADAPT, CSV>), no_static_lds(&k_mlp<H, false, false, ADAPT, CSV>)})
+    for (hipError_t e : {no_static_lds(&k_mlp<H, true, true, ADAPT, CSV, RANK>), no_static_lds(&k_mlp<H, false, true, ADAPT, CSV, RANK>),
+                         no_static_lds(&k_mlp<H, true, false, ADAPT, CSV, RANK>), no_static_lds(&k_mlp<H, false, false, ADAPT, CSV, RANK>)})
         if (e != hipSuccess) return e;
-    SET_LDS((k_mlp<H, true, true, ADAPT, CSV>), (MlpCfg<H, CSV>::total(sets, true, ADAPT)));
-    SET_LDS((k_mlp<H, true, false, ADAPT, CSV>), (MlpCfg<H, CSV>::total(sets, true, ADAPT)));
-    SET_LDS((k_mlp<H, false, true, ADAPT, CSV>), (MlpCfg<H, CSV>::total(sets, false, ADAPT)));
-    SET_LDS((k_mlp<H, false, false, ADAPT, CSV>), (MlpCfg<H, CSV>::total(sets, false, ADAPT)));
-    return prepare_qkv<H, ADAPT, CSV>(T);
+    SET_LDS((k_mlp<H, true, true, ADAPT, CSV, RANK>), (MlpCfg<H, CSV>::total(sets, true, ADAPT, RANK)));
+    SET_LDS((k_mlp<H, true, false, ADAPT, CSV, RANK>), (MlpCfg<H, CSV>::total(sets, true, ADAPT, RANK)));
+    SET_LDS((k_mlp<H, false, true, ADAPT, CSV, RANK>), (MlpCfg<H, CSV>::total(sets, false, ADAPT, RANK)));
+    SET_LDS((k_mlp<H, false, false, ADAPT, CSV, RANK>), (MlpCfg<H, CSV>::total(sets, false, ADAPT, RANK)));
+    return hipSuccess;
+}
+template <int H, bool ADAPT, int CSV>
+static hipError_t prepare_cs(int T) {
+    hipError_t e = prepare_mlp<H, ADAPT, CSV, false>(T);
+    if constexpr (!ADAPT && MlpCfg<H, CSV>::RANK1) if (e == hipSuccess) e = prepare_mlp<H, false, CSV, true>(T);
+    return e == hipSuccess ? prepare_qkv<H, ADAPT, CSV>(T) : e;
 }
 template <int H>
 static hipError_t prepare_h(int T) {
