@@ -752,7 +752,8 @@ static int forward_chunk(egg_ctx *ctx, const uint8_t *d_data, int64_t len, const
     const size_t act_bytes = (size_t)nm * c.seq_len * H;
     FwdCommon f = make_common(ctx, d_data, len, d_start, d_seed, first_member, nm);
     if (range) { f.t0 = range->t0; f.tn = range->tn; }
-    {
+    const int64_t hh = (int64_t)H * H, h4 = (int64_t)H * 4 * H;
+    auto first_params = [&]() {
         MlpParams p; memset(&p, 0, sizeof(p)); p.c = f; p.seed_base = 0;
         p.off_ln_a = OFF_LN_INIT_A; p.off_ln_b = OFF_LN_INIT_B; p.off_lnb_a = OFF_LN_INIT_BIAS_A; p.off_lnb_b = OFF_LN_INIT_BIAS_B;
         p.off_up_a = OFF_EMB_MLP_UP_A; p.off_up_b = OFF_EMB_MLP_UP_B; p.off_bup_a = OFF_EMB_MLP_BIAS_UP_A; p.off_bup_b = OFF_EMB_MLP_BIAS_UP_B;
@@ -767,53 +768,63 @@ static int forward_chunk(egg_ctx *ctx, const uint8_t *d_data, int64_t len, const
             p.q_ln_w = Q + L.ln_init; p.q_ln_b = Q + L.ln_init_bias; p.q_b_up = Q + L.mlp_emb_bias_up; p.q_b_dn = Q + L.mlp_emb_bias_down;
             p.q_up = Q + L.w_emb_mlp_up; p.q_dn = Q + L.w_emb_mlp_down; p.q_emb = Q + L.embedding; p.q_emb_bias = Q + L.emb_bias;
         }
-        { SpanScope span(ctx, EGG_K_MLP_FIRST); HIP_TRY(egg_launch_mlp(p, true, s)); }
+        return p;
+    };
+    auto qkv_params = [&](int l) {
+        QkvParams p; memset(&p, 0, sizeof(p)); p.c = f; p.seed_base = l * 1000;
+        p.ln_w = M + L.ln_1 + (int64_t)l * H; p.ln_b = M + L.ln_1_bias + (int64_t)l * H;
+        p.w_q = F + L.w_q + l * hh; p.w_k = F + L.w_k + l * hh; p.w_v = F + L.w_v + l * hh;
+        p.x = ctx->d_x; p.q = ctx->d_q; p.k = ctx->d_k; p.v = ctx->d_v;
+        if (range && range->kv) { p.k = range->kv + (size_t)(2 * l) * act_bytes; p.v = range->kv + (size_t)(2 * l + 1) * act_bytes; }
+        if (Q) {
+            p.q_ln_w = Q + L.ln_1 + (int64_t)l * H; p.q_ln_b = Q + L.ln_1_bias + (int64_t)l * H;
+            p.q_wq = Q + L.w_q + l * hh; p.q_wk = Q + L.w_k + l * hh; p.q_wv = Q + L.w_v + l * hh;
+        }
+        return p;
+    };
+    auto attn_params = [&](int l) {
+        AttnParams p; memset(&p, 0, sizeof(p)); p.c = f; p.q = ctx->d_q; p.k = ctx->d_k; p.v = ctx->d_v; p.ao = ctx->d_ao;
+        if (range && range->kv) { p.k = range->kv + (size_t)(2 * l) * act_bytes; p.v = range->kv + (size_t)(2 * l + 1) * act_bytes; }
+        return p;
+    };
+    auto mlp_params = [&](int l) {
+        MlpParams p; memset(&p, 0, sizeof(p)); p.c = f; p.seed_base = l * 1000;
+        p.off_ln_a = OFF_LN_2_A; p.off_ln_b = OFF_LN_2_B; p.off_lnb_a = OFF_LN_2_BIAS_A; p.off_lnb_b = OFF_LN_2_BIAS_B;
+        p.off_up_a = OFF_MLP_UP_A; p.off_up_b = OFF_MLP_UP_B; p.off_bup_a = OFF_MLP_BIAS_UP_A; p.off_bup_b = OFF_MLP_BIAS_UP_B;
+        p.off_dn_a = OFF_MLP_DOWN_A; p.off_dn_b = OFF_MLP_DOWN_B; p.off_bdn_a = OFF_MLP_BIAS_DOWN_A; p.off_bdn_b = OFF_MLP_BIAS_DOWN_B;
+        p.ln_w = M + L.ln_2 + (int64_t)l * H; p.ln_b = M + L.ln_2_bias + (int64_t)l * H;
+        p.w_up = F + L.w_up + l * h4; p.b_up = M + L.mlp_bias_up + (int64_t)l * 4 * H;
+        p.w_dn = F + L.w_down + l * h4; p.b_dn = M + L.mlp_bias_down + (int64_t)l * H;
+        p.w_o = F + L.w_o + l * hh; p.ao = ctx->d_ao; p.x = ctx->d_x;
+        p.x_mid = taps ? tap_ptr(ctx, 1 + 6 * l + 4) : nullptr;
+        if (Q) {
+            p.q_ln_w = Q + L.ln_2 + (int64_t)l * H; p.q_ln_b = Q + L.ln_2_bias + (int64_t)l * H;
+            p.q_b_up = Q + L.mlp_bias_up + (int64_t)l * 4 * H; p.q_b_dn = Q + L.mlp_bias_down + (int64_t)l * H;
+            p.q_up = Q + L.w_up + l * h4; p.q_dn = Q + L.w_down + l * h4; p.q_o = Q + L.w_o + l * hh;
+        }
+        return p;
+    };
+    bool taken = false;
+    if (!taps && !Q && !range && !ctx->timing && c.n_layers > 0) {
+        const BlocksParams p = {first_params(), mlp_params(0), qkv_params(0), attn_params(0), c.n_layers};
+        HIP_TRY(egg_launch_blocks(p, &taken, s));
+    }
+    if (!taken) {
+        { SpanScope span(ctx, EGG_K_MLP_FIRST); HIP_TRY(egg_launch_mlp(first_params(), true, s)); }
         if (taps) HIP_TRY(hipMemcpyAsync(tap_ptr(ctx, 0), ctx->d_x, act_bytes, hipMemcpyDeviceToDevice, s));
     }
-    for (int l = 0; l < c.n_layers; l++) {
-        const int64_t hh = (int64_t)H * H, h4 = (int64_t)H * 4 * H;
-        {
-            QkvParams p; memset(&p, 0, sizeof(p)); p.c = f; p.seed_base = l * 1000;
-            p.ln_w = M + L.ln_1 + (int64_t)l * H; p.ln_b = M + L.ln_1_bias + (int64_t)l * H;
-            p.w_q = F + L.w_q + l * hh; p.w_k = F + L.w_k + l * hh; p.w_v = F + L.w_v + l * hh;
-            p.x = ctx->d_x; p.q = ctx->d_q; p.k = ctx->d_k; p.v = ctx->d_v;
-            if (range && range->kv) { p.k = range->kv + (size_t)(2 * l) * act_bytes; p.v = range->kv + (size_t)(2 * l + 1) * act_bytes; }
-            if (Q) {
-                p.q_ln_w = Q + L.ln_1 + (int64_t)l * H; p.q_ln_b = Q + L.ln_1_bias + (int64_t)l * H;
-                p.q_wq = Q + L.w_q + l * hh; p.q_wk = Q + L.w_k + l * hh; p.q_wv = Q + L.w_v + l * hh;
-            }
-            { SpanScope span(ctx, EGG_K_QKV); HIP_TRY(egg_launch_qkv(p, s)); }
-            if (taps) {
-                HIP_TRY(hipMemcpyAsync(tap_ptr(ctx, 1 + 6 * l + 0), ctx->d_q, act_bytes, hipMemcpyDeviceToDevice, s));
-                HIP_TRY(hipMemcpyAsync(tap_ptr(ctx, 1 + 6 * l + 1), ctx->d_k, act_bytes, hipMemcpyDeviceToDevice, s));
-                HIP_TRY(hipMemcpyAsync(tap_ptr(ctx, 1 + 6 * l + 2), ctx->d_v, act_bytes, hipMemcpyDeviceToDevice, s));
-            }
-            if (range && range->kv_only && l + 1 == c.n_layers) return EGG_OK;
+    for (int l = 0; l < c.n_layers && !taken; l++) {
+        { SpanScope span(ctx, EGG_K_QKV); HIP_TRY(egg_launch_qkv(qkv_params(l), s)); }
+        if (taps) {
+            HIP_TRY(hipMemcpyAsync(tap_ptr(ctx, 1 + 6 * l + 0), ctx->d_q, act_bytes, hipMemcpyDeviceToDevice, s));
+            HIP_TRY(hipMemcpyAsync(tap_ptr(ctx, 1 + 6 * l + 1), ctx->d_k, act_bytes, hipMemcpyDeviceToDevice, s));
+            HIP_TRY(hipMemcpyAsync(tap_ptr(ctx, 1 + 6 * l + 2), ctx->d_v, act_bytes, hipMemcpyDeviceToDevice, s));
         }
-        {
-            AttnParams p; memset(&p, 0, sizeof(p)); p.c = f; p.q = ctx->d_q; p.k = ctx->d_k; p.v = ctx->d_v; p.ao = ctx->d_ao;
-            if (range && range->kv) { p.k = range->kv + (size_t)(2 * l) * act_bytes; p.v = range->kv + (size_t)(2 * l + 1) * act_bytes; }
-            { SpanScope span(ctx, EGG_K_ATTN); HIP_TRY(egg_launch_attn(p, s)); }
-            if (taps) HIP_TRY(hipMemcpyAsync(tap_ptr(ctx, 1 + 6 * l + 3), ctx->d_ao, act_bytes, hipMemcpyDeviceToDevice, s));
-        }
-        {
-            MlpParams p; memset(&p, 0, sizeof(p)); p.c = f; p.seed_base = l * 1000;
-            p.off_ln_a = OFF_LN_2_A; p.off_ln_b = OFF_LN_2_B; p.off_lnb_a = OFF_LN_2_BIAS_A; p.off_lnb_b = OFF_LN_2_BIAS_B;
-            p.off_up_a = OFF_MLP_UP_A; p.off_up_b = OFF_MLP_UP_B; p.off_bup_a = OFF_MLP_BIAS_UP_A; p.off_bup_b = OFF_MLP_BIAS_UP_B;
-            p.off_dn_a = OFF_MLP_DOWN_A; p.off_dn_b = OFF_MLP_DOWN_B; p.off_bdn_a = OFF_MLP_BIAS_DOWN_A; p.off_bdn_b = OFF_MLP_BIAS_DOWN_B;
-            p.ln_w = M + L.ln_2 + (int64_t)l * H; p.ln_b = M + L.ln_2_bias + (int64_t)l * H;
-            p.w_up = F + L.w_up + l * h4; p.b_up = M + L.mlp_bias_up + (int64_t)l * 4 * H;
-            p.w_dn = F + L.w_down + l * h4; p.b_dn = M + L.mlp_bias_down + (int64_t)l * H;
-            p.w_o = F + L.w_o + l * hh; p.ao = ctx->d_ao; p.x = ctx->d_x;
-            p.x_mid = taps ? tap_ptr(ctx, 1 + 6 * l + 4) : nullptr;
-            if (Q) {
-                p.q_ln_w = Q + L.ln_2 + (int64_t)l * H; p.q_ln_b = Q + L.ln_2_bias + (int64_t)l * H;
-                p.q_b_up = Q + L.mlp_bias_up + (int64_t)l * 4 * H; p.q_b_dn = Q + L.mlp_bias_down + (int64_t)l * H;
-                p.q_up = Q + L.w_up + l * h4; p.q_dn = Q + L.w_down + l * h4; p.q_o = Q + L.w_o + l * hh;
-            }
-            { SpanScope span(ctx, EGG_K_MLP); HIP_TRY(egg_launch_mlp(p, false, s)); }
-            if (taps) HIP_TRY(hipMemcpyAsync(tap_ptr(ctx, 1 + 6 * l + 5), ctx->d_x, act_bytes, hipMemcpyDeviceToDevice, s));
-        }
+        if (range && range->kv_only && l + 1 == c.n_layers) return EGG_OK;
+        { SpanScope span(ctx, EGG_K_ATTN); HIP_TRY(egg_launch_attn(attn_params(l), s)); }
+        if (taps) HIP_TRY(hipMemcpyAsync(tap_ptr(ctx, 1 + 6 * l + 3), ctx->d_ao, act_bytes, hipMemcpyDeviceToDevice, s));
+        { SpanScope span(ctx, EGG_K_MLP); HIP_TRY(egg_launch_mlp(mlp_params(l), false, s)); }
+        if (taps) HIP_TRY(hipMemcpyAsync(tap_ptr(ctx, 1 + 6 * l + 5), ctx->d_x, act_bytes, hipMemcpyDeviceToDevice, s));
     }
     {
         HeadParams p; memset(&p, 0, sizeof(p)); p.c = f;

@@ -176,8 +176,9 @@ struct MlpCfg {
 // hidden unit, which adds its four terms (k = unit, unit + H, ...) into an int one float addition at a time; the
 // sub-chunks are therefore visited so that those four are consecutive.  At hidden 256, 2048 members x 256 tokens the overlay's
 // kernel took 0.91 ms with integer terms, spilling at three workgroups per CU; 0.63 ms as it is (0.47 without the overlay).
+// l: layers behind the one that p describes
 template <int H, bool FIRST, bool SEED, bool ADAPT, int CSV, bool RANK>
-__global__ void __launch_bounds__(EGG_THREADS, (MlpCfg<H, CSV>::occ(ADAPT))) k_mlp(MlpParams p) {
+__device__ __forceinline__ void mlp_block(const MlpParams &p, int l) {
     typedef MlpCfg<H, CSV> M;
     constexpr int CS = M::CS, KS = M::KS, NTS = M::NTS, HS = M::HS, NTU = M::NTU, SC = M::SC;
     // fragments read ahead of their MFMAs: at hidden 512 the accumulators and operands leave room for four
@@ -191,7 +192,9 @@ __global__ void __launch_bounds__(EGG_THREADS, (MlpCfg<H, CSV>::occ(ADAPT))) k_m
     typedef const __attribute__((address_space(3))) int8_t *lds_i8_ptr;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const FwdCommon &c = p.c;
-    const int T = c.T;
+    const int T = c.T, seed_base = p.seed_base + 1000 * l, l1 = l * H, l4 = 4 * l * H * H;
+    const int8_t *const ln_w = p.ln_w + l1, *const ln_b = p.ln_b + l1, *const b_up = p.b_up + 4 * l1, *const b_dn = p.b_dn + l1;
+    const int8_t *const w_up = p.w_up + l4, *const w_dn = p.w_dn + l4, *const w_o = FIRST ? nullptr : p.w_o + l1 * H;
     const TileMap tm = tile_map<CS>(c.tn, wave, blockIdx.x);
     const int col0 = tm.cs * HS;                      // first output column of this wave's slice
     constexpr int PSET = M::per_set(FIRST, ADAPT, RANK), WB = ADAPT ? 4 : 1;        // WB: bytes of an input-side noise entry
@@ -217,17 +220,17 @@ __global__ void __launch_bounds__(EGG_THREADS, (MlpCfg<H, CSV>::occ(ADAPT))) k_m
     const DmaPlan<M::PRO, H> plan_o = dma_plan<M::PRO, H>(H);
     auto pf_up = [&](int s, int ku) {
         const int n = s * SC;
-        w_prefetch2<M::PRUP, SC>(ws, p.w_up + (size_t)(n / H) * H * H + ((size_t)ku * M::PRUP * H + n % H) * 16, plan_up);
+        w_prefetch2<M::PRUP, SC>(ws, w_up + (size_t)(n / H) * H * H + ((size_t)ku * M::PRUP * H + n % H) * 16, plan_up);
     };
     auto pf_dn = [&](int s, int du) {
         const int k = s * SC;
-        w_prefetch2<M::PRDN, H>(ws, p.w_dn + (size_t)(k / H) * H * H + (size_t)((k % H) / 16 + du * M::PRDN) * H * 16, plan_dn);
+        w_prefetch2<M::PRDN, H>(ws, w_dn + (size_t)(k / H) * H * H + (size_t)((k % H) / 16 + du * M::PRDN) * H * 16, plan_dn);
     };
     // (the unit index passes through an empty asm so that the four unit addresses are formed where they are used:
     // precomputed in front of the pass loop they overflow the scalar registers and are spilled through scratch)
     auto pf_o = [&](int u) {
         asm volatile("" : "+s"(u));
-        w_prefetch2<M::PRO, H>(ws, p.w_o + (size_t)(unsigned)u * (M::PRO * H * 16), plan_o);
+        w_prefetch2<M::PRO, H>(ws, w_o + (size_t)(unsigned)u * (M::PRO * H * 16), plan_o);
     };
     auto pf_pass_first = [&]() { if (FIRST) pf_up(0, 0); else pf_o(0); };
     pf_pass_first();
@@ -237,7 +240,7 @@ __global__ void __launch_bounds__(EGG_THREADS, (MlpCfg<H, CSV>::occ(ADAPT))) k_m
     for (int ss = 0; ss < tm.sets; ss++) {
         int ml = blockIdx.x * tm.sets + ss; if (ml >= c.n_members) ml = c.n_members - 1;
         const int mem = c.pop_offset + ml, nsx = (mem & 1) ? -1 : 1;
-        const uint32_t pseed = *c.d_step_seed + (uint32_t)(mem / 2), sbx = pseed + (uint32_t)p.seed_base;
+        const uint32_t pseed = *c.d_step_seed + (uint32_t)(mem / 2), sbx = pseed + (uint32_t)seed_base;
         int8_t *t2 = act + M::ACT + ss * PSET;
         int *e0 = reinterpret_cast<int *>(t2), *e1 = e0 + H, *lw = e1 + (FIRST ? H : 0), *lb = lw + H, *bu = lb + H, *bd = bu + 4 * H;
         int8_t *eB = reinterpret_cast<int8_t *>(bd + H), *uB = eB + WB * H, *dB = uB + WB * H, *uA = dB + 4 * WB * H, *dA = uA + (UPA32 ? 16 : 4) * H;
@@ -251,13 +254,13 @@ __global__ void __launch_bounds__(EGG_THREADS, (MlpCfg<H, CSV>::occ(ADAPT))) k_m
                 fill_noise_i32_ov(e0, sbx + OFF_O_A, H, c.mask, nsx << c.a_shift, tid, EGG_THREADS, p.q_o + H);
                 fill_noise_f32_ov(reinterpret_cast<float *>(eB), sbx + OFF_O_B, H, c.mask, tid, EGG_THREADS, p.q_o);
             }
-            fill_vec_i32_ov(lw, p.ln_w, sbx + p.off_ln_a, sbx + p.off_ln_b, H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS, 2, p.q_ln_w);
-            fill_vec_i32_ov(lb, p.ln_b, sbx + p.off_lnb_a, sbx + p.off_lnb_b, H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS, 0, p.q_ln_b);
+            fill_vec_i32_ov(lw, ln_w, sbx + p.off_ln_a, sbx + p.off_ln_b, H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS, 2, p.q_ln_w);
+            fill_vec_i32_ov(lb, ln_b, sbx + p.off_lnb_a, sbx + p.off_lnb_b, H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS, 0, p.q_ln_b);
             if (UPA32) fill_noise_i32_ov(reinterpret_cast<int *>(uA), sbx + p.off_up_a, 4 * H, c.mask, nsx << c.a_shift, tid, EGG_THREADS, p.q_up + H);
             else fill_noise_i8_ov(uA, sbx + p.off_up_a, 4 * H, c.mask, tid, EGG_THREADS, nsx, p.q_up + H);
-            fill_vec_i32_ov(bu, p.b_up, sbx + p.off_bup_a, sbx + p.off_bup_b, 4 * H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS, c.shift_mlp_up, p.q_b_up, 128);
+            fill_vec_i32_ov(bu, b_up, sbx + p.off_bup_a, sbx + p.off_bup_b, 4 * H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS, c.shift_mlp_up, p.q_b_up, 128);
             fill_noise_i32_ov(reinterpret_cast<int *>(dA), sbx + p.off_dn_a, H, c.mask, nsx << c.a_shift, tid, EGG_THREADS, p.q_dn + 4 * H);
-            fill_vec_i32_ov(bd, p.b_dn, sbx + p.off_bdn_a, sbx + p.off_bdn_b, H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS, SEED ? c.shift_mlp_down : 0, p.q_b_dn);
+            fill_vec_i32_ov(bd, b_dn, sbx + p.off_bdn_a, sbx + p.off_bdn_b, H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS, SEED ? c.shift_mlp_down : 0, p.q_b_dn);
             fill_noise_f32_ov(reinterpret_cast<float *>(uB), sbx + p.off_up_b, H, c.mask, tid, EGG_THREADS, p.q_up);
             fill_noise_f32_ov(reinterpret_cast<float *>(dB), sbx + p.off_dn_b, 4 * H, c.mask, tid, EGG_THREADS, p.q_dn);
             continue;
@@ -269,15 +272,15 @@ __global__ void __launch_bounds__(EGG_THREADS, (MlpCfg<H, CSV>::occ(ADAPT))) k_m
             fill_noise_i32(e0, sbx + OFF_O_A, H, c.mask, nsx << c.a_shift, tid, EGG_THREADS);
             fill_noise_i8(eB, sbx + OFF_O_B, H, c.mask, tid, EGG_THREADS);
         }
-        fill_vec_i32(lw, p.ln_w, sbx + p.off_ln_a, sbx + p.off_ln_b, H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS, 2);     // 4 * gain, see standard_scale
-        fill_vec_i32(lb, p.ln_b, sbx + p.off_lnb_a, sbx + p.off_lnb_b, H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS);
+        fill_vec_i32(lw, ln_w, sbx + p.off_ln_a, sbx + p.off_ln_b, H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS, 2);     // 4 * gain, see standard_scale
+        fill_vec_i32(lb, ln_b, sbx + p.off_lnb_a, sbx + p.off_lnb_b, H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS);
         if (UPA32) fill_noise_i32(reinterpret_cast<int *>(uA), sbx + p.off_up_a, 4 * H, c.mask, nsx << c.a_shift, tid, EGG_THREADS);
         else fill_noise_i8(uA, sbx + p.off_up_a, 4 * H, c.mask, tid, EGG_THREADS, nsx, RANK ? 15 : 0);       // RANK: the number of its row
         // the up bias is stored as (b + 128) << shift_mlp_up and seeds the up accumulator: ((a + (b << s)) >> s) == (a >> s) + b;
         // the 128 makes the clamped result (1..255) the GELU table's index
-        fill_vec_i32(bu, p.b_up, sbx + p.off_bup_a, sbx + p.off_bup_b, 4 * H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS, c.shift_mlp_up, 128);
+        fill_vec_i32(bu, b_up, sbx + p.off_bup_a, sbx + p.off_bup_b, 4 * H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS, c.shift_mlp_up, 128);
         fill_noise_i32(reinterpret_cast<int *>(dA), sbx + p.off_dn_a, H, c.mask, nsx << c.a_shift, tid, EGG_THREADS);
-        fill_vec_i32(bd, p.b_dn, sbx + p.off_bdn_a, sbx + p.off_bdn_b, H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS, SEED ? c.shift_mlp_down : 0);
+        fill_vec_i32(bd, b_dn, sbx + p.off_bdn_a, sbx + p.off_bdn_b, H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS, SEED ? c.shift_mlp_down : 0);
         fill_noise_i8(uB, sbx + p.off_up_b, H, c.mask, tid, EGG_THREADS);
         fill_noise_i8(dB, sbx + p.off_dn_b, 4 * H, c.mask, tid, EGG_THREADS);
     }
@@ -606,6 +609,9 @@ __global__ void __launch_bounds__(EGG_THREADS, (MlpCfg<H, CSV>::occ(ADAPT))) k_m
     }
 }
 
+template <int H, bool FIRST, bool SEED, bool ADAPT, int CSV, bool RANK>
+__global__ void __launch_bounds__(EGG_THREADS, (MlpCfg<H, CSV>::occ(ADAPT))) k_mlp(MlpParams p) { mlp_block<H, FIRST, SEED, ADAPT, CSV, RANK>(p, 0); }
+
 // ============================================================================ QKV
 template <int H, int CSV>
 struct QkvCfg {
@@ -657,14 +663,16 @@ __device__ __forceinline__ void rope_inplace(v16i *acc, const int32_t *rope_row,
 // noise are scaled when the per-member tables are filled, the input-side sums are taken term by term (dot_noise_ov), each
 // wave of a tile over its own column slice, and added up with the exchange of the normalised input.  Hidden 256, 2048
 // members x 256 tokens: 0.49 -> 0.32 ms with that and the float terms; without the overlay 0.29.
+// l: layers behind the one that p describes
 template <int H, bool ADAPT, int CSV>
-__global__ void __launch_bounds__(EGG_THREADS, (QkvCfg<H, CSV>::OCC)) k_qkv(QkvParams p) {
+__device__ __forceinline__ void qkv_block(const QkvParams &p, int l) {
     typedef QkvCfg<H, CSV> Q;
     constexpr int CS = Q::CS, KS = Q::KS, NTS = Q::NTS, HS = Q::HS;
     extern __shared__ __align__(16) int8_t smem[];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, g = lane >> 5, j = lane & 31;
     const FwdCommon &c = p.c;
-    const int T = c.T;
+    const int T = c.T, seed_base = p.seed_base + 1000 * l;
+    const int8_t *const ln_w = p.ln_w + l * H, *const ln_b = p.ln_b + l * H, *const w_q = p.w_q + l * H * H, *const w_k = p.w_k + l * H * H, *const w_v = p.w_v + l * H * H;
     const TileMap tm = tile_map<CS>(c.tn, wave, blockIdx.x);
     const int col0 = tm.cs * HS;
     constexpr int PSET = Q::per_set(ADAPT);
@@ -678,20 +686,20 @@ __global__ void __launch_bounds__(EGG_THREADS, (QkvCfg<H, CSV>::OCC)) k_qkv(QkvP
     WStream ws; wstream_init(ws, smem, Q::UNIT);
     const DmaPlan<Q::PR, H> plan = dma_plan<Q::PR, H>(H);
     auto pf = [&](const int8_t *W, int u) { w_prefetch2<Q::PR, H>(ws, W + (size_t)u * Q::PR * H * 16, plan); };
-    pf(p.w_q, 0);
+    pf(w_q, 0);
 
     for (int ss = 0; ss < tm.sets; ss++) {
         int ml = blockIdx.x * tm.sets + ss; if (ml >= c.n_members) ml = c.n_members - 1;
         const int mem = c.pop_offset + ml, nsx = (mem & 1) ? -1 : 1;
-        const uint32_t sbx = *c.d_step_seed + (uint32_t)(mem / 2) + (uint32_t)p.seed_base;
+        const uint32_t sbx = *c.d_step_seed + (uint32_t)(mem / 2) + (uint32_t)seed_base;
         int8_t *t2 = smem + Q::WBYTES + ss * PSET;
         int *lw = reinterpret_cast<int *>(t2), *lb = lw + H;
         int *a0 = lb + H, *a1 = a0 + H, *a2 = a1 + H;
         int8_t *b0 = reinterpret_cast<int8_t *>(a2 + H), *b1 = b0 + H, *b2 = b1 + H;
         const int tid = threadIdx.x;
         if (ADAPT) {
-            fill_vec_i32_ov(lw, p.ln_w, sbx + OFF_LN_1_A, sbx + OFF_LN_1_B, H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS, 2, p.q_ln_w);
-            fill_vec_i32_ov(lb, p.ln_b, sbx + OFF_LN_1_BIAS_A, sbx + OFF_LN_1_BIAS_B, H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS, 0, p.q_ln_b);
+            fill_vec_i32_ov(lw, ln_w, sbx + OFF_LN_1_A, sbx + OFF_LN_1_B, H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS, 2, p.q_ln_w);
+            fill_vec_i32_ov(lb, ln_b, sbx + OFF_LN_1_BIAS_A, sbx + OFF_LN_1_BIAS_B, H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS, 0, p.q_ln_b);
             fill_noise_i32_ov(a0, sbx + OFF_Q_A, H, c.mask, nsx << c.a_shift, tid, EGG_THREADS, p.q_wq + H);
             fill_noise_i32_ov(a1, sbx + OFF_K_A, H, c.mask, nsx << c.a_shift, tid, EGG_THREADS, p.q_wk + H);
             fill_noise_i32_ov(a2, sbx + OFF_V_A, H, c.mask, nsx << c.a_shift, tid, EGG_THREADS, p.q_wv + H);
@@ -700,8 +708,8 @@ __global__ void __launch_bounds__(EGG_THREADS, (QkvCfg<H, CSV>::OCC)) k_qkv(QkvP
             fill_noise_f32_ov(f0 + H, sbx + OFF_K_B, H, c.mask, tid, EGG_THREADS, p.q_wk);
             fill_noise_f32_ov(f0 + 2 * H, sbx + OFF_V_B, H, c.mask, tid, EGG_THREADS, p.q_wv);
         } else {
-            fill_vec_i32(lw, p.ln_w, sbx + OFF_LN_1_A, sbx + OFF_LN_1_B, H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS, 2);     // 4 * gain, see standard_scale
-            fill_vec_i32(lb, p.ln_b, sbx + OFF_LN_1_BIAS_A, sbx + OFF_LN_1_BIAS_B, H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS);
+            fill_vec_i32(lw, ln_w, sbx + OFF_LN_1_A, sbx + OFF_LN_1_B, H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS, 2);     // 4 * gain, see standard_scale
+            fill_vec_i32(lb, ln_b, sbx + OFF_LN_1_BIAS_A, sbx + OFF_LN_1_BIAS_B, H, c.mask, nsx, c.sigma_vec, tid, EGG_THREADS);
             fill_noise_i32(a0, sbx + OFF_Q_A, H, c.mask, nsx << c.a_shift, tid, EGG_THREADS);
             fill_noise_i32(a1, sbx + OFF_K_A, H, c.mask, nsx << c.a_shift, tid, EGG_THREADS);
             fill_noise_i32(a2, sbx + OFF_V_A, H, c.mask, nsx << c.a_shift, tid, EGG_THREADS);
@@ -744,8 +752,8 @@ __global__ void __launch_bounds__(EGG_THREADS, (QkvCfg<H, CSV>::OCC)) k_qkv(QkvP
         if (ADAPT && CS == 1) dot_noise_ov<KS, 3>(nrm, reinterpret_cast<const float *>(qB), H, g, sb3);
 #pragma unroll 1
         for (int which = 0; which < 3; which++) {
-            const int8_t *W = which == 0 ? p.w_q : (which == 1 ? p.w_k : p.w_v);
-            const int8_t *nw = which == 0 ? p.w_k : (which == 1 ? p.w_v : ((pass + 1 < tm.passes) ? p.w_q : nullptr));
+            const int8_t *W = which == 0 ? w_q : (which == 1 ? w_k : w_v);
+            const int8_t *nw = which == 0 ? w_k : (which == 1 ? w_v : ((pass + 1 < tm.passes) ? w_q : nullptr));
             const int8_t *Bn = which == 0 ? qB : (which == 1 ? kB : vB);
             const int *An = which == 0 ? qA : (which == 1 ? kA : vA);
             int8_t *dst = which == 0 ? p.q : (which == 1 ? p.k : p.v);
@@ -770,6 +778,9 @@ __global__ void __launch_bounds__(EGG_THREADS, (QkvCfg<H, CSV>::OCC)) k_qkv(QkvP
         }
     }
 }
+
+template <int H, bool ADAPT, int CSV>
+__global__ void __launch_bounds__(EGG_THREADS, (QkvCfg<H, CSV>::OCC)) k_qkv(QkvParams p) { qkv_block<H, ADAPT, CSV>(p, 0); }
 
 // ============================================================================ attention core
 // One wave per (member, head).  S^T = K.Q^T per 32x32 tile (lane = query token), two passes over the
@@ -830,8 +841,9 @@ __device__ __forceinline__ void attn_weights(const v16i &s, const int *lut, int 
 }
 __device__ __forceinline__ int attn_den(const int *den) { return den[0] + (den[1] << 7) + (den[2] << 14); }
 
+// one (member, head) by this wave; every wave of the workgroup calls it.  The table starts the LDS block.
 template <int HD, int CT>
-__global__ void __launch_bounds__(EGG_THREADS, (CT > 8 ? 1 : 2)) k_attn(AttnParams p) {
+__device__ __forceinline__ void attn_unit(const AttnParams &p, int unit, bool valid, int last4) {
     constexpr int KS = HD / 32, DT = HD / 32;
     constexpr int T = CT * 32;
     extern __shared__ __align__(16) int8_t smem[];
@@ -842,17 +854,9 @@ __global__ void __launch_bounds__(EGG_THREADS, (CT > 8 ? 1 : 2)) k_attn(AttnPara
 
     const FwdCommon &c = p.c;
     const int H = c.H, NH = H / HD;
-    int unit = blockIdx.x * EGG_WAVES + wave;
-    const bool valid = unit < c.n_members * NH;
-    if (!valid) unit = c.n_members * NH - 1;
     const int mloc = unit / NH, h = unit % NH;
     const size_t base = (size_t)mloc * T * H + (size_t)h * HD;
 
-    for (int i = threadIdx.x; i < 256; i += EGG_THREADS) {
-        const int w = c.exp_lut[i];
-        lut[i] = (w & 127) | (((w >> 7) & 127) << 8) | ((w >> 14) << 16);
-    }
-    const int last4 = attn_lut_last4(c.exp_lut, lut + 256, wave, lane);
     // All three row sets of this (member, head) are requested at once, so the wave waits for global memory once: the K
     // rows stay in registers until the V rows have left the row area, the Q rows go to LDS in the K rows' layout
     // (chunk c of row r at c ^ ((r / RPL) % CH), see below), the V rows to LDS rows [ctx][HD].
@@ -995,6 +999,60 @@ __global__ void __launch_bounds__(EGG_THREADS, (CT > 8 ? 1 : 2)) k_attn(AttnPara
             }
             if (valid) store_op(p.ao + base + (size_t)t * H, dt, g, outp);
         }
+    }
+}
+// the units [first, end), a wave each
+template <int HD, int CT>
+__device__ __forceinline__ void attn_block(const AttnParams &p, int first, int end) {
+    extern __shared__ __align__(16) int8_t smem[];
+    int *lut = reinterpret_cast<int *>(smem);
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    for (int i = threadIdx.x; i < 256; i += EGG_THREADS) {
+        const int w = p.c.exp_lut[i];
+        lut[i] = (w & 127) | (((w >> 7) & 127) << 8) | ((w >> 14) << 16);
+    }
+    const int last4 = attn_lut_last4(p.c.exp_lut, lut + 256, wave, lane);
+#pragma unroll 1
+    for (; first < end; first += EGG_WAVES) attn_unit<HD, CT>(p, min(first + wave, end - 1), first + wave < end, last4);
+}
+template <int HD, int CT>
+__global__ void __launch_bounds__(EGG_THREADS, (CT > 8 ? 1 : 2)) k_attn(AttnParams p) {
+    const int first = blockIdx.x * EGG_WAVES;
+    attn_block<HD, CT>(p, first, min(first + EGG_WAVES, p.c.n_members * (p.c.H / HD)));
+}
+
+// ============================================================================ short windows: the blocks of a model in one launch
+// Up to the head every stage of a member depends on that member alone, and k_mlp and k_qkv deal whole members to the workgroups in the same way.
+// Where all workgroups are resident at once, a launch of each stage costs more than its start: the next one begins when the last workgroup of the one
+// in front is through, and its tables and first weights are fetched with nothing else to do.  Here a workgroup goes through the embedding, the
+// initial MLP and all layers by itself; what its waves pass on (q, k, v, ao, x) they write and read through their CU's cache, and a barrier is all that
+// separates the stages.  Forward with the head, members x tokens: hidden 64, 2 layers 64 x 32 56 -> 52 us, 2,048 x 32 106 -> 84; hidden 64, 3 layers
+// 1,000 x 64 120 -> 101; hidden 128, 3 layers 1,002 x 64 217 -> 182, 2,000 x 32 225 -> 196; head width 64 gains the same.
+// Up to 512 workgroups, two to a CU: the stages by themselves hold three or four, and with a second round 1,026 x 64 take
+// 285 us instead of 240 at hidden 128 and 155 instead of 132 at 64.  (At 168 and 128 registers, for three and four workgroups, hidden 64 loses up to 8 and
+// 40 % of what it gains: the attention spills.)
+constexpr int BLOCKS_GROUPS = 512;
+template <int H, int HD, int CT, int CSV>
+struct Blocks {
+    static int cmax(int a, int b) { return a > b ? a : b; }
+    static int lds(int sets) {
+        return cmax(cmax(MlpCfg<H, CSV>::total(sets, true, false, true), MlpCfg<H, CSV>::total(sets, false, false, true)),
+                    cmax(QkvCfg<H, CSV>::total(sets, false), 2048 + EGG_WAVES * 2 * CT * 32 * HD));
+    }
+};
+template <int H, int HD, int CT, int CSV>
+__global__ void __launch_bounds__(EGG_THREADS, 2) k_blocks(BlocksParams p) {
+    const int sets = tile_map<CSV>(CT * 32, 0, 0).sets, NH = H / HD;
+    const int first = blockIdx.x * sets * NH, end = min(first + sets * NH, p.attn.c.n_members * NH);
+    mlp_block<H, true, true, false, CSV, true>(p.first, 0);
+#pragma unroll 1
+    for (int l = 0; l < p.layers; l++) {
+        __syncthreads();
+        qkv_block<H, false, CSV>(p.qkv, l);
+        __syncthreads();
+        attn_block<HD, CT>(p.attn, first, end);
+        __syncthreads();
+        mlp_block<H, false, true, false, CSV, true>(p.mlp, l);
     }
 }
 
@@ -1646,6 +1704,37 @@ hipError_t egg_launch_attn(const AttnParams &p, hipStream_t s) {
     }
 }
 
+template <int H, int HD, int CT, int CSV>
+static hipError_t launch_blocks_cs(const BlocksParams &p, bool *taken, hipStream_t s) {
+    const int sets = tile_map_sets(CT * 32, CSV), groups = (p.qkv.c.n_members + sets - 1) / sets, lds = Blocks<H, HD, CT, CSV>::lds(sets);
+    *taken = groups <= BLOCKS_GROUPS && lds <= 80 * 1024;
+    if (!*taken) return hipSuccess;
+    hipLaunchKernelGGL((k_blocks<H, HD, CT, CSV>), dim3(groups), dim3(EGG_THREADS), lds, s, p);
+    return hipGetLastError();
+}
+template <int H, int HD, int CT>
+static hipError_t launch_blocks_ct(const BlocksParams &p, bool *taken, hipStream_t s) {
+    if (use_many_slices<H>(p.qkv.c)) return launch_blocks_cs<H, HD, CT, many_slices<H>()>(p, taken, s);
+    return launch_blocks_cs<H, HD, CT, few_slices<H>()>(p, taken, s);
+}
+template <int H>
+static hipError_t launch_blocks_h(const BlocksParams &p, bool *taken, hipStream_t s) {
+    const FwdCommon &c = p.qkv.c;
+    // the forms that the stages would take, of which k_blocks holds one each
+    if (egg_mlp_up_acc_bound(H, c.mask, c.sigma_vec, c.shift_mlp_up) >= (1LL << 31) || egg_mlp_down_acc_bound(H, c.mask, c.sigma_vec, c.shift_mlp_down) >= (1LL << 31) ||
+        egg_out_acc_bound(H, c.mask, c.shift_out) >= (1LL << 31) || !egg_rank1_kstep(H, c.mask, c.sigma)) return hipSuccess;
+    if (c.T == 32) return c.head_dim == 32 ? launch_blocks_ct<H, 32, 1>(p, taken, s) : launch_blocks_ct<H, 64, 1>(p, taken, s);
+    return c.head_dim == 32 ? launch_blocks_ct<H, 32, 2>(p, taken, s) : launch_blocks_ct<H, 64, 2>(p, taken, s);
+}
+hipError_t egg_launch_blocks(const BlocksParams &p, bool *taken, hipStream_t s) {
+    *taken = false;
+    const FwdCommon &c = p.qkv.c;
+    if (c.t0 || c.tn != c.T || (c.T != 32 && c.T != 64) || (c.head_dim != 32 && c.head_dim != 64)) return hipSuccess;
+    if (c.H == 64) return launch_blocks_h<64>(p, taken, s);
+    if (c.H == 128) return launch_blocks_h<128>(p, taken, s);
+    return hipSuccess;
+}
+
 template <int H, bool ADAPT>
 static hipError_t launch_head_big(const HeadParams &p, hipStream_t s) {
     const int sets = tile_map_sets(p.c.tn, 1), tiles = p.c.tn / 32;
@@ -1736,6 +1825,20 @@ static hipError_t prepare_h(int T) {
     SET_LDS((k_head_big<H, true, true>), BigHead<H>::total(hsets, true, true));
     return hipSuccess;
 }
+template <int H, int HD, int CT, int CSV>
+static hipError_t prepare_blocks_cs() {
+    const hipError_t e = no_static_lds(&k_blocks<H, HD, CT, CSV>);
+    if (e != hipSuccess) return e;
+    SET_LDS((k_blocks<H, HD, CT, CSV>), (Blocks<H, HD, CT, CSV>::lds(tile_map_sets(CT * 32, CSV))));
+    return hipSuccess;
+}
+template <int H, int HD>
+static hipError_t prepare_blocks(int T) {
+    for (hipError_t e : {T == 32 ? prepare_blocks_cs<H, HD, 1, few_slices<H>()>() : prepare_blocks_cs<H, HD, 2, few_slices<H>()>(),
+                         T == 32 ? prepare_blocks_cs<H, HD, 1, many_slices<H>()>() : prepare_blocks_cs<H, HD, 2, many_slices<H>()>()})
+        if (e != hipSuccess) return e;
+    return hipSuccess;
+}
 template <int HD, int CT>
 static hipError_t prepare_attn() {
     if constexpr (CT % 8 == 0) SET_LDS((k_attn_wg<HD, CT>), (AttnWg<HD, CT>::LDS));
@@ -1762,6 +1865,8 @@ hipError_t egg_prepare_forward(int H, int head_dim, int T) {
         case 512: e = prepare_h<512>(T); break;
         default: return hipErrorInvalidValue;
     }
+    if (e == hipSuccess && (H == 64 || H == 128) && T <= 64)
+        e = H == 64 ? (head_dim == 32 ? prepare_blocks<64, 32>(T) : prepare_blocks<64, 64>(T)) : (head_dim == 32 ? prepare_blocks<128, 32>(T) : prepare_blocks<128, 64>(T));
     if (e != hipSuccess) return e;
     return head_dim == 32 ? prepare_attn_hd<32>(T / 32) : (head_dim == 64 ? prepare_attn_hd<64>(T / 32) : hipErrorInvalidValue);
 }

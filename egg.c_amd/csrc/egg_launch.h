@@ -8,6 +8,7 @@
 hipError_t egg_launch_mlp(const MlpParams &p, bool first, hipStream_t s);
 hipError_t egg_launch_qkv(const QkvParams &p, hipStream_t s);
 hipError_t egg_launch_attn(const AttnParams &p, hipStream_t s);
+hipError_t egg_launch_blocks(const BlocksParams &p, bool *taken, hipStream_t s);      // taken: false where the stages are to be launched one by one
 hipError_t egg_launch_head(const HeadParams &p, hipStream_t s);
 hipError_t egg_prepare_forward(int H, int head_dim, int T);
 

@@ -126,6 +126,14 @@ struct AttnParams {
     int8_t *ao;
 };
 
+// the blocks of a whole model; qkv and mlp describe layer 0, the others follow it in the blob and in the fragment-major copies
+struct BlocksParams {
+    MlpParams first, mlp;
+    QkvParams qkv;
+    AttnParams attn;
+    int layers;
+};
+
 struct HeadParams {
     FwdCommon c;
     const int8_t *ln_w, *ln_b;
