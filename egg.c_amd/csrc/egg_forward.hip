@@ -8,6 +8,7 @@
 //   k_qkv<H,..>     LN1 + Q/K/V projections + RoPE + norms (mgpu.cu:769-784)
 //   k_attn<HD,CT>   causal exp-LUT attention core          (mgpu.cu:787-825)
 //   k_mlp<H,false>  O-projection + residual norm + MLP     (mgpu.cu:827-831, :708-759)
+//   k_blocks<..>    all of the above in one launch, for small populations of short windows
 //   k_head<H>       final norm + tied head + loss          (mgpu.cu:955-1028)
 #include <algorithm>
 #include "egg_device.h"
@@ -151,7 +152,7 @@ struct MlpCfg {
     static constexpr int per_set(bool first, bool adapt, bool rank) { return PER_SET + (!rank && up32(first) ? UPA32 : 0) - (first ? 0 : 4 * H) + (adapt ? 3 * 6 * H : 0); }
     // The up projection's rank-one term as one more k-step (rank1_token) instead of a multiply, an add and a quarter of an LDS read an element, for
     // the noise that egg_rank1_kstep allows.  It costs the registers of the token's operand and of a row: 8,192 members x 256 tokens at hidden 256
-    // 1.64 -> 1.58 ms, 2,048 x 512 at hidden 512 3.01 -> 2.96 (7 more registers in scratch across a pass), 16,384 x 128 at hidden 64 0.246 -> 0.235,
+    // 1.64 -> 1.58 ms, 2,048 x 512 at hidden 512 3.01 -> 2.96 (9 registers in scratch across a pass, not 6), 16,384 x 128 at hidden 64 0.246 -> 0.235,
     // 8,192 x 128 at hidden 128 0.296 -> 0.291 at three workgroups per CU as before (0.335 at two, which its 178 registers would give).  Hidden 256 with two
     // slices would keep 8 registers in scratch: 80 -> 83 us for 2,048 members of 32 tokens, so it has the other form only.
     static constexpr bool RANK1 = !(H == 256 && CS == 2);
@@ -169,8 +170,8 @@ struct MlpCfg {
 // read again, 2 of 5 bytes that the kernel moves -- and the epilogue neither extracts nor adds it.  Hidden 256, 40,960
 // members x 256 tokens: 9.33 -> 8.97 ms a launch, hidden 512, 2,048 x 512: 3.12 -> 3.05 ms (the residual stays in
 // registers until the accumulator is live: seeded in front of the norm, hidden 512 spills in its sub-chunk loop and takes
-// 3.85 ms.  As it is, hidden 512 still keeps 6 registers -- the first block 21 -- in scratch across a pass: 7 and 30 accesses a
-// pass, none in the sub-chunk loop; without SEED it keeps none).
+// 3.85 ms.  As it is, hidden 512 still keeps 6 to 9 registers -- the first block 23 -- in scratch across a pass: 7 and 31 accesses a
+// pass, none in the sub-chunk loop; without SEED none, or 4).
 // ADAPT: the d-eggs adaptive noise overlay is on (de/include/model/layers.cuh:215-296, :432-438,
 // de/src/kernels.cu:139-158); see k_qkv.  The down projection's input-side sum follows the reference thread of a
 // hidden unit, which adds its four terms (k = unit, unit + H, ...) into an int one float addition at a time; the
