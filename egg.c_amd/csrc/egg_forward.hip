@@ -1028,16 +1028,19 @@ __global__ void __launch_bounds__(EGG_THREADS, (CT > 8 ? 1 : 2)) k_attn(AttnPara
 // in front is through, and its tables and first weights are fetched with nothing else to do.  Here a workgroup goes through the embedding, the
 // initial MLP and all layers by itself; what its waves pass on (q, k, v, ao, x) they write and read through their CU's cache, and a barrier is all that
 // separates the stages.  Forward with the head, members x tokens: hidden 64, 2 layers 64 x 32 56 -> 52 us, 2,048 x 32 106 -> 84; hidden 64, 3 layers
-// 1,000 x 64 120 -> 101; hidden 128, 3 layers 1,002 x 64 217 -> 182, 2,000 x 32 225 -> 196; head width 64 gains the same.
+// 1,000 x 64 120 -> 101; hidden 128, 3 layers 1,002 x 64 217 -> 182, 2,000 x 32 225 -> 196; hidden 256, 4 layers 64 x 32 187 -> 180,
+// 1,000 x 32 331 -> 288, 400 x 64 305 -> 273; head width 64 gains the same.
 // Up to 512 workgroups, two to a CU: the stages by themselves hold three or four, and with a second round 1,026 x 64 take
 // 285 us instead of 240 at hidden 128 and 155 instead of 132 at 64.  (At 168 and 128 registers, for three and four workgroups, hidden 64 loses up to 8 and
-// 40 % of what it gains: the attention spills.)
+// 40 % of what it gains: the attention spills.)  With one column slice at hidden 256, half as many workgroups of twice the work, 770 x 64 take 296 us instead
+// of 276: not taken.
 constexpr int BLOCKS_GROUPS = 512;
 template <int H, int HD, int CT, int CSV>
 struct Blocks {
+    static constexpr bool RANK = MlpCfg<H, CSV>::RANK1;
     static int cmax(int a, int b) { return a > b ? a : b; }
     static int lds(int sets) {
-        return cmax(cmax(MlpCfg<H, CSV>::total(sets, true, false, true), MlpCfg<H, CSV>::total(sets, false, false, true)),
+        return cmax(cmax(MlpCfg<H, CSV>::total(sets, true, false, RANK), MlpCfg<H, CSV>::total(sets, false, false, RANK)),
                     cmax(QkvCfg<H, CSV>::total(sets, false), 2048 + EGG_WAVES * 2 * CT * 32 * HD));
     }
 };
@@ -1045,7 +1048,8 @@ template <int H, int HD, int CT, int CSV>
 __global__ void __launch_bounds__(EGG_THREADS, 2) k_blocks(BlocksParams p) {
     const int sets = tile_map<CSV>(CT * 32, 0, 0).sets, NH = H / HD;
     const int first = blockIdx.x * sets * NH, end = min(first + sets * NH, p.attn.c.n_members * NH);
-    mlp_block<H, true, true, false, CSV, true>(p.first, 0);
+    constexpr bool RANK = Blocks<H, HD, CT, CSV>::RANK;
+    mlp_block<H, true, true, false, CSV, RANK>(p.first, 0);
 #pragma unroll 1
     for (int l = 0; l < p.layers; l++) {
         __syncthreads();
@@ -1053,7 +1057,7 @@ __global__ void __launch_bounds__(EGG_THREADS, 2) k_blocks(BlocksParams p) {
         __syncthreads();
         attn_block<HD, CT>(p.attn, first, end);
         __syncthreads();
-        mlp_block<H, false, true, false, CSV, true>(p.mlp, l);
+        mlp_block<H, false, true, false, CSV, RANK>(p.mlp, l);
     }
 }
 
@@ -1716,6 +1720,7 @@ static hipError_t launch_blocks_cs(const BlocksParams &p, bool *taken, hipStream
 template <int H, int HD, int CT>
 static hipError_t launch_blocks_ct(const BlocksParams &p, bool *taken, hipStream_t s) {
     if (use_many_slices<H>(p.qkv.c)) return launch_blocks_cs<H, HD, CT, many_slices<H>()>(p, taken, s);
+    if constexpr (H == 256) if (use_one_slice_qkv(p.qkv.c)) return hipSuccess;
     return launch_blocks_cs<H, HD, CT, few_slices<H>()>(p, taken, s);
 }
 template <int H>
@@ -1733,6 +1738,7 @@ hipError_t egg_launch_blocks(const BlocksParams &p, bool *taken, hipStream_t s) 
     if (c.t0 || c.tn != c.T || (c.T != 32 && c.T != 64) || (c.head_dim != 32 && c.head_dim != 64)) return hipSuccess;
     if (c.H == 64) return launch_blocks_h<64>(p, taken, s);
     if (c.H == 128) return launch_blocks_h<128>(p, taken, s);
+    if (c.H == 256) return launch_blocks_h<256>(p, taken, s);
     return hipSuccess;
 }
 
@@ -1866,8 +1872,9 @@ hipError_t egg_prepare_forward(int H, int head_dim, int T) {
         case 512: e = prepare_h<512>(T); break;
         default: return hipErrorInvalidValue;
     }
-    if (e == hipSuccess && (H == 64 || H == 128) && T <= 64)
-        e = H == 64 ? (head_dim == 32 ? prepare_blocks<64, 32>(T) : prepare_blocks<64, 64>(T)) : (head_dim == 32 ? prepare_blocks<128, 32>(T) : prepare_blocks<128, 64>(T));
+    if (e == hipSuccess && H <= 256 && T <= 64)
+        e = H == 64 ? (head_dim == 32 ? prepare_blocks<64, 32>(T) : prepare_blocks<64, 64>(T)) : H == 128 ? (head_dim == 32 ? prepare_blocks<128, 32>(T) : prepare_blocks<128, 64>(T))
+                    : (head_dim == 32 ? prepare_blocks<256, 32>(T) : prepare_blocks<256, 64>(T));
     if (e != hipSuccess) return e;
     return head_dim == 32 ? prepare_attn_hd<32>(T / 32) : (head_dim == 64 ? prepare_attn_hd<64>(T / 32) : hipErrorInvalidValue);
 }

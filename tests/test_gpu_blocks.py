@@ -1,5 +1,5 @@
 """A model's blocks in one launch (k_blocks) against the same stages launched one by one (which timed contexts take) and, for sampled members, against
-the oracle: short windows, both head widths, full and partial last workgroups, few and many column slices, and populations on both sides of the line."""
+the oracle: short windows, all hidden sizes that take it, both head widths, full and partial last workgroups, few and many column slices, and populations on both sides of the line."""
 import numpy as np
 import pytest
 
@@ -17,6 +17,12 @@ pytestmark = pytest.mark.gpu
     dict(hidden=128, head_dim=64, seq_len=64, population=1024, n_layers=1),
     dict(hidden=128, head_dim=32, seq_len=32, population=1030, n_layers=2),
     dict(hidden=128, head_dim=64, seq_len=32, population=6, n_layers=2, vocab=512),
+    dict(hidden=256, head_dim=64, seq_len=32, population=6, n_layers=2),
+    dict(hidden=256, head_dim=32, seq_len=64, population=250, n_layers=2),          # two passes: the first block once per byte value
+    dict(hidden=256, head_dim=64, seq_len=64, population=512, n_layers=1),
+    dict(hidden=256, head_dim=64, seq_len=64, population=514, n_layers=1),
+    dict(hidden=256, head_dim=64, seq_len=32, population=1002, n_layers=2),
+    dict(hidden=256, head_dim=64, seq_len=64, population=770, n_layers=1),          # one column slice: stage by stage
     dict(hidden=128, head_dim=32, seq_len=32, population=130, n_layers=2, noise_mask=31),     # noise that the launch does not take
     dict(hidden=64, head_dim=32, seq_len=32, population=130, n_layers=2, use_same_data=1)],
     ids=lambda kw: "h%(hidden)d_d%(head_dim)d_t%(seq_len)d_p%(population)d" % kw)
