@@ -1029,7 +1029,7 @@ __global__ void __launch_bounds__(EGG_THREADS, (CT > 8 ? 1 : 2)) k_attn(AttnPara
 // initial MLP and all layers by itself; what its waves pass on (q, k, v, ao, x) they write and read through their CU's cache, and a barrier is all that
 // separates the stages.  Forward with the head, members x tokens: hidden 64, 2 layers 64 x 32 56 -> 52 us, 2,048 x 32 106 -> 84; hidden 64, 3 layers
 // 1,000 x 64 120 -> 101; hidden 128, 3 layers 1,002 x 64 217 -> 182, 2,000 x 32 225 -> 196; hidden 256, 4 layers 64 x 32 187 -> 180,
-// 1,000 x 32 331 -> 288, 400 x 64 305 -> 273; head width 64 gains the same.
+// 1,000 x 32 331 -> 288, 400 x 64 305 -> 273; 250 x 128 450 -> 422, hidden 128, 3 layers 300 x 128 208 -> 185; head width 64 gains the same.
 // Up to 512 workgroups, two to a CU: the stages by themselves hold three or four, and with a second round 1,026 x 64 take
 // 285 us instead of 240 at hidden 128 and 155 instead of 132 at 64.  (At 168 and 128 registers, for three and four workgroups, hidden 64 loses up to 8 and
 // 40 % of what it gains: the attention spills.)  With one column slice at hidden 256, half as many workgroups of twice the work, 770 x 64 take 296 us instead
@@ -1730,12 +1730,13 @@ static hipError_t launch_blocks_h(const BlocksParams &p, bool *taken, hipStream_
     if (egg_mlp_up_acc_bound(H, c.mask, c.sigma_vec, c.shift_mlp_up) >= (1LL << 31) || egg_mlp_down_acc_bound(H, c.mask, c.sigma_vec, c.shift_mlp_down) >= (1LL << 31) ||
         egg_out_acc_bound(H, c.mask, c.shift_out) >= (1LL << 31) || !egg_rank1_kstep(H, c.mask, c.sigma)) return hipSuccess;
     if (c.T == 32) return c.head_dim == 32 ? launch_blocks_ct<H, 32, 1>(p, taken, s) : launch_blocks_ct<H, 64, 1>(p, taken, s);
-    return c.head_dim == 32 ? launch_blocks_ct<H, 32, 2>(p, taken, s) : launch_blocks_ct<H, 64, 2>(p, taken, s);
+    if (c.T == 64) return c.head_dim == 32 ? launch_blocks_ct<H, 32, 2>(p, taken, s) : launch_blocks_ct<H, 64, 2>(p, taken, s);
+    return c.head_dim == 32 ? launch_blocks_ct<H, 32, 4>(p, taken, s) : launch_blocks_ct<H, 64, 4>(p, taken, s);
 }
 hipError_t egg_launch_blocks(const BlocksParams &p, bool *taken, hipStream_t s) {
     *taken = false;
     const FwdCommon &c = p.qkv.c;
-    if (c.t0 || c.tn != c.T || (c.T != 32 && c.T != 64) || (c.head_dim != 32 && c.head_dim != 64)) return hipSuccess;
+    if (c.t0 || c.tn != c.T || (c.T != 32 && c.T != 64 && c.T != 128) || (c.head_dim != 32 && c.head_dim != 64)) return hipSuccess;
     if (c.H == 64) return launch_blocks_h<64>(p, taken, s);
     if (c.H == 128) return launch_blocks_h<128>(p, taken, s);
     if (c.H == 256) return launch_blocks_h<256>(p, taken, s);
@@ -1841,8 +1842,8 @@ static hipError_t prepare_blocks_cs() {
 }
 template <int H, int HD>
 static hipError_t prepare_blocks(int T) {
-    for (hipError_t e : {T == 32 ? prepare_blocks_cs<H, HD, 1, few_slices<H>()>() : prepare_blocks_cs<H, HD, 2, few_slices<H>()>(),
-                         T == 32 ? prepare_blocks_cs<H, HD, 1, many_slices<H>()>() : prepare_blocks_cs<H, HD, 2, many_slices<H>()>()})
+    for (hipError_t e : {T == 32 ? prepare_blocks_cs<H, HD, 1, few_slices<H>()>() : T == 64 ? prepare_blocks_cs<H, HD, 2, few_slices<H>()>() : prepare_blocks_cs<H, HD, 4, few_slices<H>()>(),
+                         T == 32 ? prepare_blocks_cs<H, HD, 1, many_slices<H>()>() : T == 64 ? prepare_blocks_cs<H, HD, 2, many_slices<H>()>() : prepare_blocks_cs<H, HD, 4, many_slices<H>()>()})
         if (e != hipSuccess) return e;
     return hipSuccess;
 }
@@ -1872,7 +1873,7 @@ hipError_t egg_prepare_forward(int H, int head_dim, int T) {
         case 512: e = prepare_h<512>(T); break;
         default: return hipErrorInvalidValue;
     }
-    if (e == hipSuccess && H <= 256 && T <= 64)
+    if (e == hipSuccess && H <= 256 && T <= 128)
         e = H == 64 ? (head_dim == 32 ? prepare_blocks<64, 32>(T) : prepare_blocks<64, 64>(T)) : H == 128 ? (head_dim == 32 ? prepare_blocks<128, 32>(T) : prepare_blocks<128, 64>(T))
                     : (head_dim == 32 ? prepare_blocks<256, 32>(T) : prepare_blocks<256, 64>(T));
     if (e != hipSuccess) return e;

@@ -18,6 +18,12 @@ pytestmark = pytest.mark.gpu
     dict(hidden=128, head_dim=32, seq_len=32, population=1030, n_layers=2),
     dict(hidden=128, head_dim=64, seq_len=32, population=6, n_layers=2, vocab=512),
     dict(hidden=256, head_dim=64, seq_len=32, population=6, n_layers=2),
+    dict(hidden=64, head_dim=64, seq_len=128, population=130, n_layers=2),
+    dict(hidden=64, head_dim=32, seq_len=128, population=512, n_layers=1),
+    dict(hidden=128, head_dim=64, seq_len=128, population=66, n_layers=2),
+    dict(hidden=128, head_dim=32, seq_len=128, population=514, n_layers=1),         # stage by stage
+    dict(hidden=256, head_dim=64, seq_len=128, population=130, n_layers=2),
+    dict(hidden=256, head_dim=32, seq_len=128, population=302, n_layers=1),
     dict(hidden=256, head_dim=32, seq_len=64, population=250, n_layers=2),          # two passes: the first block once per byte value
     dict(hidden=256, head_dim=64, seq_len=64, population=512, n_layers=1),
     dict(hidden=256, head_dim=64, seq_len=64, population=514, n_layers=1),
