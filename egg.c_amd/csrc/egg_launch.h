@@ -135,7 +135,7 @@ hipError_t egg_launch_ternary_unpack(const uint8_t *packed, int8_t *dst, int n_e
 hipError_t egg_launch_ternary_pack(const int8_t *src, uint8_t *packed, int n_elems, int *d_bad, hipStream_t s);
 
 // Muon chain (muon_internal.cuh:15-342): momentum + gather (epilogue of the votes), Frobenius normalisation,
-// 5 Newton-Schulz iterations on fp32 MFMA, quantised apply (egg_launch_muon_apply).
+// 5 Newton-Schulz iterations with products at float32 accuracy, quantised apply (egg_launch_muon_apply).
 struct MuonWork { float *x, *swap, *gram, *bterm, *partials, *norm; };   // x/swap: rows*cols, gram/bterm: K*K, partials: 1024
 hipError_t egg_launch_newton_schulz(const MuonWork &w, int rows, int cols, int iters, hipStream_t s);
 hipError_t egg_launch_newton_schulz_batched(const MuonWork &w, int rows, int cols, int iters, int batch, hipStream_t s, const float **result);

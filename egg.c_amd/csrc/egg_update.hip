@@ -351,12 +351,19 @@ __global__ void __launch_bounds__(EGG_THREADS) k_sgemm(const float *A, long lda,
 // current one run, and those of the one behind it).
 // The float32 matrix instruction does 64 multiplications a clock and SIMD, the bf16 one 1,024, so every operand is taken apart on its
 // way into LDS: x = x0 + x1 + x2, each the nearest bf16 of what is left (8 + 8 + 8 bits: 24, the float's own), and a product is
-// the six partial products of at least 2^-18 of it: x0 y0, x0 y1, x1 y0, x1 y1, x0 y2, x2 y0.  They are exact, what is left out is below 2^-26 of
-// the product, a quarter of the rounding of one float32 addition; they are added in float32, the smallest first.  Five iterations
-// against 64 bits are nearer than with the float32 instruction: relative error of random matrices 9.1e-7 -> 6.0e-7 at 512 x 512, 4.2e-7 -> 2.7e-7 at
-// 512 x 2048, 3.3e-7 -> 2.6e-7 at 64 x 64, rank one 6.2e-6 -> 4.0e-6 (rows scaled over e^4 4.2e-7 -> 4.3e-7 and 9.7e-7 -> 6.8e-7).  Times: G (upper half) of 32
-// matrices of 512 x 512 63 -> 60 us, X B of them 89 -> 64, 2048 x 512 x 512 of nine 127 -> 82, and the products of nine 512 x 512 38 -> 26.5:
-// those are 16 chunks one after the other, at one to three workgroups a CU.
+// eight exact partial products: all but x2 y2, which is below 2^-34 of it.  (x1 y2 and x2 y1 reach 2^-24, half a unit of the last place.)
+// The bf16 instruction aligns its sixteen products and its addend to the largest of them, so a product that meets a smaller sum can be off by
+// a whole unit of the last place and a long sum is rounded once for each instruction.  Therefore the sum over k does not pass through
+// it: x0 y0 of a chunk of 32 k and the seven others, smallest first, each start from zero, and their sum is added to the accumulator by the
+// vector unit, one rounding for 32 k where the float32 instruction has sixteen; a single product is rounded as float32 multiplication rounds it.
+// Relative errors of five iterations against 64 bits, float32 instruction -> this: random matrices 9.1e-7 -> 2.7e-7 at 512 x 512, 4.2e-7 -> 1.3e-7 at
+// 512 x 2048, 3.3e-7 -> 1.7e-7 at 64 x 64; rank one 6.2e-6 -> 1.4e-6; rows scaled over e^4 9.7e-7 -> 2.7e-7 and 3.9e-7 -> 1.6e-7, columns 3.5e-7 -> 2.3e-7 and
+// 1.05e-6 -> 3.8e-7; two elements a row, where hardly anything is summed, 1.3e-7 -> 1.3e-7 (0.83 to 1.03 of it over the sizes).  (One
+// accumulator through all instructions: 6.0e-7, 2.7e-7, 2.5e-7, 3.9e-6; 1.6 times the float32 instruction's for columns scaled over e^4 at 2048 x 512, 1.3 times for
+// two elements a row.)  Parts below 2^-126, so of elements below 2^-110 of the matrix' norm, are lost.
+// Times, float32 instruction -> this: G (upper half) of 32 matrices of 512 x 512 56 -> 61 us, X B of them 80 -> 69, G of nine 512 x 2048 83 -> 76 and
+// 2048 x 512 84 -> 87, their X P 111 and 123 -> 102, products of nine 512 x 512 30 -> 25, of eighteen 41 -> 34: those are 16 chunks one after the other, at one to three workgroups a CU.
+// The whole chain of a model of hidden 64 / 128 / 256 / 512: 0.26 / 0.33 / 0.48 / 1.76 -> 0.25 / 0.32 / 0.47 / 1.60 ms.
 // An operand sits in LDS as three planes [row][k] of bf16 with rows 80 bytes apart (a lane reads eight consecutive k of its row as 16
 // bytes; 16 such rows fall on all banks once).  One whose k stride is not 1 is turned over on the way: a thread
 // takes four rows at two consecutive k.
@@ -407,7 +414,7 @@ __device__ __forceinline__ void split_bf16(float a, float b, uint32_t *pl) {
 template <bool AK, bool BK, int WT, bool SYM>
 __global__ void __launch_bounds__(EGG_THREADS, WT == 1 ? 3 : 2) k_sgemm_lds(SgemmJobs jobs, long lda, const float *B, long ldb, long batch_b, int M, int N, int K) {
     constexpr int TILE = 64 * WT, KC = 32, ROW = 80, PLANE = TILE * ROW, PIECES = TILE * KC / 4 / EGG_THREADS;
-    constexpr int AHEAD = 2;
+    constexpr int AHEAD = WT == 2 ? 1 : 2;      // (two chunks ahead do not fit the registers beside WT = 2's accumulators)
     __shared__ __align__(16) int8_t As[NS_PLANES * PLANE];
     __shared__ __align__(16) int8_t Bs[NS_PLANES * PLANE];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 5, j = lane & 31, tid = threadIdx.x;
@@ -484,25 +491,30 @@ __global__ void __launch_bounds__(EGG_THREADS, WT == 1 ? 3 : 2) k_sgemm_lds(Sgem
         store_operand(b_kone, Bs, rb[n]);
         __syncthreads();
         load_chunk(n, k0 + AHEAD * KC);
+        constexpr int STEPS = KC / 16, LOW = 7, PA[LOW] = {2, 1, 2, 0, 1, 1, 0}, PB[LOW] = {1, 2, 0, 2, 1, 0, 1};      // the partial products below x0 y0, smallest first
+        v8bf a[STEPS][WT][NS_PLANES], b[STEPS][WT][NS_PLANES];
 #pragma unroll
-        for (int c = 0; c < KC / 16; c++) {
-            v8bf a[WT][NS_PLANES], b[WT][NS_PLANES];
+        for (int c = 0; c < STEPS; c++)
 #pragma unroll
             for (int t = 0; t < WT; t++)
 #pragma unroll
                 for (int pl = 0; pl < NS_PLANES; pl++) {
-                    a[t][pl] = *reinterpret_cast<const v8bf *>(As + pl * PLANE + (32 * WT * wm + 32 * t + j) * ROW + 32 * c + 16 * g);
-                    b[t][pl] = *reinterpret_cast<const v8bf *>(Bs + pl * PLANE + (32 * WT * wn + 32 * t + j) * ROW + 32 * c + 16 * g);
+                    a[c][t][pl] = *reinterpret_cast<const v8bf *>(As + pl * PLANE + (32 * WT * wm + 32 * t + j) * ROW + 32 * c + 16 * g);
+                    b[c][t][pl] = *reinterpret_cast<const v8bf *>(Bs + pl * PLANE + (32 * WT * wn + 32 * t + j) * ROW + 32 * c + 16 * g);
                 }
-            constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};
 #pragma unroll
-            for (int m = 0; m < 6; m++)
+        for (int ta = 0; ta < WT; ta++)
 #pragma unroll
-                for (int ta = 0; ta < WT; ta++)
+            for (int tb = 0; tb < WT; tb++) {
+                v16f top = {}, low = {};
 #pragma unroll
-                    for (int tb = 0; tb < WT; tb++)
-                        acc[ta][tb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[ta][PA[m]], b[tb][PB[m]], acc[ta][tb], 0, 0, 0);
-        }
+                for (int c = 0; c < STEPS; c++) top = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[c][ta][0], b[c][tb][0], top, 0, 0, 0);
+#pragma unroll
+                for (int c = 0; c < STEPS; c++)
+#pragma unroll
+                    for (int m = 0; m < LOW; m++) low = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[c][ta][PA[m]], b[c][tb][PB[m]], low, 0, 0, 0);
+                acc[ta][tb] += top + low;
+            }
     };
 #pragma unroll
     for (int n = 0; n < AHEAD; n++) load_chunk(n, n * KC);
