@@ -315,7 +315,8 @@ static std::vector<MatDesc> matrix_descs(egg_ctx *ctx) {
             MatDesc d;
             d.W = ctx->d_model + t.offset; d.frag = ctx->d_wfrag + t.offset; d.offset = t.offset;
             d.state = reinterpret_cast<float *>(ctx->d_state + ctx->t_state_off[ids[b]]);
-            d.muon_x = muon ? ctx->muon.x + b * (size_t)t.rows * t.cols : nullptr;
+            d.muon_at = (int64_t)b * t.rows * t.cols;
+            d.muon_x = muon ? ctx->muon.x + d.muon_at : nullptr;
             d.rows = t.rows; d.cols = t.cols; d.tile_first = l.tiles;
             // hidden x hidden blocks for the layer matrices; the embedding (hidden x vocab) is cut into <= 256-wide blocks
             d.block = (t.cols == c.vocab && t.rows == c.hidden && c.hidden > 256) ? 256 : c.hidden;
@@ -916,7 +917,7 @@ extern "C" int egg_update_tensor(egg_ctx *ctx, int id, const int32_t *d_fit, con
     if (t.is_matrix && t.muon && ctx->cfg.use_muon) {
         // LAUNCH_ADAM_MATRIX under USE_MUON (mgpu.cu:1587-1595)
         HIP_TRY(egg_launch_newton_schulz(ctx->muon, t.rows, t.cols, 5, ctx->stream));
-        HIP_TRY(egg_launch_muon_apply(p, ctx->cfg.adam_weight_decay, 0, ctx->stream));
+        HIP_TRY(egg_launch_muon_apply(p, ctx->cfg.adam_weight_decay, ctx->muon.x, ctx->stream));
     }
     return EGG_OK;
 }
@@ -971,7 +972,7 @@ static int es_update(egg_ctx *ctx, const int32_t *d_fit, const StepEnd &end, con
             { SpanScope span(ctx, EGG_K_UPDATE_MATRIX); HIP_TRY(egg_launch_update(p, ctx->stream)); }
             const float *result = ctx->muon.x;
             { SpanScope span(ctx, EGG_K_MUON_NS); HIP_TRY(egg_launch_newton_schulz_batched(ctx->muon, t0.rows, t0.cols, 5, p.n_mat, ctx->stream, &result)); }
-            { SpanScope span(ctx, EGG_K_UPDATE_MATRIX); HIP_TRY(egg_launch_muon_apply(p, c.adam_weight_decay, result - ctx->muon.x, ctx->stream)); }
+            { SpanScope span(ctx, EGG_K_UPDATE_MATRIX); HIP_TRY(egg_launch_muon_apply(p, c.adam_weight_decay, result, ctx->stream)); }
         }
     }
     // d-eggs runs the overlay rule after each tensor's update (de/src/worker.cu:446-523); tensors and their overlay

@@ -70,7 +70,7 @@ hipError_t egg_launch_noise_table(const NoiseTable &nt, const uint32_t *d_seed, 
                                   int t_lo, int t_hi, int n_layers, unsigned long long *counter, hipStream_t s);
 struct MatDesc {
     int8_t *W, *frag; float *state;    // canonical weights, their fragment-major copy, optimizer state ({m,v,acc} or Muon's {m,acc})
-    float *muon_x;                     // Muon: the matrix's [rows][cols] slot of the workspace, else null
+    float *muon_x; int64_t muon_at;    // Muon: the matrix's [rows][cols] slot of the workspace, else null; the slot's place in it, in floats
     int64_t offset;                    // in the model blob (and in the overlay's flags)
     int rows, cols, block;             // rows = input dim (k), cols = output dim (n); block: edge of the fragment-major blocks
     int tile_first;                    // number of 64 x 64 tiles of the matrices in front of it in its list
@@ -96,7 +96,7 @@ int egg_update_blocks(const UpdLaunch &p);             // its workgroups
 size_t egg_noise_ld(int entries);                      // bytes of a table row that holds so many entries
 size_t egg_noise_mask_ld(int pairs_pad);
 hipError_t egg_launch_update(const UpdLaunch &p, hipStream_t s);
-hipError_t egg_launch_muon_apply(const UpdLaunch &p, float wd, ptrdiff_t moved, hipStream_t s);      // moved: from MatDesc::muon_x to the orthogonalised matrix, in floats
+hipError_t egg_launch_muon_apply(const UpdLaunch &p, float wd, const float *x, hipStream_t s);      // x: the orthogonalised matrices, each at its MatDesc::muon_at
 hipError_t egg_launch_frag(const MatDesc *d_mat, int n_mat, int tiles, hipStream_t s);
 
 // adaptive noise overlay (de/src/kernels.cu:61-77): for every entry of every segment, +inc where the flag is set, -dec

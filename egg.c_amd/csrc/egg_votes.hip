@@ -534,7 +534,7 @@ hipError_t egg_launch_update(const UpdLaunch &p, hipStream_t s) {
 // muon_apply_update_kernel (muon_internal.cuh:112-170) for every matrix of a list: a thread takes one 16-byte unit of the
 // fragment-major copy (16 rows of one column), so neighbouring lanes read and write neighbouring columns throughout.
 // Bound by memory (22 bytes an element).
-__global__ void __launch_bounds__(256) k_muon_apply(UpdLaunch p, float wd, ptrdiff_t moved) {
+__global__ void __launch_bounds__(256) k_muon_apply(UpdLaunch p, float wd, const float *ortho) {
     __shared__ int sums[EGG_WAVES];
     const MatDesc t = p.mat[find_last(p.n_mat, blockIdx.x, [&](int i) { return p.mat[i].tile_first; })];
     const int u = ((int)blockIdx.x - t.tile_first) * 256 + (int)threadIdx.x;       // 256 units to a 64 x 64 tile
@@ -554,7 +554,7 @@ __global__ void __launch_bounds__(256) k_muon_apply(UpdLaunch p, float wd, ptrdi
         w4[q] = *reinterpret_cast<const int *>(t.W + idx);
         s0[q] = sp[0]; s1[q] = sp[1];
 #pragma unroll
-        for (int e = 0; e < 4; e++) x[q][e] = (t.muon_x + moved)[(size_t)(kr + e) * t.cols + n];
+        for (int e = 0; e < 4; e++) x[q][e] = ortho[t.muon_at + (size_t)(kr + e) * t.cols + n];
     }
 #pragma unroll
     for (int q = 0; q < 4; q++) {
@@ -580,9 +580,9 @@ __global__ void __launch_bounds__(256) k_muon_apply(UpdLaunch p, float wd, ptrdi
     for (int off = 32; off > 0; off >>= 1) changes += __shfl_xor(changes, off, 64);
     count_changes(p, changes, sums);
 }
-hipError_t egg_launch_muon_apply(const UpdLaunch &p, float wd, ptrdiff_t moved, hipStream_t s) {
-    if (p.tiles < 1) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_muon_apply, dim3(p.tiles), dim3(256), 0, s, p, wd, moved);
+hipError_t egg_launch_muon_apply(const UpdLaunch &p, float wd, const float *x, hipStream_t s) {
+    if (p.tiles < 1 || !x) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_muon_apply, dim3(p.tiles), dim3(256), 0, s, p, wd, x);
     return hipGetLastError();
 }
 
