@@ -57,7 +57,7 @@ EXPORTS = [
     "egg_gru_model_init", "egg_gru_model_upload", "egg_gru_model_download", "egg_gru_state_reset",
     "egg_gru_state_download", "egg_gru_step", "egg_gru_losses", "egg_gru_forward_mode",
 ]
-KCLASSES = ["mlp_first", "qkv", "attn", "mlp", "head", "update_matrix", "update_vector", "plinear", "muon_ns"]
+KCLASSES = ["mlp_first", "qkv", "attn", "mlp", "head", "update_matrix", "update_vector", "plinear", "muon_ns", "blocks"]
 
 
 def build(force=True):
@@ -458,8 +458,9 @@ class Context:
         return out
 
 
-def _enable_timing(self, on=True):
-    self._ck(lib().egg_ctx_enable_timing(self._h, 1 if on else 0), "egg_ctx_enable_timing")
+def _enable_timing(self, on=True, stages=False):
+    """stages: the forward's stages one by one also where they would share a launch ("blocks")"""
+    self._ck(lib().egg_ctx_enable_timing(self._h, (2 if stages else 1) if on else 0), "egg_ctx_enable_timing")
 
 
 def _timing_reset(self):

@@ -73,7 +73,7 @@ struct egg_ctx {
     // taps
     bool taps = false; int8_t *d_tap = nullptr; int32_t *d_tap_logits = nullptr; int tap_members = 0;
     // per-kernel-class event timing (egg_ctx_enable_timing)
-    bool timing = false;
+    bool timing = false, timing_stages = false;
     struct Span { int cls; hipEvent_t a, b; };
     std::vector<Span> spans; size_t spans_used = 0;
     double t_ms[EGG_KCLASS_COUNT] = {0}; long t_n[EGG_KCLASS_COUNT] = {0};
@@ -126,9 +126,9 @@ static void span_end(egg_ctx *ctx) {
 }
 // closes the span on every way out of a scope, error returns included
 struct SpanScope {
-    egg_ctx *ctx;
+    egg_ctx *ctx; bool launched = true;
     SpanScope(egg_ctx *c, int cls) : ctx(c) { span_begin(c, cls); }
-    ~SpanScope() { span_end(ctx); }
+    ~SpanScope() { if (launched) span_end(ctx); }        // (its events serve the next span otherwise)
 };
 static void spans_collect(egg_ctx *ctx) {
     for (size_t i = 0; i < ctx->spans_used; i++) {
@@ -806,9 +806,12 @@ static int forward_chunk(egg_ctx *ctx, const uint8_t *d_data, int64_t len, const
         return p;
     };
     bool taken = false;
-    if (!taps && !Q && !range && !ctx->timing && c.n_layers > 0) {
+    if (!taps && !Q && !range && !ctx->timing_stages && c.n_layers > 0) {
         const BlocksParams p = {first_params(), mlp_params(0), qkv_params(0), attn_params(0), c.n_layers};
-        HIP_TRY(egg_launch_blocks(p, &taken, s));
+        SpanScope span(ctx, EGG_K_BLOCKS);
+        const hipError_t e = egg_launch_blocks(p, &taken, s);
+        span.launched = taken;
+        HIP_TRY(e);
     }
     if (!taken) {
         { SpanScope span(ctx, EGG_K_MLP_FIRST); HIP_TRY(egg_launch_mlp(first_params(), true, s)); }
@@ -1359,6 +1362,7 @@ extern "C" int egg_ctx_enable_timing(egg_ctx *ctx, int enable) {
     HIP_TRY(hipStreamSynchronize(ctx->stream));
     spans_collect(ctx);
     ctx->timing = enable != 0;
+    ctx->timing_stages = enable == EGG_TIMING_STAGES;
     return EGG_OK;
 }
 extern "C" int egg_timing_reset(egg_ctx *ctx) {

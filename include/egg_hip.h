@@ -347,11 +347,16 @@ int  egg_gru_forward_mode(egg_gru_ctx *ctx, int staged);
 
 /* per-kernel-class timing with hipEvent pairs recorded on the context's stream around each launch (the
  * reference only splits Fwd/Host/Upd wall time, full_cuda_train_egg.cu:1116-1126).  Not usable while capturing.  An
- * untimed update takes the vector tensors in the launch of the matrices; timed, they have one of their own. */
+ * untimed update takes the vector tensors in the launch of the matrices; timed, they have one of their own.
+ * enable: 0 off; 1 times the forward's launches as an untimed context makes them; EGG_TIMING_STAGES has every stage of the forward
+ * launched by itself (MLP_FIRST, QKV, ATTN, MLP) also where an untimed context takes them in one launch (BLOCKS: small populations
+ * of short windows).  Same results. */
 enum { EGG_K_MLP_FIRST = 0, EGG_K_QKV = 1, EGG_K_ATTN = 2, EGG_K_MLP = 3, EGG_K_HEAD = 4,
        EGG_K_UPDATE_MATRIX = 5, EGG_K_UPDATE_VECTOR = 6, EGG_K_PLINEAR = 7,
        EGG_K_MUON_NS = 8 /* the Newton-Schulz chain of a Muon batch; votes, momentum and apply count as UPDATE_MATRIX */,
-       EGG_KCLASS_COUNT = 9 };
+       EGG_K_BLOCKS = 9 /* embedding, initial MLP and all layers in one launch */,
+       EGG_KCLASS_COUNT = 10 };
+enum { EGG_TIMING_STAGES = 2 };
 int  egg_ctx_enable_timing(egg_ctx *ctx, int enable);
 int  egg_timing_reset(egg_ctx *ctx);
 int  egg_timing_get(egg_ctx *ctx, int kclass, int64_t *launches, double *total_ms);   /* synchronises */

@@ -1,4 +1,4 @@
-"""A model's blocks in one launch (k_blocks) against the same stages launched one by one (which timed contexts take) and, for sampled members, against
+"""A model's blocks in one launch (k_blocks) against the same stages launched one by one (which a context that times its stages takes) and, for sampled members, against
 the oracle: short windows, all hidden sizes that take it, both head widths, full and partial last workgroups, few and many column slices, and populations on both sides of the line."""
 import numpy as np
 import pytest
@@ -54,7 +54,7 @@ def test_blocks_equal_the_stages(pkg, orc, kw):
         return out.cpu().numpy()
 
     def stages(seed, *part):
-        ctx.enable_timing(True)
+        ctx.enable_timing(True, stages=True)
         got = losses(seed, *part)
         ctx.enable_timing(False)
         return got
@@ -66,4 +66,26 @@ def test_blocks_equal_the_stages(pkg, orc, kw):
         assert [int(got[m]) for m in members] == [r[0] if isinstance(r, tuple) else r for r in ref]
     if P > 4:                                           # a worker's part of the population
         assert np.array_equal(losses(4321, 2, P - 3), stages(4321, 2, P - 3))
+    ctx.close()
+
+
+@pytest.mark.parametrize("overlay", [False, True])
+def test_timing_describes_the_launches_of_an_untimed_forward(pkg, orc, overlay):
+    import torch
+    layers = 3
+    ctx = pkg.Context(pkg.default_config(hidden=128, head_dim=32, seq_len=64, population=66, n_layers=layers))
+    ctx.model_init(42)
+    if overlay:                                         # the launch for all blocks does not take it
+        ctx.adaptive_enable()
+    data = torch.from_numpy(orc.zipf_bytes(1 << 14)).cuda()
+    loss = torch.zeros(66, dtype=torch.int32, device="cuda")
+    for stages in (False, True, False):
+        ctx.enable_timing(True, stages=stages)
+        ctx.timing_reset()
+        for seed in (1, 2):
+            ctx.population_forward(data.data_ptr(), data.numel(), 0, seed, 0, 66, loss.data_ptr())
+        got = {k: v[0] for k, v in ctx.timing().items() if v[0]}
+        one = not stages and not overlay
+        assert got == ({"blocks": 2, "head": 2} if one else {"mlp_first": 2, "qkv": 2 * layers, "attn": 2 * layers, "mlp": 2 * layers, "head": 2}), got
+        assert all(ms > 0 for n, ms in ctx.timing().values() if n)
     ctx.close()
