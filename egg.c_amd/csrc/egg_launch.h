@@ -70,12 +70,13 @@ hipError_t egg_launch_noise_table(const NoiseTable &nt, const uint32_t *d_seed, 
                                   int t_lo, int t_hi, int n_layers, unsigned long long *counter, hipStream_t s);
 struct MatDesc {
     int8_t *W, *frag; float *state;    // canonical weights, their fragment-major copy, optimizer state ({m,v,acc} or Muon's {m,acc})
-    float *muon_x; int64_t muon_at;    // Muon: the matrix's [rows][cols] slot of the workspace, else null; the slot's place in it, in floats
+    float *muon_x;                     // Muon: the matrix's [rows][cols] slot of the workspace, else null
     int64_t offset;                    // in the model blob (and in the overlay's flags)
     int rows, cols, block;             // rows = input dim (k), cols = output dim (n); block: edge of the fragment-major blocks
     int tile_first;                    // number of 64 x 64 tiles of the matrices in front of it in its list
     int t_a, t_b;                      // first table entry of its output-side and input-side noise
     int limit; float lr_scale;         // weights saturate at +-limit: 127 (mgpu.cu:1056-1062), or the configured limit
+    int64_t muon_at;                   // the slot's place in the workspace, in floats (last: in front of what k_update reads it costs that 8 spilled registers)
 };
 // a vector tensor; `first` is the running element count.  flags (adaptive noise overlay), per element, or null
 struct VecDesc { int8_t *W; float *state; int n, first, off_a, off_b, seed_base; float lr_scale; int8_t *flags; };
