@@ -85,9 +85,10 @@ __device__ __forceinline__ void wait_vmcnt_upto(int n) {
 // stands (to [-127 * 256, 127 * 256 + 255]) and the result is its second byte, which the pack's byte permute picks,
 // so the shift costs no instruction; 4 and 5 = perturbed, with the rank-one term as one more k-step (rank1_token) and the epilogues of 0
 // and 3: a tile's x.B are known in the middle of its own k-loop, so the term joins the accumulators while they are still in the matrix pipe.  Four
-// matrix instructions more a tile and about 45 vector ones for the token's operand, in place of three a result.  8,192 members x 128 tokens x 512 x 512,
-// int8:
-// 347 -> 334 us and, a noise of its own for every member, 329 -> 320; K = 256 218 -> 208 (at the power limit: 2.2 vector instructions a result fewer, of 5.4).
+// matrix instructions more a tile and about 45 vector ones for the token's operand, in place of three a result: 5.85 -> 3.82 vector instructions an
+// MFMA of the product.  A tile takes no fewer clocks for it (497 K -> 504 K a workgroup), but they come faster: the clock is held between 1.3 and 1.8 GHz by the
+// power that the kernel draws.  8,192 members x 128 tokens x 512 x 512, int8, back to back and in turn with the former epilogue: 322 -> 317 us and, a noise of
+// its own for every member, 314 -> 309; K = 256 222 -> 215 and 220 -> 211; equal at 512 members (27 us), K = 256 21.4 -> 20.5 and 21.0 -> 20.2.
 // int32 results do not gain, 516 -> 522 us, and keep the vector epilogue
 template <int K, int N, bool OUT32, int MODE>
 __global__ void __launch_bounds__(EGG_THREADS, 1) k_plinear_ws(PlinParams p) {

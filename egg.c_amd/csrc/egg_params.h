@@ -49,7 +49,7 @@ static inline long long egg_out_acc_bound(int hidden, int mask, int shift_out) {
 
 // (sb * a) >> sigma of a rank-one term is the high word of (sb << sb_shift) * (a << a_shift), one instruction where the output
 // side's table holds the shifted noise: sb_shift + a_shift = 32 - sigma, with as little on sb as keeps a below 2^31 (sb has
-// 24 bits, the magnitude at most 7: at most 8 more are ever needed).
+// 24 bits, the magnitude at most 127: at most 8 more are ever needed, at sigma = 0).
 static inline void egg_rank1_shifts(int mask, int sigma, int *sb_shift, int *a_shift) {
     int t = 0;
     while (sigma + t < 32 && egg_noise_magnitude(mask) >= (1LL << (sigma + t)) / 2) t++;

@@ -75,8 +75,8 @@ def test_products_round_as_float32_does(pkg, rows, cols, power_of_two):
     got = d.cpu().numpy().astype(np.float64)
     got = got[at + 1, at + 1]
     want = -0.5 * r.astype(np.float64) * p * q           # exact: 48 bits
-    # half a unit of the last place (2^-24) from the one rounding; the small parts are 2^-8 of the product, and each of the seven steps of their sum is off by
-    # at most a unit of its last place, 2^-31 of the product: 2^-28 in all
+    # half a unit of the last place (2^-24) from the one rounding; the sum of the small parts is at most 2^-7 of the product and of its seven steps two reach that
+    # size, each off by at most a unit of its last place (2^-31 and 2^-30); what is left out is below 2^-34: 2^-29 in all, of which the limit allows twice
     err = np.abs(got - want) / np.abs(want)
     assert err.max() <= 2.0 ** -24 * (1 + 2.0 ** -4), err.max() * 2 ** 24
     ctx.close()
