@@ -323,8 +323,8 @@ def main():
               "kernel_frac_mfma_note": "algorithmic int8 ops of the shared products at every position over event-timed kernel time, against 5.0 POP/s; "
                                        "mlp_first evaluates its block once per distinct byte value of a member's window, so its figure is not a pipe utilisation",
               "muon": {"newton_schulz_ms": ns_ms, "matrices": sum(g["members"] for g in groups), "TFLOP/s_fp32": ns_flops / (ns_ms * 1e-3) / 1e12 if ns_ms > 0 else None,
-                       # a float32 product is six of bf16 (three parts an operand), against 2.5 PFLOP/s
-                       "frac_bf16_mfma_peak": 6 * ns_flops / (ns_ms * 1e-3) / 2.5e15 if ns_ms > 0 else None,
+                       # a float32 product is eight of bf16 (three parts an operand), against 2.5 PFLOP/s
+                       "frac_bf16_mfma_peak": 8 * ns_flops / (ns_ms * 1e-3) / 2.5e15 if ns_ms > 0 else None,
                        "votes_momentum_apply_ms": tm["update_matrix"][1],
                        "parity": "fp32 matrix products in a fixed order of the library's own; the reference leaves the order to cuBLAS, so Muon "
                                  "state is compared within a tolerance (relative Frobenius error <= 1e-5 against fp64 Newton-Schulz, "

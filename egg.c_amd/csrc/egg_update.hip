@@ -632,11 +632,11 @@ hipError_t egg_launch_newton_schulz_batched(const MuonWork &w, int rows, int col
     // iterations can be multiplied up among short x short matrices and X once with their product: with k = the short side
     // and r = long / short, 3/2 r + 6 products of k^3 for five iterations where each one on X itself takes 15/2 r (counting
     // a symmetric product as half).  Used from r = 4 on, which is also where the second matrix buffer holds the four
-    // k x k matrices it needs; r = 1, the other shape of the models, would gain nothing.  In float32 it is closer to the
-    // exact iteration than that on X (relative error 3e-7 against 6e-7 for random matrices, 1.4e-6 against 4.3e-6 at rank
-    // one); but G is not computed from X again, and an eigenvalue that should be 0 grows 9/4-fold an iteration, so it is kept to
-    // eight iterations.  9 matrices of 512 x 2048, 5 iterations: 1.23 -> 0.50 ms; 32 of 512 x 512 (G from its upper
-    // half): 0.83 -> 0.67 ms.
+    // k x k matrices it needs; r = 1, the other shape of the models, would gain nothing.  With the products above it is closer to the
+    // exact iteration than that on X for dense matrices (512 x 2048: relative error 1.3e-7 against 2.8e-7 for random ones, 7.0e-7 against 1.4e-6 at rank
+    // one) and further with the long side scaled over e^4 (3.7e-7 against 2.8e-7); but G is not computed from X again, and an eigenvalue that should be 0 grows 9/4-fold
+    // an iteration, so it is kept to eight iterations.  9 matrices of 512 x 2048, 5 iterations: 0.85 -> 0.43 ms; the products of 32 of 512 x 512 (G from its upper
+    // half): 0.71 -> 0.65 ms.
     if (K % 64 == 0 && iters >= 1 && iters <= 8 && (long)rows * cols >= 4 * kk) {
         float *G = w.swap, *S = w.swap + kk * batch, *next = w.swap + 2 * kk * batch;
         float *P = iters & 1 ? w.bterm : w.swap + 3 * kk * batch, *Pn = iters & 1 ? w.swap + 3 * kk * batch : w.bterm;      // the last one in bterm
